@@ -41,11 +41,9 @@ __device__ __forceinline__ short bf(float f) {
     return __builtin_bit_cast(short, h);
 }
 
-__device__ __forceinline__ int64_t nb_voxel(int64_t v, int t, int G) {
-    const int x = int(v / (int64_t(G) * G)), y = int((v / G) % G), z = int(v % G);
-    const int nx = x + t / 9 - 1, ny = y + (t / 3) % 3 - 1, nz = z + t % 3 - 1;
-    if (nx < 0 || ny < 0 || nz < 0 || nx >= G || ny >= G || nz >= G) return -1;
-    return (int64_t(nx) * G + ny) * G + nz;
+// two values as BF16 in one word, the first in the low half
+__device__ __forceinline__ uint32_t bf2(float a, float b) {
+    return uint32_t(uint16_t(bf(a))) | (uint32_t(uint16_t(bf(b))) << 16);
 }
 
 // Input of a convolution: channels [0, clo) come from `lo` (grid G / 2,
@@ -222,42 +220,156 @@ __global__ void __launch_bounds__(kT) k_conv3(ConvIn src, const short* __restric
 }
 
 // dW partials: part[ch][t][co][ci] = sum over the chunk's voxels v of
-// bf16(g[v, co]) * bf16(in[v + off_t, ci]); one wave per (chunk, t, co tile, ci tile).
-__global__ void __launch_bounds__(kT) k_conv3_wgrad(const float* __restrict__ in, int cin,
-                                                   const float* __restrict__ g, int cout, int G, int nchunk,
+// bf16(g[v, co]) * bf16(in[v + off_t, ci]), 16 voxels per MFMA in voxel order.
+//
+// On grids of 8^3 and more (k_wgrad_rows): one workgroup per (chunk, dx, co
+// tile, ci tile), one wave per dy, the three dz of a wave's taps in three
+// accumulators.  The chunk passes through LDS in stages of 512 voxels, the
+// gradient and the input's rows (one more on either side) as BF16, channel by
+// channel with z innermost, so a lane's four voxels of one channel are one
+// 8-byte read; the fragments shifted by dz = -1 and 1 are funnel shifts of it
+// and the two words beside it.  Rows carry zeros on both ends in z, rows
+// outside the grid in x are staged as zeros and rows outside in y are
+// replaced by zeros.  The channel strides are 4 words past a multiple of 32
+// (no bank conflict beyond the two cycles a half-wave's 256 bytes need).
+// What bounds it is the staging (each element is read for 3 dx and per tile
+// of the other operand), not the matrix cores.  One wave per (chunk, tap,
+// tiles) with scalar loads straight from memory and 64-bit divisions per
+// element took 440 us for 16 -> 16 channels on 64^3 and 990 us for 48 -> 16.
+constexpr int kWStage = 512;  // voxels per stage
+
+template <int LG>
+__global__ void __launch_bounds__(192) k_wgrad_rows(ConvIn src, const float* __restrict__ g, int cout, int nchunk,
+                                                   float* __restrict__ part) {
+    constexpr int G = 1 << LG, V = G * G * G, R = kWStage / G, ROWS = R + 2, RS = G + 8;
+    constexpr int CW0 = ROWS * RS / 2, CW = CW0 + ((4 - CW0) & 31);  // words per input channel
+    constexpr int GW = kWStage / 2 + 4;                               // words per gradient channel
+    __shared__ __align__(16) uint32_t si[16 * CW];
+    __shared__ __align__(16) uint32_t sg[16 * GW];
+    const int cin = src.clo + src.cskip;
+    const int ntc = cout >> 4, nti = cin >> 4;
+    int b = blockIdx.x;
+    const int ch = b % nchunk;  // fastest: workgroups of one chunk meet on few XCDs
+    b /= nchunk;
+    const int cit = b % nti;
+    b /= nti;
+    const int cot = b % ntc;
+    const int dx = b / ntc - 1;
+    const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63;
+    const int i = l & 15, kq = l >> 4, dy = wave - 1;
+    const bool lo = cit * 16 < src.clo;
+    const int sc = lo ? src.clo : src.cskip;  // channels of the source tensor
+    const float* sp = lo ? src.lo + cit * 16 : src.skip + (cit * 16 - src.clo);
+    const float* gp = g + cot * 16;
+    // the zeros beyond both ends of every row
+    for (int t = tid; t < 16 * ROWS; t += 192) {
+        uint32_t* r = si + (t / ROWS) * CW + (t % ROWS) * (RS / 2);
+        r[1] = 0;
+        r[G / 2 + 2] = 0;
+    }
+    f4 acc[3];
+#pragma unroll
+    for (int z = 0; z < 3; z++) acc[z] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    const int v0 = ch * kWChunk, v1 = v0 + kWChunk < V ? v0 + kWChunk : V;
+    for (int vs = v0; vs < v1; vs += kWStage) {
+        __syncthreads();  // the previous stage's reads
+        const int row0 = vs >> LG;  // first row (x G + y) of the stage
+#pragma unroll 4
+        for (int t = tid; t < ROWS * G * 2; t += 192) {
+            const int cq = t & 3, zp = (t >> 2) & (G / 2 - 1), r = t >> (LG + 1);
+            const int row = row0 - 1 + r, x = (row >> LG) + dx, y = row & (G - 1);
+            float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f), c = a;
+            if (row >= 0 && row < G * G && x >= 0 && x < G) {
+                if (lo) {
+                    a = *reinterpret_cast<const float4*>(
+                        sp + int64_t((((x >> 1) << (LG - 1)) + (y >> 1)) * (G / 2) + zp) * sc + 4 * cq);
+                    c = a;
+                } else {
+                    const float* q = sp + int64_t(((x << LG) + y) * G + 2 * zp) * sc + 4 * cq;
+                    a = *reinterpret_cast<const float4*>(q);
+                    c = *reinterpret_cast<const float4*>(q + sc);
+                }
+            }
+            uint32_t* d = si + 4 * cq * CW + r * (RS / 2) + 2 + zp;
+            d[0] = bf2(a.x, c.x);
+            d[CW] = bf2(a.y, c.y);
+            d[2 * CW] = bf2(a.z, c.z);
+            d[3 * CW] = bf2(a.w, c.w);
+        }
+#pragma unroll 4
+        for (int t = tid; t < kWStage * 2; t += 192) {
+            const int cq = t & 3, vp = t >> 2;
+            const float* q = gp + int64_t(vs + 2 * vp) * cout + 4 * cq;
+            const float4 a = *reinterpret_cast<const float4*>(q);
+            const float4 c = *reinterpret_cast<const float4*>(q + cout);
+            uint32_t* d = sg + 4 * cq * GW + vp;
+            d[0] = bf2(a.x, c.x);
+            d[GW] = bf2(a.y, c.y);
+            d[2 * GW] = bf2(a.z, c.z);
+            d[3 * GW] = bf2(a.w, c.w);
+        }
+        __syncthreads();
+#pragma unroll 4
+        for (int st = 0; st < kWStage / 16; st++) {
+            const int v = st * 16 + 4 * kq;  // the lane's first voxel in the stage
+            const int r = v >> LG, z = v & (G - 1), y = (row0 + r) & (G - 1);
+            const uint2 ga = *reinterpret_cast<const uint2*>(sg + i * GW + (v >> 1));
+            const uint32_t* q = si + i * CW + (r + 1 + dy) * (RS / 2) + 2 + (z >> 1);
+            uint2 m = *reinterpret_cast<const uint2*>(q);
+            uint32_t w0 = q[-1], w3 = q[2];
+            if (y + dy < 0 || y + dy >= G) m.x = m.y = w0 = w3 = 0;
+            const uint32_t s0 = __builtin_amdgcn_alignbit(m.x, w0, 16), s1 = __builtin_amdgcn_alignbit(m.y, m.x, 16),
+                           s2 = __builtin_amdgcn_alignbit(w3, m.y, 16);
+            const s4 av = __builtin_bit_cast(s4, ga);
+            acc[0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, __builtin_bit_cast(s4, make_uint2(s0, s1)), acc[0],
+                                                               0, 0, 0);
+            acc[1] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, __builtin_bit_cast(s4, m), acc[1], 0, 0, 0);
+            acc[2] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, __builtin_bit_cast(s4, make_uint2(s1, s2)), acc[2],
+                                                               0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int z = 0; z < 3; z++) {
+        const int t = 9 * (dx + 1) + 3 * (dy + 1) + z;
+        float* dst = part + (int64_t(ch) * 27 + t) * cout * cin;
+#pragma unroll
+        for (int e = 0; e < 4; e++) dst[int64_t(cot * 16 + 4 * kq + e) * cin + cit * 16 + i] = acc[z][e];
+    }
+}
+
+// The same on grids under 8^3 (at most 64 voxels, which need not fill an
+// MFMA): one wave per (tap, co tile, ci tile).
+__global__ void __launch_bounds__(kT) k_wgrad_small(ConvIn src, const float* __restrict__ g, int cout, int G,
                                                    float* __restrict__ part) {
     const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
+    const int cin = src.clo + src.cskip;
     const int ntc = cout / 16, nti = cin / 16;
-    const int64_t job = int64_t(blockIdx.x) * 4 + wave;
-    const int64_t njobs = int64_t(nchunk) * 27 * ntc * nti;
-    if (job >= njobs) return;
-    const int cit = int(job % nti);
-    const int cot = int((job / nti) % ntc);
-    const int t = int((job / (int64_t(nti) * ntc)) % 27);
-    const int ch = int(job / (int64_t(nti) * ntc * 27));
-    const int64_t V = int64_t(G) * G * G;
+    const int job = int(blockIdx.x) * 4 + wave;
+    if (job >= 27 * ntc * nti) return;
+    const int cit = job % nti, cot = (job / nti) % ntc, t = job / (nti * ntc);
+    const int V = G * G * G;
     const int i = l & 15, kq = l >> 4;
     const int co = cot * 16 + i, ci = cit * 16 + i;
     f4 acc = f4{0.0f, 0.0f, 0.0f, 0.0f};
-    const int64_t vb0 = int64_t(ch) * kWChunk;
-    const int64_t vb1 = vb0 + kWChunk < V ? vb0 + kWChunk : V;
-    for (int64_t vb = vb0; vb < vb1; vb += 16) {
+    for (int vb = 0; vb < V; vb += 16) {
         s4 a, b;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const int64_t v = vb + 4 * kq + e;
+            const int v = vb + 4 * kq + e;
             float ga = 0.0f, xb = 0.0f;
-            if (v < vb1) {
+            if (v < V) {
                 ga = g[v * cout + co];
-                const int64_t nv = nb_voxel(v, t, G);
-                if (nv >= 0) xb = in[nv * cin + ci];
+                const int x = v / (G * G) + t / 9 - 1, y = (v / G) % G + (t / 3) % 3 - 1, z = v % G + t % 3 - 1;
+                if (x >= 0 && y >= 0 && z >= 0 && x < G && y < G && z < G)
+                    xb = ci < src.clo ? src.lo[(((x >> 1) * (G / 2) + (y >> 1)) * (G / 2) + (z >> 1)) * src.clo + ci]
+                                      : src.skip[((x * G + y) * G + z) * src.cskip + (ci - src.clo)];
             }
             a[e] = bf(ga);
             b[e] = bf(xb);
         }
         acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
     }
-    float* dst = part + ((int64_t(ch) * 27 + t) * cout) * cin;
+    float* dst = part + int64_t(t) * cout * cin;
 #pragma unroll
     for (int e = 0; e < 4; e++) dst[int64_t(cot * 16 + 4 * kq + e) * cin + ci] = acc[e];
 }
@@ -267,6 +379,7 @@ __global__ void k_sum_chunks(const float* part, int nchunk, int64_t n, float* gr
     const int64_t k = int64_t(blockIdx.x) * kT + threadIdx.x;
     if (k >= n) return;
     float s = 0.0f;
+#pragma unroll 16
     for (int c = 0; c < nchunk; c++) s += part[int64_t(c) * n + k];
     grad[k] += s;
 }
@@ -330,23 +443,8 @@ __global__ void k_pool_back(const float* g, int G, int C, float* gin, int accumu
     gin[k] = accumulate ? gin[k] + val : val;
 }
 
-// nearest upsampling (G/2 -> G) into channels [0, C) of a concat tensor of
-// width W, and the skip tensor into channels [C, C + S)
-__global__ void k_up_concat(const float* lo, int C, const float* skip, int S, int G, float* out) {
-    const int W = C + S, H = G / 2;
-    const int64_t k = int64_t(blockIdx.x) * kT + threadIdx.x;
-    if (k >= int64_t(G) * G * G * W) return;
-    const int c = int(k % W);
-    const int64_t u = k / W;
-    if (c < C) {
-        const int x = int(u / (int64_t(G) * G)), y = int((u / G) % G), z = int(u % G);
-        out[k] = lo[((int64_t(x / 2) * H + y / 2) * H + z / 2) * C + c];
-    } else {
-        out[k] = skip[u * S + (c - C)];
-    }
-}
-
-// gradient of k_up_concat: g_lo (sum of 8 children, fixed order) and the skip part
+// gradient of a decoder input, concat(nearest upsampling of lo, skip): g_lo
+// (sum of 8 children, fixed order) and the skip part
 __global__ void k_up_concat_back_lo(const float* g, int C, int S, int G, float* glo) {
     const int W = C + S, H = G / 2;
     const int64_t k = int64_t(blockIdx.x) * kT + threadIdx.x;
@@ -525,11 +623,9 @@ unsigned blocks(int64_t n) { return unsigned((n + kT - 1) / kT); }
 struct UNetConv {
     int cin, cout, G;
     int64_t woff, boff;
-    const float* in;  // the input tensor (cin channels) the weight gradient reads
     const float* lo;  // decoder convolutions: the upsampled part of the input (clo channels, grid G / 2)
     int clo;          // 0 for a plain input
     const float* skip;
-    float* cat;  // decoder convolutions: `in`, written only for the backward pass
     float* out;
     DBuf<short> wb, wf;
 };
@@ -546,7 +642,7 @@ struct prg_unet {
     int64_t adam_t = 0;
     prg::UNetConv conv[14];  // the convolutions, encoder to decoder
     // activations
-    prg::DBuf<float> x0, p1, p2, p3, c2, c1, c0, pred, target, mask, bgrid;
+    prg::DBuf<float> x0, p1, p2, p3, pred, target, mask, bgrid;
     prg::DBuf<float> act[14];
     // gradients
     prg::DBuf<float> ga, gb, ge0, ge1, ge2, gpred, part;
@@ -673,15 +769,19 @@ void conv_back(prg_unet* n, int k, float* g, float* gin) {
     PRG_CHECK_LAUNCH();
     k_bias_grad<<<L.cout, kT, 0, s>>>(g, V, L.cout, n->grads.get() + L.boff);
     PRG_CHECK_LAUNCH();
-    if (L.clo) {
-        // the decoder input the forward pass read through its fused loader
-        k_up_concat<<<blocks(V * L.cin), kT, 0, s>>>(L.lo, L.clo, L.skip, L.cin - L.clo, L.G, L.cat);
-        PRG_CHECK_LAUNCH();
-    }
     const int nchunk = int((V + kWChunk - 1) / kWChunk);
     const int64_t nw = int64_t(27) * L.cout * L.cin;
-    const int64_t jobs = int64_t(nchunk) * 27 * (L.cout / 16) * (L.cin / 16);
-    k_conv3_wgrad<<<unsigned((jobs + 3) / 4), kT, 0, s>>>(L.in, L.cin, g, L.cout, L.G, nchunk, n->part.get());
+    const ConvIn src{L.lo, L.clo, L.skip, L.cin - L.clo};
+    const unsigned jobs = unsigned(nchunk * 3 * (L.cout / 16) * (L.cin / 16));
+    switch (L.G) {
+        case 128: k_wgrad_rows<7><<<jobs, 192, 0, s>>>(src, g, L.cout, nchunk, n->part.get()); break;
+        case 64: k_wgrad_rows<6><<<jobs, 192, 0, s>>>(src, g, L.cout, nchunk, n->part.get()); break;
+        case 32: k_wgrad_rows<5><<<jobs, 192, 0, s>>>(src, g, L.cout, nchunk, n->part.get()); break;
+        case 16: k_wgrad_rows<4><<<jobs, 192, 0, s>>>(src, g, L.cout, nchunk, n->part.get()); break;
+        case 8: k_wgrad_rows<3><<<jobs, 192, 0, s>>>(src, g, L.cout, nchunk, n->part.get()); break;
+        default:  // 4 or 2
+            k_wgrad_small<<<unsigned((9 * jobs + 3) / 4), kT, 0, s>>>(src, g, L.cout, L.G, n->part.get());
+    }
     PRG_CHECK_LAUNCH();
     k_sum_chunks<<<blocks(nw), kT, 0, s>>>(n->part.get(), nchunk, nw, n->grads.get() + L.woff);
     PRG_CHECK_LAUNCH();
@@ -849,9 +949,6 @@ prg_status prg_unet_create(prg_unet** out, int32_t device, int32_t grid, uint64_
         n->p1.reserve(V0 / 8 * 16);
         n->p2.reserve(V0 / 64 * 32);
         n->p3.reserve(V0 / 512 * 64);
-        n->c2.reserve(V0 / 64 * 128);
-        n->c1.reserve(V0 / 8 * 96);
-        n->c0.reserve(V0 * 48);
         n->pred.reserve(V0);
         n->target.reserve(V0);
         n->mask.reserve(V0);
@@ -870,35 +967,22 @@ prg_status prg_unet_create(prg_unet** out, int32_t device, int32_t grid, uint64_
         }
         n->part.reserve(pc);
         auto& C = n->conv;
-        C[0].in = n->x0.get();
-        C[1].in = C[0].out;
-        C[2].in = n->p1.get();
-        C[3].in = C[2].out;
-        C[4].in = n->p2.get();
-        C[5].in = C[4].out;
-        C[6].in = n->p3.get();
-        C[7].in = C[6].out;
-        C[8].in = n->c2.get();
-        C[9].in = C[8].out;
-        C[10].in = n->c1.get();
-        C[11].in = C[10].out;
-        C[12].in = n->c0.get();
-        C[13].in = C[12].out;
+        // inputs: the previous output, or a pooled one at the encoder's levels
         for (int k = 0; k < 14; k++) {
             C[k].lo = nullptr;
             C[k].clo = 0;
-            C[k].skip = C[k].in;
-            C[k].cat = nullptr;
+            C[k].skip = k ? C[k - 1].out : n->x0.get();
         }
+        C[2].skip = n->p1.get();
+        C[4].skip = n->p2.get();
+        C[6].skip = n->p3.get();
         // decoder inputs: concat(upsampled coarser output, encoder skip)
         const int dec[3][3] = {{8, 7, 5}, {10, 9, 3}, {12, 11, 1}};
-        float* cats[3] = {n->c2.get(), n->c1.get(), n->c0.get()};
         for (int j = 0; j < 3; j++) {
             auto& L = C[dec[j][0]];
             L.lo = C[dec[j][1]].out;
             L.clo = C[dec[j][1]].cout;
             L.skip = C[dec[j][2]].out;
-            L.cat = cats[j];
         }
         // He-normal initial weights (splitmix64 + Box-Muller), zero biases
         std::vector<float> h(size_t(n->nparams), 0.0f);

@@ -153,3 +153,88 @@ def test_worse_than_zero_warm_start_falls_back(prg, monkeypatch, grid):
         warm.close()
         plain.close()
         net.close()
+
+
+def _torch_gradients(params, b, m, t):
+    """oracle.unet_ref's loss and gradient (the same BF16 rounding points) in
+    float32 torch on the CPU, fast enough for 128^3; one 2-D product per tap."""
+    import torch
+    import torch.nn.functional as F
+
+    def bf16(a):
+        return a.bfloat16().float()
+
+    def taps(p, G):
+        for k in range(27):
+            x, y, z = k // 9, (k // 3) % 3, k % 3
+            yield k, p[x:x + G, y:y + G, z:z + G]
+
+    class Conv(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, a, w):
+            G, ci = a.shape[0], a.shape[3]
+            p, wb = F.pad(bf16(a), (0, 0, 1, 1, 1, 1, 1, 1)), bf16(w)
+            ctx.save_for_backward(p, wb)
+            return sum(s.reshape(-1, ci) @ wb[k].T for k, s in taps(p, G)).reshape(G, G, G, -1)
+
+        @staticmethod
+        def backward(ctx, g):
+            p, wb = ctx.saved_tensors
+            G, ci, co = g.shape[0], p.shape[3], g.shape[3]
+            gb = bf16(g)
+            dw = torch.stack([gb.reshape(-1, co).T @ s.reshape(-1, ci) for _, s in taps(p, G)])
+            gp = F.pad(gb, (0, 0, 1, 1, 1, 1, 1, 1))
+            da = sum(s.reshape(-1, co) @ wb[26 - k] for k, s in taps(gp, G)).reshape(G, G, G, ci)
+            return da, dw
+
+    flat = torch.from_numpy(params).requires_grad_(True)
+    conv, o = [], 0
+    for _, ci, co in U.CONVS:
+        conv.append((flat[o:o + 27 * ci * co].reshape(27, co, ci), flat[o + 27 * ci * co:o + 27 * ci * co + co]))
+        o += 27 * ci * co + co
+
+    def run(k, a):
+        return torch.relu(Conv.apply(a, conv[k][0]) + conv[k][1])
+
+    def pool(a):
+        H = a.shape[0] // 2
+        return a.reshape(H, 2, H, 2, H, 2, -1).mean(dim=(1, 3, 5))
+
+    def up(a):
+        H, c = a.shape[0], a.shape[3]
+        return a[:, None, :, None, :, None].expand(H, 2, H, 2, H, 2, c).reshape(2 * H, 2 * H, 2 * H, c)
+
+    db, dm, dt = (torch.from_numpy(a) for a in (b, m, t))
+    x = torch.stack([db, dm] + [torch.zeros_like(db)] * 14, dim=3)
+    e0 = run(1, run(0, x))
+    e1 = run(3, run(2, pool(e0)))
+    e2 = run(5, run(4, pool(e1)))
+    bt = run(7, run(6, pool(e2)))
+    d2 = run(9, run(8, torch.cat([up(bt), e2], 3)))
+    d1 = run(11, run(10, torch.cat([up(d2), e1], 3)))
+    d0 = run(13, run(12, torch.cat([up(d1), e0], 3)))
+    pred = d0 @ flat[o:o + 16] + flat[o + 16]
+    loss = (dm * (pred - dt) ** 2).sum() / dm.sum()
+    loss.backward()
+    return float(loss.detach()), flat.grad.numpy()
+
+
+@pytest.mark.parametrize("grid", [32, 64, 128])
+def test_gradients_on_larger_grids(prg, grid):
+    """Every level's weight-gradient instance (grids 4 to 128; 16 and 2 are in
+    the 16^3 test above), with that test's tolerance: the rounding points are
+    the same, so only BF16 roundings and ReLU masks that flip by an
+    accumulation's last bits differ.  A lost tap, row or halo is over 0.1."""
+    print(f"\n[unet gradients G={grid}]", flush=True)
+    b, m, t = _sample(grid, 20 + grid)
+    net = prg.UNet(grid=grid, seed=7)
+    try:
+        loss_ref, ref = _torch_gradients(net.get_params(), b, m, t)
+        loss, g = net.gradients(b, m, t, 1.0)
+    finally:
+        net.close()
+    assert abs(loss - loss_ref) <= 1e-3 * abs(loss_ref)
+    gd, rd = U.unflatten(g), U.unflatten(ref)
+    for name, _ in U.param_layout():
+        err = _rel(gd[name], rd[name])
+        assert err <= 3e-2, (name, err)
