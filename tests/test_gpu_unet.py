@@ -238,3 +238,30 @@ def test_gradients_on_larger_grids(prg, grid):
     for name, _ in U.param_layout():
         err = _rel(gd[name], rd[name])
         assert err <= 3e-2, (name, err)
+
+
+@pytest.mark.parametrize("batch", [1, 3, 18])
+def test_train_step_is_one_adam_step_on_the_mean_gradient(prg, batch):
+    """Samples that share launches (18: two launches of 16 and 2) give the sum
+    of their single gradients.  The first Adam step is lr g / (|g| + eps):
+    with float moments, divisions and a parameter below 2 the result is
+    within 1e-6 lr + 2^-23 of it where |g| is far above eps."""
+    print(f"\n[unet train step G=16 batch {batch}]", flush=True)
+    lr, G = 1e-3, 16
+    net = prg.UNet(grid=G, seed=13)
+    try:
+        s = [_sample(G, 40 + k) for k in range(batch)]
+        scales = np.linspace(0.5, 2.0, batch).astype(np.float32)
+        p0 = net.get_params()
+        losses, grads = zip(*[net.gradients(b, m, t, float(f)) for (b, m, t), f in zip(s, scales)])
+        g = np.sum(np.array(grads, np.float64), axis=0) / batch
+        loss = net.train_step(*(np.stack(a) for a in zip(*s)), scales, lr)
+        p1 = net.get_params()
+    finally:
+        net.close()
+    assert abs(loss - np.mean(losses)) <= 1e-12 * abs(np.mean(losses))
+    big = np.abs(g) > 1e-3 * np.abs(g).max()  # (sums of up to 18 floats: signs are certain here)
+    assert big.any()
+    want = p0 - lr * np.sign(g)
+    assert np.abs(p1 - want)[big].max() <= 1e-6 * lr + 2.0 ** -23 + lr * 1e-8 / np.abs(g[big]).min()
+    assert np.abs(p1 - p0).max() <= lr * (1 + 1e-5) + 2.0 ** -23
