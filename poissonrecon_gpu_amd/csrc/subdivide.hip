@@ -38,6 +38,8 @@
 //             of another brick found through that brick's table
 // Memory grows with the number of bricks (about 1 M for 506 M virtual
 // leaves) and with the bricks that carry output, never with the virtual leaves.
+// Roots of 2^3 and 4^3 leaves (one brick each) take a path of their own, with
+// several roots to a wave and no certificates (k_small_values and on).
 #include <algorithm>
 #include <vector>
 
@@ -87,7 +89,8 @@ __constant__ int8_t c_children_vertex_kind[8] = {0, 1, 3, 2, 4, 5, 7, 6};
 enum { kCntCoarse = 0, kCntCorners = 1, kCntRoots = 2, kCntBricks = 3, kCntVerts = 4, kCntTris = 5, kCntActive = 6,
        kCntLeaves = 7, kCntErr = 8, kCntDense = 9, kCntDepBricks = 10, kCntDepPairs = 11, kCntWork = 12,
        kCntExact = 13, kCntSuper = 14, kCntList2 = 15, kCntWork2 = 16, kCntExactSorted = 17, kCntWork3 = 18,
-       kCntWork4 = 19, kCntDenseSorted = 20, kCntList2Sorted = 21, kCntSlots = 32 };
+       kCntWork4 = 19, kCntDenseSorted = 20, kCntList2Sorted = 21, kCntSmall1 = 22, kCntSmall2 = 23,
+       kCntSlots = 32 };
 static_assert(kCntSlots * 4 <= 128, "the pinned counter copy holds 32 ints");
 
 __device__ __forceinline__ int depth_of(int64_t i, const Levels& L, int D) {
@@ -400,6 +403,36 @@ __global__ void __launch_bounds__(kBlockS) k_root_info(const int32_t* cl, const 
 __global__ void __launch_bounds__(kBlockS) k_root_of(const int32_t* roots, const int32_t* nroots, int32_t* root_of) {
     const int64_t i = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
     if (i < *nroots) root_of[roots[i]] = int32_t(i);
+}
+
+// The place in a list (its length in *counter) of each lane with `want`: one
+// atomic per wave, lanes in order.
+__device__ __forceinline__ int32_t wave_append(bool want, int32_t* counter) {
+    const uint64_t m = __builtin_amdgcn_ballot_w64(want);
+    if (m == 0) return 0;
+    const int lane = threadIdx.x & 63, first = int(__builtin_ctzll(m));
+    int32_t at = 0;
+    if (lane == first) at = atomicAdd(counter, int32_t(__popcll(m)));
+    at = __shfl(at, first, 64);
+    return at + int32_t(__popcll(m & ((uint64_t(1) << lane) - 1)));
+}
+
+// The roots of 2^3 and of 4^3 leaves in lists of their own, and each one's
+// place in its list (sidx).
+__global__ void __launch_bounds__(kBlockS) k_list_small_roots(const int32_t* roots, const int32_t* nroots, Levels L,
+                                                              int D, int32_t* list1, int32_t* list2, int32_t* sidx,
+                                                              int32_t* cnt) {
+    const int64_t q = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
+    const int kb = q < *nroots ? D - depth_of(roots[q], L, D) : 0;
+    const int32_t a1 = wave_append(kb == 1, cnt + kCntSmall1), a2 = wave_append(kb == 2, cnt + kCntSmall2);
+    if (kb == 1) {
+        list1[a1] = int32_t(q);
+        sidx[q] = a1;
+    }
+    if (kb == 2) {
+        list2[a2] = int32_t(q);
+        sidx[q] = a2;
+    }
 }
 
 struct SubArgs {
@@ -991,7 +1024,8 @@ __device__ __forceinline__ void edge_owner(const Brick& B, const L& S, int D, co
 
 // Cube index and owned crossing edges of leaf l of the brick
 // (generateSubdivideVexNums, main.cu:2481-2531; generateTriNums, :2562-2582).
-template <class L>
+// (G: the brick's corner values, (i, j, k) at (k kStride + j) kStride + i)
+template <int kStride = kP, class L>
 __device__ __forceinline__ void leaf_cube(const Brick& B, const L& S, const float* G, int D, int l, int32_t v[3],
                                           float cv[8], int* cube, int* emask) {
     const int lx = int(compact3(uint32_t(l) >> 2)), ly = int(compact3(uint32_t(l) >> 1)), lz = int(compact3(uint32_t(l)));
@@ -1002,7 +1036,7 @@ __device__ __forceinline__ void leaf_cube(const Brick& B, const L& S, const floa
 #pragma unroll
     for (int q = 0; q < 8; q++) {
         const int y = (q >> 1) & 1, xx = (q & 1) ^ y, z = q >> 2;
-        cv[q] = G[((lz + z) * kP + (ly + y)) * kP + (lx + xx)];
+        cv[q] = G[((lz + z) * kStride + (ly + y)) * kStride + (lx + xx)];
         if (cv[q] < 0) cb |= 1 << q;
     }
     *cube = cb;
@@ -1595,12 +1629,14 @@ __global__ void __launch_bounds__(kWave, 5) k_brick_screen_super(SubArgs A, cons
     }
 }
 
-// The bricks of the roots with fewer than 8 bricks, for the brick screen.
-__global__ void __launch_bounds__(kBlockS) k_list_small_root_bricks(const int32_t* bmap, const int32_t* rbricks,
-                                                                    int64_t nb, int32_t* list2, int32_t* cnt) {
-    const int64_t b = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
-    if (b >= nb) return;
-    if (rbricks[bmap[b]] < 8) list2[atomicAdd(cnt + kCntList2, 1)] = int32_t(b);
+// The roots of one 8^3 brick, for the brick screen.
+__global__ void __launch_bounds__(kBlockS) k_list_one_brick_roots(const int32_t* roots, const int32_t* boff,
+                                                                  int64_t nr, Levels L, int D, int32_t* list2,
+                                                                  int32_t* cnt) {
+    const int64_t q = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
+    const bool one = q < nr && depth_of(roots[q], L, D) == D - kBrickLog;
+    const int32_t at = wave_append(one, cnt + kCntList2);
+    if (one) list2[at] = boff[q];
 }
 
 // Per root: its super-brick count (a root of at least 8 bricks has a
@@ -1779,10 +1815,11 @@ __global__ void __launch_bounds__(kWave) k_brick_count(SubArgs A, const int32_t*
     }
 }
 
-__global__ void __launch_bounds__(kBlockS) k_brick_active(const int32_t* bnv, const int32_t* bnt, int64_t n,
-                                                          int32_t* flag) {
+// (sign 2: a small root's brick, whose tables are its own)
+__global__ void __launch_bounds__(kBlockS) k_brick_active(const int32_t* bnv, const int32_t* bnt, const int8_t* sign,
+                                                          int64_t n, int32_t* flag) {
     const int64_t i = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
-    if (i < n) flag[i] = (bnv[i] | bnt[i]) ? 1 : 0;
+    if (i < n) flag[i] = ((bnv[i] | bnt[i]) && sign[i] != 2) ? 1 : 0;
 }
 
 __global__ void __launch_bounds__(kBlockS) k_brick_compact(const int32_t* flag, const int32_t* off, int64_t n,
@@ -1795,6 +1832,63 @@ __global__ void __launch_bounds__(kBlockS) k_brick_compact(const int32_t* flag, 
     } else {
         amap[i] = -1;
     }
+}
+
+// The vertices of the leaf with key k on the edges of mask em, from its corner
+// values (interpolatePoint and generateSubdivideIntersectionPoint,
+// main.cu:2584-2597, 2629-2697); returns their number.
+__device__ __forceinline__ int emit_leaf_vertices(uint32_t k, int D, int em, const float cv[8], float* out) {
+    float c[3];
+    node_center(k, D, D, c);
+    const float hw = 1.0f / float(1 << (D + 1));
+    int n = 0;
+#pragma unroll
+    for (int e = 0; e < 12; e++) {
+        if (!(em & (1 << e))) continue;
+        const int q1 = c_edge_vertex_h[e][0], q2 = c_edge_vertex_h[e][1];
+        float p1[3], p2[3];
+        {
+            const int y = (q1 >> 1) & 1, xx = (q1 & 1) ^ y, z = q1 >> 2;
+            p1[0] = c[0] + float(2 * xx - 1) * hw;
+            p1[1] = c[1] + float(2 * y - 1) * hw;
+            p1[2] = c[2] + float(2 * z - 1) * hw;
+        }
+        {
+            const int y = (q2 >> 1) & 1, xx = (q2 & 1) ^ y, z = q2 >> 2;
+            p2[0] = c[0] + float(2 * xx - 1) * hw;
+            p2[1] = c[1] + float(2 * y - 1) * hw;
+            p2[2] = c[2] + float(2 * z - 1) * hw;
+        }
+        const float f1 = cv[q1], f2 = cv[q2];
+        const int dim = e >> 2;
+        float o3[3] = {p1[0], p1[1], p1[2]};
+        const float pivot = f1 / (f1 - f2);
+        const float another = 1 - pivot;
+        const float s1 = p2[dim] * pivot;
+        const float s2 = p1[dim] * another;
+        o3[dim] = s1 + s2;
+        out[3 * n + 0] = o3[0];
+        out[3 * n + 1] = o3[1];
+        out[3 * n + 2] = o3[2];
+        n++;
+    }
+    return n;
+}
+
+// The vertex of edge e of leaf v: its owner leaf's place (root number q2, -1
+// if none, and Morton offset mort in the root) and the edge kind seen there.
+// root_of_slot(j): the root number of the brick's root's neighbour j.
+template <class L, class RootFn>
+__device__ __forceinline__ int32_t edge_vertex_place(const Brick& B, const L& S, int D, const int32_t v[3], int e,
+                                                     RootFn root_of_slot, uint32_t* mort, int* eo) {
+    int32_t ow[3];
+    edge_owner(B, S, D, v, e, ow, eo);
+    int sl = 13;
+    cell_virtual(B, S, D, ow, &sl);
+    const int sh = 3 * (D - B.r);
+    const uint32_t rmask = sh >= 32 ? 0xffffffffu : ((1u << sh) - 1u);
+    *mort = cell_key(uint32_t(ow[0]), uint32_t(ow[1]), uint32_t(ow[2])) & rmask;
+    return sl == 13 ? B.q : root_of_slot(sl);
 }
 
 // Pass 2 (bricks with output): per-leaf edge masks, cube indices and vertex
@@ -1828,7 +1922,6 @@ __global__ void __launch_bounds__(kWave) k_brick_vertices(SubArgs A, const int32
         cnt += __popc(uint32_t(em));
     }
     int run = wave_excl_scan(cnt);
-    const float hw = 1.0f / float(1 << (D + 1));
     for (int l = l0; l < l1; l++) {
         lofs_tab[int64_t(ai) * kBrickLeaves + l] = uint16_t(run);
         const int em = emask_tab[int64_t(ai) * kBrickLeaves + l];
@@ -1837,37 +1930,7 @@ __global__ void __launch_bounds__(kWave) k_brick_vertices(SubArgs A, const int32
         float cv[8];
         int cube, em2;
         leaf_cube(B, S, S.G, D, l, v, cv, &cube, &em2);
-        float c[3];
-        node_center(B.bkey | uint32_t(l), D, D, c);
-        for (int e = 0; e < 12; e++) {
-            if (!(em & (1 << e))) continue;
-            const int q1 = c_edge_vertex[e][0], q2 = c_edge_vertex[e][1];
-            float p1[3], p2[3];
-            {
-                const int y = (q1 >> 1) & 1, xx = (q1 & 1) ^ y, z = q1 >> 2;
-                p1[0] = c[0] + float(2 * xx - 1) * hw;
-                p1[1] = c[1] + float(2 * y - 1) * hw;
-                p1[2] = c[2] + float(2 * z - 1) * hw;
-            }
-            {
-                const int y = (q2 >> 1) & 1, xx = (q2 & 1) ^ y, z = q2 >> 2;
-                p2[0] = c[0] + float(2 * xx - 1) * hw;
-                p2[1] = c[1] + float(2 * y - 1) * hw;
-                p2[2] = c[2] + float(2 * z - 1) * hw;
-            }
-            const float f1 = cv[q1], f2 = cv[q2];
-            const int dim = e >> 2;
-            float o3[3] = {p1[0], p1[1], p1[2]};
-            const float pivot = f1 / (f1 - f2);
-            const float another = 1 - pivot;
-            const float s1 = p2[dim] * pivot;
-            const float s2 = p1[dim] * another;
-            o3[dim] = s1 + s2;
-            const int64_t id = int64_t(bvoff[b]) + run++;
-            out_v[3 * id + 0] = o3[0];
-            out_v[3 * id + 1] = o3[1];
-            out_v[3 * id + 2] = o3[2];
-        }
+        run += emit_leaf_vertices(B.bkey | uint32_t(l), D, em, cv, out_v + 3 * (int64_t(bvoff[b]) + run));
     }
 }
 
@@ -1891,8 +1954,6 @@ __global__ void __launch_bounds__(kWave) k_brick_triangles(SubArgs A, const int3
     int cnt = 0;
     for (int l = l0; l < l1; l++) cnt += tri_count(cube_tab[int64_t(ai) * kBrickLeaves + l]);
     int64_t o = 3 * (int64_t(btoff[b]) + wave_excl_scan(cnt));
-    const int sh = 3 * (D - B.r);
-    const uint32_t rmask = sh >= 32 ? 0xffffffffu : ((1u << sh) - 1u);
     for (int l = l0; l < l1; l++) {
         const int cube = cube_tab[int64_t(ai) * kBrickLeaves + l];
         const int n = 3 * tri_count(cube);
@@ -1900,14 +1961,10 @@ __global__ void __launch_bounds__(kWave) k_brick_triangles(SubArgs A, const int3
         const int32_t v[3] = {B.org[0] + int32_t(compact3(uint32_t(l) >> 2)),
                               B.org[1] + int32_t(compact3(uint32_t(l) >> 1)), B.org[2] + int32_t(compact3(uint32_t(l)))};
         for (int k = 0; k < n; k++) {
-            const int e = c_tri[cube][k];
-            int32_t ow[3];
+            uint32_t mort;
             int eo;
-            edge_owner(B, S, D, v, e, ow, &eo);
-            int sl = 13;
-            cell_virtual(B, S, D, ow, &sl);
-            const int32_t q2 = sl == 13 ? B.q : S.NBR[sl];
-            const uint32_t mort = cell_key(uint32_t(ow[0]), uint32_t(ow[1]), uint32_t(ow[2])) & rmask;
+            const int32_t q2 =
+                edge_vertex_place(B, S, D, v, c_tri[cube][k], [&](int j) { return S.NBR[j]; }, &mort, &eo);
             const int32_t bi = q2 < 0 ? 0 : A.boff[q2] + int32_t(mort >> (3 * B.kb));
             const int32_t lu = int32_t(mort & ((1u << (3 * B.kb)) - 1u));
             const int32_t au = q2 < 0 ? -1 : amap[bi];
@@ -1921,6 +1978,351 @@ __global__ void __launch_bounds__(kWave) k_brick_triangles(SubArgs A, const int3
             out_t[o + k] = id;
         }
         o += n;
+    }
+}
+
+// ---- small roots -----------------------------------------------------------------------
+// A root of 2^3 (KB = 1) or 4^3 leaves (KB = 2) is one brick of 27 or 125
+// corner values.  Such roots lie at the surface: certificates settle few of
+// them (on a sparse 150,000-point cloud at depth 10, 2% of 235,000), and a
+// certificate costs about what the values cost.  So every small root is
+// evaluated.  A wave of its own per root left 37 of 64 lanes idle in each of
+// three rounds (27 points strewn over an 8^3 brick's numbering); here a wave
+// takes two 2^3 roots or two rounds of a 4^3 root.  Corners that a leaf of another
+// root of the group owns are not evaluated at all: the roots of a group have
+// one depth, so the owner's root is small too and computes the value as its
+// own corner (the same owner, table entries and order); gref says where.
+// Bound by the exact sums' issue: 27 products in the reference's order per
+// depth and corner.  A whole pass over
+// 150,000 points at depth 10 (294,344 roots, 282,635 of them small) went from
+// 35.8 to 14.2 ms, over 35,947 points at depth 8 from 5.4 to 3.9 ms.
+template <int KB>
+struct SmallRoots {
+    static constexpr int kS = 1 << KB, kPts1 = kS + 1, kPts = kPts1 * kPts1 * kPts1;
+    static constexpr int kLanes = KB == 1 ? 32 : 64, kPerWave = kWave / kLanes;  // value pass
+    static constexpr int kLeaves = 1 << (3 * KB), kLeafRoots = kWave / kLeaves;  // leaf passes
+};
+
+template <int KB>
+struct SmallLds {
+    // the chain's neighbour values, 28 floats per depth (16-byte reads)
+    alignas(16) float X[(kMaxDepth + 1) * 28];
+    BasisT T[(kMaxDepth + 1) * 3 * SmallRoots<KB>::kPts1];  // per depth and axis, each grid coordinate's owner's
+    // coefficients of the real cells around the root: 4^3 at depth r + 1 and,
+    // for 4^3 leaves, 6^3 at depth D (0 where virtual or absent)
+    float XB[KB == 1 ? 64 : 64 + 216];
+    int32_t CB[KB == 1 ? 1 : 64];  // child bases of the depth r + 1 cells
+    int32_t NBK[27], NBR[27];
+};
+
+// Adds the 27 terms of one block depth (W cells a side, the owner's low
+// neighbour at cx, cy, cz) in the reference's order.
+template <int W>
+__device__ __forceinline__ float small_block_sum(const float* Xb, int cx, int cy, int cz, BasisT tx, BasisT ty,
+                                                 BasisT tz, float f) {
+    const float bx[3] = {tx.x, tx.y, tx.z}, by[3] = {ty.x, ty.y, ty.z}, bz[3] = {tz.x, tz.y, tz.z};
+    const float* X0 = Xb + (cx * W + cy) * W + cz;
+    float xv[27];
+#pragma unroll
+    for (int k = 0; k < 27; k++) xv[k] = X0[((k / 9) * W + (k / 3) % 3) * W + k % 3];
+#pragma unroll
+    for (int k = 0; k < 27; k++) {
+        float tt = xv[k] * bx[k / 9];
+        tt = tt * by[(k / 3) % 3];
+        tt = tt * bz[k % 3];
+        f = f + tt;
+    }
+    return f;
+}
+
+// A small root's geometry (Brick's fields that the owner tests read).
+__device__ __forceinline__ void small_brick(Brick& B, const int32_t* R, int32_t q, int D, int kb) {
+    B.q = q;
+    B.r = D - kb;
+    B.kb = kb;
+    B.bkey = uint32_t(R[kRecKey]);
+    B.Sr = 1 << kb;
+    decode_cell(B.bkey, B.org);
+    for (int a = 0; a < 3; a++) {
+        B.R[a] = B.org[a] >> kb;
+        B.R0[a] = B.org[a];
+    }
+}
+
+// The corner values its own leaves own, of every small root: gv[slot kPts + p]
+// (f - iso at grid point p = (k kPts1 + j) kPts1 + i), and for every corner
+// where its value is (gref).
+template <int KB>
+__global__ void __launch_bounds__(kWave) k_small_values(SubArgs A, const int32_t* slist, int32_t ns,
+                                                        const int32_t* sidx, float* gv, int32_t* gref) {
+    using C = SmallRoots<KB>;
+    constexpr int P = C::kPts1, LP = C::kLanes;
+    __shared__ SmallLds<KB> SS[C::kPerWave];
+    const int D = A.D, r = D - KB, lane = threadIdx.x, l = lane % LP;
+    SmallLds<KB>& S = SS[lane / LP];
+    const int32_t slot = int32_t(blockIdx.x) * C::kPerWave + lane / LP;
+    const bool live = slot < ns;
+    const int32_t q = slist[live ? slot : ns - 1];
+    const int32_t* R = A.rec + int64_t(q) * kRecWords;
+    Brick B;
+    small_brick(B, R, q, D, KB);
+    if (l < 27) {
+        S.NBK[l] = R[kRecNBK + l];
+        S.NBR[l] = R[kRecNBR + l];
+#pragma unroll
+        for (int d = 0; d <= kMaxDepth; d++)
+            if (d <= r) S.X[28 * d + l] = __int_as_float(R[kRecX + 27 * d + l]);
+    }
+    for (int e = l; e < (D + 1) * 3 * P; e += LP) {
+        const int d = e / (3 * P), a = (e / P) % 3, i = e % P;
+        const int32_t g = (a == 0 ? B.org[0] : a == 1 ? B.org[1] : B.org[2]) + i;
+        const int32_t o = i == 0 ? g : g - 1;  // own_cell
+        const float4 t = A.btab[((int64_t(d) << D) + o) * 2 + (g - o)];
+        S.T[e] = BasisT{t.x, t.y, t.z};
+    }
+    __syncthreads();
+    // depth r + 1: the root's 2^3 cells (virtual) and one more on every side
+    bool kids = false;
+#pragma unroll
+    for (int e = l; e < 64; e += LP) {
+        const int x = e >> 4, y = (e >> 2) & 3, z = e & 3;
+        const int ox = x == 0 ? -1 : x == 3, oy = y == 0 ? -1 : y == 3, oz = z == 0 ? -1 : z == 3;
+        const int32_t cb = (ox | oy | oz) ? S.NBK[nidx(ox, oy, oz)] : -1;
+        // (the root's first cell is even along every axis)
+        const int32_t node = cb < 0 ? -1 : cb + ((((x + 1) & 1) << 2) | (((y + 1) & 1) << 1) | ((z + 1) & 1));
+        S.XB[e] = node < 0 ? 0.0f : A.x[node];
+        if constexpr (KB == 2) {
+            const int32_t c2 = node < 0 ? -1 : A.child_base[node];
+            S.CB[e] = c2;
+            kids = kids || c2 >= 0;
+        }
+    }
+    if constexpr (KB == 2) {  // depth D: the children of those cells around the 4^3 leaves
+        kids = __builtin_amdgcn_ballot_w64(kids) != 0;
+        __syncthreads();
+        if (kids) {
+            for (int e = l; e < 216; e += kWave) {
+                const int x = e / 36, y = (e / 6) % 6, z = e % 6;
+                const int32_t cb = S.CB[(((x + 1) >> 1) * 4 + ((y + 1) >> 1)) * 4 + ((z + 1) >> 1)];
+                const int32_t node = cb < 0 ? -1 : cb + ((((x + 1) & 1) << 2) | (((y + 1) & 1) << 1) | ((z + 1) & 1));
+                S.XB[64 + e] = node < 0 ? 0.0f : A.x[node];
+            }
+        }
+    }
+    __syncthreads();
+    const float iso = *A.iso;
+    for (int p = l; p < C::kPts; p += LP) {
+        const int gi[3] = {p % P, (p / P) % P, p / (P * P)};
+        const int32_t g[3] = {B.org[0] + gi[0], B.org[1] + gi[1], B.org[2] + gi[2]};
+        int32_t o[3] = {0, 0, 0};
+        const int sl = corner_owner(B, S, D, g, o);
+        int32_t ref = slot * C::kPts + p;
+        if (sl != 13) {
+            const int li = gi[0] - (sl / 9 - 1) * C::kS, lj = gi[1] - ((sl / 3) % 3 - 1) * C::kS,
+                      lk = gi[2] - (sl % 3 - 1) * C::kS;
+            ref = sidx[S.NBR[sl]] * C::kPts + (lk * P + lj) * P + li;
+        } else {
+            // the owner is own_cell along every axis; its cell in the root
+            const int c[3] = {gi[0] - (gi[0] > 0), gi[1] - (gi[1] > 0), gi[2] - (gi[2] > 0)};
+            const BasisT* Tx = S.T + gi[0];
+            const BasisT* Ty = S.T + P + gi[1];
+            const BasisT* Tz = S.T + 2 * P + gi[2];
+            // real nodes below the root, depth D up to r + 1 (a virtual,
+            // absent or outside neighbour adds +-0, which leaves a float sum
+            // that started at +0 unchanged)
+            float f = 0.0f;
+            if constexpr (KB == 2) {
+                if (kids) f = small_block_sum<6>(S.XB + 64, c[0], c[1], c[2], Tx[3 * P * D], Ty[3 * P * D], Tz[3 * P * D], f);
+            }
+            f = small_block_sum<4>(S.XB, c[0] >> (KB - 1), c[1] >> (KB - 1), c[2] >> (KB - 1), Tx[3 * P * (r + 1)],
+                                   Ty[3 * P * (r + 1)], Tz[3 * P * (r + 1)], f);
+            // the root's chain (chain_lds's order)
+            for (int d = r; d >= 1; d--) {
+                const BasisT tx = Tx[3 * P * d], ty = Ty[3 * P * d], tz = Tz[3 * P * d];
+                const float bx[3] = {tx.x, tx.y, tx.z}, by[3] = {ty.x, ty.y, ty.z}, bz[3] = {tz.x, tz.y, tz.z};
+                float xv[28];
+#pragma unroll
+                for (int j = 0; j < 7; j++)
+                    *reinterpret_cast<float4*>(xv + 4 * j) = *reinterpret_cast<const float4*>(S.X + 28 * d + 4 * j);
+#pragma unroll
+                for (int j = 0; j < 27; j++) {
+                    float tt = xv[j] * bx[j / 9];
+                    tt = tt * by[(j / 3) % 3];
+                    tt = tt * bz[j % 3];
+                    f = f + tt;
+                }
+            }
+            float tt = S.X[0] * Tx[0].y;
+            tt = tt * Ty[0].y;
+            tt = tt * Tz[0].y;
+            f = f + tt;
+            if (live) gv[ref] = f - iso;
+        }
+        if (live) gref[int64_t(slot) * C::kPts + p] = ref;
+    }
+}
+
+// The group's roots around a small root as a bit mask, for the owner tests
+// (which only ask whether a neighbour is in the group).
+struct GroupMask {
+    struct {
+        uint32_t m;
+        __device__ __forceinline__ int32_t operator[](int j) const { return ((m >> j) & 1u) ? 0 : -1; }
+    } NBR;
+};
+
+// The leaf passes' lanes: kLeafRoots roots to a wave, one leaf per lane.  Sets
+// the lane's root geometry and group.
+template <int KB>
+__device__ __forceinline__ void small_leaf_setup(const SubArgs& A, int32_t q, Brick& B, GroupMask& S) {
+    constexpr int LV = SmallRoots<KB>::kLeaves;
+    const int32_t* R = A.rec + int64_t(q) * kRecWords;
+    small_brick(B, R, q, A.D, KB);
+    const int l = threadIdx.x % LV;
+    uint32_t m = 0;
+#pragma unroll
+    for (int j = l; j < 27; j += LV)
+        if (R[kRecNBR + j] >= 0) m |= 1u << j;
+#pragma unroll
+    for (int o = 1; o < (LV < 32 ? LV : 32); o <<= 1) m |= uint32_t(__shfl_xor(int(m), o, kWave));
+    if constexpr (LV == 64) m |= uint32_t(__shfl_xor(int(m), 32, kWave));
+    S.NBR.m = m;
+}
+
+// Exclusive sums of v over the leaves of the lane's root, and the total.
+template <int LV>
+__device__ __forceinline__ int leaf_excl_scan(int v, int* total) {
+    int inc = v;
+#pragma unroll
+    for (int o = 1; o < LV; o <<= 1) {
+        const int t = __shfl_up(inc, o, LV);
+        if (int(threadIdx.x % LV) >= o) inc += t;
+    }
+    *total = __shfl(inc, LV - 1, LV);
+    return inc - v;
+}
+
+// Per-leaf tables of the small roots (slot kLeaves + leaf): owned crossing
+// edges, cube index, first vertex within the root.
+struct SmallTabs {
+    uint16_t* emask;
+    uint16_t* lofs;
+    uint8_t* cube;
+};
+
+// The corner values of the wave's roots into LDS.
+template <int KB>
+__device__ __forceinline__ void small_corner_values(int32_t s0, int32_t ns, const float* gv, const int32_t* gref,
+                                                    float* G) {
+    using C = SmallRoots<KB>;
+    const int n = std::min(int(ns - s0), C::kLeafRoots) * C::kPts;
+    const int32_t* gr = gref + int64_t(s0) * C::kPts;
+#pragma unroll
+    for (int t = threadIdx.x; t < C::kLeafRoots * C::kPts; t += kWave) G[t] = t < n ? gv[gr[t]] : 1.0f;
+    __syncthreads();
+}
+
+// Cube indices and owned crossing edges of every small root's leaves, and the
+// root's vertex and triangle counts.
+template <int KB>
+__global__ void __launch_bounds__(kWave) k_small_cubes(SubArgs A, const int32_t* slist, int32_t ns, const float* gv,
+                                                       const int32_t* gref, SmallTabs T, int32_t* bnv, int32_t* bnt,
+                                                       int8_t* sign) {
+    using C = SmallRoots<KB>;
+    constexpr int LV = C::kLeaves;
+    __shared__ float G[C::kLeafRoots * C::kPts];
+    const int lane = threadIdx.x, l = lane % LV;
+    const int32_t s0 = int32_t(blockIdx.x) * C::kLeafRoots, slot = s0 + lane / LV;
+    const bool live = slot < ns;
+    const int32_t q = slist[live ? slot : ns - 1];
+    Brick B;
+    GroupMask S;
+    small_leaf_setup<KB>(A, q, B, S);
+    small_corner_values<KB>(s0, ns, gv, gref, G);
+    int32_t v[3];
+    float cv[8];
+    int cube, em;
+    leaf_cube<C::kPts1>(B, S, G + (lane / LV) * C::kPts, A.D, l, v, cv, &cube, &em);
+    int nv, nt;
+    const int ofs = leaf_excl_scan<LV>(__popc(uint32_t(em)), &nv);
+    (void)leaf_excl_scan<LV>(tri_count(cube), &nt);
+    if (!live) return;
+    const int64_t at = int64_t(slot) * LV + l;
+    T.emask[at] = uint16_t(em);
+    T.lofs[at] = uint16_t(ofs);
+    T.cube[at] = uint8_t(cube);
+    if (l == 0) {
+        const int32_t b = A.boff[q];
+        bnv[b] = nv;
+        bnt[b] = nt;
+        sign[b] = 2;
+    }
+}
+
+template <int KB>
+__global__ void __launch_bounds__(kWave) k_small_vertices(SubArgs A, const int32_t* slist, int32_t ns, const float* gv,
+                                                          const int32_t* gref, SmallTabs T, const int32_t* bvoff,
+                                                          float* out_v) {
+    using C = SmallRoots<KB>;
+    constexpr int LV = C::kLeaves, P = C::kPts1;
+    __shared__ float Gs[C::kLeafRoots * C::kPts];
+    const int lane = threadIdx.x, l = lane % LV;
+    const int32_t s0 = int32_t(blockIdx.x) * C::kLeafRoots, slot = s0 + lane / LV;
+    const int64_t at = int64_t(slot) * LV + l;
+    const int em = slot < ns ? T.emask[at] : 0;
+    if (__builtin_amdgcn_ballot_w64(em != 0) == 0) return;
+    small_corner_values<KB>(s0, ns, gv, gref, Gs);
+    if (!em) return;
+    const int32_t q = slist[slot];
+    const uint32_t key = uint32_t(A.rec[int64_t(q) * kRecWords + kRecKey]) | uint32_t(l);
+    const int lx = int(compact3(uint32_t(l) >> 2)), ly = int(compact3(uint32_t(l) >> 1)), lz = int(compact3(uint32_t(l)));
+    const float* G = Gs + (lane / LV) * C::kPts;
+    float cv[8];
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+        const int y = (c >> 1) & 1, xx = (c & 1) ^ y, z = c >> 2;
+        cv[c] = G[((lz + z) * P + (ly + y)) * P + (lx + xx)];
+    }
+    (void)emit_leaf_vertices(key, A.D, em, cv, out_v + 3 * (int64_t(bvoff[A.boff[q]]) + T.lofs[at]));
+}
+
+template <int KB>
+__global__ void __launch_bounds__(kWave) k_small_triangles(SubArgs A, const int32_t* slist, int32_t ns,
+                                                           const int32_t* sidx, SmallTabs T, const int32_t* bvoff,
+                                                           const int32_t* btoff, int64_t vbase, int32_t* out_t,
+                                                           int32_t* err) {
+    using C = SmallRoots<KB>;
+    constexpr int LV = C::kLeaves;
+    const int lane = threadIdx.x, l = lane % LV;
+    const int32_t slot = int32_t(blockIdx.x) * C::kLeafRoots + lane / LV;
+    const bool live = slot < ns;
+    const int cube = live ? T.cube[int64_t(slot) * LV + l] : 0;
+    const int nt = tri_count(cube);
+    if (__builtin_amdgcn_ballot_w64(nt != 0) == 0) return;
+    const int32_t q = slist[live ? slot : ns - 1];
+    Brick B;
+    GroupMask S;
+    small_leaf_setup<KB>(A, q, B, S);
+    int total;
+    const int first = leaf_excl_scan<LV>(nt, &total);
+    if (!nt) return;
+    int32_t* out = out_t + 3 * (int64_t(btoff[A.boff[q]]) + first);
+    const int32_t v[3] = {B.org[0] + int32_t(compact3(uint32_t(l) >> 2)), B.org[1] + int32_t(compact3(uint32_t(l) >> 1)),
+                          B.org[2] + int32_t(compact3(uint32_t(l)))};
+    const int32_t* NBR = A.rec + int64_t(q) * kRecWords + kRecNBR;
+    for (int k = 0; k < 3 * nt; k++) {
+        uint32_t mort;
+        int eo;
+        const int32_t q2 = edge_vertex_place(B, S, A.D, v, c_tri[cube][k], [&](int j) { return NBR[j]; }, &mort, &eo);
+        const int64_t t = q2 < 0 ? 0 : int64_t(sidx[q2]) * LV + mort;
+        const uint32_t em = q2 < 0 ? 0 : T.emask[t];
+        int32_t id = 0;
+        if (!((em >> eo) & 1u)) {
+            err[0] = 1;  // the owner has no vertex on the edge
+        } else {
+            id = int32_t(vbase + bvoff[A.boff[q2]] + T.lofs[t] + __popc(em & ((1u << eo) - 1u)));
+        }
+        out[k] = id;
     }
 }
 
@@ -1945,7 +2347,7 @@ void extract_subdivision(prg_ctx* c) {
     const int rd = ensure_coarse_rows(c, s);
     if (rd < D - 1) throw Error{PRG_E_STATE, "coarse rows missing"};
 
-    // pool slots 97..139
+    // pool slots 97..159
     PoolBuf<uint8_t> inter{&c->pool[97]};
     PoolBuf<int32_t> cnt{&c->pool[98]}, flag{&c->pool[99]}, off{&c->pool[100]}, cl{&c->pool[101]},
         oref{&c->pool[102]}, need{&c->pool[103]}, nid{&c->pool[104]}, clist{&c->pool[105]}, rflag{&c->pool[107]},
@@ -2027,6 +2429,13 @@ void extract_subdivision(prg_ctx* c) {
     PRG_CHECK_LAUNCH();
     scan_exclusive2(rbricks.get(), boff.get(), C + kCntBricks, rleaves.get(), loff.get(), C + kCntLeaves, baseD, s,
                     c->scratch, kt);
+    PoolBuf<int32_t> slist1{&c->pool[144]}, slist2{&c->pool[145]}, sidx{&c->pool[146]};
+    slist1.reserve(baseD);
+    slist2.reserve(baseD);
+    sidx.reserve(baseD);
+    k_list_small_roots<<<grid_for(baseD, kBlockS), kBlockS, 0, s>>>(roots.get(), C + kCntRoots, Lv, D, slist1.get(),
+                                                                     slist2.get(), sidx.get(), C);
+    PRG_CHECK_LAUNCH();
     int32_t* H = c->sub_host;
     PRG_HIP(hipMemcpyAsync(H, C, kCntSlots * 4, hipMemcpyDeviceToHost, s));
     PRG_HIP(hipStreamSynchronize(s));
@@ -2079,7 +2488,48 @@ void extract_subdivision(prg_ctx* c) {
     dbricks.reserve(3 * nb);
     dpairs.reserve(26 * nb);
     bsign.reserve(nb);
+    // the small roots: values, cubes and counts
+    const int32_t n1 = H[kCntSmall1], n2 = H[kCntSmall2];
+    const int64_t nb3 = nb - n1 - n2;  // 8^3 bricks
+    PoolBuf<float> gv1{&c->pool[147]}, gv2{&c->pool[148]};
+    PoolBuf<int32_t> gref1{&c->pool[149]}, gref2{&c->pool[150]};
+    PoolBuf<uint16_t> semask{&c->pool[151]}, slofs{&c->pool[152]};
+    PoolBuf<uint8_t> scube{&c->pool[153]};
+    using Small1 = SmallRoots<1>;
+    using Small2 = SmallRoots<2>;
+    if (int64_t(n1) * Small1::kPts >= (int64_t(1) << 31) || int64_t(n2) * Small2::kPts >= (int64_t(1) << 31))
+        throw Error{PRG_E_NOMEM, "too many small subdivision roots"};
+    const size_t tab2 = size_t(n1) * Small1::kLeaves, tabn = tab2 + size_t(n2) * Small2::kLeaves;
+    semask.reserve(tabn);
+    slofs.reserve(tabn);
+    scube.reserve(tabn);
+    const SmallTabs T1{semask.get(), slofs.get(), scube.get()};
+    const SmallTabs T2{semask.get() + tab2, slofs.get() + tab2, scube.get() + tab2};
+    const unsigned lw1 = grid_for(n1, Small1::kLeafRoots), lw2 = grid_for(n2, Small2::kLeafRoots);
     {
+        TimedScope ts(kt, "subdivide_small_values", 0.0);  // issue-bound: no byte figure
+        if (n1) {
+            gv1.reserve(size_t(n1) * Small1::kPts);
+            gref1.reserve(size_t(n1) * Small1::kPts);
+            k_small_values<1><<<grid_for(n1, Small1::kPerWave), kWave, 0, s>>>(A, slist1.get(), n1, sidx.get(),
+                                                                               gv1.get(), gref1.get());
+            PRG_CHECK_LAUNCH();
+            k_small_cubes<1><<<lw1, kWave, 0, s>>>(A, slist1.get(), n1, gv1.get(), gref1.get(), T1, bnv.get(),
+                                                   bnt.get(), bsign.get());
+            PRG_CHECK_LAUNCH();
+        }
+        if (n2) {
+            gv2.reserve(size_t(n2) * Small2::kPts);
+            gref2.reserve(size_t(n2) * Small2::kPts);
+            k_small_values<2><<<grid_for(n2, Small2::kPerWave), kWave, 0, s>>>(A, slist2.get(), n2, sidx.get(),
+                                                                               gv2.get(), gref2.get());
+            PRG_CHECK_LAUNCH();
+            k_small_cubes<2><<<lw2, kWave, 0, s>>>(A, slist2.get(), n2, gv2.get(), gref2.get(), T2, bnv.get(),
+                                                   bnt.get(), bsign.get());
+            PRG_CHECK_LAUNCH();
+        }
+    }
+    if (nb3 > 0) {
         TimedScope ts(kt, "subdivide_screen", 0.0);  // latency- and issue-bound: no byte figure
         // super-bricks of the roots with at least 8 bricks, then the brick
         // screen over the bricks they leave and those of the smaller roots
@@ -2095,8 +2545,8 @@ void extract_subdivision(prg_ctx* c) {
                                                                                       std::max<int64_t>(1, nb / 8),
                                                                                       smap.get());
         PRG_CHECK_LAUNCH();
-        k_list_small_root_bricks<<<grid_for(nb, kBlockS), kBlockS, 0, s>>>(bmap.get(), rbricks.get(), nb,
-                                                                            list2.get(), C);
+        k_list_one_brick_roots<<<grid_for(nr, kBlockS), kBlockS, 0, s>>>(roots.get(), boff.get(), nr, Lv, D,
+                                                                          list2.get(), C);
         PRG_CHECK_LAUNCH();
         // resident grids: every workgroup walks its share
         int per_cu = 0;
@@ -2145,19 +2595,21 @@ void extract_subdivision(prg_ctx* c) {
         k_compact<<<grid_for(nb, kBlockS), kBlockS, 0, s>>>(xmark.get(), xoff.get(), nb, dlist.get());
         PRG_CHECK_LAUNCH();
     }
-    PRG_HIP(hipMemcpyAsync(H, C, kCntSlots * 4, hipMemcpyDeviceToHost, s));
-    PRG_HIP(hipStreamSynchronize(s));
-    const int64_t ndense = H[kCntDense];
+    if (nb3 > 0) {
+        PRG_HIP(hipMemcpyAsync(H, C, kCntSlots * 4, hipMemcpyDeviceToHost, s));
+        PRG_HIP(hipStreamSynchronize(s));
+    }
+    const int64_t ndense = nb3 > 0 ? H[kCntDense] : 0;
     PoolBuf<float> gvals{&c->pool[134]};
     PoolBuf<int32_t> didx{&c->pool[135]};
     gvals.reserve(size_t(std::max<int64_t>(1, ndense)) * kBrickPts);
     didx.reserve(nb);
-    {
+    if (ndense > 0) {
         TimedScope ts(kt, "subdivide_count", 0.0);
         int per_cu = 0;
         PRG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_brick_count, kWave, 0));
         const int64_t grid = std::min<int64_t>(ndense, int64_t(std::max(1, per_cu)) * std::max(1, c->num_cu));
-        if (grid > 0) {
+        {
             k_brick_count<<<unsigned(grid), kWave, 0, s>>>(A, dlist.get(), C, bnv.get(), bnt.get(), gvals.get(),
                                                            didx.get());
             PRG_CHECK_LAUNCH();
@@ -2165,7 +2617,7 @@ void extract_subdivision(prg_ctx* c) {
     }
     scan_exclusive2(bnv.get(), bvoff.get(), C + kCntVerts, bnt.get(), btoff.get(), C + kCntTris, nb, s, c->scratch,
                     kt);
-    k_brick_active<<<grid_for(nb, kBlockS), kBlockS, 0, s>>>(bnv.get(), bnt.get(), nb, aflag.get());
+    k_brick_active<<<grid_for(nb, kBlockS), kBlockS, 0, s>>>(bnv.get(), bnt.get(), bsign.get(), nb, aflag.get());
     PRG_CHECK_LAUNCH();
     scan_exclusive(aflag.get(), aoff.get(), nb, C + kCntActive, s, c->scratch, kt);
     k_brick_compact<<<grid_for(nb, kBlockS), kBlockS, 0, s>>>(aflag.get(), aoff.get(), nb, alist.get(), amap.get());
@@ -2174,13 +2626,13 @@ void extract_subdivision(prg_ctx* c) {
     PRG_HIP(hipStreamSynchronize(s));
     const int64_t snv = H[kCntVerts], snt = H[kCntTris], nact = H[kCntActive];
     c->sub_bricks = nb;
-    c->sub_exact = H[kCntExact];
-    c->sub_evaluated = H[kCntDense];
+    c->sub_exact = int64_t(H[kCntExact]) + n1 + n2;
+    c->sub_evaluated = int64_t(H[kCntDense]) + n1 + n2;
     if (snv < 0 || snt < 0 || nact < 0) throw Error{PRG_E_NOMEM, "subdivision mesh exceeds int32 counts"};
     if (c->mesh_nv + snv >= (int64_t(1) << 31)) throw Error{PRG_E_NOMEM, "mesh vertex count exceeds int32 indices"};
-    if (nact == 0) return;
+    if (snv == 0 && snt == 0) return;
 
-    // passes 2 and 3 over the bricks with output
+    // passes 2 and 3 over the small roots and the bricks with output
     PoolBuf<uint16_t> lofs_tab{&c->pool[124]}, emask_tab{&c->pool[125]};
     PoolBuf<uint8_t> cube_tab{&c->pool[126]};
     lofs_tab.reserve(size_t(nact) * kBrickLeaves);
@@ -2190,16 +2642,39 @@ void extract_subdivision(prg_ctx* c) {
     int32_t* ST = c->sub_t.reserve(size_t(3) * snt + 3);
     {
         TimedScope ts(kt, "subdivide_vertices", 12.0 * double(snv));
-        k_brick_vertices<<<unsigned(nact), kWave, 0, s>>>(A, alist.get(), bvoff.get(), lofs_tab.get(),
-                                                          emask_tab.get(), cube_tab.get(), gvals.get(), didx.get(), SV);
-        PRG_CHECK_LAUNCH();
+        if (n1) {
+            k_small_vertices<1><<<lw1, kWave, 0, s>>>(A, slist1.get(), n1, gv1.get(), gref1.get(), T1, bvoff.get(), SV);
+            PRG_CHECK_LAUNCH();
+        }
+        if (n2) {
+            k_small_vertices<2><<<lw2, kWave, 0, s>>>(A, slist2.get(), n2, gv2.get(), gref2.get(), T2, bvoff.get(), SV);
+            PRG_CHECK_LAUNCH();
+        }
+        if (nact) {
+            k_brick_vertices<<<unsigned(nact), kWave, 0, s>>>(A, alist.get(), bvoff.get(), lofs_tab.get(),
+                                                              emask_tab.get(), cube_tab.get(), gvals.get(),
+                                                              didx.get(), SV);
+            PRG_CHECK_LAUNCH();
+        }
     }
     {
         TimedScope ts(kt, "subdivide_triangles", 12.0 * double(snt));
-        k_brick_triangles<<<unsigned(nact), kWave, 0, s>>>(A, alist.get(), amap.get(), bvoff.get(), btoff.get(),
-                                                           lofs_tab.get(), emask_tab.get(), cube_tab.get(),
-                                                           c->mesh_nv, ST, C + kCntErr);
-        PRG_CHECK_LAUNCH();
+        if (n1) {
+            k_small_triangles<1><<<lw1, kWave, 0, s>>>(A, slist1.get(), n1, sidx.get(), T1, bvoff.get(), btoff.get(),
+                                                       c->mesh_nv, ST, C + kCntErr);
+            PRG_CHECK_LAUNCH();
+        }
+        if (n2) {
+            k_small_triangles<2><<<lw2, kWave, 0, s>>>(A, slist2.get(), n2, sidx.get(), T2, bvoff.get(), btoff.get(),
+                                                       c->mesh_nv, ST, C + kCntErr);
+            PRG_CHECK_LAUNCH();
+        }
+        if (nact) {
+            k_brick_triangles<<<unsigned(nact), kWave, 0, s>>>(A, alist.get(), amap.get(), bvoff.get(), btoff.get(),
+                                                               lofs_tab.get(), emask_tab.get(), cube_tab.get(),
+                                                               c->mesh_nv, ST, C + kCntErr);
+            PRG_CHECK_LAUNCH();
+        }
     }
     PRG_HIP(hipMemcpyAsync(H + kCntErr, C + kCntErr, 4, hipMemcpyDeviceToHost, s));
     PRG_HIP(hipStreamSynchronize(s));

@@ -43,6 +43,21 @@ CASES = ["sphere_c1_d6", "torus_d7", "superquadrics_d7", "sparse_d5", "two_point
 @pytest.mark.parametrize("name", CASES)
 def test_full_mesh_bit_exact(name, prg):
     (p, n), D = _workload(name, prg)
+    _check_full_mesh(name, p, n, D, prg)
+
+
+@pytest.mark.parametrize("D,count", [(2, 1), (2, 9), (3, 5), (3, 60), (4, 30), (4, 400), (6, 37), (6, 2001), (7, 800)])
+def test_small_roots_bit_exact(D, count, prg):
+    """Roots of 2^3 and 4^3 leaves, several to a wave: from none or one of a
+    kind to thousands (waves whose last root is missing among them), alone
+    (root depth under 3) and in groups that share corners."""
+    rng = np.random.default_rng(100 * D + count)
+    p = (rng.random((count, 3)) * [1.0, 0.7, 0.4]).astype(np.float32)
+    n = rng.standard_normal((count, 3)).astype(np.float32)
+    _check_full_mesh("random", p, n, D, prg)
+
+
+def _check_full_mesh(name, p, n, D, prg):
     print(f"\n[case {name}: N={len(p)} D={D}]", flush=True)
     o = orc.Oracle(D)
     g = prg.Reconstructor(max_depth=D)
