@@ -480,6 +480,7 @@ constexpr int kP = (1 << kBrickLog) + 1;  // grid points per brick side (at most
 // at most (D - 3 - r) blocks of 4^3 cells and blocks of 5^3, 7^3 and 11^3
 // cells at the three finest depths.
 constexpr int kXBlk = 2304;
+constexpr int kXBlkScreen = 512;  // and in the screens' LDS
 
 // LDS of one brick's wave: the root's neighbourhood, the brick's basis
 // tables and blocks (BrickCore), and for the evaluation its corner values.
@@ -502,6 +503,10 @@ struct BrickCoreT {
     float X[kXBCap > 1 ? (kMaxDepth + 1) * 27 : 1];  // the root's chain: neighbour values at depths 0..r
     float XB[kXBCap];                  // per depth below the root: its block (xb_off)
     int32_t xb_off[kMaxDepth + 1];     // start of depth dd's block in XB, or -1 (no real node in it)
+    // child bases of a block's cells while the blocks are filled, at depths
+    // D, D - 2, .. and D - 1, D - 3, ..: up to 5^3 and 7^3 cells (the
+    // screens take blocks of up to 5^3 above depth D)
+    int32_t CB0[kXBCap > 1 ? 125 : 1], CB1[kXBCap > kXBlkScreen ? 343 : kXBCap > 1 ? 125 : 1];
     int32_t NB[27], NBK[27], NBR[27];  // the root's neighbours, their child bases, their root numbers (group)
     float tmax[kMaxDepth + 1];         // brick_abs_bound: per depth, the largest |basis value|
     float xsum[kMaxDepth + 1];         // and the sum of |coefficients|
@@ -515,7 +520,6 @@ using BrickCore = BrickCoreT<kXBlk>;
 // The certificate screen's LDS: blocks up to kXBlkScreen floats (the depths
 // where the brick lies in one cell, and the first finer one); bricks that
 // need more go to the exact certificate, whose LDS holds every block.
-constexpr int kXBlkScreen = 512;
 using BrickScreenLds = BrickCoreT<kXBlkScreen, kP, false>;
 // The super-brick screen's: 2x2x2 bricks, 17 grid coordinates per axis.
 constexpr int kPSuper = 2 * (1 << kBrickLog) + 1;
@@ -665,95 +669,70 @@ __device__ __forceinline__ void brick_tables(const SubArgs& A, const Brick& B, L
     }
 }
 
-// Fills the brick's blocks (depths r+1..D): each cell's coefficient.  A
-// depth's block is needed when it reaches outside the root into a
-// neighbour with children; the parents of a block's cells lie in the block
-// one depth up, so the depths that need one are r+1 .. some dmax, and the
-// blocks are filled level by level: the cells of depth r+1 from the
-// neighbours' child bases, each deeper cell from its parent's node (one
-// child-base load per cell).  A block holds its cells' node indices until
-// the next depth has read them, then their coefficients.  A depth whose
-// block holds no real node gets none.
+// Fills the brick's blocks (depths r+1..D), level by level: each cell's
+// coefficient, 0 where it is virtual or absent.  The cells of depth r+1 come
+// from the neighbours' child bases, each deeper cell from its parent's, which
+// lies in the block one depth up; a cell's coefficient and child base load
+// together.  The levels end where no cell of a block has children: most
+// bricks of a large root see real nodes of the first depths below it only,
+// and blocks of 5^3, 7^3 and 11^3 empty cells neither take time nor fill the
+// LDS (109,000 of 160,000 bricks missed the interval screen for those alone).
+// A depth whose block holds no nonzero coefficient gets none.  Returns false
+// when the caller's LDS cannot hold the blocks.
 template <class L>
 __device__ __forceinline__ bool brick_blocks(const SubArgs& A, const Brick& B, L& S) {
     constexpr int kCap = int(sizeof(S.XB) / sizeof(float));
+    constexpr int kCapC[2] = {int(sizeof(S.CB0) / sizeof(int32_t)), int(sizeof(S.CB1) / sizeof(int32_t))};
     const int D = A.D, lane = threadIdx.x;
-    int off[kMaxDepth + 1];  // uniform: constant indices below keep it in scalar registers
-    int total = 0, dmax = B.r;
+    bool on = B.deep;  // (uniform) the next depth may have real cells
+    int total = 0;
+    if (lane <= kMaxDepth) S.xb_off[lane] = -1;
 #pragma unroll
-    for (int dd = 0; dd <= kMaxDepth; dd++) {
-        off[dd] = -1;
-        if (dd > D || dd <= B.r || !B.deep || dmax != dd - 1) continue;
-        const int W = block_width(D, B.kb, dd), sh = D - dd, up = dd - B.r;
-        // the root slots the block touches: filled only if one of them has children
-        uint32_t in[3];  // per axis, bit t: offset t - 1 is touched
-        for (int a = 0; a < 3; a++) {
-            const int32_t lo = (B.org[a] >> sh) - 2;
-            const int slo = (lo >> up) - B.R[a], shi = ((lo + W - 1) >> up) - B.R[a];
-            in[a] = (slo <= -1 ? 1u : 0u) | (slo <= 0 && shi >= 0 ? 2u : 0u) | (shi >= 1 ? 4u : 0u);
-        }
-        uint32_t touched = 0;
-#pragma unroll
-        for (int j = 0; j < 27; j++)
-            if (((in[0] >> (j / 9)) & (in[1] >> ((j / 3) % 3)) & (in[2] >> (j % 3))) & 1u) touched |= 1u << j;
-        if (!(touched & B.kids)) continue;
-        if (total + W * W * W > kCap) return false;  // (uniform) the caller's LDS cannot hold the blocks
-        off[dd] = total;
-        total += W * W * W;
-        dmax = dd;
-    }
-    int32_t* NI = reinterpret_cast<int32_t*>(S.XB);
-    uint32_t nz = 0;  // depths where this lane found a real node
-#pragma unroll
-    for (int dd = 1; dd <= kMaxDepth + 1; dd++) {
-        if (dd <= kMaxDepth && dd > B.r && dd <= dmax) {
-            // node indices of depth dd
-            const int W = block_width(D, B.kb, dd), sh = D - dd, n = W * W * W;
-            const uint32_t rw = (65536u + uint32_t(W) - 1u) / uint32_t(W);
-            const int32_t lo[3] = {(B.org[0] >> sh) - 2, (B.org[1] >> sh) - 2, (B.org[2] >> sh) - 2};
-            const int32_t width = 1 << dd;
-            const int Wp = dd > B.r + 1 ? block_width(D, B.kb, dd - 1) : 0;
-            const int32_t plo[3] = {(B.org[0] >> (sh + 1)) - 2, (B.org[1] >> (sh + 1)) - 2, (B.org[2] >> (sh + 1)) - 2};
-            for (int e = lane; e < n; e += kWave) {
-                // l / W and l / W^2 for l < W^3 <= 1331 by a 16-bit reciprocal (exact: l / W
-                // has a fractional part of at most (W-1)/W, the reciprocal's excess adds < 0.03)
-                const int q1 = int((uint32_t(e) * rw) >> 16), q2 = int((uint32_t(q1) * rw) >> 16);
-                const int32_t c[3] = {lo[0] + q2, lo[1] + (q1 - q2 * W), lo[2] + (e - q1 * W)};
-                const int oct = ((c[0] & 1) << 2) | ((c[1] & 1) << 1) | (c[2] & 1);
-                int32_t node = -1;
-                if (c[0] >= 0 && c[1] >= 0 && c[2] >= 0 && c[0] < width && c[1] < width && c[2] < width) {
-                    if (dd == B.r + 1) {
-                        const int ox = (c[0] >> 1) - B.R[0], oy = (c[1] >> 1) - B.R[1], oz = (c[2] >> 1) - B.R[2];
-                        const int32_t kids = (ox | oy | oz) ? S.NBK[nidx(ox, oy, oz)] : -1;
-                        node = kids < 0 ? -1 : kids + oct;
-                    } else {
-                        const int32_t pe =
-                            (((c[0] >> 1) - plo[0]) * Wp + ((c[1] >> 1) - plo[1])) * Wp + ((c[2] >> 1) - plo[2]);
-                        const int32_t par = NI[off[dd - 1] + pe];
-                        const int32_t cb = par < 0 ? -1 : A.child_base[par];
-                        node = cb < 0 ? -1 : cb + oct;
-                    }
+    for (int dd = 1; dd <= kMaxDepth; dd++) {
+        if (!on || dd <= B.r || dd > D) continue;
+        const int W = block_width(D, B.kb, dd), sh = D - dd, n = W * W * W;
+        // child bases of depth dd - 1 in one buffer, of dd in the other
+        const bool odd = (sh & 1) != 0;
+        if (total + n > kCap || (dd < D && n > kCapC[odd ? 1 : 0])) return false;
+        const int32_t* CBp = odd ? S.CB0 : S.CB1;
+        int32_t* CBn = odd ? S.CB1 : S.CB0;
+        const uint32_t rw = (65536u + uint32_t(W) - 1u) / uint32_t(W);
+        const int32_t lo[3] = {(B.org[0] >> sh) - 2, (B.org[1] >> sh) - 2, (B.org[2] >> sh) - 2};
+        const int32_t width = 1 << dd;
+        const int Wp = dd > B.r + 1 ? block_width(D, B.kb, dd - 1) : 0;
+        const int32_t plo[3] = {(B.org[0] >> (sh + 1)) - 2, (B.org[1] >> (sh + 1)) - 2, (B.org[2] >> (sh + 1)) - 2};
+        bool kids = false, nz = false;
+        for (int e = lane; e < n; e += kWave) {
+            // l / W and l / W^2 for l < W^3 <= 1331 by a 16-bit reciprocal (exact: l / W
+            // has a fractional part of at most (W-1)/W, the reciprocal's excess adds < 0.03)
+            const int q1 = int((uint32_t(e) * rw) >> 16), q2 = int((uint32_t(q1) * rw) >> 16);
+            const int32_t c[3] = {lo[0] + q2, lo[1] + (q1 - q2 * W), lo[2] + (e - q1 * W)};
+            int32_t cb = -1;
+            if (uint32_t(c[0]) < uint32_t(width) && uint32_t(c[1]) < uint32_t(width) && uint32_t(c[2]) < uint32_t(width)) {
+                if (dd == B.r + 1) {
+                    const int ox = (c[0] >> 1) - B.R[0], oy = (c[1] >> 1) - B.R[1], oz = (c[2] >> 1) - B.R[2];
+                    cb = (ox | oy | oz) ? S.NBK[nidx(ox, oy, oz)] : -1;
+                } else {
+                    cb = CBp[(((c[0] >> 1) - plo[0]) * Wp + ((c[1] >> 1) - plo[1])) * Wp + ((c[2] >> 1) - plo[2])];
                 }
-                NI[off[dd] + e] = node;
             }
-        }
-        // coefficients of depth dd - 1, whose node indices depth dd has read
-        const int dc = dd - 1;
-        if (dc > B.r && dc <= dmax) {
-            const int W = block_width(D, B.kb, dc), n = W * W * W;
-            for (int e = lane; e < n; e += kWave) {
-                const int32_t node = NI[off[dc] + e];
-                const float xv = node < 0 ? 0.0f : A.x[node];
-                S.XB[off[dc] + e] = xv;
-                if (xv != 0.0f) nz |= 1u << dc;
+            float xv = 0.0f;
+            int32_t ck = -1;
+            if (cb >= 0) {
+                const int32_t node = cb + (((c[0] & 1) << 2) | ((c[1] & 1) << 1) | (c[2] & 1));
+                xv = A.x[node];
+                if (dd < D) ck = A.child_base[node];
             }
+            S.XB[total + e] = xv;
+            if (dd < D) CBn[e] = ck;
+            nz = nz || xv != 0.0f;
+            kids = kids || ck >= 0;
         }
-        if (dd <= dmax + 1) __syncthreads();  // this depth's node indices are read by the next
-    }
-#pragma unroll
-    for (int dd = 0; dd <= kMaxDepth; dd++) {
-        const bool any = __builtin_amdgcn_ballot_w64((nz >> dd) & 1u) != 0;
-        if (lane == 0) S.xb_off[dd] = any ? off[dd] : -1;
+        const bool any = __builtin_amdgcn_ballot_w64(nz) != 0;
+        on = __builtin_amdgcn_ballot_w64(kids) != 0;
+        if (any && lane == 0) S.xb_off[dd] = total;
+        total += n;
+        __syncthreads();  // this depth's child bases are read by the next
     }
     __syncthreads();
     return true;
