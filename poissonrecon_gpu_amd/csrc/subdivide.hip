@@ -27,15 +27,15 @@
 // order, so one scan numbers every batch's vertices and triangles.
 //
 // Work is split into bricks: Morton-contiguous blocks of up to 8^3 virtual
-// leaves of one root (the whole root when it is smaller), one wavefront each.
-// A wave computes the brick's (S+1)^3 corner values into LDS, each from its
-// owner's point of view (the owner fixes the summation order), then the
-// leaves' cubes and owned crossing edges from LDS.  Three passes:
-//   count     every brick: vertex and triangle counts      (k_brick_count)
-//   vertices  bricks with output: per-leaf edge masks, cube indices and
-//             vertex offsets into small per-brick tables, and the vertices
-//   triangles bricks with output: triangle entries, a vertex owned by a leaf
-//             of another brick found through that brick's table
+// leaves of one root (the whole root when it is smaller).  Certificates settle
+// the 8^3 bricks without a sign change, one wavefront each; for the others
+//   values    the 9^3 corner values, each from its owner's point of view (the
+//             owner fixes the summation order)
+//   cubes     per leaf: cube index and owned crossing edges, into per-brick
+//             tables, and the brick's vertex and triangle counts
+//   vertices  the vertices, numbered by scans of the counts
+//   triangles triangle entries, a vertex owned by a leaf of another brick
+//             found through that brick's tables
 // Memory grows with the number of bricks (about 1 M for 506 M virtual
 // leaves) and with the bricks that carry output, never with the virtual leaves.
 // Roots of 2^3 and 4^3 leaves (one brick each) take a path of their own, with
@@ -86,10 +86,10 @@ __constant__ CubeFaces c_cube_faces = make_cube_faces();
 __constant__ int8_t c_children_vertex_kind[8] = {0, 1, 3, 2, 4, 5, 7, 6};
 
 // slots of the device counter array
-enum { kCntCoarse = 0, kCntCorners = 1, kCntRoots = 2, kCntBricks = 3, kCntVerts = 4, kCntTris = 5, kCntActive = 6,
+enum { kCntCoarse = 0, kCntCorners = 1, kCntRoots = 2, kCntBricks = 3, kCntVerts = 4, kCntTris = 5,
        kCntLeaves = 7, kCntErr = 8, kCntDense = 9, kCntDepBricks = 10, kCntDepPairs = 11, kCntWork = 12,
-       kCntExact = 13, kCntSuper = 14, kCntList2 = 15, kCntWork2 = 16, kCntExactSorted = 17, kCntWork3 = 18,
-       kCntWork4 = 19, kCntDenseSorted = 20, kCntList2Sorted = 21, kCntSmall1 = 22, kCntSmall2 = 23,
+       kCntExact = 13, kCntSuper = 14, kCntList2 = 15, kCntWork2 = 16, kCntWork3 = 17, kCntSmall1 = 18,
+       kCntSmall2 = 19,
        kCntSlots = 32 };
 static_assert(kCntSlots * 4 <= 128, "the pinned counter copy holds 32 ints");
 
@@ -201,13 +201,6 @@ __global__ void __launch_bounds__(kBlockS) k_flag_coarse_leaves(const int32_t* c
 __global__ void __launch_bounds__(kBlockS) k_compact(const int32_t* flag, const int32_t* off, int64_t n, int32_t* out) {
     const int64_t i = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
     if (i < n && flag[i]) out[off[i]] = int32_t(i);
-}
-
-// mark[list[i]] = 1 for the *n entries of a list of brick numbers below nb
-__global__ void __launch_bounds__(kBlockS) k_mark_listed(const int32_t* list, const int32_t* n, int64_t nb,
-                                                         int32_t* mark) {
-    const int64_t i = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
-    if (i < nb && i < *n) mark[list[i]] = 1;
 }
 
 // Corner owners of the coarse leaves' corners among the same-depth nodes
@@ -483,7 +476,7 @@ constexpr int kXBlk = 2304;
 constexpr int kXBlkScreen = 512;  // and in the screens' LDS
 
 // LDS of one brick's wave: the root's neighbourhood, the brick's basis
-// tables and blocks (BrickCore), and for the evaluation its corner values.
+// tables and blocks (BrickCore).
 // One basis table entry of the brick (the owner's three values along one
 // axis): 12 bytes, the corner basis table's fourth float is never read.
 struct BasisT {
@@ -492,21 +485,20 @@ struct BasisT {
 
 template <int kXBCap, int kTP = kP, bool kHasT = true>
 struct BrickCoreT {
+    static_assert(kXBCap > 1, "a layout holds blocks");
     static constexpr int kTPts = kTP;  // grid coordinates per axis (of T, or of the screen's ranges)
     // per depth d, axis a and grid coordinate i: the corner basis table entry
     // of the owner (own_cell) of grid coordinate org[a] + i, (d, a, i) at
     // d * 3 kP + a kP + i (the screens reduce the entries straight from the
     // global table and keep no T)
-    // (a layout without blocks, kXBCap = 1, is for the mesh passes, which
-    // evaluate nothing: no table and no chain)
-    BasisT T[kHasT && kXBCap > 1 ? (kMaxDepth + 1) * 3 * kTP : 1];
-    float X[kXBCap > 1 ? (kMaxDepth + 1) * 27 : 1];  // the root's chain: neighbour values at depths 0..r
+    BasisT T[kHasT ? (kMaxDepth + 1) * 3 * kTP : 1];
+    float X[(kMaxDepth + 1) * 27];  // the root's chain: neighbour values at depths 0..r
     float XB[kXBCap];                  // per depth below the root: its block (xb_off)
     int32_t xb_off[kMaxDepth + 1];     // start of depth dd's block in XB, or -1 (no real node in it)
     // child bases of a block's cells while the blocks are filled, at depths
     // D, D - 2, .. and D - 1, D - 3, ..: up to 5^3 and 7^3 cells (the
     // screens take blocks of up to 5^3 above depth D)
-    int32_t CB0[kXBCap > 1 ? 125 : 1], CB1[kXBCap > kXBlkScreen ? 343 : kXBCap > 1 ? 125 : 1];
+    int32_t CB0[125], CB1[kXBCap > kXBlkScreen ? 343 : 125];
     int32_t NB[27], NBK[27], NBR[27];  // the root's neighbours, their child bases, their root numbers (group)
     float tmax[kMaxDepth + 1];         // brick_abs_bound: per depth, the largest |basis value|
     float xsum[kMaxDepth + 1];         // and the sum of |coefficients|
@@ -524,12 +516,6 @@ using BrickScreenLds = BrickCoreT<kXBlkScreen, kP, false>;
 // The super-brick screen's: 2x2x2 bricks, 17 grid coordinates per axis.
 constexpr int kPSuper = 2 * (1 << kBrickLog) + 1;
 using BrickSuperLds = BrickCoreT<kXBlkScreen, kPSuper, false>;
-
-// The vertex and triangle passes read the corner values the count pass
-// stored (the count pass keeps them over its blocks): no blocks.
-struct BrickMeshLds : BrickCoreT<1> {
-    float G[kBrickPts];  // f - iso at the brick's corners: (i, j, k) at (k kP + j) kP + i
-};
 
 __device__ __forceinline__ void decode_cell(uint32_t k, int32_t c[3]) {
     c[0] = int32_t(compact3(k >> 2));
@@ -580,12 +566,12 @@ __global__ void __launch_bounds__(kBlockS) k_brick_map(const int32_t* boff, cons
     bmap[b] = lo;
 }
 
-// Loads brick b's root record into LDS (with the chain's neighbour values
-// when kChain) and sets the brick's geometry.
+// Loads brick b's root record into LDS (its neighbours and its chain's
+// values) and sets the brick's geometry.
 // q_loaded: the root whose record S already holds (the previous brick's, in a
 // kernel that walks consecutive bricks), or -1.  up = 1 sets up the
 // super-brick of the 2x2x2 bricks that start at brick b.
-template <bool kChain, class L>
+template <class L>
 __device__ __forceinline__ void brick_setup(const SubArgs& A, int32_t b, Brick& B, L& S, int32_t q_loaded = -1,
                                             int up = 0) {
     const int D = A.D, lane = threadIdx.x;
@@ -601,10 +587,7 @@ __device__ __forceinline__ void brick_setup(const SubArgs& A, int32_t b, Brick& 
             else if (w < kRecNBR) S.NBK[w - kRecNBK] = v;
             else S.NBR[w - kRecNBR] = v;
         }
-        if constexpr (kChain) {
-            static_assert(sizeof(S.X) == (kMaxDepth + 1) * 27 * sizeof(float), "the layout holds the chain");
-            for (int w = lane; w < 27 * (B.r + 1); w += kWave) S.X[w] = __int_as_float(R[kRecX + w]);
-        }
+        for (int w = lane; w < 27 * (B.r + 1); w += kWave) S.X[w] = __int_as_float(R[kRecX + w]);
     }
     B.kb = brick_log(D, B.r) + up;  // up = 1: the 2x2x2 bricks from brick b (a multiple of 8 in the root)
     int32_t rc[3];
@@ -782,10 +765,12 @@ __device__ __forceinline__ float deep_sum_lds(const SubArgs& A, const Brick& B, 
 // corner of owner leaf o on sides s, in the reference's order: depth D up to
 // r + 1, neighbours j = 0..26 of the owner's virtual ancestor
 // (computeSubdivideVertexImplicitFunctionValue, main.cu:2346-2372).  R is the
-// owner's root at depth r; nb(j) its neighbour j and kids(j) that neighbour's
-// child base.
-template <class NbFn, class KidsFn>
-__device__ __forceinline__ float deep_sum(const SubArgs& A, int r, const int32_t R[3], const int32_t o[3], const int s[3], NbFn nb,
+// owner's root at depth r; kids(j) the child base of its neighbour j.  All 27
+// neighbours descend together, one level's loads in flight at once: walking
+// them one after another took a memory round trip per neighbour and level,
+// 0.4 ms for the one brick per wave that a small cloud leaves to evaluate.
+template <class KidsFn>
+__device__ __forceinline__ float deep_sum(const SubArgs& A, int r, const int32_t R[3], const int32_t o[3], const int s[3],
                           KidsFn kids) {
     const int D = A.D;
     float f = 0.0f;
@@ -803,25 +788,39 @@ __device__ __forceinline__ float deep_sum(const SubArgs& A, int r, const int32_t
         const float4 tz = A.btab[((int64_t(dd) << D) + o[2]) * 2 + s[2]];
         const float bx[3] = {tx.x, tx.y, tx.z}, by[3] = {ty.x, ty.y, ty.z}, bz[3] = {tz.x, tz.y, tz.z};
         const int32_t width = 1 << dd;
+        // the node of each neighbour, from the child base one level up; -1
+        // where it is outside the domain, inside the root (virtual), absent
+        // or below a coarse leaf
+        int32_t cur[27];
 #pragma unroll
         for (int k = 0; k < 27; k++) {
             const int32_t nx = ax + (k / 9 - 1), ny = ay + ((k / 3) % 3 - 1), nz = az + (k % 3 - 1);
-            if (nx < 0 || ny < 0 || nz < 0 || nx >= width || ny >= width || nz >= width) continue;
             const int cx = (nx >> up) - R[0], cy = (ny >> up) - R[1], cz = (nz >> up) - R[2];
-            if (!(cx | cy | cz)) continue;  // inside the root: virtual
-            const int jn = nidx(cx, cy, cz);
-            if (kids(jn) < 0) continue;  // absent, or a coarse leaf: no real node below
-            int32_t cur = nb(jn);
-            for (int l = r + 1; l <= dd && cur >= 0; l++) {
-                const int32_t cb = A.child_base[cur];
-                const int s2 = dd - l;
-                cur = cb < 0 ? -1 : cb + ((((nx >> s2) & 1) << 2) | (((ny >> s2) & 1) << 1) | ((nz >> s2) & 1));
+            const bool in = nx >= 0 && ny >= 0 && nz >= 0 && nx < width && ny < width && nz < width && (cx | cy | cz);
+            cur[k] = in ? kids(nidx(cx, cy, cz)) : -1;
+        }
+        for (int l = r + 1; l <= dd; l++) {
+            const int s2 = dd - l;
+#pragma unroll
+            for (int k = 0; k < 27; k++) {
+                const int32_t nx = ax + (k / 9 - 1), ny = ay + ((k / 3) % 3 - 1), nz = az + (k % 3 - 1);
+                const int oct = (((nx >> s2) & 1) << 2) | (((ny >> s2) & 1) << 1) | ((nz >> s2) & 1);
+                cur[k] = cur[k] < 0 ? -1 : cur[k] + oct;
             }
-            if (cur < 0) continue;
-            float tt = A.x[cur] * bx[k / 9];
+            if (l < dd) {
+#pragma unroll
+                for (int k = 0; k < 27; k++) cur[k] = cur[k] < 0 ? -1 : A.child_base[cur[k]];
+            }
+        }
+        float xv[27];
+#pragma unroll
+        for (int k = 0; k < 27; k++) xv[k] = cur[k] < 0 ? 0.0f : A.x[cur[k]];
+#pragma unroll
+        for (int k = 0; k < 27; k++) {
+            float tt = xv[k] * bx[k / 9];
             tt = tt * by[(k / 3) % 3];
             tt = tt * bz[k % 3];
-            f = f + tt;
+            f = cur[k] < 0 ? f : f + tt;
         }
     }
     return f;
@@ -907,8 +906,7 @@ __device__ __forceinline__ float grid_value(const SubArgs& A, const Brick& B, co
     // the corner basis table
     const int32_t* R2 = A.rec + int64_t(S.NBR[slot]) * kRecWords;
     const int32_t RC[3] = {B.R[0] + slot / 9 - 1, B.R[1] + (slot / 3) % 3 - 1, B.R[2] + slot % 3 - 1};
-    float f = deep_sum(
-        A, B.r, RC, o, side, [&](int j) { return R2[kRecNB + j]; }, [&](int j) { return R2[kRecNBK + j]; });
+    float f = deep_sum(A, B.r, RC, o, side, [&](int j) { return R2[kRecNBK + j]; });
     for (int d = B.r; d >= 1; d--) {
         const float4 tx = A.btab[((int64_t(d) << D) + o[0]) * 2 + side[0]];
         const float4 ty = A.btab[((int64_t(d) << D) + o[1]) * 2 + side[1]];
@@ -930,47 +928,7 @@ __device__ __forceinline__ float grid_value(const SubArgs& A, const Brick& B, co
     return f + tt - *A.iso;
 }
 
-// The brick's corner values (grid_value; 0 at the points a smaller brick
-// does not have), stored over its blocks, which nothing reads once the values
-// are known: each lane holds its values in registers until every lane's
-// block reads are done.  The blocks' LDS is then the corner values' (G), so
-// the evaluation needs no LDS beyond the certificate's.  The values also go
-// to gv (kBrickPts floats).
 constexpr int kValRounds = (kBrickPts + kWave - 1) / kWave;
-
-template <class L>
-__device__ __forceinline__ float* brick_values(const SubArgs& A, const Brick& B, L& S, float* gv) {
-    static_assert(sizeof(S.XB) >= kBrickPts * sizeof(float), "the corner values fit over the blocks");
-    const int P = (1 << B.kb) + 1;
-    float held[kValRounds];
-#pragma unroll
-    for (int t = 0; t < kValRounds; t++) held[t] = 0.0f;
-    for (int t = 0; t < kValRounds; t++) {
-        const int p = threadIdx.x + kWave * t;
-        const int i = p % kP, j = (p / kP) % kP, k = p / (kP * kP);
-        float v = 0.0f;
-        if (p < kBrickPts && i < P && j < P && k < P) {
-            const int32_t g[3] = {B.org[0] + i, B.org[1] + j, B.org[2] + k};
-            v = grid_value(A, B, S, g);
-        }
-        // (a register queue: constant indices keep held out of scratch memory)
-#pragma unroll
-        for (int q = 0; q + 1 < kValRounds; q++) held[q] = held[q + 1];
-        held[kValRounds - 1] = v;
-    }
-    __syncthreads();  // the blocks' last reads
-    float* G = S.XB;
-#pragma unroll
-    for (int t = 0; t < kValRounds; t++) {
-        const int p = threadIdx.x + kWave * t;
-        if (p < kBrickPts) {
-            G[p] = held[t];
-            gv[p] = held[t];
-        }
-    }
-    __syncthreads();
-    return G;
-}
 
 // Owner of edge e of leaf v among the virtual leaves sharing it
 // (initSubdivideEdgeArray, main.cu:1867-2019): its cell and the edge kind seen
@@ -1040,22 +998,6 @@ __device__ __forceinline__ void leaf_cube(const Brick& B, const L& S, const floa
         if (own) m |= 1 << e;
     }
     *emask = m;
-}
-
-__device__ __forceinline__ int wave_sum(int v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-    return v;
-}
-
-__device__ __forceinline__ int wave_excl_scan(int v) {
-    int inc = v;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-        const int t = __shfl_up(inc, o, kWave);
-        if (int(threadIdx.x) >= o) inc += t;
-    }
-    return inc - v;
 }
 
 // The separable contraction of one depth's coefficients over z and y for
@@ -1572,22 +1514,22 @@ __global__ void __launch_bounds__(kWave, 5) k_brick_screen_super(SubArgs A, cons
     __shared__ BrickSuperLds S;
     const int lane = threadIdx.x;
     const int32_t ns = cnt[kCntSuper];
-    constexpr int kChunk = 8;
+    const int32_t chunk = std::max(1, std::min(8, ns / (2 * int32_t(gridDim.x))));
     int32_t q_loaded = -1, sb = 0, s_end = 0;
     for (;;) {
         if (sb == s_end) {
             int32_t c0 = 0;
-            if (lane == 0) c0 = atomicAdd(cnt + kCntWork, kChunk);
+            if (lane == 0) c0 = atomicAdd(cnt + kCntWork, chunk);
             c0 = __shfl(c0, 0, kWave);
             if (c0 >= ns) break;
             sb = c0;
-            s_end = std::min(ns, c0 + kChunk);
+            s_end = std::min(ns, c0 + chunk);
         }
         const int32_t q = smap[sb];
         const int32_t b0 = A.boff[q] + 8 * (sb - soff[q]);
         Brick B;
         __syncthreads();  // the previous super-brick's LDS reads are done
-        brick_setup<true>(A, b0, B, S, q_loaded, 1);
+        brick_setup(A, b0, B, S, q_loaded, 1);
         q_loaded = B.q;
         int sgn = 0;
         if (certify && !brick_in_group(B, S) && brick_blocks(A, B, S))
@@ -1653,22 +1595,25 @@ __global__ void __launch_bounds__(kWave, 5) k_brick_screen(SubArgs A, const int3
                                                         int32_t* dpairs, int32_t* cnt, int certify) {
     __shared__ BrickScreenLds S;
     const int lane = threadIdx.x;
-    const int32_t nl = cnt[kCntList2Sorted];
-    constexpr int kChunk = 16;  // consecutive entries per grab: mostly one root, whose record stays in LDS
+    const int32_t nl = cnt[kCntList2];
+    // consecutive entries per grab (mostly one root, whose record stays in LDS):
+    // up to 16, at least about four grabs per workgroup (13,000 bricks in
+    // chunks of 16 kept 815 of 5,120 waves busy for 510 us)
+    const int32_t chunk = std::max(1, std::min(16, nl / (4 * int32_t(gridDim.x))));
     int32_t q_loaded = -1, it = 0, it_end = 0;
     for (;;) {
         if (it == it_end) {
             int32_t c0 = 0;
-            if (lane == 0) c0 = atomicAdd(cnt + kCntWork2, kChunk);
+            if (lane == 0) c0 = atomicAdd(cnt + kCntWork2, chunk);
             c0 = __shfl(c0, 0, kWave);
             if (c0 >= nl) break;
             it = c0;
-            it_end = std::min(nl, c0 + kChunk);
+            it_end = std::min(nl, c0 + chunk);
         }
         const int32_t b = list2[it];
         Brick B;
         __syncthreads();  // the previous brick's LDS reads are done
-        brick_setup<true>(A, b, B, S, q_loaded);
+        brick_setup(A, b, B, S, q_loaded);
         q_loaded = B.q;
         Certificate c;
         c.sign = 0;
@@ -1686,16 +1631,15 @@ __global__ void __launch_bounds__(kWave, 5) k_brick_screen(SubArgs A, const int3
 // Pass 0b: the exact certificate (brick_certify) for the bricks the interval
 // left (a fixed grid walks the list); the bricks it does not certify are
 // listed for the evaluation.
-// The list is in brick order (root-major), and a resident grid takes chunks
-// of consecutive entries from a counter, so consecutive bricks mostly share
-// their root and its record stays in LDS.  Compiled for three waves per SIMD
-// (168 VGPRs, a few spilled; the LDS allows eleven workgroups per CU): the
-// waves wait on memory about half their time, and two per SIMD hid less.
+// A resident grid takes chunks of consecutive entries from a counter; entries
+// of one root often follow each other, and its record then stays in LDS.
+// Compiled for three waves per SIMD (168 VGPRs, a few spilled): the waves wait
+// on memory about half their time, and two per SIMD hid less.
 __global__ void __launch_bounds__(kWave, 3) k_brick_exact(SubArgs A, const int32_t* xlist, int8_t* sign, int32_t* list,
                                                        int32_t* dbricks, int32_t* dpairs, int32_t* cnt, int certify) {
     __shared__ BrickCore S;
     const int lane = threadIdx.x;
-    const int32_t n = cnt[kCntExactSorted];
+    const int32_t n = cnt[kCntExact];
     // chunks of up to 8 entries, at least about four per workgroup
     const int32_t chunk = std::max(1, std::min(8, n / (4 * int32_t(gridDim.x))));
     int32_t q_loaded = -1, it = 0, it_end = 0;
@@ -1711,7 +1655,7 @@ __global__ void __launch_bounds__(kWave, 3) k_brick_exact(SubArgs A, const int32
         const int32_t b = xlist[it++];
         Brick B;
         __syncthreads();  // the previous brick's LDS reads are done
-        brick_setup<true>(A, b, B, S, q_loaded);
+        brick_setup(A, b, B, S, q_loaded);
         q_loaded = B.q;
         brick_tables(A, B, S);
         brick_blocks(A, B, S);
@@ -1740,76 +1684,26 @@ __global__ void __launch_bounds__(kBlockS) k_brick_deps(const int32_t* dbricks, 
     if (!ok) list[atomicAdd(cnt + kCntDense, 1)] = b;
 }
 
-// Pass 1: vertex and triangle counts of the bricks the certificate left
-// (a fixed grid walks the list).
-// The corner values go to gvals (kBrickPts per listed brick) and the
-// brick's place in the list to didx, for the vertex pass; in LDS they take
-// the place of the blocks (brick_values), so the pass needs the
-// certificate's LDS only.
-// The list is in brick order and a resident grid takes chunks of consecutive
-// entries from a counter (kCntWork4), so the root's record mostly stays in LDS.
-__global__ void __launch_bounds__(kWave) k_brick_count(SubArgs A, const int32_t* list, int32_t* cnt,
-                                                       int32_t* bnv, int32_t* bnt, float* gvals, int32_t* didx) {
+// The corner values of the bricks the certificates left (grid_value): gv at
+// kBrickPts per listed brick.  `slices` waves share a brick's rounds of 64
+// points (each sets up the brick's tables and blocks itself): a list shorter
+// than the chip's waves leaves each of them a part of a brick's serial chain
+// of loads and sums instead of all of it (921 bricks, 35,947 points at depth
+// 8: 401 us one wave per brick).
+__global__ void __launch_bounds__(kWave) k_brick_values(SubArgs A, const int32_t* list, int slices, float* gv) {
     __shared__ BrickCore S;
-    const int32_t n = cnt[kCntDenseSorted];
-    // chunks of up to 8 entries, at least about four per workgroup (a short
-    // list in long chunks leaves some workgroups with twice the others' work)
-    const int32_t chunk = std::max(1, std::min(8, n / (4 * int32_t(gridDim.x))));
-    int32_t q_loaded = -1, it = 0, it_end = 0;
-    for (;;) {
-        if (it == it_end) {
-            int32_t c0 = 0;
-            if (threadIdx.x == 0) c0 = atomicAdd(cnt + kCntWork4, chunk);
-            c0 = __shfl(c0, 0, kWave);
-            if (c0 >= n) break;
-            it = c0;
-            it_end = std::min(n, c0 + chunk);
-        }
-        Brick B;
-        const int32_t b = list[it];
-        __syncthreads();  // the previous brick's LDS reads are done
-        brick_setup<true>(A, b, B, S, q_loaded);
-        q_loaded = B.q;
-        brick_tables(A, B, S);
-        brick_blocks(A, B, S);
-        const float* G = brick_values(A, B, S, gvals + int64_t(it) * kBrickPts);
-        if (threadIdx.x == 0) didx[b] = it;
-        int nv = 0, nt = 0;
-        const int L = 1 << (3 * B.kb);
-        for (int l = threadIdx.x; l < L; l += kWave) {
-            int32_t v[3];
-            float cv[8];
-            int cube, em;
-            leaf_cube(B, S, G, A.D, l, v, cv, &cube, &em);
-            nv += __popc(uint32_t(em));
-            nt += tri_count(cube);
-        }
-        nv = wave_sum(nv);
-        nt = wave_sum(nt);
-        if (threadIdx.x == 0) {
-            bnv[b] = nv;
-            bnt[b] = nt;
-        }
-        it++;
-    }
-}
-
-// (sign 2: a small root's brick, whose tables are its own)
-__global__ void __launch_bounds__(kBlockS) k_brick_active(const int32_t* bnv, const int32_t* bnt, const int8_t* sign,
-                                                          int64_t n, int32_t* flag) {
-    const int64_t i = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
-    if (i < n) flag[i] = ((bnv[i] | bnt[i]) && sign[i] != 2) ? 1 : 0;
-}
-
-__global__ void __launch_bounds__(kBlockS) k_brick_compact(const int32_t* flag, const int32_t* off, int64_t n,
-                                                           int32_t* alist, int32_t* amap) {
-    const int64_t i = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
-    if (i >= n) return;
-    if (flag[i]) {
-        alist[off[i]] = int32_t(i);
-        amap[i] = off[i];
-    } else {
-        amap[i] = -1;
+    const int32_t it = int32_t(blockIdx.x) / slices;
+    const int slice = int(blockIdx.x) % slices, per = (kValRounds + slices - 1) / slices;
+    Brick B;
+    brick_setup(A, list[it], B, S);
+    brick_tables(A, B, S);
+    brick_blocks(A, B, S);
+    float* out = gv + int64_t(it) * kBrickPts;
+    for (int t = slice * per; t < std::min(kValRounds, slice * per + per); t++) {
+        const int p = threadIdx.x + kWave * t;
+        if (p >= kBrickPts) break;
+        const int32_t g[3] = {B.org[0] + p % kP, B.org[1] + (p / kP) % kP, B.org[2] + p / (kP * kP)};
+        out[p] = grid_value(A, B, S, g);
     }
 }
 
@@ -1870,93 +1764,158 @@ __device__ __forceinline__ int32_t edge_vertex_place(const Brick& B, const L& S,
     return sl == 13 ? B.q : root_of_slot(sl);
 }
 
-// Pass 2 (bricks with output): per-leaf edge masks, cube indices and vertex
-// offsets into the brick's tables; the vertices (interpolatePoint and
-// generateSubdivideIntersectionPoint, main.cu:2584-2597, 2629-2697).
-__global__ void __launch_bounds__(kWave) k_brick_vertices(SubArgs A, const int32_t* alist, const int32_t* bvoff,
-                                                          uint16_t* lofs_tab, uint16_t* emask_tab, uint8_t* cube_tab,
-                                                          const float* gvals, const int32_t* didx, float* out_v) {
-    __shared__ BrickMeshLds S;
+// Per-leaf tables (the evaluated bricks': place in the list x 512 + leaf; the
+// small roots': place x leaves + leaf): owned crossing edges, first vertex
+// within the brick, cube index.
+struct LeafTabs {
+    uint16_t* emask;
+    uint16_t* lofs;
+    uint8_t* cube;
+};
+
+// The group's roots around a root as a bit mask, for the owner tests (which
+// only ask whether a neighbour is in the group).
+struct GroupMask {
+    struct {
+        uint32_t m;
+        __device__ __forceinline__ int32_t operator[](int j) const { return ((m >> j) & 1u) ? 0 : -1; }
+    } NBR;
+};
+
+// An 8^3 brick's geometry and group, for the leaf passes (one thread per
+// leaf, every wave for itself).
+__device__ __forceinline__ void brick_geometry(const SubArgs& A, int32_t b, Brick& B, GroupMask& S) {
+    const int D = A.D, lane = threadIdx.x & 63;
+    B.q = __builtin_amdgcn_readfirstlane(A.bmap[b]);
+    const int32_t* R = A.rec + int64_t(B.q) * kRecWords;
+    B.r = __builtin_amdgcn_readfirstlane(R[kRecR]);
+    const uint32_t rkey = uint32_t(__builtin_amdgcn_readfirstlane(R[kRecKey]));
+    B.kb = kBrickLog;
+    B.Sr = 1 << (D - B.r);
+    B.bkey = rkey | (uint32_t(b - A.boff[B.q]) << (3 * kBrickLog));
+    int32_t rc[3];
+    decode_cell(rkey, rc);
+    decode_cell(B.bkey, B.org);
+    for (int a = 0; a < 3; a++) {
+        B.R[a] = rc[a] >> (D - B.r);
+        B.R0[a] = rc[a];
+    }
+    S.NBR.m = uint32_t(__builtin_amdgcn_ballot_w64(lane < 27 && R[kRecNBR + (lane < 27 ? lane : 0)] >= 0));
+}
+
+// Exclusive sum of v over the workgroup's 512 threads, and the total.
+__device__ __forceinline__ int block_excl_scan(int v, int* total) {
+    __shared__ int sums[kBrickLeaves / kWave];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int inc = v;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const int t = __shfl_up(inc, o, kWave);
+        if (lane >= o) inc += t;
+    }
+    __syncthreads();
+    if (lane == kWave - 1) sums[wave] = inc;
+    __syncthreads();
+    int base = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < kBrickLeaves / kWave; w++) {
+        if (w < wave) base += sums[w];
+        all += sums[w];
+    }
+    *total = all;
+    return base + inc - v;
+}
+
+// Cube indices and owned crossing edges of the evaluated bricks' leaves, the
+// bricks' vertex and triangle counts, and their places in the list (didx).
+__global__ void __launch_bounds__(kBrickLeaves) k_brick_cubes(SubArgs A, const int32_t* list, const float* gv,
+                                                              LeafTabs T, int32_t* bnv, int32_t* bnt, int32_t* didx) {
+    __shared__ float G[kBrickPts];
+    const int32_t it = blockIdx.x, b = list[it], l = threadIdx.x;
+    for (int p = l; p < kBrickPts; p += kBrickLeaves) G[p] = gv[int64_t(it) * kBrickPts + p];
     Brick B;
-    const int32_t ai = blockIdx.x;
-    const int32_t b = alist[ai];
-    brick_setup<false>(A, b, B, S);
-    {  // the corner values the count pass computed
-        const float* G = gvals + int64_t(didx[b]) * kBrickPts;
-        for (int p = threadIdx.x; p < kBrickPts; p += kWave) S.G[p] = G[p];
-        __syncthreads();
-    }
-    const int D = A.D;
-    const int L = 1 << (3 * B.kb);
-    const int per = (L + kWave - 1) / kWave;
-    const int l0 = min(L, int(threadIdx.x) * per), l1 = min(L, l0 + per);
-    int cnt = 0;
-    for (int l = l0; l < l1; l++) {
-        int32_t v[3];
-        float cv[8];
-        int cube, em;
-        leaf_cube(B, S, S.G, D, l, v, cv, &cube, &em);
-        emask_tab[int64_t(ai) * kBrickLeaves + l] = uint16_t(em);
-        cube_tab[int64_t(ai) * kBrickLeaves + l] = uint8_t(cube);
-        cnt += __popc(uint32_t(em));
-    }
-    int run = wave_excl_scan(cnt);
-    for (int l = l0; l < l1; l++) {
-        lofs_tab[int64_t(ai) * kBrickLeaves + l] = uint16_t(run);
-        const int em = emask_tab[int64_t(ai) * kBrickLeaves + l];
-        if (!em) continue;
-        int32_t v[3];
-        float cv[8];
-        int cube, em2;
-        leaf_cube(B, S, S.G, D, l, v, cv, &cube, &em2);
-        run += emit_leaf_vertices(B.bkey | uint32_t(l), D, em, cv, out_v + 3 * (int64_t(bvoff[b]) + run));
+    GroupMask S;
+    brick_geometry(A, b, B, S);
+    __syncthreads();
+    int32_t v[3];
+    float cv[8];
+    int cube, em;
+    leaf_cube(B, S, G, A.D, l, v, cv, &cube, &em);
+    int nv, nt;
+    const int ofs = block_excl_scan(__popc(uint32_t(em)), &nv);
+    (void)block_excl_scan(tri_count(cube), &nt);
+    const int64_t at = int64_t(it) * kBrickLeaves + l;
+    T.emask[at] = uint16_t(em);
+    T.lofs[at] = uint16_t(ofs);
+    T.cube[at] = uint8_t(cube);
+    if (l == 0) {
+        bnv[b] = nv;
+        bnt[b] = nt;
+        didx[b] = it;
     }
 }
 
-// Pass 3 (bricks with output): triangle entries (generateSubdivideTrianglePos,
+// The vertices of the evaluated bricks.
+__global__ void __launch_bounds__(kBrickLeaves) k_brick_vertices(SubArgs A, const int32_t* list, const float* gv,
+                                                                 LeafTabs T, const int32_t* bnv, const int32_t* bvoff,
+                                                                 float* out_v) {
+    __shared__ float G[kBrickPts];
+    const int32_t it = blockIdx.x, b = list[it], l = threadIdx.x;
+    if (bnv[b] == 0) return;
+    for (int p = l; p < kBrickPts; p += kBrickLeaves) G[p] = gv[int64_t(it) * kBrickPts + p];
+    __syncthreads();
+    const int64_t at = int64_t(it) * kBrickLeaves + l;
+    const int em = T.emask[at];
+    if (!em) return;
+    const int32_t q = A.bmap[b];
+    const uint32_t key = uint32_t(A.rec[int64_t(q) * kRecWords + kRecKey]) |
+                         (uint32_t(b - A.boff[q]) << (3 * kBrickLog)) | uint32_t(l);
+    const int lx = int(compact3(uint32_t(l) >> 2)), ly = int(compact3(uint32_t(l) >> 1)), lz = int(compact3(uint32_t(l)));
+    float cv[8];
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+        const int y = (c >> 1) & 1, xx = (c & 1) ^ y, z = c >> 2;
+        cv[c] = G[((lz + z) * kP + (ly + y)) * kP + (lx + xx)];
+    }
+    emit_leaf_vertices(key, A.D, em, cv, out_v + 3 * (int64_t(bvoff[b]) + T.lofs[at]));
+}
+
+// Triangle entries of the evaluated bricks (generateSubdivideTrianglePos,
 // main.cu:2759-2825).  A vertex owned by a leaf of another brick (of this
 // root or of another root of the group) is found through that brick's tables.
-__global__ void __launch_bounds__(kWave) k_brick_triangles(SubArgs A, const int32_t* alist, const int32_t* amap,
-                                                           const int32_t* bvoff, const int32_t* btoff,
-                                                           const uint16_t* lofs_tab, const uint16_t* emask_tab,
-                                                           const uint8_t* cube_tab, int64_t vbase, int32_t* out_t,
-                                                           int32_t* err) {
-    __shared__ BrickCoreT<1> S;  // the root's neighbours only
+__global__ void __launch_bounds__(kBrickLeaves) k_brick_triangles(SubArgs A, const int32_t* list, const int32_t* didx,
+                                                                  LeafTabs T, const int32_t* bnt, const int32_t* bvoff,
+                                                                  const int32_t* btoff, int64_t vbase, int32_t* out_t,
+                                                                  int32_t* err) {
+    const int32_t it = blockIdx.x, b = list[it], l = threadIdx.x;
+    if (bnt[b] == 0) return;
     Brick B;
-    const int32_t ai = blockIdx.x;
-    const int32_t b = alist[ai];
-    brick_setup<false>(A, b, B, S);
-    const int D = A.D;
-    const int L = 1 << (3 * B.kb);
-    const int per = (L + kWave - 1) / kWave;
-    const int l0 = min(L, int(threadIdx.x) * per), l1 = min(L, l0 + per);
-    int cnt = 0;
-    for (int l = l0; l < l1; l++) cnt += tri_count(cube_tab[int64_t(ai) * kBrickLeaves + l]);
-    int64_t o = 3 * (int64_t(btoff[b]) + wave_excl_scan(cnt));
-    for (int l = l0; l < l1; l++) {
-        const int cube = cube_tab[int64_t(ai) * kBrickLeaves + l];
-        const int n = 3 * tri_count(cube);
-        if (!n) continue;
-        const int32_t v[3] = {B.org[0] + int32_t(compact3(uint32_t(l) >> 2)),
-                              B.org[1] + int32_t(compact3(uint32_t(l) >> 1)), B.org[2] + int32_t(compact3(uint32_t(l)))};
-        for (int k = 0; k < n; k++) {
-            uint32_t mort;
-            int eo;
-            const int32_t q2 =
-                edge_vertex_place(B, S, D, v, c_tri[cube][k], [&](int j) { return S.NBR[j]; }, &mort, &eo);
-            const int32_t bi = q2 < 0 ? 0 : A.boff[q2] + int32_t(mort >> (3 * B.kb));
-            const int32_t lu = int32_t(mort & ((1u << (3 * B.kb)) - 1u));
-            const int32_t au = q2 < 0 ? -1 : amap[bi];
-            int32_t id = 0;
-            if (au < 0) {
-                err[0] = 1;  // a crossing edge whose owner brick has no output: inconsistent counts
-            } else {
-                const int64_t t = int64_t(au) * kBrickLeaves + lu;
-                id = int32_t(vbase + bvoff[bi] + lofs_tab[t] + __popc(uint32_t(emask_tab[t]) & ((1u << eo) - 1u)));
-            }
-            out_t[o + k] = id;
+    GroupMask S;
+    brick_geometry(A, b, B, S);
+    const int cube = T.cube[int64_t(it) * kBrickLeaves + l];
+    const int nt = tri_count(cube);
+    int total;
+    const int first = block_excl_scan(nt, &total);
+    if (!nt) return;
+    int32_t* out = out_t + 3 * (int64_t(btoff[b]) + first);
+    const int32_t v[3] = {B.org[0] + int32_t(compact3(uint32_t(l) >> 2)), B.org[1] + int32_t(compact3(uint32_t(l) >> 1)),
+                          B.org[2] + int32_t(compact3(uint32_t(l)))};
+    const int32_t* NBR = A.rec + int64_t(B.q) * kRecWords + kRecNBR;
+    for (int k = 0; k < 3 * nt; k++) {
+        uint32_t mort;
+        int eo;
+        const int32_t q2 = edge_vertex_place(B, S, A.D, v, c_tri[cube][k], [&](int j) { return NBR[j]; }, &mort, &eo);
+        const int32_t b2 = q2 < 0 ? 0 : A.boff[q2] + int32_t(mort >> (3 * kBrickLog));
+        const int32_t at = q2 < 0 ? -1 : didx[b2];
+        const int64_t t = at < 0 ? 0 : int64_t(at) * kBrickLeaves + (mort & (kBrickLeaves - 1));
+        const uint32_t em = at < 0 ? 0 : T.emask[t];
+        int32_t id = 0;
+        if (!((em >> eo) & 1u)) {
+            err[0] = 1;  // a crossing edge whose owner has no vertex on it: inconsistent counts
+        } else {
+            id = int32_t(vbase + bvoff[b2] + T.lofs[t] + __popc(em & ((1u << eo) - 1u)));
         }
-        o += n;
+        out[k] = id;
     }
 }
 
@@ -2141,15 +2100,6 @@ __global__ void __launch_bounds__(kWave) k_small_values(SubArgs A, const int32_t
     }
 }
 
-// The group's roots around a small root as a bit mask, for the owner tests
-// (which only ask whether a neighbour is in the group).
-struct GroupMask {
-    struct {
-        uint32_t m;
-        __device__ __forceinline__ int32_t operator[](int j) const { return ((m >> j) & 1u) ? 0 : -1; }
-    } NBR;
-};
-
 // The leaf passes' lanes: kLeafRoots roots to a wave, one leaf per lane.  Sets
 // the lane's root geometry and group.
 template <int KB>
@@ -2181,14 +2131,6 @@ __device__ __forceinline__ int leaf_excl_scan(int v, int* total) {
     return inc - v;
 }
 
-// Per-leaf tables of the small roots (slot kLeaves + leaf): owned crossing
-// edges, cube index, first vertex within the root.
-struct SmallTabs {
-    uint16_t* emask;
-    uint16_t* lofs;
-    uint8_t* cube;
-};
-
 // The corner values of the wave's roots into LDS.
 template <int KB>
 __device__ __forceinline__ void small_corner_values(int32_t s0, int32_t ns, const float* gv, const int32_t* gref,
@@ -2205,8 +2147,7 @@ __device__ __forceinline__ void small_corner_values(int32_t s0, int32_t ns, cons
 // root's vertex and triangle counts.
 template <int KB>
 __global__ void __launch_bounds__(kWave) k_small_cubes(SubArgs A, const int32_t* slist, int32_t ns, const float* gv,
-                                                       const int32_t* gref, SmallTabs T, int32_t* bnv, int32_t* bnt,
-                                                       int8_t* sign) {
+                                                       const int32_t* gref, LeafTabs T, int32_t* bnv, int32_t* bnt) {
     using C = SmallRoots<KB>;
     constexpr int LV = C::kLeaves;
     __shared__ float G[C::kLeafRoots * C::kPts];
@@ -2234,13 +2175,12 @@ __global__ void __launch_bounds__(kWave) k_small_cubes(SubArgs A, const int32_t*
         const int32_t b = A.boff[q];
         bnv[b] = nv;
         bnt[b] = nt;
-        sign[b] = 2;
     }
 }
 
 template <int KB>
 __global__ void __launch_bounds__(kWave) k_small_vertices(SubArgs A, const int32_t* slist, int32_t ns, const float* gv,
-                                                          const int32_t* gref, SmallTabs T, const int32_t* bvoff,
+                                                          const int32_t* gref, LeafTabs T, const int32_t* bvoff,
                                                           float* out_v) {
     using C = SmallRoots<KB>;
     constexpr int LV = C::kLeaves, P = C::kPts1;
@@ -2267,7 +2207,7 @@ __global__ void __launch_bounds__(kWave) k_small_vertices(SubArgs A, const int32
 
 template <int KB>
 __global__ void __launch_bounds__(kWave) k_small_triangles(SubArgs A, const int32_t* slist, int32_t ns,
-                                                           const int32_t* sidx, SmallTabs T, const int32_t* bvoff,
+                                                           const int32_t* sidx, LeafTabs T, const int32_t* bvoff,
                                                            const int32_t* btoff, int64_t vbase, int32_t* out_t,
                                                            int32_t* err) {
     using C = SmallRoots<KB>;
@@ -2449,16 +2389,11 @@ void extract_subdivision(prg_ctx* c) {
     PRG_CHECK_LAUNCH();
 
     // pass 1: counts per brick
-    PoolBuf<int32_t> bnv{&c->pool[116]}, bnt{&c->pool[117]}, bvoff{&c->pool[118]}, btoff{&c->pool[119]},
-        aflag{&c->pool[120]}, aoff{&c->pool[121]}, alist{&c->pool[122]}, amap{&c->pool[123]};
+    PoolBuf<int32_t> bnv{&c->pool[116]}, bnt{&c->pool[117]}, bvoff{&c->pool[118]}, btoff{&c->pool[119]};
     bnv.reserve(nb);
     bnt.reserve(nb);
     bvoff.reserve(nb);
     btoff.reserve(nb);
-    aflag.reserve(nb);
-    aoff.reserve(nb);
-    alist.reserve(nb);
-    amap.reserve(nb);
     // pass 0: certificates; pass 1: counts of the bricks left
     PoolBuf<int32_t> dlist{&c->pool[129]}, dbricks{&c->pool[130]}, dpairs{&c->pool[131]}, xlist{&c->pool[133]};
     PoolBuf<int8_t> bsign{&c->pool[132]};
@@ -2482,8 +2417,8 @@ void extract_subdivision(prg_ctx* c) {
     semask.reserve(tabn);
     slofs.reserve(tabn);
     scube.reserve(tabn);
-    const SmallTabs T1{semask.get(), slofs.get(), scube.get()};
-    const SmallTabs T2{semask.get() + tab2, slofs.get() + tab2, scube.get() + tab2};
+    const LeafTabs T1{semask.get(), slofs.get(), scube.get()};
+    const LeafTabs T2{semask.get() + tab2, slofs.get() + tab2, scube.get() + tab2};
     const unsigned lw1 = grid_for(n1, Small1::kLeafRoots), lw2 = grid_for(n2, Small2::kLeafRoots);
     {
         TimedScope ts(kt, "subdivide_small_values", 0.0);  // issue-bound: no byte figure
@@ -2494,7 +2429,7 @@ void extract_subdivision(prg_ctx* c) {
                                                                                gv1.get(), gref1.get());
             PRG_CHECK_LAUNCH();
             k_small_cubes<1><<<lw1, kWave, 0, s>>>(A, slist1.get(), n1, gv1.get(), gref1.get(), T1, bnv.get(),
-                                                   bnt.get(), bsign.get());
+                                                   bnt.get());
             PRG_CHECK_LAUNCH();
         }
         if (n2) {
@@ -2504,7 +2439,7 @@ void extract_subdivision(prg_ctx* c) {
                                                                                gv2.get(), gref2.get());
             PRG_CHECK_LAUNCH();
             k_small_cubes<2><<<lw2, kWave, 0, s>>>(A, slist2.get(), n2, gv2.get(), gref2.get(), T2, bnv.get(),
-                                                   bnt.get(), bsign.get());
+                                                   bnt.get());
             PRG_CHECK_LAUNCH();
         }
     }
@@ -2534,44 +2469,18 @@ void extract_subdivision(prg_ctx* c) {
         k_brick_screen_super<<<unsigned(grid), kWave, 0, s>>>(A, smap.get(), soff.get(), bnv.get(), bnt.get(),
                                                               bsign.get(), list2.get(), C, int(c->sub_certify));
         PRG_CHECK_LAUNCH();
-        // the lists the passes append to, each put in brick order (marks,
-        // scan, compact) before the next pass walks it
-        PoolBuf<int32_t> xmark{&c->pool[141]}, xoff{&c->pool[142]}, xsorted{&c->pool[143]};
-        xmark.reserve(nb);
-        xoff.reserve(nb);
-        xsorted.reserve(nb);
-        PRG_HIP(hipMemsetAsync(xmark.get(), 0, size_t(nb) * 4, s));
-        k_mark_listed<<<grid_for(nb, kBlockS), kBlockS, 0, s>>>(list2.get(), C + kCntList2, nb, xmark.get());
-        PRG_CHECK_LAUNCH();
-        scan_exclusive(xmark.get(), xoff.get(), nb, C + kCntList2Sorted, s, c->scratch, kt);
-        k_compact<<<grid_for(nb, kBlockS), kBlockS, 0, s>>>(xmark.get(), xoff.get(), nb, list2.get());
-        PRG_CHECK_LAUNCH();
         PRG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_brick_screen, kWave, 0));
         grid = std::min<int64_t>(nb, int64_t(std::max(1, per_cu)) * std::max(1, c->num_cu));
         k_brick_screen<<<unsigned(grid), kWave, 0, s>>>(A, list2.get(), bnv.get(), bnt.get(), bsign.get(), xlist.get(),
                                                         dbricks.get(), dpairs.get(), C, int(c->sub_certify));
         PRG_CHECK_LAUNCH();
-        // the exact certificate's list
-        PRG_HIP(hipMemsetAsync(xmark.get(), 0, size_t(nb) * 4, s));
-        k_mark_listed<<<grid_for(nb, kBlockS), kBlockS, 0, s>>>(xlist.get(), C + kCntExact, nb, xmark.get());
-        PRG_CHECK_LAUNCH();
-        scan_exclusive(xmark.get(), xoff.get(), nb, C + kCntExactSorted, s, c->scratch, kt);
-        k_compact<<<grid_for(nb, kBlockS), kBlockS, 0, s>>>(xmark.get(), xoff.get(), nb, xsorted.get());
-        PRG_CHECK_LAUNCH();
         PRG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_brick_exact, kWave, 0));
         grid = std::min<int64_t>(nb, int64_t(std::max(1, per_cu)) * std::max(1, c->num_cu));
-        k_brick_exact<<<unsigned(grid), kWave, 0, s>>>(A, xsorted.get(), bsign.get(), dlist.get(), dbricks.get(),
+        k_brick_exact<<<unsigned(grid), kWave, 0, s>>>(A, xlist.get(), bsign.get(), dlist.get(), dbricks.get(),
                                                        dpairs.get(), C, int(c->sub_certify));
         PRG_CHECK_LAUNCH();
         k_brick_deps<<<grid_for(nb, kBlockS), kBlockS, 0, s>>>(dbricks.get(), dpairs.get(), bsign.get(),
                                                                 dlist.get(), C);
-        PRG_CHECK_LAUNCH();
-        // the evaluation's list in brick order, in place of the unordered one
-        PRG_HIP(hipMemsetAsync(xmark.get(), 0, size_t(nb) * 4, s));
-        k_mark_listed<<<grid_for(nb, kBlockS), kBlockS, 0, s>>>(dlist.get(), C + kCntDense, nb, xmark.get());
-        PRG_CHECK_LAUNCH();
-        scan_exclusive(xmark.get(), xoff.get(), nb, C + kCntDenseSorted, s, c->scratch, kt);
-        k_compact<<<grid_for(nb, kBlockS), kBlockS, 0, s>>>(xmark.get(), xoff.get(), nb, dlist.get());
         PRG_CHECK_LAUNCH();
     }
     if (nb3 > 0) {
@@ -2581,42 +2490,43 @@ void extract_subdivision(prg_ctx* c) {
     const int64_t ndense = nb3 > 0 ? H[kCntDense] : 0;
     PoolBuf<float> gvals{&c->pool[134]};
     PoolBuf<int32_t> didx{&c->pool[135]};
-    gvals.reserve(size_t(std::max<int64_t>(1, ndense)) * kBrickPts);
-    didx.reserve(nb);
+    PoolBuf<uint16_t> lofs_tab{&c->pool[124]}, emask_tab{&c->pool[125]};
+    PoolBuf<uint8_t> cube_tab{&c->pool[126]};
+    LeafTabs T3{};
     if (ndense > 0) {
+        gvals.reserve(size_t(ndense) * kBrickPts);
+        didx.reserve(nb);
+        T3.lofs = lofs_tab.reserve(size_t(ndense) * kBrickLeaves);
+        T3.emask = emask_tab.reserve(size_t(ndense) * kBrickLeaves);
+        T3.cube = cube_tab.reserve(size_t(ndense) * kBrickLeaves);
         TimedScope ts(kt, "subdivide_count", 0.0);
+        PRG_HIP(hipMemsetAsync(didx.get(), 0xff, size_t(nb) * 4, s));
         int per_cu = 0;
-        PRG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_brick_count, kWave, 0));
-        const int64_t grid = std::min<int64_t>(ndense, int64_t(std::max(1, per_cu)) * std::max(1, c->num_cu));
-        {
-            k_brick_count<<<unsigned(grid), kWave, 0, s>>>(A, dlist.get(), C, bnv.get(), bnt.get(), gvals.get(),
-                                                           didx.get());
-            PRG_CHECK_LAUNCH();
-        }
+        PRG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_brick_values, kWave, 0));
+        const int64_t resident = int64_t(std::max(1, per_cu)) * std::max(1, c->num_cu);
+        // about two resident grids of waves, in whole rounds
+        int slices = int(std::min<int64_t>(kValRounds, std::max<int64_t>(1, 2 * resident / ndense)));
+        while (kValRounds % slices) slices--;
+        if (ndense * slices >= (int64_t(1) << 31)) throw Error{PRG_E_NOMEM, "too many bricks to evaluate"};
+        k_brick_values<<<unsigned(ndense * slices), kWave, 0, s>>>(A, dlist.get(), slices, gvals.get());
+        PRG_CHECK_LAUNCH();
+        k_brick_cubes<<<unsigned(ndense), kBrickLeaves, 0, s>>>(A, dlist.get(), gvals.get(), T3, bnv.get(), bnt.get(),
+                                                                didx.get());
+        PRG_CHECK_LAUNCH();
     }
     scan_exclusive2(bnv.get(), bvoff.get(), C + kCntVerts, bnt.get(), btoff.get(), C + kCntTris, nb, s, c->scratch,
                     kt);
-    k_brick_active<<<grid_for(nb, kBlockS), kBlockS, 0, s>>>(bnv.get(), bnt.get(), bsign.get(), nb, aflag.get());
-    PRG_CHECK_LAUNCH();
-    scan_exclusive(aflag.get(), aoff.get(), nb, C + kCntActive, s, c->scratch, kt);
-    k_brick_compact<<<grid_for(nb, kBlockS), kBlockS, 0, s>>>(aflag.get(), aoff.get(), nb, alist.get(), amap.get());
-    PRG_CHECK_LAUNCH();
     PRG_HIP(hipMemcpyAsync(H, C, kCntSlots * 4, hipMemcpyDeviceToHost, s));
     PRG_HIP(hipStreamSynchronize(s));
-    const int64_t snv = H[kCntVerts], snt = H[kCntTris], nact = H[kCntActive];
+    const int64_t snv = H[kCntVerts], snt = H[kCntTris];
     c->sub_bricks = nb;
     c->sub_exact = int64_t(H[kCntExact]) + n1 + n2;
     c->sub_evaluated = int64_t(H[kCntDense]) + n1 + n2;
-    if (snv < 0 || snt < 0 || nact < 0) throw Error{PRG_E_NOMEM, "subdivision mesh exceeds int32 counts"};
+    if (snv < 0 || snt < 0) throw Error{PRG_E_NOMEM, "subdivision mesh exceeds int32 counts"};
     if (c->mesh_nv + snv >= (int64_t(1) << 31)) throw Error{PRG_E_NOMEM, "mesh vertex count exceeds int32 indices"};
     if (snv == 0 && snt == 0) return;
 
-    // passes 2 and 3 over the small roots and the bricks with output
-    PoolBuf<uint16_t> lofs_tab{&c->pool[124]}, emask_tab{&c->pool[125]};
-    PoolBuf<uint8_t> cube_tab{&c->pool[126]};
-    lofs_tab.reserve(size_t(nact) * kBrickLeaves);
-    emask_tab.reserve(size_t(nact) * kBrickLeaves);
-    cube_tab.reserve(size_t(nact) * kBrickLeaves);
+    // the vertices and triangles of the small roots and the evaluated bricks
     float* SV = c->sub_v.reserve(size_t(3) * snv + 3);
     int32_t* ST = c->sub_t.reserve(size_t(3) * snt + 3);
     {
@@ -2629,10 +2539,9 @@ void extract_subdivision(prg_ctx* c) {
             k_small_vertices<2><<<lw2, kWave, 0, s>>>(A, slist2.get(), n2, gv2.get(), gref2.get(), T2, bvoff.get(), SV);
             PRG_CHECK_LAUNCH();
         }
-        if (nact) {
-            k_brick_vertices<<<unsigned(nact), kWave, 0, s>>>(A, alist.get(), bvoff.get(), lofs_tab.get(),
-                                                              emask_tab.get(), cube_tab.get(), gvals.get(),
-                                                              didx.get(), SV);
+        if (ndense > 0) {
+            k_brick_vertices<<<unsigned(ndense), kBrickLeaves, 0, s>>>(A, dlist.get(), gvals.get(), T3, bnv.get(),
+                                                                       bvoff.get(), SV);
             PRG_CHECK_LAUNCH();
         }
     }
@@ -2648,10 +2557,10 @@ void extract_subdivision(prg_ctx* c) {
                                                        c->mesh_nv, ST, C + kCntErr);
             PRG_CHECK_LAUNCH();
         }
-        if (nact) {
-            k_brick_triangles<<<unsigned(nact), kWave, 0, s>>>(A, alist.get(), amap.get(), bvoff.get(), btoff.get(),
-                                                               lofs_tab.get(), emask_tab.get(), cube_tab.get(),
-                                                               c->mesh_nv, ST, C + kCntErr);
+        if (ndense > 0) {
+            k_brick_triangles<<<unsigned(ndense), kBrickLeaves, 0, s>>>(A, dlist.get(), didx.get(), T3, bnt.get(),
+                                                                        bvoff.get(), btoff.get(), c->mesh_nv, ST,
+                                                                        C + kCntErr);
             PRG_CHECK_LAUNCH();
         }
     }
