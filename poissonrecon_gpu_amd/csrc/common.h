@@ -171,6 +171,10 @@ struct FsTables {
     // divergence weights per node depth d: 3 * 2^(D-d) floats starting at div_off[d]
     std::vector<float> div_table;
     std::vector<int64_t> div_off;
+    // per depth: the largest difference, over all grid points of depth D and
+    // the three cells around them, between a base function's float value and
+    // the quadratic B-spline it stands for (1 at the centre)
+    std::vector<float> corner_dev;
 };
 void build_fs_tables(int D, FsTables* out);
 

@@ -302,6 +302,42 @@ void build_fs_tables(int D, FsTables* out) {
         for (int64_t u = 0; u < 3 * s; u++)
             out->div_table[size_t(out->div_off[d] + u)] = float(sp.entry(1, d, 0, D, u - s));
     }
+    // deviation of the corner values from the spline, by the float operations
+    // of the corner basis table (cell centre, half a cell to a side, the
+    // pieces' sums)
+    out->corner_dev.assign(D + 1, 0.0f);
+    const float hw = 1.0f / float(int64_t(1) << (D + 1));
+    for (int64_t ix = 0; ix < (int64_t(1) << D); ix++) {
+        float c = 0.5f, w = 0.25f;
+        for (int i = D - 1; i >= 0; --i) {
+            c = ((ix >> i) & 1) ? c + w : c - w;
+            w = w / 2;
+        }
+        for (int side = 0; side < 2; side++) {
+            const float p = c + float(2 * side - 1) * hw;
+            const double at = double(ix + side) / double(int64_t(1) << D);
+            for (int d = 0; d <= D; d++) {
+                const int64_t width = int64_t(1) << d;
+                for (int64_t u = (ix >> (D - d)) - 1; u <= (ix >> (D - d)) + 1; u++) {
+                    if (u < 0 || u >= width) continue;
+                    const float* f = &out->base_fn[size_t(width - 1 + u) * 20];
+                    float v = 0.0f;
+                    for (int i = 0; i < 4 && p > f[5 * i]; i++) {
+                        float t = 1.0f, q = 0.0f;
+                        for (int j = 0; j < 4; j++) {
+                            q = q + t * f[5 * i + 1 + j];
+                            t = t * p;
+                        }
+                        v = v + q;
+                    }
+                    const double a = std::fabs(at * double(width) - (double(u) + 0.5));
+                    const double e = a <= 0.5 ? 1.0 - a * a / 0.75 : a < 1.5 ? (1.5 - a) * (1.5 - a) / 1.5 : 0.0;
+                    out->corner_dev[d] = std::max(out->corner_dev[d], float(std::fabs(double(v) - e)));
+                }
+            }
+        }
+    }
+    for (float& v : out->corner_dev) v = 1.01f * v + 1e-6f;
 }
 
 }  // namespace prg

@@ -85,13 +85,13 @@ __constant__ CubeFaces c_cube_faces = make_cube_faces();
 // childrenVertexKind (MarchingCubes.cuh:720-723), used literally
 __constant__ int8_t c_children_vertex_kind[8] = {0, 1, 3, 2, 4, 5, 7, 6};
 
-// slots of the device counter array
-enum { kCntCoarse = 0, kCntCorners = 1, kCntRoots = 2, kCntBricks = 3, kCntVerts = 4, kCntTris = 5,
-       kCntLeaves = 7, kCntErr = 8, kCntDense = 9, kCntDepBricks = 10, kCntDepPairs = 11, kCntWork = 12,
-       kCntExact = 13, kCntSuper = 14, kCntList2 = 15, kCntWork2 = 16, kCntWork3 = 17, kCntSmall1 = 18,
-       kCntSmall2 = 19,
-       kCntSlots = 32 };
-static_assert(kCntSlots * 4 <= 128, "the pinned counter copy holds 32 ints");
+// slots of the device counter array; the cells of 2^k leaves a side listed at
+// kCntCells + k, and taken from the list at kCntTaken + k
+enum { kCntCoarse = 0, kCntCorners = 1, kCntRoots = 2, kCntBricks = 3, kCntVerts = 4, kCntTris = 5, kCntLeaves = 6,
+       kCntErr = 7, kCntDense = 8, kCntExact = 9, kCntExactTaken = 10, kCntSmall1 = 11, kCntSmall2 = 12,
+       kCntGroup = 13, kCntCells = 16, kCntTaken = 32, kCntSlots = 48 };
+static_assert(kCntSlots * 4 <= 256 && kCntCells + kMaxDepth < kCntTaken && kCntTaken + kMaxDepth < kCntSlots,
+              "the pinned counter copy holds 64 ints");
 
 __device__ __forceinline__ int depth_of(int64_t i, const Levels& L, int D) {
     int d = 0;
@@ -428,6 +428,15 @@ __global__ void __launch_bounds__(kBlockS) k_list_small_roots(const int32_t* roo
     }
 }
 
+// counts and signs of n bricks to 0
+__global__ void __launch_bounds__(kBlockS) k_clear_bricks(int32_t* bnv, int32_t* bnt, int8_t* sign, int64_t n) {
+    const int64_t i = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
+    if (i >= n) return;
+    bnv[i] = 0;
+    bnt[i] = 0;
+    sign[i] = 0;
+}
+
 struct SubArgs {
     const uint32_t* key;
     const int32_t* child_base;
@@ -446,14 +455,21 @@ struct SubArgs {
     const int32_t* cnt;      // device counters
     const int32_t* bmap;     // root number of each brick
     const int32_t* rec;      // per root: its record (kRecWords words, root_record)
+    // per depth: the largest corner value of sum |x_k b_x b_y b_z| over 27
+    // neighbours for coefficients up to 1, and the largest difference between
+    // the evaluation's value and the spline's there (depth_bounds)
+    float big[kMaxDepth + 1], dev[kMaxDepth + 1];
 };
 
 // Per-root record, built once per root and loaded by each of its bricks in
 // one coalesced read: the root's 27 neighbours, their child bases and root
 // numbers (group), its ancestor chain's neighbour values (27 per depth
-// 0..r), the root's index, depth and key.
-constexpr int kRecWords = 384;
+// 0..r), the root's index, depth and key; for roots of 8^3 leaves and more the
+// chain's values over the root as one polynomial (27 Bezier control values)
+// and the bound of what the evaluation's chain sum differs from it.
+constexpr int kRecWords = 416;
 constexpr int kRecNB = 0, kRecNBK = 27, kRecNBR = 54, kRecX = 81, kRecRho = 378, kRecR = 379, kRecKey = 380;
+constexpr int kRecPoly = 384, kRecErr = 411;
 
 // A brick and its root (wave-uniform).
 struct Brick {
@@ -483,44 +499,91 @@ struct BasisT {
     float x, y, z;
 };
 
-template <int kXBCap, int kTP = kP, bool kHasT = true>
-struct BrickCoreT {
-    static_assert(kXBCap > 1, "a layout holds blocks");
-    static constexpr int kTPts = kTP;  // grid coordinates per axis (of T, or of the screen's ranges)
+struct BrickCore {
     // per depth d, axis a and grid coordinate i: the corner basis table entry
     // of the owner (own_cell) of grid coordinate org[a] + i, (d, a, i) at
-    // d * 3 kP + a kP + i (the screens reduce the entries straight from the
-    // global table and keep no T)
-    BasisT T[kHasT ? (kMaxDepth + 1) * 3 * kTP : 1];
-    float X[(kMaxDepth + 1) * 27];  // the root's chain: neighbour values at depths 0..r
-    float XB[kXBCap];                  // per depth below the root: its block (xb_off)
+    // d * 3 kP + a kP + i
+    BasisT T[(kMaxDepth + 1) * 3 * kP];
+    float X[(kMaxDepth + 1) * 27];     // the root's chain: neighbour values at depths 0..r
+    float XB[kXBlk];                   // per depth below the root: its block (xb_off)
     int32_t xb_off[kMaxDepth + 1];     // start of depth dd's block in XB, or -1 (no real node in it)
     // child bases of a block's cells while the blocks are filled, at depths
-    // D, D - 2, .. and D - 1, D - 3, ..: up to 5^3 and 7^3 cells (the
-    // screens take blocks of up to 5^3 above depth D)
-    int32_t CB0[125], CB1[kXBCap > kXBlkScreen ? 343 : 125];
+    // D, D - 2, .. and D - 1, D - 3, ..: up to 5^3 and 7^3 cells
+    int32_t CB0[125], CB1[343];
     int32_t NB[27], NBK[27], NBR[27];  // the root's neighbours, their child bases, their root numbers (group)
     float tmax[kMaxDepth + 1];         // brick_abs_bound: per depth, the largest |basis value|
     float xsum[kMaxDepth + 1];         // and the sum of |coefficients|
-    // brick_interval_sign (the screens, which keep no T): per depth, axis and
-    // block slot, the range of the weight over the brick's points
-    float wlo[kHasT ? 1 : (kMaxDepth + 1) * 12];
-    float whi[kHasT ? 1 : (kMaxDepth + 1) * 12];
 };
 
-using BrickCore = BrickCoreT<kXBlk>;
-// The certificate screen's LDS: blocks up to kXBlkScreen floats (the depths
-// where the brick lies in one cell, and the first finer one); bricks that
-// need more go to the exact certificate, whose LDS holds every block.
-using BrickScreenLds = BrickCoreT<kXBlkScreen, kP, false>;
-// The super-brick screen's: 2x2x2 bricks, 17 grid coordinates per axis.
-constexpr int kPSuper = 2 * (1 << kBrickLog) + 1;
-using BrickSuperLds = BrickCoreT<kXBlkScreen, kPSuper, false>;
+// A screened cell's: the chain's polynomial and blocks of up to kXBlkScreen
+// floats and 5^3 cells above depth D (a cell that needs more is not settled).
+struct CellLds {
+    float P[27];
+    float XB[kXBlkScreen];
+    int32_t xb_off[kMaxDepth + 1];
+    int32_t CB0[125], CB1[125];
+    int32_t NBK[27], NBR[27];
+};
 
 __device__ __forceinline__ void decode_cell(uint32_t k, int32_t c[3]) {
     c[0] = int32_t(compact3(k >> 2));
     c[1] = int32_t(compact3(k >> 1));
     c[2] = int32_t(compact3(k));
+}
+
+// ---- the implicit function over a cell as a polynomial ----
+// Depth d's functions are quadratic B-splines of the depth's cell width (1 at
+// the node's centre, 4/3 summed over the three that overlap a point), whose
+// pieces meet at the depth's cell faces.  Over a cell of depth c, the sum of
+// all depths up to c is therefore one polynomial, quadratic along each axis;
+// its 27 Bezier control values bound it on the cell, and they are linear in
+// the depths' coefficients, so the depths add up (and cancel) before any
+// bound is taken.
+
+// Weights of the Bernstein control values of [0, 1] in control value i (0, 1,
+// 2) of the interval [t0, t0 + h]: the blossom at (t0, t0), (t0, t1), (t1, t1).
+__device__ __forceinline__ void bernstein_weights(float t0, float h, int i, float w[3]) {
+    const float s = i < 2 ? t0 : t0 + h, t = i < 1 ? t0 : t0 + h;
+    w[0] = (1.0f - s) * (1.0f - t);
+    w[1] = s * (1.0f - t) + t * (1.0f - s);
+    w[2] = s * t;
+}
+
+// Weights of the coefficients of a depth's three cells around cell A (A - 1,
+// A, A + 1) in control value i of the cell at coordinate c, `up` depths below
+// A: the spline's control values over A are (2/3)(x- + x), (4/3) x,
+// (2/3)(x + x+).
+__device__ __forceinline__ void spline_weights(int32_t c, int up, int i, float w[3]) {
+    const float h = 1.0f / float(1 << up), t0 = float(c & ((1 << up) - 1)) * h;
+    float b[3];
+    bernstein_weights(t0, h, i, b);
+    w[0] = (2.0f / 3.0f) * b[0];
+    w[1] = (2.0f / 3.0f) * (b[0] + b[2]) + (4.0f / 3.0f) * b[1];
+    w[2] = (2.0f / 3.0f) * b[2];
+}
+
+// sum over m, n, l of w[0][m] w[1][n] w[2][l] X[sx m + sy n + l]
+__device__ __forceinline__ float sum27(const float* X, int sx, int sy, const float w[3][3]) {
+    float v = 0.0f;
+#pragma unroll
+    for (int m = 0; m < 3; m++) {
+        float y = 0.0f;
+#pragma unroll
+        for (int n = 0; n < 3; n++) {
+            float z = 0.0f;
+#pragma unroll
+            for (int l = 0; l < 3; l++) z = __builtin_fmaf(X[sx * m + sy * n + l], w[2][l], z);
+            y = __builtin_fmaf(z, w[1][n], y);
+        }
+        v = __builtin_fmaf(y, w[0][m], v);
+    }
+    return v;
+}
+
+__device__ __forceinline__ float wave_max(float v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
+    return v;
 }
 
 // The record of root q (one wave per root).
@@ -530,18 +593,24 @@ __global__ void __launch_bounds__(kWave) k_root_records(SubArgs A, int32_t* rec)
     const int32_t rho = A.roots[q];
     const int r = depth_of(rho, A.L, D);
     int32_t* R = rec + int64_t(q) * kRecWords;
+    __shared__ float X[(kMaxDepth + 1) * 27];
     if (lane < 27) {
         const int32_t nb = neighbour_of(A.pnt, A.L, r, rho, lane);
         R[kRecNB + lane] = nb;
         R[kRecNBK + lane] = nb < 0 ? -1 : A.child_base[nb];
         R[kRecNBR + lane] = (nb < 0 || r < kFinerDepth) ? -1 : A.root_of[nb];
-        R[kRecX + 27 * r + lane] = __float_as_int(nb < 0 ? 0.0f : A.x[nb]);
+        const float xv = nb < 0 ? 0.0f : A.x[nb];
+        R[kRecX + 27 * r + lane] = __float_as_int(xv);
+        X[27 * r + lane] = xv;
     }
     // ancestors' rows (their 27 neighbour values, then the parent), depths r-1 .. 1
     int32_t a = A.parent[rho];
     for (int d = r - 1; d >= 1; d--) {
         const float* Row = A.rows + kRowFloats * (int64_t(a) - A.L.base[1]);
-        if (lane < 27) R[kRecX + 27 * d + lane] = __float_as_int(Row[lane]);
+        if (lane < 27) {
+            R[kRecX + 27 * d + lane] = __float_as_int(Row[lane]);
+            X[27 * d + lane] = Row[lane];
+        }
         a = __builtin_amdgcn_readfirstlane(__float_as_int(Row[27]));
     }
     if (lane == 0) {
@@ -550,6 +619,23 @@ __global__ void __launch_bounds__(kWave) k_root_records(SubArgs A, int32_t* rec)
         R[kRecR] = r;
         R[kRecKey] = int32_t(A.key[rho]);
     }
+    if (D - r < kBrickLog) return;  // (uniform) no cells to screen
+    if (lane < 27) X[lane] = lane == 13 ? A.x[0] : 0.0f;  // depth 0: the tree's root has no neighbours
+    __syncthreads();
+    int32_t rc[3];
+    decode_cell(A.key[rho], rc);
+    const int l27 = lane < 27 ? lane : 0;
+    float val = 0.0f, err = 0.0f;
+    for (int d = 0; d <= r; d++) {
+        float w[3][3];
+#pragma unroll
+        for (int a3 = 0; a3 < 3; a3++)
+            spline_weights(rc[a3] >> (D - r), r - d, a3 == 0 ? l27 / 9 : a3 == 1 ? (l27 / 3) % 3 : l27 % 3, w[a3]);
+        val += sum27(X + 27 * d, 9, 3, w);
+        err += A.dev[d] * wave_max(fabsf(X[27 * d + l27]));
+    }
+    if (lane < 27) R[kRecPoly + lane] = __float_as_int(val);
+    if (lane == 0) R[kRecErr] = __float_as_int(err);
 }
 
 // bmap[b] = the root of brick b (binary search of the brick offsets).
@@ -566,20 +652,43 @@ __global__ void __launch_bounds__(kBlockS) k_brick_map(const int32_t* boff, cons
     bmap[b] = lo;
 }
 
-// Loads brick b's root record into LDS (its neighbours and its chain's
-// values) and sets the brick's geometry.
-// q_loaded: the root whose record S already holds (the previous brick's, in a
-// kernel that walks consecutive bricks), or -1.  up = 1 sets up the
-// super-brick of the 2x2x2 bricks that start at brick b.
-template <class L>
-__device__ __forceinline__ void brick_setup(const SubArgs& A, int32_t b, Brick& B, L& S, int32_t q_loaded = -1,
-                                            int up = 0) {
-    const int D = A.D, lane = threadIdx.x;
-    B.q = __builtin_amdgcn_readfirstlane(A.bmap[b]);
-    const int32_t* R = A.rec + int64_t(B.q) * kRecWords;
+// The geometry of the cell of 2^kb leaves a side (a brick, or one of a root's
+// cells above) whose first brick is b, in a root with record R.
+__device__ __forceinline__ void cell_geometry(const SubArgs& A, int32_t b, int kb, const int32_t* R, Brick& B) {
+    const int D = A.D;
     B.rho = __builtin_amdgcn_readfirstlane(R[kRecRho]);
     B.r = __builtin_amdgcn_readfirstlane(R[kRecR]);
     const uint32_t rkey = uint32_t(__builtin_amdgcn_readfirstlane(R[kRecKey]));
+    B.kb = kb;
+    B.Sr = 1 << (D - B.r);
+    B.bkey = rkey | (uint32_t(b - A.boff[B.q]) << (3 * kBrickLog));
+    int32_t rc[3];
+    decode_cell(rkey, rc);
+    decode_cell(B.bkey, B.org);
+    for (int a = 0; a < 3; a++) {
+        B.R[a] = rc[a] >> (D - B.r);
+        B.R0[a] = rc[a];
+    }
+}
+
+template <class L>
+__device__ __forceinline__ void set_kids(Brick& B, const L& S) {
+    const int lane = threadIdx.x & 63;
+    const uint64_t kids = __builtin_amdgcn_ballot_w64(lane < 27 && lane != 13 && S.NBK[lane < 27 ? lane : 0] >= 0);
+    B.kids = uint32_t(kids);
+    B.deep = B.kids != 0;
+}
+
+// Loads the root record of brick b (8^3 leaves) into LDS (its neighbours and
+// its chain's values) and sets the brick's geometry.
+// q_loaded: the root whose record S already holds (the previous brick's, in a
+// kernel that walks a list), or -1.
+template <class L>
+__device__ __forceinline__ void brick_setup(const SubArgs& A, int32_t b, Brick& B, L& S, int32_t q_loaded = -1) {
+    const int lane = threadIdx.x;
+    B.q = __builtin_amdgcn_readfirstlane(A.bmap[b]);
+    const int32_t* R = A.rec + int64_t(B.q) * kRecWords;
+    cell_geometry(A, b, kBrickLog, R, B);
     if (B.q != q_loaded) {
         for (int w = lane; w < kRecX; w += kWave) {
             const int32_t v = R[w];
@@ -589,20 +698,23 @@ __device__ __forceinline__ void brick_setup(const SubArgs& A, int32_t b, Brick& 
         }
         for (int w = lane; w < 27 * (B.r + 1); w += kWave) S.X[w] = __int_as_float(R[kRecX + w]);
     }
-    B.kb = brick_log(D, B.r) + up;  // up = 1: the 2x2x2 bricks from brick b (a multiple of 8 in the root)
-    int32_t rc[3];
-    decode_cell(rkey, rc);
-    B.Sr = 1 << (D - B.r);
-    for (int a = 0; a < 3; a++) {
-        B.R[a] = rc[a] >> (D - B.r);
-        B.R0[a] = B.R[a] << (D - B.r);
-    }
-    B.bkey = rkey | (uint32_t(b - A.boff[B.q]) << (3 * (B.kb - up)));
-    decode_cell(B.bkey, B.org);
     __syncthreads();
-    const uint64_t kids = __builtin_amdgcn_ballot_w64(lane < 27 && lane != 13 && S.NBK[lane < 27 ? lane : 0] >= 0);
-    B.kids = uint32_t(kids);
-    B.deep = B.kids != 0;
+    set_kids(B, S);
+}
+
+// The same for a screened cell of 2^k leaves a side.
+__device__ __forceinline__ void cell_setup(const SubArgs& A, int32_t b, int k, Brick& B, CellLds& S, int32_t q_loaded) {
+    const int lane = threadIdx.x;
+    B.q = __builtin_amdgcn_readfirstlane(A.bmap[b]);
+    const int32_t* R = A.rec + int64_t(B.q) * kRecWords;
+    cell_geometry(A, b, k, R, B);
+    if (B.q != q_loaded && lane < 27) {
+        S.NBK[lane] = R[kRecNBK + lane];
+        S.NBR[lane] = R[kRecNBR + lane];
+        S.P[lane] = __int_as_float(R[kRecPoly + lane]);
+    }
+    __syncthreads();
+    set_kids(B, S);
 }
 
 // Whether the depth-D cell c (inside the root's 3x3x3 neighbourhood) is a
@@ -639,7 +751,7 @@ __device__ __forceinline__ int32_t own_cell(int32_t g, int32_t R0) { return g ==
 template <class L>
 __device__ __forceinline__ void brick_tables(const SubArgs& A, const Brick& B, L& S) {
     const int D = A.D, P = (1 << B.kb) + 1;
-    constexpr int TP = L::kTPts;
+    constexpr int TP = kP;
     for (int e = threadIdx.x; e < (D + 1) * TP; e += kWave) {
         const int d = e / TP, i = e % TP;
         if (i >= P) continue;
@@ -1043,18 +1155,6 @@ __device__ __forceinline__ void contract64(const float* X64, const float wy[4], 
     }
 }
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
-    return v;
-}
-
-__device__ __forceinline__ float wave_fsum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-    return v;
-}
-
 // An upper bound of A(g) = sum over depths and the owner's 27 neighbours of
 // |x_k b_x b_y b_z| for every corner g of the brick owned inside its root:
 // per depth, the sum of |x| over the depth's block (which holds every
@@ -1067,7 +1167,7 @@ __device__ __forceinline__ float brick_abs_bound(const Brick& B, L& S, int D) {
     if (lane <= kMaxDepth) S.tmax[lane] = S.xsum[lane] = 0.0f;
     __syncthreads();
     // |basis values| (non-negative floats order as their bit patterns)
-    constexpr int TP = L::kTPts;
+    constexpr int TP = kP;
     for (int e = lane; e < (D + 1) * 3 * TP; e += kWave) {
         const int d = e / (3 * TP), i = e % TP;
         if (i >= P || (d > B.r && S.xb_off[d] < 0)) continue;
@@ -1095,78 +1195,6 @@ __device__ __forceinline__ float brick_abs_bound(const Brick& B, L& S, int D) {
     return 1.001f * bound;
 }
 
-// brick_abs_bound for the screens, and the ranges brick_interval_sign needs,
-// from the corner basis table in global memory (the screens keep no T): one
-// lane per (depth, axis) reads the owner's entry for each of the brick's grid
-// coordinates (brick_tables' entries), takes the largest |basis value| (for
-// tmax) and, at depths d <= D - kb, each block slot's weight range over the
-// points (wlo, whi).  The figures are those brick_abs_bound and the range
-// pass of the T path compute.
-template <class L>
-__device__ __forceinline__ float brick_screen_bound(const SubArgs& A, const Brick& B, L& S) {
-    static_assert(sizeof(S.wlo) == (kMaxDepth + 1) * 12 * sizeof(float), "the screens' LDS holds the slot ranges");
-    const int D = A.D, lane = threadIdx.x, P = (1 << B.kb) + 1, dlast = D - B.kb;
-    if (lane <= kMaxDepth) S.tmax[lane] = S.xsum[lane] = 0.0f;
-    __syncthreads();
-    if (lane < 3 * (D + 1)) {
-        const int d = lane / 3, a = lane % 3;
-        if (d <= B.r || S.xb_off[d] >= 0) {
-            // (arithmetic selects: an index by a would put B in scratch memory)
-            const int32_t og = (a == 0) * B.org[0] + (a == 1) * B.org[1] + (a == 2) * B.org[2];
-            const int32_t r0 = (a == 0) * B.R0[0] + (a == 1) * B.R0[1] + (a == 2) * B.R0[2];
-            float mx = 0.0f, lo[4], hi[4];
-#pragma unroll
-            for (int m = 0; m < 4; m++) {
-                lo[m] = 3.4e38f;
-                hi[m] = -3.4e38f;
-            }
-#pragma unroll
-            for (int i = 0; i < L::kTPts; i++) {
-                if (i < P) {
-                    const int32_t g = og + i, o = own_cell(g, r0);
-                    const float4 t = A.btab[((int64_t(d) << D) + o) * 2 + (g - o)];
-                    mx = fmaxf(mx, fmaxf(fabsf(t.x), fmaxf(fabsf(t.y), fabsf(t.z))));
-                    // the owner's ancestor is the brick's (slots 1..3) or the one below (0..2)
-                    const bool below = d > B.r && (o >> (D - d)) != (og >> (D - d));
-                    const float w0 = below ? t.x : 0.0f, w1 = below ? t.y : t.x, w2 = below ? t.z : t.y,
-                                w3 = below ? 0.0f : t.z;
-                    lo[0] = fminf(lo[0], w0), hi[0] = fmaxf(hi[0], w0);
-                    lo[1] = fminf(lo[1], w1), hi[1] = fmaxf(hi[1], w1);
-                    lo[2] = fminf(lo[2], w2), hi[2] = fmaxf(hi[2], w2);
-                    lo[3] = fminf(lo[3], w3), hi[3] = fmaxf(hi[3], w3);
-                }
-            }
-            // |basis values| (non-negative floats order as their bit patterns)
-            atomicMax(reinterpret_cast<int*>(&S.tmax[d]), __float_as_int(mx));
-            if (d <= dlast) {
-#pragma unroll
-                for (int m = 0; m < 4; m++) {
-                    S.wlo[12 * d + 4 * a + m] = lo[m];
-                    S.whi[12 * d + 4 * a + m] = hi[m];
-                }
-            }
-        }
-    }
-    // |coefficients|: the chain, then the blocks (as brick_abs_bound)
-    for (int e = lane; e < 27 * B.r; e += kWave) atomicAdd(&S.xsum[1 + e / 27], fabsf(S.X[27 + e]));
-    if (lane == 0) atomicAdd(&S.xsum[0], fabsf(S.X[0]));
-    for (int d = B.r + 1; d <= D; d++) {
-        if (S.xb_off[d] < 0) continue;
-        const int W = d <= dlast ? 4 : block_width(D, B.kb, d), n = W * W * W;
-        float sx = 0.0f;
-        for (int e = lane; e < n; e += kWave) sx += fabsf(S.XB[S.xb_off[d] + e]);
-        if (sx != 0.0f) atomicAdd(&S.xsum[d], sx);
-    }
-    __syncthreads();
-    float bound = 0.0f;
-#pragma unroll
-    for (int d = 0; d <= kMaxDepth; d++) {
-        const float tm = S.tmax[d];
-        if (d <= D) bound += S.xsum[d] * (tm * tm * tm);
-    }
-    return 1.001f * bound;
-}
-
 // The basis weights over the 4 block slots along axis ax for grid coordinate
 // org[ax] + i at depth d <= D - kb: the owner's three values, placed at its
 // ancestor's offset (-1 or 0) from the brick's ancestor.
@@ -1175,7 +1203,7 @@ __device__ __forceinline__ void axis_weights4(const Brick& B, const L& S, int D,
                                               float w[4]) {
     const int32_t g = B.org[ax] + i, o = own_cell(g, B.R0[ax]);
     const int delta = (o >> (D - d)) - (B.org[ax] >> (D - d));
-    const BasisT t = S.T[3 * L::kTPts * d + L::kTPts * ax + i];
+    const BasisT t = S.T[3 * kP * d + kP * ax + i];
     if (delta == 0) {
         w[0] = 0.0f;
         w[1] = t.x;
@@ -1189,61 +1217,56 @@ __device__ __forceinline__ void axis_weights4(const Brick& B, const L& S, int D,
     }
 }
 
-// A sign for every corner the brick's root owns from one interval for the
-// whole brick.  With slot weights (zero outside the owner's three per axis),
-// a depth's sum is sum over the block's slots (m, n, l) of
-// X[m][n][l] w_x(i)[m] w_y(j)[n] w_z(k)[l] exactly; each weight lies in its
-// slot's range over the brick's points, so each term lies in X times the
-// product of three ranges.  The finer depths, where the brick spans several
-// cells, are bounded by sum |x| times the cube of their largest basis value
-// (brick_abs_bound's per-depth figures).  The float evaluation differs from
-// the exact sum by at most 351 2^-24 A(g) (the certificate's analysis below)
-// and the interval's own float sums by less than 40 2^-24 of the same bound:
-// the brick is certified when the interval clears iso by 700 2^-24 times
-// the bound of A (plus the rounding of the subtraction).
-template <class L>
-__device__ __forceinline__ int brick_interval_sign(const SubArgs& A, const Brick& B, L& S, float abound) {
-    const int D = A.D, lane = threadIdx.x, dlast = D - B.kb;
-    // (the slot ranges wlo, whi come from brick_screen_bound, which ended with a barrier)
-    const int m = lane >> 4, n = (lane >> 2) & 3, l = lane & 3;
-    float lo = 0.0f, hi = 0.0f;
+// A sign for every corner of the cell that its root owns.  The depths up to
+// the cell's own are one polynomial over the cell: the chain's (restricted
+// from the root's) plus, per depth r + 1 .. D - k, the spline of the block's
+// three cells per axis around the cell's ancestor.  A corner's owner may be a
+// leaf of the cell below along an axis; its 27 neighbours then reach one cell
+// further down and one less up, and the spline of the cell left out is 0
+// there.  Its range lies between the smallest and the largest control value.
+// The depths below the cell's add at most their largest |x| times big[d]
+// each; the float evaluation differs from the spline by at most dev[d] times
+// the largest |x| per depth (depth_bounds, the rounding of all sums
+// included).  The cell is settled when all of that is clear of iso.
+__device__ __forceinline__ int cell_sign(const SubArgs& A, const Brick& B, const CellLds& S) {
+    const int D = A.D, lane = threadIdx.x, c = D - B.kb;
+    const int l27 = lane < 27 ? lane : 0;
+    const int i3[3] = {l27 / 9, (l27 / 3) % 3, l27 % 3};
+    float w[3][3];
+    const float inv = 1.0f / float(B.Sr);
 #pragma unroll
-    for (int d = 0; d <= kMaxDepth; d++) {
-        float x = 0.0f;
-        if (d == 0) {
-            x = (m == 2 && n == 2 && l == 2) ? S.X[0] : 0.0f;
-        } else if (d <= B.r) {
-            x = (m && n && l) ? S.X[27 * d + 9 * (m - 1) + 3 * (n - 1) + (l - 1)] : 0.0f;
-        } else if (d <= dlast) {
-            const int o = S.xb_off[d];
-            x = o < 0 ? 0.0f : S.XB[o + lane];
+    for (int a = 0; a < 3; a++)
+        bernstein_weights(float(B.org[a] - B.R0[a]) * inv, float(1 << B.kb) * inv, i3[a], w[a]);
+    float val = sum27(S.P, 9, 3, w);
+    bool finite = true;
+    float slack = __int_as_float(__builtin_amdgcn_readfirstlane(A.rec[int64_t(B.q) * kRecWords + kRecErr]));
+    for (int d = B.r + 1; d <= D; d++) {
+        const int o = S.xb_off[d];  // (uniform)
+        if (o < 0) continue;
+        const int W = block_width(D, B.kb, d), n = W * W * W;
+        float m = 0.0f;
+        for (int e = lane; e < n; e += kWave) {
+            const float x = fabsf(S.XB[o + e]);
+            m = fmaxf(m, x);
+            finite = finite && x < INFINITY;
         }
-        if (d <= dlast) {
-            const float a1 = S.wlo[12 * d + m], a2 = S.whi[12 * d + m];
-            const float b1 = S.wlo[12 * d + 4 + n], b2 = S.whi[12 * d + 4 + n];
-            const float c1 = S.wlo[12 * d + 8 + l], c2 = S.whi[12 * d + 8 + l];
-            const float u1 = fminf(fminf(a1 * b1, a1 * b2), fminf(a2 * b1, a2 * b2));
-            const float u2 = fmaxf(fmaxf(a1 * b1, a1 * b2), fmaxf(a2 * b1, a2 * b2));
-            const float p1 = fminf(fminf(u1 * c1, u1 * c2), fminf(u2 * c1, u2 * c2));
-            const float p2 = fmaxf(fmaxf(u1 * c1, u1 * c2), fmaxf(u2 * c1, u2 * c2));
-            if (x != 0.0f) {
-                lo += x >= 0.0f ? x * p1 : x * p2;
-                hi += x >= 0.0f ? x * p2 : x * p1;
-            }
+        m = wave_max(m);
+        if (d <= c) {
+#pragma unroll
+            for (int a = 0; a < 3; a++) spline_weights(B.org[a] >> B.kb, c - d, i3[a], w[a]);
+            val += sum27(S.XB + o + 21, 16, 4, w);  // slots 1..3 along each axis
+            slack += A.dev[d] * m;
+        } else {
+            slack += (A.big[d] + A.dev[d]) * m;
         }
     }
-    lo = wave_fsum(lo);
-    hi = wave_fsum(hi);
-    float fine = 0.0f;
-    for (int d = dlast + 1; d <= D; d++) {
-        if (S.xb_off[d] < 0) continue;
-        const float t = S.tmax[d];
-        fine += S.xsum[d] * (t * t * t);
-    }
-    lo -= 1.001f * fine;
-    hi += 1.001f * fine;
+    // (a maximum passes over NaN; a coefficient that is not finite makes every
+    // control value NaN, or is one of the deeper depths')
+    finite = finite && fabsf(val) < INFINITY;
+    if (__builtin_amdgcn_ballot_w64(!finite) != 0) return 0;
+    const float hi = wave_max(val), lo = -wave_max(-val);
     const float iso = *A.iso;
-    const float margin = 700.0f * 5.9604645e-8f * abound + 1.2e-7f * (fabsf(lo) + fabsf(hi) + 2.0f * fabsf(iso)) + 1e-15f;
+    const float margin = 1.001f * slack + 1.2e-7f * (fabsf(lo) + fabsf(hi) + 2.0f * fabsf(iso)) + 1e-15f;
     if (lo - iso > margin) return 1;
     if (hi - iso < -margin) return -1;
     return 0;
@@ -1294,13 +1317,9 @@ __device__ __forceinline__ uint32_t brick_group_deps(const Brick& B, const L& S,
 // subtraction) with one sign at every corner its root owns.  A corner on the
 // root's boundary may be owned by a leaf of another root of the group: its
 // value is the one that root's brick holding the owner computes for its own
-// corner (the same owner, table entries and order), so the brick records
-// that brick's offset instead (deps) and the sign is compared with that
-// brick's certificate afterwards (k_brick_deps).
-struct Certificate {
-    int sign;       // +1 / -1: every corner the brick's root owns has this sign; 0: not proven
-    uint32_t deps;  // bit nidx(delta): a corner owned by a leaf of another root, in the brick at offset delta
-};
+// corner (the same owner, table entries and order), so the sign is compared
+// with that brick's afterwards (k_group_check).  Returns +1 or -1 (every
+// corner the brick's root owns has this sign) or 0 (not proven).
 
 // Whether the brick touches a face, edge or corner its root shares with
 // another root of the group (whose leaves may own corners of the brick).
@@ -1324,26 +1343,14 @@ __device__ __forceinline__ bool brick_in_group(const Brick& B, const L& S) {
     return group;
 }
 
-// The interval certificate (brick_interval_sign) with the brick's
-// dependencies on other roots' bricks.
 template <class L>
-__device__ __forceinline__ Certificate brick_certify_interval(const SubArgs& A, const Brick& B, L& S) {
-    Certificate c;
-    c.sign = brick_interval_sign(A, B, S, brick_screen_bound(A, B, S));
-    c.deps = (c.sign != 0 && brick_in_group(B, S)) ? brick_group_deps(B, S, A.D) : 0;
-    return c;
-}
-
-template <class L>
-__device__ __forceinline__ Certificate brick_certify(const SubArgs& A, const Brick& B, L& S) {
-    const int D = A.D, kb = B.kb, Sb = 1 << kb, P = Sb + 1;
+__device__ __forceinline__ int brick_certify(const SubArgs& A, const Brick& B, L& S, bool group) {
+    const int D = A.D, kb = B.kb, P = (1 << kb) + 1;
     const int lane = threadIdx.x;
-    const bool group = brick_in_group(B, S);
     const float iso = *A.iso;
     const int dlast = D - kb;  // deepest depth whose cell holds the whole brick
     const float marginA = 560.0f * 5.9604645e-8f * brick_abs_bound(B, S, D) + 1e-15f;
     bool ok = true, pos = false, neg = false;
-    uint32_t deps = 0;
     for (int pp = lane; pp < kP * kP; pp += kWave) {
         const int j = pp % kP, k = pp / kP;
         if (j >= P || k >= P) continue;
@@ -1433,12 +1440,7 @@ __device__ __forceinline__ Certificate brick_certify(const SubArgs& A, const Bri
                 // on the root's boundary: is the owner a leaf of another root?
                 const int32_t g[3] = {gx, B.org[1] + j, B.org[2] + k};
                 int32_t o[3];
-                if (corner_owner(B, S, D, g, o) != 13) {
-                    int dv[3];
-                    for (int a = 0; a < 3; a++) dv[a] = o[a] < B.org[a] ? -1 : (o[a] >= B.org[a] + Sb ? 1 : 0);
-                    deps |= 1u << nidx(dv[0], dv[1], dv[2]);
-                    continue;
-                }
+                if (corner_owner(B, S, D, g, o) != 13) continue;
             }
             const float val = v[i] - iso;
             const float margin = marginA + 1.2e-7f * (fabsf(v[i]) + fabsf(iso));
@@ -1450,193 +1452,113 @@ __device__ __forceinline__ Certificate brick_certify(const SubArgs& A, const Bri
     const bool lane_good = ok && !(pos && neg);
     const uint64_t good = __builtin_amdgcn_ballot_w64(lane_good);
     const uint64_t anypos = __builtin_amdgcn_ballot_w64(pos), anyneg = __builtin_amdgcn_ballot_w64(neg);
+    return (good == ~uint64_t(0) && !(anypos && anyneg)) ? (anypos ? 1 : -1) : 0;
+}
+
+// The roots of 8^3 leaves and more: each is the first cell of its size to be
+// screened (lists: the cells of 2^k leaves a side at lists.at[k], as the
+// number of their first brick).
+struct CellLists {
+    int32_t* at[kMaxDepth + 1];
+};
+
+__global__ void __launch_bounds__(kBlockS) k_list_roots(const int32_t* roots, const int32_t* boff, int64_t nr, Levels L,
+                                                        int D, CellLists lists, int32_t* cnt) {
+    const int64_t q = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
+    const int kb = q < nr ? D - depth_of(roots[q], L, D) : 0;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) deps |= uint32_t(__shfl_xor(int(deps), o, kWave));
-    Certificate c;
-    c.sign = (good == ~uint64_t(0) && !(anypos && anyneg)) ? (anypos ? 1 : -1) : 0;
-    c.deps = deps;
-    return c;
-}
-
-// Records a brick's certificate: its sign, and either its dependencies
-// (dbricks: (b, first, count); dpairs: the bricks it depends on) or, when
-// not certified, its place in `list`.
-template <class L>
-__device__ __forceinline__ void record_certificate(const SubArgs& A, const Brick& B, const L& S, int32_t b,
-                                                   const Certificate& c, int8_t* sign, int32_t* list, int list_slot,
-                                                   int32_t* dbricks, int32_t* dpairs, int32_t* cnt) {
-    const int lane = threadIdx.x, D = A.D;
-    int32_t first = 0;
-    if (lane == 0) {
-        sign[b] = int8_t(c.sign);
-        if (c.sign == 0) {
-            list[atomicAdd(cnt + list_slot, 1)] = b;
-        } else if (c.deps) {
-            const int n = __popc(c.deps);
-            first = atomicAdd(cnt + kCntDepPairs, n);
-            const int32_t e = atomicAdd(cnt + kCntDepBricks, 1);
-            dbricks[3 * e] = b;
-            dbricks[3 * e + 1] = first;
-            dbricks[3 * e + 2] = n;
-        }
-    }
-    first = __shfl(first, 0, kWave);
-    if (c.sign != 0 && lane < 27 && ((c.deps >> lane) & 1u)) {
-        // the brick at offset delta(lane), in the root of the group that holds it
-        const int Sb = 1 << B.kb, sh = D - B.r;
-        const int dv[3] = {lane / 9 - 1, (lane / 3) % 3 - 1, lane % 3 - 1};
-        int32_t cc[3];
-        int ro[3];
-        for (int a = 0; a < 3; a++) {
-            cc[a] = B.org[a] + dv[a] * Sb;
-            ro[a] = (cc[a] >> sh) - B.R[a];
-        }
-        const int slot = nidx(ro[0], ro[1], ro[2]);
-        const int32_t q2 = slot == 13 ? B.q : S.NBR[slot];
-        const uint32_t rmask = 3 * sh >= 32 ? 0xffffffffu : ((1u << (3 * sh)) - 1u);
-        const int32_t b2 =
-            q2 < 0 ? -1
-                   : A.boff[q2] + int32_t((cell_key(uint32_t(cc[0]), uint32_t(cc[1]), uint32_t(cc[2])) & rmask) >>
-                                          (3 * B.kb));
-        dpairs[first + __popc(c.deps & ((1u << lane) - 1u))] = b2;
+    for (int k = kBrickLog; k <= kMaxDepth; k++) {
+        if (k >= D) break;
+        const int32_t at = wave_append(kb == k, cnt + kCntCells + k);
+        if (kb == k) lists.at[k][at] = boff[q];
     }
 }
 
-// Pass 0a: the interval certificate for the super-bricks (2x2x2 bricks) of
-// the roots with at least 8 bricks (a fixed grid takes chunks of consecutive
-// super-bricks from a counter).  A certified super-brick settles its 8
-// bricks (counts 0, its sign); the bricks of the others, and of super-bricks
-// that touch another root of the group (whose leaves may own corners) or
-// whose blocks the LDS cannot hold, are listed for the brick screen.
-__global__ void __launch_bounds__(kWave, 5) k_brick_screen_super(SubArgs A, const int32_t* smap, const int32_t* soff,
-                                                              int32_t* bnv, int32_t* bnt, int8_t* sign,
-                                                              int32_t* list2, int32_t* cnt, int certify) {
-    __shared__ BrickSuperLds S;
+// Pass 0: screens the listed cells of 2^k leaves a side, one wave each (a
+// resident grid takes chunks of the list from a counter).  A settled cell
+// gives its bricks its sign (their counts stay 0), and lists those that touch
+// another root of the group for k_group_check; of the others, a cell of more
+// than one brick lists its eight parts for the next size and a brick goes to
+// the per-corner certificate.  Most of the refined volume is far from the
+// surface and settles in large cells: the 1,036,945 bricks of 2 M points at
+// depth 10 took 1.85 ms as 122,256 cells of 16^3 and then 238,786 bricks, each
+// bounded by intervals depth by depth.
+__global__ void __launch_bounds__(kWave, 5) k_cell_screen(SubArgs A, int k, const int32_t* list, int32_t* parts,
+                                                       int32_t* xlist, int8_t* sign, int32_t* glist, int32_t* cnt,
+                                                       int certify) {
+    __shared__ CellLds S;
     const int lane = threadIdx.x;
-    const int32_t ns = cnt[kCntSuper];
-    const int32_t chunk = std::max(1, std::min(8, ns / (2 * int32_t(gridDim.x))));
-    int32_t q_loaded = -1, sb = 0, s_end = 0;
-    for (;;) {
-        if (sb == s_end) {
-            int32_t c0 = 0;
-            if (lane == 0) c0 = atomicAdd(cnt + kCntWork, chunk);
-            c0 = __shfl(c0, 0, kWave);
-            if (c0 >= ns) break;
-            sb = c0;
-            s_end = std::min(ns, c0 + chunk);
-        }
-        const int32_t q = smap[sb];
-        const int32_t b0 = A.boff[q] + 8 * (sb - soff[q]);
-        Brick B;
-        __syncthreads();  // the previous super-brick's LDS reads are done
-        brick_setup(A, b0, B, S, q_loaded, 1);
-        q_loaded = B.q;
-        int sgn = 0;
-        if (certify && !brick_in_group(B, S) && brick_blocks(A, B, S))
-            sgn = brick_interval_sign(A, B, S, brick_screen_bound(A, B, S));
-        if (sgn != 0) {
-            if (lane < 8) {
-                bnv[b0 + lane] = 0;
-                bnt[b0 + lane] = 0;
-                sign[b0 + lane] = int8_t(sgn);
-            }
-        } else {
-            int32_t at = 0;
-            if (lane == 0) at = atomicAdd(cnt + kCntList2, 8);
-            at = __shfl(at, 0, kWave);
-            if (lane < 8) list2[at + lane] = b0 + lane;
-        }
-        sb++;
-    }
-}
-
-// The roots of one 8^3 brick, for the brick screen.
-__global__ void __launch_bounds__(kBlockS) k_list_one_brick_roots(const int32_t* roots, const int32_t* boff,
-                                                                  int64_t nr, Levels L, int D, int32_t* list2,
-                                                                  int32_t* cnt) {
-    const int64_t q = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
-    const bool one = q < nr && depth_of(roots[q], L, D) == D - kBrickLog;
-    const int32_t at = wave_append(one, cnt + kCntList2);
-    if (one) list2[at] = boff[q];
-}
-
-// Per root: its super-brick count (a root of at least 8 bricks has a
-// multiple of 8, in 2x2x2 blocks of Morton-consecutive bricks).
-__global__ void __launch_bounds__(kBlockS) k_super_count(const int32_t* rbricks, const int32_t* cnt, int64_t nr_max,
-                                                         int32_t* nsup) {
-    const int64_t q = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
-    if (q >= nr_max) return;
-    int32_t n = 0;
-    if (q < cnt[kCntRoots]) n = rbricks[q] >= 8 ? rbricks[q] / 8 : 0;
-    nsup[q] = n;
-}
-
-// smap[s] = the root of super-brick s (binary search of the super-brick offsets).
-__global__ void __launch_bounds__(kBlockS) k_super_map(const int32_t* soff, const int32_t* cnt, int64_t ns_max,
-                                                       int32_t* smap) {
-    const int64_t sb = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
-    if (sb >= ns_max || sb >= cnt[kCntSuper]) return;
-    int32_t lo = 0, hi = cnt[kCntRoots] - 1;
-    while (lo < hi) {
-        const int32_t mid = (lo + hi + 1) >> 1;
-        if (soff[mid] <= sb) lo = mid;
-        else hi = mid - 1;
-    }
-    smap[sb] = lo;
-}
-
-// Pass 0b: the interval certificate for the listed bricks (a fixed grid takes
-// chunks of the list from a counter).  Every listed brick's counts start at
-// 0; a certified brick keeps them unless a brick it depends on has another
-// sign (k_brick_deps); the others are listed for the exact certificate
-// (k_brick_exact).
-__global__ void __launch_bounds__(kWave, 5) k_brick_screen(SubArgs A, const int32_t* list2, int32_t* bnv, int32_t* bnt,
-                                                        int8_t* sign, int32_t* xlist, int32_t* dbricks,
-                                                        int32_t* dpairs, int32_t* cnt, int certify) {
-    __shared__ BrickScreenLds S;
-    const int lane = threadIdx.x;
-    const int32_t nl = cnt[kCntList2];
-    // consecutive entries per grab (mostly one root, whose record stays in LDS):
-    // up to 16, at least about four grabs per workgroup (13,000 bricks in
-    // chunks of 16 kept 815 of 5,120 waves busy for 510 us)
-    const int32_t chunk = std::max(1, std::min(16, nl / (4 * int32_t(gridDim.x))));
+    const int32_t n = cnt[kCntCells + k];
+    // up to 16 entries, at least about four grabs per workgroup
+    const int32_t chunk = std::max(1, std::min(16, n / (4 * int32_t(gridDim.x))));
     int32_t q_loaded = -1, it = 0, it_end = 0;
     for (;;) {
         if (it == it_end) {
             int32_t c0 = 0;
-            if (lane == 0) c0 = atomicAdd(cnt + kCntWork2, chunk);
+            if (lane == 0) c0 = atomicAdd(cnt + kCntTaken + k, chunk);
             c0 = __shfl(c0, 0, kWave);
-            if (c0 >= nl) break;
+            if (c0 >= n) break;
             it = c0;
-            it_end = std::min(nl, c0 + chunk);
+            it_end = std::min(n, c0 + chunk);
         }
-        const int32_t b = list2[it];
+        const int32_t b = list[it++];
         Brick B;
-        __syncthreads();  // the previous brick's LDS reads are done
-        brick_setup(A, b, B, S, q_loaded);
+        __syncthreads();  // the previous cell's LDS reads are done
+        cell_setup(A, b, k, B, S, q_loaded);
         q_loaded = B.q;
-        Certificate c;
-        c.sign = 0;
-        c.deps = 0;
-        if (brick_blocks(A, B, S) && certify) c = brick_certify_interval(A, B, S);  // else: to the exact certificate
-        if (lane == 0) {
-            bnv[b] = 0;
-            bnt[b] = 0;
+        int s = 0;
+        if (certify && brick_blocks(A, B, S)) s = cell_sign(A, B, S);
+        if (s == 0) {
+            const int32_t np = k > kBrickLog ? 8 : 1;
+            int32_t at = 0;
+            if (lane == 0) at = atomicAdd(cnt + (k > kBrickLog ? kCntCells + k - 1 : int(kCntExact)), np);
+            at = __shfl(at, 0, kWave);
+            if (k > kBrickLog) {
+                if (lane < 8) parts[at + lane] = b + (lane << (3 * (k - 1 - kBrickLog)));
+            } else if (lane == 0) {
+                xlist[at] = b;
+            }
+            continue;
         }
-        record_certificate(A, B, S, b, c, sign, xlist, kCntExact, dbricks, dpairs, cnt);
-        it++;
+        // the cell's bricks; those on a face, edge or corner shared with the group
+        const uint64_t in_group = __builtin_amdgcn_ballot_w64(lane < 27 && lane != 13 && S.NBR[lane < 27 ? lane : 0] >= 0);
+        const uint32_t gm = uint32_t(in_group);
+        const bool touches = gm && brick_in_group(B, S);
+        const int32_t nbk = 1 << (3 * (k - kBrickLog));
+        for (int32_t i0 = 0; i0 < nbk; i0 += kWave) {
+            const int32_t i = i0 + lane;
+            const bool in = i < nbk;
+            if (in) sign[b + i] = int8_t(s);
+            if (touches) {
+                int32_t o[3];
+                decode_cell(uint32_t(i), o);
+                uint32_t m[3];
+#pragma unroll
+                for (int a = 0; a < 3; a++) {
+                    // neighbour slots with offset -1, 0, +1 along axis a
+                    const uint32_t z = a == 0 ? 0x000001ffu : a == 1 ? 0x001c0e07u : 0x01249249u;
+                    const int step = a == 0 ? 9 : a == 1 ? 3 : 1;
+                    const int32_t g = B.org[a] + (o[a] << kBrickLog);
+                    m[a] = z << step;
+                    if (g == B.R0[a]) m[a] |= z;
+                    if (g + (1 << kBrickLog) == B.R0[a] + B.Sr) m[a] |= z << (2 * step);
+                }
+                const bool want = in && (m[0] & m[1] & m[2] & gm) != 0;
+                const int32_t at = wave_append(want, cnt + kCntGroup);
+                if (want) glist[at] = b + i;
+            }
+        }
     }
 }
 
-// Pass 0b: the exact certificate (brick_certify) for the bricks the interval
-// left (a fixed grid walks the list); the bricks it does not certify are
-// listed for the evaluation.
+// Pass 0b: the per-corner certificate (brick_certify) for the bricks the
+// screen left; the bricks it does not settle are listed for the evaluation.
 // A resident grid takes chunks of consecutive entries from a counter; entries
 // of one root often follow each other, and its record then stays in LDS.
 // Compiled for three waves per SIMD (168 VGPRs, a few spilled): the waves wait
 // on memory about half their time, and two per SIMD hid less.
 __global__ void __launch_bounds__(kWave, 3) k_brick_exact(SubArgs A, const int32_t* xlist, int8_t* sign, int32_t* list,
-                                                       int32_t* dbricks, int32_t* dpairs, int32_t* cnt, int certify) {
+                                                       int32_t* glist, int32_t* cnt, int certify) {
     __shared__ BrickCore S;
     const int lane = threadIdx.x;
     const int32_t n = cnt[kCntExact];
@@ -1646,7 +1568,7 @@ __global__ void __launch_bounds__(kWave, 3) k_brick_exact(SubArgs A, const int32
     for (;;) {
         if (it == it_end) {
             int32_t c0 = 0;
-            if (lane == 0) c0 = atomicAdd(cnt + kCntWork3, chunk);
+            if (lane == 0) c0 = atomicAdd(cnt + kCntExactTaken, chunk);
             c0 = __shfl(c0, 0, kWave);
             if (c0 >= n) break;
             it = c0;
@@ -1659,29 +1581,14 @@ __global__ void __launch_bounds__(kWave, 3) k_brick_exact(SubArgs A, const int32
         q_loaded = B.q;
         brick_tables(A, B, S);
         brick_blocks(A, B, S);
-        Certificate c;
-        c.sign = 0;
-        c.deps = 0;
-        if (certify) c = brick_certify(A, B, S);
-        record_certificate(A, B, S, b, c, sign, list, kCntDense, dbricks, dpairs, cnt);
+        const bool group = brick_in_group(B, S);
+        const int s = certify ? brick_certify(A, B, S, group) : 0;
+        if (lane == 0) {
+            sign[b] = int8_t(s);
+            if (s == 0) list[atomicAdd(cnt + kCntDense, 1)] = b;
+            else if (group) glist[atomicAdd(cnt + kCntGroup, 1)] = b;
+        }
     }
-}
-
-// The certified bricks with corners owned by other roots: certified only when
-// every brick they depend on carries the same sign; the others are listed
-// for the evaluation.
-__global__ void __launch_bounds__(kBlockS) k_brick_deps(const int32_t* dbricks, const int32_t* dpairs,
-                                                        const int8_t* sign, int32_t* list, int32_t* cnt) {
-    const int32_t e = blockIdx.x * kBlockS + threadIdx.x;
-    if (e >= cnt[kCntDepBricks]) return;
-    const int32_t b = dbricks[3 * e], first = dbricks[3 * e + 1], n = dbricks[3 * e + 2];
-    const int8_t sb = sign[b];
-    bool ok = true;
-    for (int t = 0; t < n; t++) {
-        const int32_t b2 = dpairs[first + t];
-        ok = ok && b2 >= 0 && sign[b2] == sb;
-    }
-    if (!ok) list[atomicAdd(cnt + kCntDense, 1)] = b;
 }
 
 // The corner values of the bricks the certificates left (grid_value): gv at
@@ -1782,25 +1689,58 @@ struct GroupMask {
     } NBR;
 };
 
-// An 8^3 brick's geometry and group, for the leaf passes (one thread per
-// leaf, every wave for itself).
+// An 8^3 brick's geometry and group, for passes without its root's record in
+// LDS (every wave for itself).
 __device__ __forceinline__ void brick_geometry(const SubArgs& A, int32_t b, Brick& B, GroupMask& S) {
-    const int D = A.D, lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63;
     B.q = __builtin_amdgcn_readfirstlane(A.bmap[b]);
     const int32_t* R = A.rec + int64_t(B.q) * kRecWords;
-    B.r = __builtin_amdgcn_readfirstlane(R[kRecR]);
-    const uint32_t rkey = uint32_t(__builtin_amdgcn_readfirstlane(R[kRecKey]));
-    B.kb = kBrickLog;
-    B.Sr = 1 << (D - B.r);
-    B.bkey = rkey | (uint32_t(b - A.boff[B.q]) << (3 * kBrickLog));
-    int32_t rc[3];
-    decode_cell(rkey, rc);
-    decode_cell(B.bkey, B.org);
-    for (int a = 0; a < 3; a++) {
-        B.R[a] = rc[a] >> (D - B.r);
-        B.R0[a] = rc[a];
-    }
+    cell_geometry(A, b, kBrickLog, R, B);
     S.NBR.m = uint32_t(__builtin_amdgcn_ballot_w64(lane < 27 && R[kRecNBR + (lane < 27 ? lane : 0)] >= 0));
+}
+
+// The settled bricks with corners that leaves of other roots of the group
+// own: settled only when every brick holding such an owner carries the same
+// sign; the others are listed for the evaluation.  The bricks around it in
+// other roots of the group include all of those, and mostly agree, so the
+// owners themselves are looked up only when one does not.
+__global__ void __launch_bounds__(kWave) k_group_check(SubArgs A, const int32_t* glist, const int8_t* sign,
+                                                       int32_t* list, int32_t* cnt) {
+    const int lane = threadIdx.x, D = A.D;
+    const int32_t n = cnt[kCntGroup];
+    for (int32_t it = blockIdx.x; it < n; it += int32_t(gridDim.x)) {
+        const int32_t b = glist[it];
+        Brick B;
+        GroupMask S;
+        brick_geometry(A, b, B, S);
+        // the brick at offset nidx = lane, when another root of the group holds it
+        bool other = false, differs = false;
+        if (lane < 27) {
+            int32_t cc[3];
+            int ro[3];
+            const int sh = D - B.r;
+            for (int a = 0; a < 3; a++) {
+                const int dv = (a == 0 ? lane / 9 : a == 1 ? (lane / 3) % 3 : lane % 3) - 1;
+                cc[a] = B.org[a] + (dv << kBrickLog);
+                ro[a] = (cc[a] >> sh) - B.R[a];
+            }
+            const int slot = nidx(ro[0], ro[1], ro[2]);
+            const int32_t q2 = slot == 13 ? -1 : A.rec[int64_t(B.q) * kRecWords + kRecNBR + slot];
+            if (q2 >= 0) {
+                const uint32_t rmask = 3 * sh >= 32 ? 0xffffffffu : ((1u << (3 * sh)) - 1u);
+                const uint32_t mort = cell_key(uint32_t(cc[0]), uint32_t(cc[1]), uint32_t(cc[2])) & rmask;
+                other = true;
+                differs = sign[A.boff[q2] + int32_t(mort >> (3 * kBrickLog))] != sign[b];
+            }
+        }
+        const uint64_t bad = __builtin_amdgcn_ballot_w64(differs);
+        if (bad == 0) continue;
+        const uint64_t around = __builtin_amdgcn_ballot_w64(other);
+        const uint32_t deps = brick_group_deps(B, S, D);
+        // (an owner in a brick outside the group's roots cannot be)
+        if ((deps & uint32_t(bad)) || (deps & ~uint32_t(around)))
+            if (lane == 0) list[atomicAdd(cnt + kCntDense, 1)] = b;
+    }
 }
 
 // Exclusive sum of v over the workgroup's 512 threads, and the total.
@@ -2247,6 +2187,22 @@ __global__ void __launch_bounds__(kWave) k_small_triangles(SubArgs A, const int3
 
 }  // namespace
 
+// Per depth, with the coefficients bounded by 1: the basis functions of three
+// cells sum to 4/3 along an axis, and a table value differs from the spline's
+// by at most t = corner_dev[d], so 27 products sum to at most
+// big = (4/3 + 3 t)^3 in absolute value, and differ from the spline's products
+// by at most 3 (3 t) (4/3 + 3 t)^2 in all.  A corner's float sum of
+// n <= 27 (D + 1) + 1 products of three roundings lies within (n + 3) 2^-24 of
+// its terms' absolute sum; the polynomial's own float sums within 300 of that
+// unit: 700 covers both.
+static void depth_bounds(const FsTables& fs, SubArgs* A) {
+    for (int d = 0; d <= kMaxDepth; d++) {
+        const double t = d <= fs.D ? double(fs.corner_dev[d]) : 0.0, m = 4.0 / 3.0 + 3.0 * t;
+        A->big[d] = float(1.001 * m * m * m);
+        A->dev[d] = float(1.001 * (9.0 * t * m * m + 700.0 * 5.9604645e-8 * m * m * m));
+    }
+}
+
 // the coarse rows of the current solution (mc.hip)
 int ensure_coarse_rows(prg_ctx* c, hipStream_t s);
 
@@ -2375,8 +2331,9 @@ void extract_subdivision(prg_ctx* c) {
                     reinterpret_cast<const float4*>(btab.get()), c->coarse_rows.get(), D,
                     c->iso_dev.get(),  roots.get(),     boff.get(),
                     root_of.get(),     C,               nullptr,
-                    nullptr};
+                    nullptr,           {},              {}};
 
+    depth_bounds(*c->fs, &A);
     // per-root records and the brick -> root map
     PoolBuf<int32_t> rec{&c->pool[127]}, bmap{&c->pool[128]};
     rec.reserve(size_t(nr) * kRecWords);
@@ -2395,13 +2352,14 @@ void extract_subdivision(prg_ctx* c) {
     bvoff.reserve(nb);
     btoff.reserve(nb);
     // pass 0: certificates; pass 1: counts of the bricks left
-    PoolBuf<int32_t> dlist{&c->pool[129]}, dbricks{&c->pool[130]}, dpairs{&c->pool[131]}, xlist{&c->pool[133]};
+    PoolBuf<int32_t> dlist{&c->pool[129]}, glist{&c->pool[130]}, xlist{&c->pool[133]}, cells{&c->pool[136]};
     PoolBuf<int8_t> bsign{&c->pool[132]};
     dlist.reserve(nb);
     xlist.reserve(nb);
-    dbricks.reserve(3 * nb);
-    dpairs.reserve(26 * nb);
+    glist.reserve(nb);
     bsign.reserve(nb);
+    k_clear_bricks<<<grid_for(nb, kBlockS), kBlockS, 0, s>>>(bnv.get(), bnt.get(), bsign.get(), nb);
+    PRG_CHECK_LAUNCH();
     // the small roots: values, cubes and counts
     const int32_t n1 = H[kCntSmall1], n2 = H[kCntSmall2];
     const int64_t nb3 = nb - n1 - n2;  // 8^3 bricks
@@ -2445,42 +2403,37 @@ void extract_subdivision(prg_ctx* c) {
     }
     if (nb3 > 0) {
         TimedScope ts(kt, "subdivide_screen", 0.0);  // latency- and issue-bound: no byte figure
-        // super-bricks of the roots with at least 8 bricks, then the brick
-        // screen over the bricks they leave and those of the smaller roots
-        PoolBuf<int32_t> nsup{&c->pool[136]}, soff{&c->pool[137]}, smap{&c->pool[138]}, list2{&c->pool[139]};
-        nsup.reserve(nr);
-        soff.reserve(nr);
-        smap.reserve(std::max<int64_t>(1, nb / 8));
-        list2.reserve(nb);
-        k_super_count<<<grid_for(nr, kBlockS), kBlockS, 0, s>>>(rbricks.get(), C, nr, nsup.get());
-        PRG_CHECK_LAUNCH();
-        scan_exclusive(nsup.get(), soff.get(), nr, C + kCntSuper, s, c->scratch, kt);
-        k_super_map<<<grid_for(std::max<int64_t>(1, nb / 8), kBlockS), kBlockS, 0, s>>>(soff.get(), C,
-                                                                                      std::max<int64_t>(1, nb / 8),
-                                                                                      smap.get());
-        PRG_CHECK_LAUNCH();
-        k_list_one_brick_roots<<<grid_for(nr, kBlockS), kBlockS, 0, s>>>(roots.get(), boff.get(), nr, Lv, D,
-                                                                          list2.get(), C);
+        // per size, at most as many cells as the bricks fill
+        CellLists lists{};
+        int64_t total = 0;
+        for (int k = kBrickLog; k < D; k++) total += (nb3 >> (3 * (k - kBrickLog))) + 1;
+        int32_t* at = cells.reserve(total);
+        for (int k = kBrickLog; k < D; k++) {
+            lists.at[k] = at;
+            at += (nb3 >> (3 * (k - kBrickLog))) + 1;
+        }
+        k_list_roots<<<grid_for(nr, kBlockS), kBlockS, 0, s>>>(roots.get(), boff.get(), nr, Lv, D, lists, C);
         PRG_CHECK_LAUNCH();
         // resident grids: every workgroup walks its share
-        int per_cu = 0;
-        PRG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_brick_screen_super, kWave, 0));
-        int64_t grid = std::min<int64_t>(std::max<int64_t>(1, nb / 8), int64_t(std::max(1, per_cu)) * std::max(1, c->num_cu));
-        k_brick_screen_super<<<unsigned(grid), kWave, 0, s>>>(A, smap.get(), soff.get(), bnv.get(), bnt.get(),
-                                                              bsign.get(), list2.get(), C, int(c->sub_certify));
+        auto resident = [&](const void* kernel, int64_t most) {
+            int per_cu = 0;
+            PRG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kWave, 0));
+            return unsigned(std::max<int64_t>(1, std::min<int64_t>(most, int64_t(std::max(1, per_cu)) * c->num_cu)));
+        };
+        // largest root: no cell is larger
+        int kmax = D - 1;
+        while (kmax > kBrickLog && (int64_t(1) << (3 * (kmax - kBrickLog))) > nb3) kmax--;
+        for (int k = kmax; k >= kBrickLog; k--) {
+            k_cell_screen<<<resident(reinterpret_cast<const void*>(k_cell_screen), (nb3 >> (3 * (k - kBrickLog))) + 1),
+                            kWave, 0, s>>>(A, k, lists.at[k], k > kBrickLog ? lists.at[k - 1] : nullptr, xlist.get(),
+                                           bsign.get(), glist.get(), C, int(c->sub_certify));
+            PRG_CHECK_LAUNCH();
+        }
+        k_brick_exact<<<resident(reinterpret_cast<const void*>(k_brick_exact), nb3), kWave, 0, s>>>(
+            A, xlist.get(), bsign.get(), dlist.get(), glist.get(), C, int(c->sub_certify));
         PRG_CHECK_LAUNCH();
-        PRG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_brick_screen, kWave, 0));
-        grid = std::min<int64_t>(nb, int64_t(std::max(1, per_cu)) * std::max(1, c->num_cu));
-        k_brick_screen<<<unsigned(grid), kWave, 0, s>>>(A, list2.get(), bnv.get(), bnt.get(), bsign.get(), xlist.get(),
-                                                        dbricks.get(), dpairs.get(), C, int(c->sub_certify));
-        PRG_CHECK_LAUNCH();
-        PRG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_brick_exact, kWave, 0));
-        grid = std::min<int64_t>(nb, int64_t(std::max(1, per_cu)) * std::max(1, c->num_cu));
-        k_brick_exact<<<unsigned(grid), kWave, 0, s>>>(A, xlist.get(), bsign.get(), dlist.get(), dbricks.get(),
-                                                       dpairs.get(), C, int(c->sub_certify));
-        PRG_CHECK_LAUNCH();
-        k_brick_deps<<<grid_for(nb, kBlockS), kBlockS, 0, s>>>(dbricks.get(), dpairs.get(), bsign.get(),
-                                                                dlist.get(), C);
+        k_group_check<<<resident(reinterpret_cast<const void*>(k_group_check), nb3), kWave, 0, s>>>(
+            A, glist.get(), bsign.get(), dlist.get(), C);
         PRG_CHECK_LAUNCH();
     }
     if (nb3 > 0) {
