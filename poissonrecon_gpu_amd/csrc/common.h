@@ -184,6 +184,8 @@ struct Scratch;  // grows on demand
 // two arrays of the same length (exclusive scans and totals), in one pass each
 void scan_exclusive2(const int32_t* a_in, int32_t* a_out, int32_t* a_total, const int32_t* b_in, int32_t* b_out,
                      int32_t* b_total, int64_t n, hipStream_t s, Scratch& scratch, KernelTimer& kt);
+// the state of the single-pass scans of one stream, with room for `words` tiles
+uint64_t* look_state(Scratch& scratch, int64_t words, hipStream_t s);
 void scan_exclusive(const int32_t* d_in, int32_t* d_out, int64_t n, int32_t* d_total, hipStream_t s,
                     Scratch& scratch, KernelTimer& kt);
 // Stable LSD radix sort of (key, value) pairs on the low `bits` bits of the key.
@@ -192,7 +194,8 @@ void radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32
                       int bits, hipStream_t s, Scratch& scratch, KernelTimer& kt);
 
 struct Scratch {
-    DBuf<int32_t> a, b, c;
+    DBuf<uint64_t> look;  // the single-pass scans' state (look_state)
+    DBuf<int32_t> b, c;
     DBuf<uint8_t> bytes;
 };
 

@@ -20,6 +20,7 @@
 #include <cmath>
 
 #include "ctx.h"
+#include "lookback.h"
 #include "pnt.h"
 
 namespace prg {
@@ -196,27 +197,55 @@ __global__ void __launch_bounds__(kBlock) k_gather_points(const uint32_t* perm, 
     nz[r] = b.y;
 }
 
-// run heads of the sorted keys (generateMark, main.cu:195-211)
-__global__ void __launch_bounds__(kBlock) k_heads(const uint32_t* key, int64_t n, int shift, int32_t* flag) {
-    const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-    if (i >= n) return;
-    flag[i] = (i == 0 || (key[i] >> shift) != (key[i - 1] >> shift)) ? 1 : 0;
-}
-
-// the same over the first *count of ub entries (0 beyond)
-__global__ void __launch_bounds__(kBlock) k_unique(const uint32_t* key, const int32_t* flag, const int32_t* rank,
-                                                   int64_t n, uint32_t* uk, int32_t* upidx) {
-    const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-    if (i >= n || !flag[i]) return;
-    uk[rank[i]] = key[i];
-    upidx[rank[i]] = int32_t(i);
-}
-
-// exclusive head count -> index of the run containing each element
-__global__ void __launch_bounds__(kBlock) k_excl_to_incl(int32_t* out, const int32_t* excl, const int32_t* flag,
-                                                         int64_t n) {
-    const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-    if (i < n) out[i] = excl[i] + flag[i] - 1;
+// Run heads of the sorted keys (generateMark, main.cu:195-211), their scan and
+// the unique leaves in one pass (lookback.h): rank[i] = the run of sorted point
+// i, and per run its key and first point; the number of runs to *count.
+constexpr int kRunItems = 16;
+constexpr int kRunTile = kBlock * kRunItems;
+__global__ void __launch_bounds__(kBlock) k_unique(const uint32_t* __restrict__ key, int64_t n, uint32_t tiles,
+                                                   uint64_t* state, int32_t* __restrict__ rank,
+                                                   uint32_t* __restrict__ uk, int32_t* __restrict__ upidx,
+                                                   int32_t* count) {
+    __shared__ int32_t lds[kBlock / 64];
+    __shared__ int32_t s_before;
+    const LookTile t = look_begin(state, tiles);
+    if (t.tile >= tiles) return;
+    const int64_t base = int64_t(t.tile) * kRunTile + int64_t(threadIdx.x) * kRunItems;
+    uint32_t k[kRunItems];
+    const uint32_t prev = base > 0 && base - 1 < n ? key[base - 1] : 0u;
+    if (base + kRunItems <= n) {
+#pragma unroll
+        for (int j = 0; j < kRunItems; j += 4) *reinterpret_cast<uint4*>(k + j) = *reinterpret_cast<const uint4*>(key + base + j);
+    } else {
+#pragma unroll
+        for (int j = 0; j < kRunItems; j++) k[j] = base + j < n ? key[base + j] : 0u;
+    }
+    uint32_t heads = 0;
+#pragma unroll
+    for (int j = 0; j < kRunItems; j++)
+        if (base + j < n && (base + j == 0 || k[j] != (j ? k[j - 1] : prev))) heads |= 1u << j;
+    int32_t total;
+    const int32_t ex = block_exclusive_scan(__popc(heads), lds, total);
+    if (threadIdx.x < 64) {
+        const int32_t b = look_back(state + kLookHeader, t, tiles, total);
+        if (threadIdx.x == 0) {
+            s_before = b;
+            if (t.tile == tiles - 1) *count = b + total;
+        }
+    }
+    __syncthreads();
+    look_end(state, t, tiles);
+    int32_t r = s_before + ex - 1;
+#pragma unroll
+    for (int j = 0; j < kRunItems; j++) {
+        if (base + j >= n) break;
+        if ((heads >> j) & 1u) {
+            r++;
+            uk[r] = k[j];
+            upidx[r] = int32_t(base + j);
+        }
+        rank[base + j] = r;
+    }
 }
 
 __device__ __forceinline__ void level_init_slot(int64_t base, int64_t s, bool leaf, int32_t* pnum, int32_t* dnum,
@@ -224,13 +253,6 @@ __device__ __forceinline__ void level_init_slot(int64_t base, int64_t s, bool le
     pnum[base + s] = 0;
     dnum[base + s] = leaf ? 1 : 0;
     child_base[base + s] = -1;
-}
-
-__global__ void __launch_bounds__(kBlock) k_level_init(int64_t base, int64_t count, bool leaf, int32_t* pnum,
-                                                       int32_t* dnum, int32_t* child_base) {
-    const int64_t s = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-    if (s >= count) return;
-    level_init_slot(base, s, leaf, pnum, dnum, child_base);
 }
 
 // Scatter the non-empty nodes of depth d into their slots.
@@ -254,18 +276,6 @@ __device__ __forceinline__ void level_scatter_node(int64_t q, const uint32_t* nk
     }
 }
 
-__global__ void __launch_bounds__(kBlock) k_level_scatter(const uint32_t* nk, const int32_t* np, const int32_t* ndi,
-                                                          const int32_t* pos, int64_t ne, int64_t npoints,
-                                                          int64_t nleaf_slots, bool leaf, int64_t base,
-                                                          int64_t child_level_base, uint32_t* key, int32_t* pidx,
-                                                          int32_t* pnum, int32_t* didx, int32_t* dnum,
-                                                          int32_t* child_base) {
-    const int64_t q = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-    if (q >= ne) return;
-    level_scatter_node(q, nk, np, ndi, pos, ne, npoints, nleaf_slots, leaf, base, child_level_base, key, pidx, pnum,
-                       didx, dnum, child_base);
-}
-
 // Every slot of depth d: key, running pidx / didx inside the sibling block and
 // the parent index (updateEmptyNodeInfo's intent, main.cu:433-490).
 __device__ __forceinline__ void level_fill_slot(int64_t s, const uint32_t* pk, const int32_t* pp,
@@ -285,16 +295,6 @@ __device__ __forceinline__ void level_fill_slot(int64_t s, const uint32_t* pk, c
     pidx[g] = run_p;
     didx[g] = (d != D) ? run_d : int32_t(s);  // leaf level: every slot is its own first leaf slot
     parent[g] = int32_t(parent_base + ppos[b]);
-}
-
-__global__ void __launch_bounds__(kBlock) k_level_fill(const uint32_t* pk, const int32_t* pp, const int32_t* pdi,
-                                                       const int32_t* ppos, int64_t count, int D, int d, int64_t base,
-                                                       int64_t parent_base, uint32_t* key, int32_t* pidx,
-                                                       const int32_t* pnum, int32_t* didx, const int32_t* dnum,
-                                                       int32_t* parent) {
-    const int64_t s = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-    if (s >= count) return;
-    level_fill_slot(s, pk, pp, pdi, ppos, D, d, base, parent_base, key, pidx, pnum, didx, dnum, parent);
 }
 
 __global__ void __launch_bounds__(kBlock) k_point_leaf(const int32_t* rank, const int32_t* pos_leaf, int64_t n,
@@ -361,13 +361,12 @@ __global__ void __launch_bounds__(kBlock) k_parent_neighbor_table(const int32_t*
     pnt_block(b, parent, child_base, pnt_prev, base_prev, base, pnt);
 }
 
-// ---- the bottom-up step of a large depth in three launches ---------------------------
+// ---- the bottom-up step of a large depth in one launch -------------------------------
 // The non-empty nodes of depth d (compact, key order) give their slot in the
 // depth-d level array and the compact arrays of depth d - 1: the parent-run
-// heads are counted per tile, the tile counts scanned (their total is the
-// parent depth's non-empty count), and the apply pass recomputes the heads,
-// scans them inside the tile and writes each node's slot and, per head, its
-// parent's key, first point and first leaf-level slot.
+// heads are scanned (lookback.h; their number is the parent depth's non-empty
+// count), and each node's slot and, per head, its parent's key, first point
+// and first leaf-level slot are written.
 constexpr int kLvlBlock = 256;
 constexpr int kLvlItems = 8;
 constexpr int kLvlTile = kLvlBlock * kLvlItems;
@@ -376,60 +375,15 @@ __device__ __forceinline__ int32_t head_flag(const uint32_t* nk, int64_t i, int6
     return (i < n && (i == 0 || (nk[i] >> hs) != (nk[i - 1] >> hs))) ? 1 : 0;
 }
 
-// exclusive scan of one value per thread over the workgroup, and its total
-__device__ __forceinline__ int32_t lvl_block_scan(int32_t v, int32_t* lds, int32_t& total) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int32_t x = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int32_t y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
-    if (lane == 63) lds[wave] = x;
-    __syncthreads();
-    int32_t before = 0, tot = 0;
-    for (int w = 0; w < int(blockDim.x >> 6); w++) {
-        const int32_t t = lds[w];
-        if (w < wave) before += t;
-        tot += t;
-    }
-    __syncthreads();
-    total = tot;
-    return before + x - v;
-}
-
-__global__ void __launch_bounds__(kLvlBlock) k_lvl_reduce(const uint32_t* nk, const int32_t* ne, int hs,
-                                                          int32_t* sums) {
+__global__ void __launch_bounds__(kLvlBlock) k_level_up(const uint32_t* nk, const int32_t* np, const int32_t* ndi,
+                                                        int32_t* ne, int hs, int D, int d, uint32_t tiles,
+                                                        uint64_t* state, int32_t* pos, uint32_t* pk, int32_t* pp,
+                                                        int32_t* pdi) {
     __shared__ int32_t lds[kLvlBlock / 64];
-    const int64_t n = *ne, base = int64_t(blockIdx.x) * kLvlTile;
-    int32_t acc = 0;
-#pragma unroll
-    for (int k = 0; k < kLvlItems; k++) acc += head_flag(nk, base + int64_t(k) * kLvlBlock + threadIdx.x, n, hs);
-    int32_t tot;
-    (void)lvl_block_scan(acc, lds, tot);
-    if (threadIdx.x == 0) sums[blockIdx.x] = tot;
-}
-
-// single workgroup: exclusive scan of the tile counts in place, total to *ne_parent
-__global__ void __launch_bounds__(1024) k_lvl_sums(int32_t* sums, int64_t tiles, int32_t* ne_parent) {
-    __shared__ int32_t lds[16];
-    int32_t carry = 0;
-    for (int64_t base = 0; base < tiles; base += 1024) {
-        const int64_t i = base + threadIdx.x;
-        const int32_t v = i < tiles ? sums[i] : 0;
-        int32_t tot;
-        const int32_t ex = lvl_block_scan(v, lds, tot);
-        if (i < tiles) sums[i] = carry + ex;
-        carry += tot;
-    }
-    if (threadIdx.x == 0) *ne_parent = carry;
-}
-
-__global__ void __launch_bounds__(kLvlBlock) k_lvl_apply(const uint32_t* nk, const int32_t* np, const int32_t* ndi,
-                                                         const int32_t* ne, int hs, int D, int d, const int32_t* sums,
-                                                         int32_t* pos, uint32_t* pk, int32_t* pp, int32_t* pdi) {
-    __shared__ int32_t lds[kLvlBlock / 64];
-    const int64_t n = *ne, base = int64_t(blockIdx.x) * kLvlTile + int64_t(threadIdx.x) * kLvlItems;
+    __shared__ int32_t s_before;
+    const LookTile t = look_begin(state, tiles);
+    if (t.tile >= tiles) return;
+    const int64_t n = ne[d], base = int64_t(t.tile) * kLvlTile + int64_t(threadIdx.x) * kLvlItems;
     const int sh = 3 * (D - d);
     int32_t f[kLvlItems];
     int32_t acc = 0;
@@ -439,7 +393,17 @@ __global__ void __launch_bounds__(kLvlBlock) k_lvl_apply(const uint32_t* nk, con
         acc += f[k];
     }
     int32_t tot;
-    int32_t ex = lvl_block_scan(acc, lds, tot) + sums[blockIdx.x];
+    int32_t ex = block_exclusive_scan(acc, lds, tot);
+    if (threadIdx.x < 64) {
+        const int32_t b = look_back(state + kLookHeader, t, tiles, tot);
+        if (threadIdx.x == 0) {
+            s_before = b;
+            if (t.tile == tiles - 1) ne[d - 1] = b + tot;
+        }
+    }
+    __syncthreads();
+    look_end(state, t, tiles);
+    ex += s_before;
 #pragma unroll
     for (int k = 0; k < kLvlItems; k++) {
         const int64_t i = base + k;
@@ -471,13 +435,14 @@ struct LevelArrays {
     int32_t* pos[kMaxDepth + 1];  // and slot in the depth's level array
 };
 
-// The bottom-up step (k_lvl_reduce, k_lvl_sums, k_lvl_apply) for depths
+// The bottom-up step (k_level_up) for depths
 // ds .. 1: per depth, chunks of the compact nodes with a workgroup scan of
 // the parent-run heads carried across chunks.
 __global__ void __launch_bounds__(kSmallThreads) k_levels_up_small(LevelArrays A, int32_t* ne, int ds, int D) {
     __shared__ int32_t sc[kSmallThreads];
     __shared__ int32_t carry;
     const int tid = threadIdx.x;
+    if (tid == 0) A.pos[0][0] = 0;  // the root's slot
     for (int d = ds; d >= 1; --d) {
         const int64_t n = ne[d];
         const int hs = 3 * (D - d + 1), sh = 3 * (D - d);
@@ -522,9 +487,47 @@ struct SmallLevels {
     int64_t base[kMaxDepth + 1], count[kMaxDepth + 1], ne[kMaxDepth + 1], pnt_off[kMaxDepth + 2];
 };
 
-// Root, then for depths 1 .. df: slot defaults and non-empty nodes (k_level_init,
-// k_level_scatter), every slot's fields (k_level_fill) and the parent-neighbour
-// rows (k_parent_neighbor_table, top-down).
+// The depths df + 1 .. D in one launch per step: slot defaults of the nodes
+// base[df + 1] .. M, the non-empty nodes into their slots (thread t takes
+// compact node t of the depths' concatenation), every slot's fields.  A launch
+// per depth and step was 15 of them at depth 10, most a few workgroups.
+__global__ void __launch_bounds__(kBlock) k_levels_init(int64_t base, int64_t M, int64_t baseD, int32_t* pnum,
+                                                        int32_t* dnum, int32_t* child_base) {
+    const int64_t g = base + int64_t(blockIdx.x) * kBlock + threadIdx.x;
+    if (g < M) level_init_slot(0, g, g >= baseD, pnum, dnum, child_base);
+}
+
+__global__ void __launch_bounds__(kBlock) k_levels_scatter(LevelArrays A, SmallLevels S, int df, int D,
+                                                           int64_t npoints, int64_t MD, uint32_t* key, int32_t* pidx,
+                                                           int32_t* pnum, int32_t* didx, int32_t* dnum,
+                                                           int32_t* child_base) {
+    int64_t q = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+    for (int d = df + 1; d <= D; d++) {
+        if (q < S.ne[d]) {
+            level_scatter_node(q, A.nk[d], A.np[d], A.ndi[d], A.pos[d], S.ne[d], npoints, MD, d == D, S.base[d],
+                               d == D ? 0 : S.base[d + 1], key, pidx, pnum, didx, dnum, child_base);
+            return;
+        }
+        q -= S.ne[d];
+    }
+}
+
+__global__ void __launch_bounds__(kBlock) k_levels_fill(LevelArrays A, SmallLevels S, int df, int D, uint32_t* key,
+                                                        int32_t* pidx, const int32_t* pnum, int32_t* didx,
+                                                        const int32_t* dnum, int32_t* parent) {
+    int64_t s = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+    for (int d = df + 1; d <= D; d++) {
+        if (s < S.count[d]) {
+            level_fill_slot(s, A.nk[d - 1], A.np[d - 1], A.ndi[d - 1], A.pos[d - 1], D, d, S.base[d], S.base[d - 1],
+                            key, pidx, pnum, didx, dnum, parent);
+            return;
+        }
+        s -= S.count[d];
+    }
+}
+
+// Root, then for depths 1 .. df: slot defaults, non-empty nodes, every slot's
+// fields and the parent-neighbour rows (k_parent_neighbor_table, top-down).
 __global__ void __launch_bounds__(kSmallThreads) k_levels_small(LevelArrays A, SmallLevels S, int df, int D,
                                                                 int64_t M, int64_t npoints, int64_t MD,
                                                                 uint32_t* key, int32_t* pidx, int32_t* pnum,
@@ -669,18 +672,10 @@ void build_octree(prg_ctx* c) {
     c->points_sorted = true;
 
     // 2. unique leaves
-    PoolBuf<int32_t> flag{&c->pool[7]}, rank{&c->pool[8]}, tot{&c->pool[9]};
-    flag.reserve(n);
+    PoolBuf<int32_t> rank{&c->pool[8]};  // unique-leaf rank of every sorted point
     rank.reserve(n);
-    tot.reserve(1);
-    {
-        TimedScope ts(kt, "heads", 12.0 * double(n));
-        k_heads<<<grid_for(n, kBlock), kBlock, 0, s>>>(key.get(), n, 0, flag.get());
-        PRG_CHECK_LAUNCH();
-    }
     PoolBuf<int32_t> ne_dev{&c->pool[14]};  // non-empty nodes per depth
     ne_dev.reserve(D + 1);
-    scan_exclusive(flag.get(), rank.get(), n, ne_dev.get() + D, s, c->scratch, kt);
     // upper bounds of the non-empty node counts, min(n, 8^d): the unique
     // leaves number at most n, and the counts stay on the device until the
     // levels are built
@@ -704,12 +699,12 @@ void build_octree(prg_ctx* c) {
     NDI[D]->reserve(U);
     {
         TimedScope ts(kt, "unique", 16.0 * double(n));
-        k_unique<<<grid_for(n, kBlock), kBlock, 0, s>>>(key.get(), flag.get(), rank.get(), n, NK[D]->get(),
-                                                         NP[D]->get());
+        const int64_t tiles = (n + kRunTile - 1) / kRunTile;
+        uint64_t* state = look_state(c->scratch, tiles, s);
+        k_unique<<<unsigned(tiles), kBlock, 0, s>>>(key.get(), n, uint32_t(tiles), state, rank.get(), NK[D]->get(),
+                                                    NP[D]->get(), ne_dev.get() + D);
         PRG_CHECK_LAUNCH();
     }
-    PoolBuf<int32_t> prank{&c->pool[10]};  // unique-leaf rank of every sorted point
-    prank.reserve(n);
 
     // 3. levels bottom-up: sizes stay on the device (upper bounds size the
     // launches); one read-back after the loop
@@ -717,23 +712,18 @@ void build_octree(prg_ctx* c) {
     // depths ds .. 1 (at most kSmallLevelUp non-empty nodes each) in one launch
     int ds = 0;
     while (ds < D && ub[ds + 1] <= kSmallLevelUp) ds++;
-    PoolBuf<int32_t> lsums{&c->pool[95]};
     for (int d = D; d > ds; --d) {
         NK[d - 1]->reserve(ub[d - 1]);
         NP[d - 1]->reserve(ub[d - 1]);
         NDI[d - 1]->reserve(ub[d - 1]);
         POS[d]->reserve(ub[d]);
         const int64_t tiles = (ub[d] + kLvlTile - 1) / kLvlTile;
-        int32_t* sums = lsums.reserve(tiles);
+        uint64_t* state = look_state(c->scratch, tiles, s);
         const int hs = 3 * (D - d + 1);
         TimedScope ts(kt, "level_up", 28.0 * double(ub[d]));
-        k_lvl_reduce<<<unsigned(tiles), kLvlBlock, 0, s>>>(NK[d]->get(), ne_dev.get() + d, hs, sums);
-        PRG_CHECK_LAUNCH();
-        k_lvl_sums<<<1, 1024, 0, s>>>(sums, tiles, ne_dev.get() + d - 1);
-        PRG_CHECK_LAUNCH();
-        k_lvl_apply<<<unsigned(tiles), kLvlBlock, 0, s>>>(NK[d]->get(), NP[d]->get(), NDI[d]->get(),
-                                                           ne_dev.get() + d, hs, D, d, sums, POS[d]->get(),
-                                                           NK[d - 1]->get(), NP[d - 1]->get(), NDI[d - 1]->get());
+        k_level_up<<<unsigned(tiles), kLvlBlock, 0, s>>>(NK[d]->get(), NP[d]->get(), NDI[d]->get(), ne_dev.get(), hs, D,
+                                                         d, uint32_t(tiles), state, POS[d]->get(), NK[d - 1]->get(),
+                                                         NP[d - 1]->get(), NDI[d - 1]->get());
         PRG_CHECK_LAUNCH();
     }
     LevelArrays LA{};
@@ -750,7 +740,8 @@ void build_octree(prg_ctx* c) {
         LA.ndi[d] = NDI[d]->get();
         LA.pos[d] = POS[d]->get();
     }
-    if (ds >= 1) {
+    {
+        // (ds >= 1: depth 1 has at most 8 nodes)
         TimedScope ts(kt, "level_up_small", 28.0 * double(ub[ds]));
         k_levels_up_small<<<1, kSmallThreads, 0, s>>>(LA, ne_dev.get(), ds, D);
         PRG_CHECK_LAUNCH();
@@ -768,9 +759,6 @@ void build_octree(prg_ctx* c) {
         for (int d = 1; d <= D; d++) counts[d] = 8 * NE[d - 1];
     }
     counts[0] = 1;
-    // root compact arrays: key 0, pidx 0, didx 0, slot 0
-    PRG_HIP(hipMemsetAsync(POS[0]->get(), 0, 4, s));
-
     std::vector<int64_t> bases(D + 1, 0);
     for (int d = 1; d <= D; d++) bases[d] = bases[d - 1] + counts[d - 1];
     const int64_t M = bases[D] + counts[D];
@@ -793,42 +781,34 @@ void build_octree(prg_ctx* c) {
     // parent-neighbour rows in one launch
     int df = 0;
     while (df < D && counts[df + 1] <= kSmallLevelSlots) df++;
+    SmallLevels SL{};
+    for (int d = 0; d <= D; d++) {
+        SL.base[d] = bases[d];
+        SL.count[d] = counts[d];
+        SL.ne[d] = NE[d];
+    }
+    for (int d = 0; d <= D + 1; d++) SL.pnt_off[d] = c->pnt_off[d];
     {
-        SmallLevels SL{};
-        for (int d = 0; d <= D; d++) {
-            SL.base[d] = bases[d];
-            SL.count[d] = counts[d];
-            SL.ne[d] = NE[d];
-        }
-        for (int d = 0; d <= D + 1; d++) SL.pnt_off[d] = c->pnt_off[d];
         TimedScope ts(kt, "levels_small", 44.0 * double(bases[df] + counts[df]));
         k_levels_small<<<1, kSmallThreads, 0, s>>>(LA, SL, df, D, M, n, MD, K, PI, PN, PA, CB, DI, DN, PT);
         PRG_CHECK_LAUNCH();
     }
-    {
+    if (df < D) {
         TimedScope ts(kt, "levels_fill", 44.0 * double(M));
-        for (int d = df + 1; d <= D; d++) {
-            const bool leaf = (d == D);
-            k_level_init<<<grid_for(counts[d], kBlock), kBlock, 0, s>>>(bases[d], counts[d], leaf, PN, DN, CB);
-            PRG_CHECK_LAUNCH();
-            k_level_scatter<<<grid_for(NE[d], kBlock), kBlock, 0, s>>>(
-                NK[d]->get(), NP[d]->get(), NDI[d]->get(), POS[d]->get(), NE[d], n, MD, leaf, bases[d],
-                leaf ? 0 : bases[d + 1], K, PI, PN, DI, DN, CB);
-            PRG_CHECK_LAUNCH();
-        }
-        for (int d = df + 1; d <= D; d++) {
-            k_level_fill<<<grid_for(counts[d], kBlock), kBlock, 0, s>>>(
-                NK[d - 1]->get(), NP[d - 1]->get(), NDI[d - 1]->get(), POS[d - 1]->get(), counts[d], D, d,
-                bases[d], bases[d - 1], K, PI, PN, DI, DN, PA);
-            PRG_CHECK_LAUNCH();
-        }
+        const int64_t slots = M - bases[df + 1];
+        int64_t nodes = 0;
+        for (int d = df + 1; d <= D; d++) nodes += NE[d];
+        k_levels_init<<<grid_for(slots, kBlock), kBlock, 0, s>>>(bases[df + 1], M, bases[D], PN, DN, CB);
+        PRG_CHECK_LAUNCH();
+        k_levels_scatter<<<grid_for(nodes, kBlock), kBlock, 0, s>>>(LA, SL, df, D, n, MD, K, PI, PN, DI, DN, CB);
+        PRG_CHECK_LAUNCH();
+        k_levels_fill<<<grid_for(slots, kBlock), kBlock, 0, s>>>(LA, SL, df, D, K, PI, PN, DI, DN, PA);
+        PRG_CHECK_LAUNCH();
     }
     // point -> leaf-level slot: rank of the run containing each sorted point
     {
         TimedScope ts(kt, "point_leaf", 12.0 * double(n));
-        k_excl_to_incl<<<grid_for(n, kBlock), kBlock, 0, s>>>(prank.get(), rank.get(), flag.get(), n);
-        PRG_CHECK_LAUNCH();
-        k_point_leaf<<<grid_for(n, kBlock), kBlock, 0, s>>>(prank.get(), POS[D]->get(), n, c->point_leaf.reserve(n));
+        k_point_leaf<<<grid_for(n, kBlock), kBlock, 0, s>>>(rank.get(), POS[D]->get(), n, c->point_leaf.reserve(n));
         PRG_CHECK_LAUNCH();
     }
     // 4. parent-neighbour tables (depths 1..D), top-down; the 27-plane

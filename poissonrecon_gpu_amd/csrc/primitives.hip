@@ -1,5 +1,5 @@
-// Device-wide primitives: exclusive scan of int32 and a stable LSD radix sort
-// of (uint32 key, uint32 value) pairs.
+// Device-wide primitives: exclusive scan of int32 (single-pass, lookback.h) and
+// a stable LSD radix sort of (uint32 key, uint32 value) pairs.
 //
 // Radix sort, one 8-bit digit per pass (3D key bits -> ceil(3D/8) passes):
 //   upsweep   - each workgroup counts the digits of its 4096-key tile in LDS
@@ -13,159 +13,81 @@
 //               stores are contiguous.
 // Stability holds because waves own consecutive sub-tiles, items are visited
 // in input order and tiles are laid out digit-major in the scan.
-#include "common.h"
+#include "lookback.h"
 
 namespace prg {
 namespace {
 
 constexpr int kScanBlock = 256;
-constexpr int kScanItems = 8;
+constexpr int kScanItems = 16;  // consecutive elements per thread
 constexpr int kScanTile = kScanBlock * kScanItems;
 
-__device__ inline int32_t block_exclusive_scan(int32_t v, int32_t* lds_waves, int32_t& total) {
-    // wave-level inclusive scan
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int32_t x = v;
+// v[k] = in[base + k], 0 from n on; `wide`: 16-byte loads where all are in range
+__device__ __forceinline__ int32_t load_items(const int32_t* __restrict__ in, int64_t base, int64_t n, bool wide,
+                                              int32_t v[kScanItems]) {
+    if (wide && base + kScanItems <= n) {
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        int32_t y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
+        for (int k = 0; k < kScanItems; k += 4) *reinterpret_cast<int4*>(v + k) = *reinterpret_cast<const int4*>(in + base + k);
+    } else {
+#pragma unroll
+        for (int k = 0; k < kScanItems; k++) v[k] = base + k < n ? in[base + k] : 0;
     }
-    if (lane == 63) lds_waves[wave] = x;
-    __syncthreads();
-    const int nw = blockDim.x >> 6;
-    int32_t wsum = 0, tot = 0;
-    for (int w = 0; w < nw; w++) {
-        int32_t t = lds_waves[w];
-        if (w < wave) wsum += t;
-        tot += t;
-    }
-    __syncthreads();
-    total = tot;
-    return wsum + x - v;
+    int32_t s = 0;
+#pragma unroll
+    for (int k = 0; k < kScanItems; k++) s += v[k];
+    return s;
 }
 
-__global__ void __launch_bounds__(kScanBlock) k_scan_reduce(const int32_t* in, int64_t n, int32_t* sums) {
-    __shared__ int32_t w[kScanBlock / 64];
-    const int64_t base = int64_t(blockIdx.x) * kScanTile;
-    int32_t acc = 0;
+__device__ __forceinline__ void store_items(int32_t* __restrict__ out, int64_t base, int64_t n, bool wide, int32_t ex,
+                                            int32_t v[kScanItems]) {
 #pragma unroll
     for (int k = 0; k < kScanItems; k++) {
-        int64_t i = base + k * kScanBlock + threadIdx.x;
-        if (i < n) acc += in[i];
+        const int32_t t = v[k];
+        v[k] = ex;
+        ex += t;
     }
-    int32_t tot;
-    (void)block_exclusive_scan(acc, w, tot);
-    if (threadIdx.x == 0) sums[blockIdx.x] = tot;
-}
-
-// Single workgroup: exclusive scan of the tile sums, in chunks with a carry.
-__global__ void __launch_bounds__(1024) k_scan_sums(int32_t* sums, int64_t n, int32_t* d_total) {
-    __shared__ int32_t w[16];
-    int32_t carry = 0;
-    for (int64_t base = 0; base < n; base += 1024) {
-        int64_t i = base + threadIdx.x;
-        int32_t v = (i < n) ? sums[i] : 0;
-        int32_t tot;
-        int32_t ex = block_exclusive_scan(v, w, tot);
-        if (i < n) sums[i] = carry + ex;
-        carry += tot;
-    }
-    if (threadIdx.x == 0 && d_total) *d_total = carry;
-}
-
-__global__ void __launch_bounds__(kScanBlock) k_scan_apply(const int32_t* in, int32_t* out, int64_t n,
-                                                             const int32_t* sums) {
-    __shared__ int32_t w[kScanBlock / 64];
-    const int64_t base = int64_t(blockIdx.x) * kScanTile;
-    // each thread owns kScanItems consecutive elements
-    int32_t v[kScanItems];
-    int32_t acc = 0;
+    if (wide && base + kScanItems <= n) {
 #pragma unroll
-    for (int k = 0; k < kScanItems; k++) {
-        int64_t i = base + int64_t(threadIdx.x) * kScanItems + k;
-        v[k] = (i < n) ? in[i] : 0;
-        acc += v[k];
-    }
-    int32_t tot;
-    int32_t ex = block_exclusive_scan(acc, w, tot) + sums[blockIdx.x];
+        for (int k = 0; k < kScanItems; k += 4) *reinterpret_cast<int4*>(out + base + k) = *reinterpret_cast<int4*>(v + k);
+    } else {
 #pragma unroll
-    for (int k = 0; k < kScanItems; k++) {
-        int64_t i = base + int64_t(threadIdx.x) * kScanItems + k;
-        if (i < n) out[i] = ex;
-        ex += v[k];
+        for (int k = 0; k < kScanItems; k++)
+            if (base + k < n) out[base + k] = v[k];
     }
 }
 
-// Two arrays of the same length scanned together: one reduce, one
-// two-workgroup sums pass and one apply (sums_a, sums_b: the tile sums).
-__global__ void __launch_bounds__(kScanBlock) k_scan_reduce2(const int32_t* in_a, const int32_t* in_b, int64_t n,
-                                                               int32_t* sums_a, int32_t* sums_b) {
+// Exclusive scan of one array, or of two of the same length (TWO), in one
+// launch (lookback.h).  Bound by its launch (about 4 us) up to about 10^5
+// elements, then by the memory it reads and writes once.
+template <bool TWO>
+__global__ void __launch_bounds__(kScanBlock) k_scan(const int32_t* in_a, int32_t* out_a, int32_t* total_a,
+                                                     const int32_t* in_b, int32_t* out_b, int32_t* total_b, int64_t n,
+                                                     uint32_t tiles, bool wide, uint64_t* state) {
     __shared__ int32_t w[kScanBlock / 64];
-    const int64_t base = int64_t(blockIdx.x) * kScanTile;
-    int32_t acc_a = 0, acc_b = 0;
-#pragma unroll
-    for (int k = 0; k < kScanItems; k++) {
-        int64_t i = base + k * kScanBlock + threadIdx.x;
-        if (i < n) {
-            acc_a += in_a[i];
-            acc_b += in_b[i];
-        }
-    }
-    int32_t tot_a, tot_b;
-    (void)block_exclusive_scan(acc_a, w, tot_a);
-    (void)block_exclusive_scan(acc_b, w, tot_b);
-    if (threadIdx.x == 0) {
-        sums_a[blockIdx.x] = tot_a;
-        sums_b[blockIdx.x] = tot_b;
-    }
-}
-
-__global__ void __launch_bounds__(1024) k_scan_sums2(int32_t* sums_a, int32_t* sums_b, int64_t n, int32_t* total_a,
-                                                     int32_t* total_b) {
-    __shared__ int32_t w[16];
-    int32_t* sums = blockIdx.x == 0 ? sums_a : sums_b;
-    int32_t* d_total = blockIdx.x == 0 ? total_a : total_b;
-    int32_t carry = 0;
-    for (int64_t base = 0; base < n; base += 1024) {
-        int64_t i = base + threadIdx.x;
-        int32_t v = (i < n) ? sums[i] : 0;
-        int32_t tot;
-        int32_t ex = block_exclusive_scan(v, w, tot);
-        if (i < n) sums[i] = carry + ex;
-        carry += tot;
-    }
-    if (threadIdx.x == 0 && d_total) *d_total = carry;
-}
-
-__global__ void __launch_bounds__(kScanBlock) k_scan_apply2(const int32_t* in_a, int32_t* out_a, const int32_t* in_b,
-                                                              int32_t* out_b, int64_t n, const int32_t* sums_a,
-                                                              const int32_t* sums_b) {
-    __shared__ int32_t w[kScanBlock / 64];
-    const int64_t base = int64_t(blockIdx.x) * kScanTile;
+    __shared__ int32_t before[2];
+    const LookTile t = look_begin(state, tiles);
+    if (t.tile >= tiles) return;  // (uniform; only if the state was damaged from outside)
+    const int64_t base = int64_t(t.tile) * kScanTile + int64_t(threadIdx.x) * kScanItems;
     int32_t va[kScanItems], vb[kScanItems];
-    int32_t acc_a = 0, acc_b = 0;
-#pragma unroll
-    for (int k = 0; k < kScanItems; k++) {
-        int64_t i = base + int64_t(threadIdx.x) * kScanItems + k;
-        va[k] = (i < n) ? in_a[i] : 0;
-        vb[k] = (i < n) ? in_b[i] : 0;
-        acc_a += va[k];
-        acc_b += vb[k];
-    }
-    int32_t tot;
-    int32_t ea = block_exclusive_scan(acc_a, w, tot) + sums_a[blockIdx.x];
-    int32_t eb = block_exclusive_scan(acc_b, w, tot) + sums_b[blockIdx.x];
-#pragma unroll
-    for (int k = 0; k < kScanItems; k++) {
-        int64_t i = base + int64_t(threadIdx.x) * kScanItems + k;
-        if (i < n) {
-            out_a[i] = ea;
-            out_b[i] = eb;
+    const int32_t sa = load_items(in_a, base, n, wide, va);
+    const int32_t sb = TWO ? load_items(in_b, base, n, wide, vb) : 0;
+    int32_t ta, tb = 0;
+    const int32_t ea = block_exclusive_scan(sa, w, ta);
+    const int32_t eb = TWO ? block_exclusive_scan(sb, w, tb) : 0;
+    const int wave = threadIdx.x >> 6;
+    if (wave == 0 || (TWO && wave == 1)) {
+        const int32_t mine = wave == 0 ? ta : tb;
+        const int32_t x = look_back(state + kLookHeader + int64_t(wave) * tiles, t, tiles, mine);
+        if ((threadIdx.x & 63) == 0) {
+            before[wave] = x;
+            int32_t* total = wave == 0 ? total_a : total_b;
+            if (t.tile == tiles - 1 && total) *total = x + mine;
         }
-        ea += va[k];
-        eb += vb[k];
     }
+    __syncthreads();
+    look_end(state, t, tiles);
+    store_items(out_a, base, n, wide, before[0] + ea, va);
+    if (TWO) store_items(out_b, base, n, wide, before[1] + eb, vb);
 }
 
 // ---- radix sort ------------------------------------------------------------------
@@ -191,7 +113,8 @@ __global__ void __launch_bounds__(kSortBlock) k_radix_upsweep(const uint32_t* ke
 
 __global__ void __launch_bounds__(kSortBlock) k_radix_downsweep(const uint32_t* keys_in, const uint32_t* vals_in,
                                                                   uint32_t* keys_out, uint32_t* vals_out, int64_t n,
-                                                                  int shift, const int32_t* offsets, int tiles) {
+                                                                  int shift, const int32_t* offsets, int tiles,
+                                                                  bool counts) {
     __shared__ int32_t wcnt[4][256];     // per-wave digit counts, then per-wave digit offsets
     __shared__ int32_t tile_off[256];    // digit start inside the tile
     __shared__ int32_t glob_off[256];    // digit start in the output
@@ -201,7 +124,20 @@ __global__ void __launch_bounds__(kSortBlock) k_radix_downsweep(const uint32_t* 
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int i = threadIdx.x; i < 4 * 256; i += kSortBlock) (&wcnt[0][0])[i] = 0;
-    glob_off[threadIdx.x] = offsets[int64_t(threadIdx.x) * tiles + blockIdx.x];
+    if (counts) {
+        // few tiles: their digit counts instead of the scanned offsets (thread
+        // t adds up digit t's)
+        int32_t before = 0, all = 0;
+        for (int i = 0; i < tiles; i++) {
+            const int32_t v = offsets[int64_t(threadIdx.x) * tiles + i];
+            before += i < int(blockIdx.x) ? v : 0;
+            all += v;
+        }
+        int32_t tot;
+        glob_off[threadIdx.x] = before + block_exclusive_scan(all, wsum, tot);
+    } else {
+        glob_off[threadIdx.x] = offsets[int64_t(threadIdx.x) * tiles + blockIdx.x];
+    }
     __syncthreads();
 
     const int64_t wbase = int64_t(blockIdx.x) * kSortTile + int64_t(wave) * kWaveTile;
@@ -271,6 +207,16 @@ __global__ void __launch_bounds__(kSortBlock) k_radix_downsweep(const uint32_t* 
 
 }  // namespace
 
+// The scan state of a stream for `words` tile words, cleared when it grows.
+uint64_t* look_state(Scratch& scratch, int64_t words, hipStream_t s) {
+    const size_t want = size_t(words) + kLookHeader;
+    if (scratch.look.n < want || !scratch.look.p) {
+        scratch.look.reserve(want + want / 4);
+        PRG_HIP(hipMemsetAsync(scratch.look.p, 0, scratch.look.n * sizeof(uint64_t), s));
+    }
+    return scratch.look.p;
+}
+
 void scan_exclusive(const int32_t* d_in, int32_t* d_out, int64_t n, int32_t* d_total, hipStream_t s,
                     Scratch& scratch, KernelTimer& kt) {
     if (n <= 0) {
@@ -278,13 +224,11 @@ void scan_exclusive(const int32_t* d_in, int32_t* d_out, int64_t n, int32_t* d_t
         return;
     }
     const int64_t tiles = (n + kScanTile - 1) / kScanTile;
-    int32_t* sums = scratch.a.reserve(size_t(tiles));
+    uint64_t* state = look_state(scratch, tiles, s);
+    const bool wide = ((reinterpret_cast<uintptr_t>(d_in) | reinterpret_cast<uintptr_t>(d_out)) & 15) == 0;
     TimedScope ts(kt, "scan_exclusive", 8.0 * double(n));
-    k_scan_reduce<<<unsigned(tiles), kScanBlock, 0, s>>>(d_in, n, sums);
-    PRG_CHECK_LAUNCH();
-    k_scan_sums<<<1, 1024, 0, s>>>(sums, tiles, d_total);
-    PRG_CHECK_LAUNCH();
-    k_scan_apply<<<unsigned(tiles), kScanBlock, 0, s>>>(d_in, d_out, n, sums);
+    k_scan<false><<<unsigned(tiles), kScanBlock, 0, s>>>(d_in, d_out, d_total, nullptr, nullptr, nullptr, n,
+                                                         uint32_t(tiles), wide, state);
     PRG_CHECK_LAUNCH();
 }
 
@@ -296,13 +240,12 @@ void scan_exclusive2(const int32_t* a_in, int32_t* a_out, int32_t* a_total, cons
         return;
     }
     const int64_t tiles = (n + kScanTile - 1) / kScanTile;
-    int32_t* sums = scratch.a.reserve(size_t(2 * tiles));
+    uint64_t* state = look_state(scratch, 2 * tiles, s);
+    const bool wide = ((reinterpret_cast<uintptr_t>(a_in) | reinterpret_cast<uintptr_t>(a_out) |
+                        reinterpret_cast<uintptr_t>(b_in) | reinterpret_cast<uintptr_t>(b_out)) & 15) == 0;
     TimedScope ts(kt, "scan_exclusive", 16.0 * double(n));
-    k_scan_reduce2<<<unsigned(tiles), kScanBlock, 0, s>>>(a_in, b_in, n, sums, sums + tiles);
-    PRG_CHECK_LAUNCH();
-    k_scan_sums2<<<2, 1024, 0, s>>>(sums, sums + tiles, tiles, a_total, b_total);
-    PRG_CHECK_LAUNCH();
-    k_scan_apply2<<<unsigned(tiles), kScanBlock, 0, s>>>(a_in, a_out, b_in, b_out, n, sums, sums + tiles);
+    k_scan<true><<<unsigned(tiles), kScanBlock, 0, s>>>(a_in, a_out, a_total, b_in, b_out, b_total, n, uint32_t(tiles),
+                                                        wide, state);
     PRG_CHECK_LAUNCH();
 }
 
@@ -322,10 +265,14 @@ void radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32
             k_radix_upsweep<<<unsigned(tiles), kSortBlock, 0, s>>>(ki, n, shift, hist, tiles);
             PRG_CHECK_LAUNCH();
         }
-        scan_exclusive(hist, offs, hn, nullptr, s, scratch, kt);
+        // up to 16 tiles (65,536 keys) each workgroup adds up the counts itself:
+        // 16 loads per thread cost less than the scan's launch (about 4 us)
+        const bool counts = tiles <= 16;
+        if (!counts) scan_exclusive(hist, offs, hn, nullptr, s, scratch, kt);
         {
             TimedScope ts(kt, "radix_downsweep", 16.0 * double(n));
-            k_radix_downsweep<<<unsigned(tiles), kSortBlock, 0, s>>>(ki, vi, ko, vo, n, shift, offs, tiles);
+            k_radix_downsweep<<<unsigned(tiles), kSortBlock, 0, s>>>(ki, vi, ko, vo, n, shift, counts ? hist : offs,
+                                                                     tiles, counts);
             PRG_CHECK_LAUNCH();
         }
         std::swap(ki, ko);

@@ -158,7 +158,7 @@ constexpr int64_t kNoAllocTriangles = PRG_WELD_NOALLOC_MAX_TRIANGLES;
 constexpr int64_t kAlign = 256;
 constexpr int64_t align_up(int64_t b) { return (b + kAlign - 1) / kAlign * kAlign; }
 constexpr int64_t kSortTiles = (kNoAllocVertices + 4095) / 4096 + 1;  // radix sort tiles (4096 keys each)
-constexpr int64_t kScanTemp = 256 * kSortTiles + 1024;               // histogram scan; >= n / 2048 scan tiles
+constexpr int64_t kScanTemp = 256 * kSortTiles + 1024;               // histogram scan; twice the scans' tiles and header
 constexpr int64_t kNoAllocBytes = 2 * align_up(12 * kNoAllocVertices) + 4 * align_up(4 * kNoAllocVertices) +
                                   7 * align_up(4 * kNoAllocVertices) + align_up(12 * kNoAllocTriangles) +
                                   align_up(16) + 3 * align_up(4 * kScanTemp);
@@ -235,16 +235,19 @@ void weld_mesh_noalloc(prg_ctx* c, float* vertices, int64_t n, int32_t* triangle
     struct Lend {
         Scratch& s;
         ~Lend() {
-            s.a.p = nullptr;
+            s.look.p = nullptr;
             s.b.p = nullptr;
             s.c.p = nullptr;
-            s.a.n = s.b.n = s.c.n = 0;
+            s.look.n = s.b.n = s.c.n = 0;
         }
     } lend{scr};
-    scr.a.p = reinterpret_cast<int32_t*>(take(4 * kScanTemp));
+    // (the scans' state is zero when the library loads, and every scan leaves
+    // it ready for the next)
+    scr.look.p = reinterpret_cast<uint64_t*>(take(4 * kScanTemp));
     scr.b.p = reinterpret_cast<int32_t*>(take(4 * kScanTemp));
     scr.c.p = reinterpret_cast<int32_t*>(take(4 * kScanTemp));
-    scr.a.n = scr.b.n = scr.c.n = size_t(kScanTemp);
+    scr.look.n = size_t(kScanTemp) / 2;
+    scr.b.n = scr.c.n = size_t(kScanTemp);
     if (off > kNoAllocBytes) throw Error{PRG_E_HIP, "weld array layout exceeds its size"};
     weld_core(c, b, scr, vertices, n, triangles, m, n_leaf, n_out, n_leaf_out);
 }
