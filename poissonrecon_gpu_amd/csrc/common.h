@@ -16,6 +16,10 @@ namespace prg {
 
 constexpr int kMaxDepth = 10;  // 3D key bits must fit in uint32
 
+// A context's pinned read-back area; its last 4 bytes hold the owned-corner count.
+constexpr size_t kCgHostBytes = 8192;
+constexpr size_t kCgHostTopo = kCgHostBytes - 4;
+
 // ---- errors ------------------------------------------------------------------
 struct Error {
     prg_status status;

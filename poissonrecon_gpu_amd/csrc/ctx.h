@@ -66,7 +66,6 @@ struct prg_ctx {
     prg::DBuf<double> cg_part[3][4];  // r.r (two slots), p.q, b.b / true-residual partials
     prg::DBuf<uint8_t> cg_state[3];
     prg::DBuf<uint8_t> cg_seg;  // the solver's per-depth segment table
-    prg::DBuf<double> cg_out;
     // SpMV tile plans of the large depths, valid for octree `plan_gen`
     prg::DBuf<int32_t> plan_count, plan_ubase;
     prg::DBuf<int16_t> plan_rowid;
@@ -135,7 +134,7 @@ struct prg_ctx {
     bool stage_pending[PRG_STAGE_COUNT] = {};
     std::vector<hipEvent_t> ev_pool;  // the solver's events, reused across solves
     int num_cu = 0;                   // compute units of the device
-    void* cg_host = nullptr;          // pinned, 4 KiB: CG state read-backs and the segment table's staging
+    void* cg_host = nullptr;          // pinned, kCgHostBytes: CG state read-backs, plan counts, the segment table's staging
     int32_t* sub_host = nullptr;      // pinned, 64 ints: the subdivision's counters
     // test setting (environment PRG_TILE_LDS_LIMIT at creation): caps the
     // listed blocks and points the leaf-level tile kernels stage in LDS, so

@@ -23,6 +23,7 @@
 #include <algorithm>
 
 #include "ctx.h"
+#include "lookback.h"
 #include "pnt.h"
 #include "tile.h"
 
@@ -489,33 +490,47 @@ __device__ __forceinline__ int depth_of(const Bases& B, int D, int64_t i) {
 // b_i = sum_j G[neighbour_j(i)][j].  The float terms are the reference's;
 // only the grouping of the double sum differs.
 
-// chunks of a node's own leaf range
-__global__ void __launch_bounds__(kBlock) k_g_chunks(const int32_t* dnum, int64_t n, int64_t first_skipped,
-                                                     int32_t* chunks, int32_t* multi) {
-    const int64_t a = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-    if (a >= n) return;
-    // nodes from first_skipped on (the depth just above the leaf level) are summed by k_g_parent_sums
-    const int32_t c = a >= first_skipped ? 0 : (dnum[a] + kChunk - 1) / kChunk;
-    chunks[a] = c;
-    multi[a] = (c > 1) ? c : 0;
-}
+struct ChunkCounts {
+    int32_t chunks, multi_chunks, multi_nodes;
+};
 
-// node of each chunk: the last node whose chunk offset is <= c (the
-// exclusive scan of chunk counts is non-decreasing; nodes without chunks
-// share their successor's offset, so the last one is the chunk's owner)
-__global__ void __launch_bounds__(kBlock) k_g_chunk_map(const int32_t* chunk_off, int64_t n, const int32_t* d_nchunks,
-                                                        int32_t* chunk_node) {
-    const int64_t c = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-    if (c >= *d_nchunks) return;
-    int64_t lo = 0, hi = n;  // invariant: chunk_off[lo] <= c, and hi is past the answer
-    while (hi - lo > 1) {
-        const int64_t mid = (lo + hi) >> 1;
-        if (chunk_off[mid] <= c)
-            lo = mid;
-        else
-            hi = mid;
+// The chunks of the nodes of depths 0 .. D-2 (those of depth D-1 are summed
+// by k_g_parent_sums), as (node, chunk of the node) in any order: a node's
+// chunks are added up by their number inside it, so the order of the list
+// changes no sum.  Nodes with several chunks also get their place among the
+// partials and in the list of such nodes.  A workgroup reserves its places
+// with one atomic each; as scans this took six launches of about 4 us.
+constexpr int kListBlock = 1024;
+__global__ void __launch_bounds__(kListBlock) k_g_list(const int32_t* dnum, int64_t n, ChunkCounts* cnt, int2* rec,
+                                                       int32_t* multi_off, int32_t* mlist) {
+    __shared__ int32_t lds[kListBlock / 64];
+    __shared__ int32_t s_base[3];
+    const int64_t a = int64_t(blockIdx.x) * kListBlock + threadIdx.x;
+    const int32_t c = a < n ? (dnum[a] + kChunk - 1) / kChunk : 0;
+    const bool multi = c > 1;
+    int32_t tot0, tot1, tot2;
+    const int32_t e0 = block_exclusive_scan(c, lds, tot0);
+    const int32_t e1 = block_exclusive_scan(multi ? c : 0, lds, tot1);
+    const int32_t e2 = block_exclusive_scan(multi ? 1 : 0, lds, tot2);
+    if (threadIdx.x == 0) {
+        s_base[0] = tot0 ? atomicAdd(&cnt->chunks, tot0) : 0;
+        s_base[1] = tot1 ? atomicAdd(&cnt->multi_chunks, tot1) : 0;
+        s_base[2] = tot2 ? atomicAdd(&cnt->multi_nodes, tot2) : 0;
     }
-    chunk_node[c] = int32_t(lo);
+    __syncthreads();
+    const int32_t pos = s_base[0] + e0;
+    if (c == 1) rec[pos] = int2{int32_t(a), 0};
+    if (multi) {
+        multi_off[a] = s_base[1] + e1;
+        mlist[s_base[2] + e2] = int32_t(a);
+    }
+    // the chunks of a large node (the root's alone are MD / kChunk) are written by its whole wave
+    const int lane = threadIdx.x & 63;
+    for (uint64_t m = __ballot(multi); m; m &= m - 1) {
+        const int l = __builtin_ctzll(m);
+        const int32_t node = __shfl(int32_t(a), l, 64), nc = __shfl(c, l, 64), p0 = __shfl(pos, l, 64);
+        for (int32_t i = lane; i < nc; i += 64) rec[p0 + i] = int2{node, i};
+    }
 }
 
 // the 27 terms of one leaf slot for a node whose cell spans sc leaf cells
@@ -537,29 +552,27 @@ constexpr int kCoarseTableFloats = 3 * ((2 << kMaxDepth) - 4);
 // The tables of depths 0 .. D-2 (table[0 .. tcount)) are staged in LDS.
 __global__ void __launch_bounds__(kBlock) k_g_sums(const uint32_t* key, const int32_t* didx, const int32_t* dnum,
                                                    const float* vfx, const float* vfy, const float* vfz,
-                                                   const float* table, int32_t tcount, const int64_t* table_off,
-                                                   const int32_t* chunk_node, const int32_t* chunk_off,
-                                                   const int32_t* chunks, const int32_t* multi_off,
-                                                   const int32_t* d_nchunks, Bases B, int D, double* G,
+                                                   const float* table, int32_t tcount, Bases table_off, const int2* rec,
+                                                   const int32_t* multi_off, const ChunkCounts* cnt, Bases B, int D, double* G,
                                                    int64_t gstride, double* partial) {
     __shared__ float tab[kCoarseTableFloats];
     for (int i = threadIdx.x; i < tcount; i += kBlock) tab[i] = table[i];
     __syncthreads();
     const int lane = threadIdx.x & 63;
-    const int64_t nchunks = *d_nchunks;
+    const int64_t nchunks = cnt->chunks;
     // the chunk, its node and their ranges are wave-uniform (scalar loads)
     const int64_t wave0 = __builtin_amdgcn_readfirstlane(int32_t((blockIdx.x * kBlock + threadIdx.x) >> 6));
     const int64_t nwaves = (int64_t(gridDim.x) * kBlock) >> 6;
     const int64_t baseD = B.b[D];
     for (int64_t c = wave0; c < nchunks; c += nwaves) {
-        const int64_t a = chunk_node[c];
-        const int64_t ci = c - chunk_off[a];
+        const int64_t a = rec[c].x;
+        const int64_t ci = rec[c].y;
         const int64_t k0 = int64_t(didx[a]) + ci * kChunk;
         const int64_t k1 = min(k0 + kChunk, int64_t(didx[a]) + dnum[a]);
         const int d = depth_of(B, D, a);
         const int sc = 1 << (D - d);
         const uint32_t rmask = uint32_t(sc - 1);
-        const float* T = tab + table_off[d];
+        const float* T = tab + table_off.b[d];
         double acc[32];
 #pragma unroll
         for (int j = 0; j < 32; j++) acc[j] = 0.0;
@@ -590,7 +603,7 @@ __global__ void __launch_bounds__(kBlock) k_g_sums(const uint32_t* key, const in
         const int q = 16 * ((lane >> 5) & 1) + 8 * ((lane >> 4) & 1) + 4 * ((lane >> 3) & 1) + 2 * ((lane >> 2) & 1) +
                       ((lane >> 1) & 1);
         if (!(lane & 1) && q < 27) {
-            if (chunks[a] == 1)
+            if (dnum[a] <= kChunk)
                 G[q * gstride + a] = tot;
             else
                 partial[27 * (int64_t(multi_off[a]) + ci) + q] = tot;
@@ -600,26 +613,15 @@ __global__ void __launch_bounds__(kBlock) k_g_sums(const uint32_t* key, const in
 
 // nodes spanning several chunks: one workgroup per such node adds its chunk
 // partials (fixed per-thread strides, fixed tree) for all 27 positions
-__global__ void __launch_bounds__(kBlock) k_g_flag_multi(const int32_t* chunks, int64_t n, int32_t* flag) {
-    const int64_t a = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-    if (a < n) flag[a] = chunks[a] > 1 ? 1 : 0;
-}
-
-__global__ void __launch_bounds__(kBlock) k_g_list_multi(const int32_t* flag, const int32_t* pos, int64_t n,
-                                                         int32_t* list) {
-    const int64_t a = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-    if (a < n && flag[a]) list[pos[a]] = int32_t(a);
-}
-
-__global__ void __launch_bounds__(kBlock) k_g_finish(const int32_t* list, const int32_t* d_count,
-                                                     const int32_t* chunks, const int32_t* multi_off,
+__global__ void __launch_bounds__(kBlock) k_g_finish(const int32_t* list, const ChunkCounts* cnt,
+                                                     const int32_t* dnum, const int32_t* multi_off,
                                                      const double* partial, double* G, int64_t gstride) {
     __shared__ double red[kBlock / 64][27];
-    const int64_t count = *d_count;  // the grid is sized by an upper bound and strides over the list
+    const int64_t count = cnt->multi_nodes;  // the grid is sized by an upper bound and strides over the list
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int64_t l = blockIdx.x; l < count; l += gridDim.x) {
         const int64_t a = list[l];
-        const int32_t c = chunks[a];
+        const int32_t c = (dnum[a] + kChunk - 1) / kChunk;
         const double* P = partial + 27 * int64_t(multi_off[a]);
         double acc[27];
 #pragma unroll
@@ -652,8 +654,9 @@ __global__ void __launch_bounds__(kBlock) k_g_finish(const int32_t* list, const 
 __global__ void __launch_bounds__(kBlock) k_g_parent_sums(const uint32_t* key, const int32_t* parent,
                                                           const float* vfx, const float* vfy, const float* vfz,
                                                           const float* T, int64_t baseD, int64_t MD, double* G,
-                                                          int64_t gstride) {
+                                                          int64_t gstride, ChunkCounts* cnt) {
     const int64_t k = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+    if (k == 0) *cnt = ChunkCounts{0, 0, 0};  // for k_g_list behind this launch
     if (k >= MD) return;  // MD is a multiple of 8 and kBlock of 8: blocks never straddle
     const uint32_t kl = key[baseD + k];
     const int rx = (kl >> 2) & 1, ry = (kl >> 1) & 1, rz = kl & 1;  // offset inside the parent's cell (s = 2)
@@ -705,7 +708,7 @@ __global__ void __launch_bounds__(kBlock) k_g_parent_sums(const uint32_t* key, c
 // G holds every position of a node with leaf-level slots below it (dnum > 0);
 // a node without any contributes no terms and its G is neither written nor
 // read.
-__global__ void __launch_bounds__(kBlock, 6) k_div_from_g(const int32_t* pnt, const int64_t* pnt_off, Bases B, int D,
+__global__ void __launch_bounds__(kBlock, 6) k_div_from_g(const int32_t* pnt, Bases pnt_off, Bases B, int D,
                                                        const int32_t* dnum, const double* G, int64_t gstride,
                                                        int64_t n, float* div) {
     const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
@@ -717,7 +720,7 @@ __global__ void __launch_bounds__(kBlock, 6) k_div_from_g(const int32_t* pnt, co
         const int d = depth_of(B, D, i);
         const int64_t t = i - B.b[d];
         int32_t nbr[27];
-        pnt_neighbours(pnt + 27 * (pnt_off[d] + (t >> 3)), int(t & 7), nbr);
+        pnt_neighbours(pnt + 27 * (pnt_off.b[d] + (t >> 3)), int(t & 7), nbr);
         // loads issued nine at a time; G of a node without leaf-level slots
         // is never written, and its value is read but not added
 #pragma unroll
@@ -808,9 +811,6 @@ void compute_divergence(prg_ctx* c) {
     }
     StageTimer st(c, PRG_STAGE_DIVERGENCE);
     float* DV = c->div.reserve(M);
-    PoolBuf<int64_t> toff{&c->pool[60]};
-    PRG_HIP(hipMemcpyAsync(toff.reserve(c->fs->div_off.size()), c->fs->div_off.data(), c->fs->div_off.size() * 8,
-                           hipMemcpyHostToDevice, s));
     {
         TimedScope ts(c->kt, "div_leaf", 124.0 * double(MD));
         TilePlan P{};
@@ -827,42 +827,39 @@ void compute_divergence(prg_ctx* c) {
     }
     const int64_t n = baseD;  // nodes of depths 0 .. D-1
     if (n > 0) {
-        PoolBuf<int32_t> chunks{&c->pool[61]}, multi{&c->pool[62]}, coff{&c->pool[63]}, moff{&c->pool[64]},
-            cnode{&c->pool[65]}, ctot{&c->pool[66]}, mtot{&c->pool[67]};
-        PoolBuf<double> G{&c->pool[68]}, partial{&c->pool[69]};
-        chunks.reserve(n);
-        multi.reserve(n);
-        coff.reserve(n);
-        moff.reserve(n);
-        ctot.reserve(1);
-        mtot.reserve(1);
+        PoolBuf<int32_t> moff{&c->pool[61]}, mlist{&c->pool[62]};
+        PoolBuf<int2> rec{&c->pool[63]};
+        PoolBuf<ChunkCounts> cnt{&c->pool[64]};
+        PoolBuf<double> G{&c->pool[65]}, partial{&c->pool[66]};
+        cnt.reserve(1);
         G.reserve(size_t(27) * n);  // written for every node with dnum > 0; only those are read
-        const int64_t first_skipped = D >= 1 ? c->bases[D - 1] : n;
-        if (D >= 1) {
+        const int64_t nl = c->bases[D - 1];  // nodes of depths 0 .. D-2 (n > 0: D >= 1)
+        {
             TimedScope ts(c->kt, "div_parent_sums", 16.0 * double(MD) + 216.0 * double(c->counts[D - 1]));
             k_g_parent_sums<<<grid_for(MD, kBlock), kBlock, 0, s>>>(c->key.get(), c->parent.get(), VX, VY, VZ,
                                                                    c->d_div_table.get() + c->fs->div_off[D - 1],
-                                                                   baseD, MD, G.get(), n);
+                                                                   baseD, MD, G.get(), n, cnt.get());
             PRG_CHECK_LAUNCH();
         }
-        k_g_chunks<<<grid_for(n, kBlock), kBlock, 0, s>>>(c->dnum.get(), n, first_skipped, chunks.get(), multi.get());
-        PRG_CHECK_LAUNCH();
-        scan_exclusive2(chunks.get(), coff.get(), ctot.get(), multi.get(), moff.get(), mtot.get(), n, s, c->scratch,
-                        c->kt);
         // Sizes from upper bounds, the counts stay on the device (no host
         // round trip): a node's chunks number at most 1 + dnum / kChunk and
         // every depth's dnum add up to the leaf-level slot count, so
-        // chunks <= n + (D - 1) (MD / kChunk + 1); a node with several chunks
+        // chunks <= nl + (D - 1) (MD / kChunk + 1); a node with several chunks
         // has dnum > kChunk, so those chunks number at most
         // 2 (D - 1) (MD / kChunk + 1), and such nodes half that.
         const int64_t per_depth = MD / kChunk + 1;
-        const int64_t nchunks = n + std::max(1, D - 1) * per_depth;
+        const int64_t nchunks = nl + std::max(1, D - 1) * per_depth;
         const int64_t nmulti = 2 * std::max(1, D - 1) * per_depth;
         const int64_t nm = std::max(1, D - 1) * per_depth;
-        cnode.reserve(nchunks);
+        moff.reserve(std::max<int64_t>(1, nl));
+        mlist.reserve(nm);
+        rec.reserve(nchunks);
         partial.reserve(size_t(27) * nmulti);
-        k_g_chunk_map<<<grid_for(nchunks, kBlock), kBlock, 0, s>>>(coff.get(), n, ctot.get(), cnode.get());
-        PRG_CHECK_LAUNCH();
+        if (nl > 0) {
+            k_g_list<<<grid_for(nl, kListBlock), kListBlock, 0, s>>>(c->dnum.get(), nl, cnt.get(), rec.get(), moff.get(),
+                                                                   mlist.get());
+            PRG_CHECK_LAUNCH();
+        }
         Bases B{};
         for (int d = 0; d <= D; d++) B.b[d] = c->bases[d];
         B.b[D + 1] = M;
@@ -870,39 +867,29 @@ void compute_divergence(prg_ctx* c) {
         // depths 0 .. D-2 come first in the table, 3 * 2^(D - d) floats each
         const int32_t tcount = D >= 2 ? int32_t(c->fs->div_off[D - 1]) : 0;
         if (tcount > kCoarseTableFloats) throw Error{PRG_E_ARG, "divergence: coarse tables exceed their LDS area"};
-        {
-            // every leaf slot read once per coarser depth (key + vector field), G written once
-            TimedScope ts(c->kt, "div_subtree_sums", 16.0 * double(MD) * double(D) + 216.0 * double(n));
-            k_g_sums<<<grid_for(waves * 64, kBlock), kBlock, 0, s>>>(
-                c->key.get(), c->didx.get(), c->dnum.get(), VX, VY, VZ, c->d_div_table.get(), tcount, toff.get(), cnode.get(),
-                coff.get(), chunks.get(), moff.get(), ctot.get(), B, D, G.get(), n, partial.get());
-            PRG_CHECK_LAUNCH();
+        Bases toff{}, poff{};
+        for (int d = 0; d <= D; d++) {
+            toff.b[d] = c->fs->div_off[d];
+            poff.b[d] = c->pnt_off[d];
         }
-        {
-            PoolBuf<int32_t> mflag{&c->pool[70]}, mpos{&c->pool[71]}, mcnt{&c->pool[72]}, mlist{&c->pool[73]};
-            mflag.reserve(n);
-            mpos.reserve(n);
-            mcnt.reserve(1);
-            k_g_flag_multi<<<grid_for(n, kBlock), kBlock, 0, s>>>(chunks.get(), n, mflag.get());
-            PRG_CHECK_LAUNCH();
-            scan_exclusive(mflag.get(), mpos.get(), n, mcnt.get(), s, c->scratch, c->kt);
-            mlist.reserve(nm);
-            k_g_list_multi<<<grid_for(n, kBlock), kBlock, 0, s>>>(mflag.get(), mpos.get(), n, mlist.get());
-            PRG_CHECK_LAUNCH();
+        if (nl > 0) {
+            {
+                // every leaf slot read once per coarser depth (key + vector field), G written once
+                TimedScope ts(c->kt, "div_subtree_sums", 16.0 * double(MD) * double(D) + 216.0 * double(n));
+                k_g_sums<<<grid_for(waves * 64, kBlock), kBlock, 0, s>>>(
+                    c->key.get(), c->didx.get(), c->dnum.get(), VX, VY, VZ, c->d_div_table.get(), tcount, toff, rec.get(),
+                    moff.get(), cnt.get(), B, D, G.get(), n, partial.get());
+                PRG_CHECK_LAUNCH();
+            }
             TimedScope ts(c->kt, "div_subtree_finish", 216.0 * double(nm));
             const unsigned fgrid = unsigned(std::min<int64_t>(nm, 2048));
-            k_g_finish<<<fgrid, kBlock, 0, s>>>(mlist.get(), mcnt.get(), chunks.get(), moff.get(), partial.get(),
+            k_g_finish<<<fgrid, kBlock, 0, s>>>(mlist.get(), cnt.get(), c->dnum.get(), moff.get(), partial.get(),
                                                 G.get(), n);
             PRG_CHECK_LAUNCH();
         }
-        {
-            PoolBuf<int64_t> poff{&c->pool[74]};
-            PRG_HIP(hipMemcpyAsync(poff.reserve(D + 2), c->pnt_off.data(), size_t(D + 2) * 8, hipMemcpyHostToDevice, s));
-            TimedScope ts(c->kt, "div_from_subtree_sums", 13.5 * double(n) + 216.0 * double(n) + 4.0 * double(n));
-            k_div_from_g<<<grid_for(n, kBlock), kBlock, 0, s>>>(c->pnt.get(), poff.get(), B, D, c->dnum.get(), G.get(),
-                                                               n, n, DV);
-            PRG_CHECK_LAUNCH();
-        }
+        TimedScope ts(c->kt, "div_from_subtree_sums", 13.5 * double(n) + 216.0 * double(n) + 4.0 * double(n));
+        k_div_from_g<<<grid_for(n, kBlock), kBlock, 0, s>>>(c->pnt.get(), poff, B, D, c->dnum.get(), G.get(), n, n, DV);
+        PRG_CHECK_LAUNCH();
     }
 }
 

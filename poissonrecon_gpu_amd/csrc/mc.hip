@@ -490,7 +490,7 @@ void compute_isovalue(prg_ctx* c) {
 
 // pinned area of the owned-corner count (the last bytes of the context's
 // pinned staging page, after the solver's areas)
-int32_t* topo_count_host(prg_ctx* c) { return reinterpret_cast<int32_t*>(static_cast<uint8_t*>(c->cg_host) + 4092); }
+int32_t* topo_count_host(prg_ctx* c) { return reinterpret_cast<int32_t*>(static_cast<uint8_t*>(c->cg_host) + kCgHostTopo); }
 
 void start_topology(prg_ctx* c) {
     ensure_tables(c);

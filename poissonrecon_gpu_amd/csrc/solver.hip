@@ -80,8 +80,30 @@ struct Seg {
     float *R, *P0, *P1, *Q, *XS;
     double *rr, *pq, *bb;  // r.r (two slots of kMaxWG), p.q, b.b partials
     CgState* st;
+    const int32_t* pnt;  // parent-neighbour rows of the depth, its right-hand side and solution
+    const float* b;
+    float* X;
+    CgState* hst;      // pinned host memory: the state when the chain ends,
+    int32_t* hdone;    // set as soon as the depth is found finished,
+    double* hout;      // and the depth's residuals and iteration count
+    int32_t zero_x;    // x0 = 0 (else x0 is read from X)
     float L[27];
 };
+
+__device__ __forceinline__ Stencil seg_stencil(const Seg& sg) {
+    Stencil S;
+#pragma unroll
+    for (int j = 0; j < 27; j++) S.L[j] = sg.L[j];
+    return S;
+}
+
+// The depth is finished: the device state, and the host's copy of the flag,
+// which the host reads while it queues iterations.
+__device__ __forceinline__ void set_done(const Seg& sg, int32_t iters) {
+    sg.st->done = 1;
+    sg.st->iters = iters;
+    __hip_atomic_store(sg.hdone, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 __device__ __forceinline__ int seg_of(const Seg* __restrict__ segs, int nseg, int b, bool vec) {
     int k = 0;
@@ -144,15 +166,21 @@ constexpr int kHashSlots = 2048;          // > kTileEntries: linear probing alwa
 static_assert(kHashSlots > kTileEntries, "hash must hold every entry of a tile");
 
 // r = b - A x0, p = r, xs = x0 (the solve works on the 16-byte-aligned copy
-// xs); partials of r.r (slot 0) and b.b.  zero_x: x0 = 0 is known, and A x0
-// is +0 (a float sum of signed zeros started at +0), so r = b - 0 without the
-// SpMV.
-__global__ void __launch_bounds__(kVecThreads) k_cg_init(const int32_t* pnt, int64_t n, Stencil S, const float* b,
-                                                         const float* x, int32_t zero_x, float* xs, float* r,
-                                                         float* p, double* rr_part, double* bb_part, CgState* st) {
+// xs) for every depth of a chain; partials of r.r (slot 0) and b.b.  zero_x:
+// x0 = 0 is known, and A x0 is +0 (a float sum of signed zeros started at
+// +0), so r = b - 0 without the SpMV.
+__global__ void __launch_bounds__(kVecThreads) k_cg_init(const Seg* __restrict__ segs, int32_t nseg) {
     __shared__ double lds[kVecThreads / 64];
+    const Seg& sg = segs[seg_of(segs, nseg, blockIdx.x, true)];
+    const int64_t n = sg.n;
+    const int bid = int(blockIdx.x) - sg.vwg0;
+    const int32_t zero_x = sg.zero_x;
+    const int32_t* pnt = sg.pnt;
+    const float *b = sg.b, *x = sg.X;
+    float *xs = sg.XS, *r = sg.R, *p = sg.P0;
+    const Stencil S = seg_stencil(sg);
     double bb = 0.0, rr = 0.0;
-    for (int64_t t = int64_t(blockIdx.x) * kVecThreads + threadIdx.x; t < n; t += int64_t(gridDim.x) * kVecThreads) {
+    for (int64_t t = int64_t(bid) * kVecThreads + threadIdx.x; t < n; t += int64_t(sg.nvwg) * kVecThreads) {
         const float ax = zero_x ? 0.0f : spmv_pnt(pnt, t, x, S);
         const float rv = b[t] - ax;
         xs[t] = zero_x ? 0.0f : x[t];
@@ -164,13 +192,13 @@ __global__ void __launch_bounds__(kVecThreads) k_cg_init(const int32_t* pnt, int
     const double sbb = block_allsum<kVecThreads>(bb, lds);
     const double srr = block_allsum<kVecThreads>(rr, lds);
     if (threadIdx.x == 0) {
-        bb_part[blockIdx.x] = sbb;
-        rr_part[blockIdx.x] = srr;
+        sg.bb[bid] = sbb;
+        sg.rr[bid] = srr;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        st->done = 0;
-        st->iters = 0;
-        st->restarted = 0;
+    if (bid == 0 && threadIdx.x == 0) {
+        sg.st->done = 0;
+        sg.st->iters = 0;
+        sg.st->restarted = 0;
     }
 }
 
@@ -432,10 +460,7 @@ __global__ void __launch_bounds__(kSpmvThreads, K <= kSpmvSmallK ? 8 : (K <= 8 ?
         if (it == 1) st->bb = bb;
         st->rr_hist[k1 & 1] = rr;
         st->rr = rr;
-        if (stop) {
-            st->done = 1;
-            st->iters = k1;
-        }
+        if (stop) set_done(sg, k1);
     }
     if (stop) return;
     load_cells(pa, va, vpa);
@@ -517,10 +542,7 @@ __global__ void __launch_bounds__(kVecThreads) k_cg_update(const Seg* __restrict
     const int bid = int(blockIdx.x) - sg.vwg0, nblocks = sg.nvwg;
     const double PQ = sum_partials<kVecThreads>(sg.pq, sg.nwg, lds);
     if (!(PQ > 0.0)) {
-        if (bid == 0 && threadIdx.x == 0) {
-            st->done = 1;
-            st->iters = it - 1;
-        }
+        if (bid == 0 && threadIdx.x == 0) set_done(sg, it - 1);
         return;
     }
     const float a = float(st->rr_hist[(it - 1) & 1] / PQ);
@@ -563,54 +585,69 @@ __global__ void __launch_bounds__(kVecThreads) k_cg_update(const Seg* __restrict
     if (bid == 0 && threadIdx.x == 0) st->iters = it;
 }
 
-// r = b - A x (every `refresh` iterations) and its r.r partial (slot it & 1)
-__global__ void __launch_bounds__(kVecThreads) k_cg_refresh(const int32_t* pnt, int64_t n, Stencil S, const float* b,
-                                                            const float* x, float* r, double* rr_part, CgState* st) {
+// r = b - A x (every `refresh` iterations) and its r.r partial (slot it & 1),
+// for the unfinished depths of a chain
+__global__ void __launch_bounds__(kVecThreads) k_cg_refresh(const Seg* __restrict__ segs, int32_t nseg, int32_t it) {
     __shared__ double lds[kVecThreads / 64];
-    if (st->done) return;
+    const Seg& sg = segs[seg_of(segs, nseg, blockIdx.x, true)];
+    if (sg.st->done) return;
+    const int64_t n = sg.n;
+    const int bid = int(blockIdx.x) - sg.vwg0;
+    const int32_t* pnt = sg.pnt;
+    const float *b = sg.b, *x = sg.XS;
+    float* r = sg.R;
+    const Stencil S = seg_stencil(sg);
     double rr = 0.0;
-    for (int64_t t = int64_t(blockIdx.x) * kVecThreads + threadIdx.x; t < n; t += int64_t(gridDim.x) * kVecThreads) {
+    for (int64_t t = int64_t(bid) * kVecThreads + threadIdx.x; t < n; t += int64_t(sg.nvwg) * kVecThreads) {
         const float ax = spmv_pnt(pnt, t, x, S);
         const float rv = b[t] - ax;
         r[t] = rv;
         rr += double(rv) * double(rv);
     }
     const double sum = block_allsum<kVecThreads>(rr, lds);
-    if (threadIdx.x == 0) rr_part[blockIdx.x] = sum;
+    if (threadIdx.x == 0) sg.rr[(it & 1) * kMaxWG + bid] = sum;
 }
 
-// ||b - A x||^2 of the final iterate, one FP64 partial per workgroup (FP32
-// SpMV, FP64 sum of squares).
-__global__ void __launch_bounds__(kVecThreads) k_true_residual(const int32_t* pnt, int64_t n, Stencil S, const float* b,
-                                                               const float* x, double* partial) {
+// The end of a chain, one launch for its depths: ||b - A x||^2 of the final
+// iterates, one FP64 partial per workgroup (FP32 SpMV, FP64 sum of squares),
+// and the solution copied out of the aligned work vector.
+__global__ void __launch_bounds__(kVecThreads) k_true_residual(const Seg* __restrict__ segs, int32_t nseg) {
     __shared__ double lds[kVecThreads / 64];
+    const Seg& sg = segs[seg_of(segs, nseg, blockIdx.x, true)];
+    const int64_t n = sg.n;
+    const int bid = int(blockIdx.x) - sg.vwg0;
+    const int32_t* pnt = sg.pnt;
+    const float *b = sg.b, *x = sg.XS;
+    float* X = sg.X;
+    const Stencil S = seg_stencil(sg);
     double rr = 0.0;
-    for (int64_t t = int64_t(blockIdx.x) * kVecThreads + threadIdx.x; t < n; t += int64_t(gridDim.x) * kVecThreads) {
+    for (int64_t t = int64_t(bid) * kVecThreads + threadIdx.x; t < n; t += int64_t(sg.nvwg) * kVecThreads) {
         const float ax = spmv_pnt(pnt, t, x, S);
+        X[t] = x[t];
         const double rv = double(b[t]) - double(ax);
         rr += rv * rv;
     }
     const double sum = block_allsum<kVecThreads>(rr, lds);
-    if (threadIdx.x == 0) partial[blockIdx.x] = sum;
+    if (threadIdx.x == 0) sg.bb[bid] = sum;
 }
 
-// One workgroup: ||b - A x|| / ||b|| from the true-residual partials (nt of
-// them), the recursive residual of the last iteration (its r.r partials, np
-// of them, in slot iters & 1) and the iteration count.
-__global__ void __launch_bounds__(kVecThreads) k_true_residual_finish(const double* partial, int32_t nt,
-                                                                      const double* rr_slots, int32_t np,
-                                                                      int32_t slot_stride, const CgState* st,
-                                                                      double* out) {
+// One workgroup per depth of a chain: ||b - A x|| / ||b|| from the
+// true-residual partials, the recursive residual of the last iteration (its
+// r.r partials, in slot iters & 1), the iteration count and the state, all
+// into pinned host memory.
+__global__ void __launch_bounds__(kVecThreads) k_true_residual_finish(const Seg* __restrict__ segs) {
     __shared__ double lds[kVecThreads / 64];
-    const double RR = sum_partials<kVecThreads>(partial, nt, lds);
-    const int32_t iters = st->iters;
-    const double rec = sum_partials<kVecThreads>(rr_slots + int64_t(iters & 1) * slot_stride, np, lds);
+    const Seg& sg = segs[blockIdx.x];
+    const double RR = sum_partials<kVecThreads>(sg.bb, sg.nvwg, lds);
+    const CgState st = *sg.st;
+    const double rec = sum_partials<kVecThreads>(sg.rr + int64_t(st.iters & 1) * kMaxWG, sg.nvwg, lds);
     if (threadIdx.x == 0) {
-        const double bb = st->bb;
-        out[0] = (bb > 0.0) ? sqrt(RR / bb) : 0.0;
-        out[1] = (bb > 0.0) ? sqrt(rec / bb) : 0.0;
-        out[2] = double(iters);
-        out[3] = double(st->restarted);
+        const double bb = st.bb;
+        sg.hout[0] = (bb > 0.0) ? sqrt(RR / bb) : 0.0;
+        sg.hout[1] = (bb > 0.0) ? sqrt(rec / bb) : 0.0;
+        sg.hout[2] = double(st.iters);
+        sg.hout[3] = double(st.restarted);
+        *sg.hst = st;
     }
 }
 
@@ -821,21 +858,33 @@ struct Chain {
     int inst = 0;                // SpMV instance (cells per thread)
     size_t lds = 0;              // SpMV dynamic LDS
     int issued = 0;              // iterations queued
-    int batch = 24;
+    int end_idx = -1;            // timing record of its latest end
     bool waiting = false;
-    bool ended = false;          // true residuals queued after the latest batch
     CgState* st = nullptr;       // device states, one per depth
     CgState* hst = nullptr;      // pinned host copies
-    hipEvent_t ev = nullptr;     // marks the state copy
+    int32_t* hdone = nullptr;    // pinned flags, one per depth
+    hipEvent_t beg = nullptr;    // before its first launch
+    hipEvent_t ev = nullptr;     // behind its latest end
     std::vector<std::pair<int, int>> launched;
 };
 
-constexpr int kFirstBatch = 24;      // iterations queued before a chain's first state read-back
+constexpr int kFirstBatch = 24;      // iterations queued before a chain's first state read-back,
+constexpr int kNextBatch = 6;        // and before each one after it
 constexpr int kMaxSegs = 12;         // depths per solve above kSmallRows rows (D <= 10 has at most 10)
-constexpr size_t kHostStates = 1024;  // pinned read-back area: states first, then the segment table
-constexpr size_t kHostPlanMax = 3840;  // then the plans' per-depth largest tile counts (kMaxDepth + 1 int32)
-constexpr size_t kHostPlanSum = 3888;  // and their per-depth sums of tile counts (kMaxDepth + 1 int64)
+// Layout of the pinned area (kCgHostBytes): the chains' states, the depths'
+// flags and results, the segment table's staging, and the plans' per-depth
+// largest tile counts and sums of tile counts.
+constexpr size_t kHostDone = 576;
+constexpr size_t kHostOut = 640;
+constexpr size_t kHostSegs = 1024;
+constexpr size_t kHostPlanMax = 4608;
+constexpr size_t kHostPlanSum = 4656;
+static_assert(kMaxSegs * sizeof(CgState) <= kHostDone, "chain states exceed their pinned area");
+static_assert(kHostDone + kMaxSegs * 4 <= kHostOut, "flags exceed their pinned area");
+static_assert(kHostOut + (kMaxDepth + 1) * 4 * 8 <= kHostSegs, "results exceed their pinned area");
+static_assert(kHostSegs + kMaxSegs * sizeof(Seg) <= kHostPlanMax, "segment table exceeds the pinned staging area");
 static_assert(kHostPlanMax + (kMaxDepth + 1) * 4 <= kHostPlanSum && kHostPlanSum % 8 == 0, "plan read-back layout");
+static_assert(kHostPlanSum + (kMaxDepth + 1) * 8 <= kCgHostTopo, "plan counts exceed the pinned area");
 
 int32_t* plan_maxcount_host(prg_ctx* c) {
     return reinterpret_cast<int32_t*>(static_cast<uint8_t*>(c->cg_host) + kHostPlanMax);
@@ -980,8 +1029,9 @@ prg_status solve_all(prg_ctx* c, prg_solve_stats* stats) {
         while ((int64_t(1) << g) < prg_unet_grid(c->warm_net)) g++;
         if (g <= D && c->counts[g] > 0) warm_depth = g;
     }
-    double* outv = c->cg_out.reserve(size_t(4) * (D + 1));
-    PRG_HIP(hipMemsetAsync(outv, 0, size_t(4) * (D + 1) * 8, s));
+    // every depth's residuals and iteration count, written by its solve
+    double* ov = reinterpret_cast<double*>(static_cast<uint8_t*>(c->cg_host) + kHostOut);
+    std::fill(ov, ov + 4 * (D + 1), 0.0);
     const float tol = c->cfg.cg_tol;
     const int32_t fixed = c->cfg.cg_fixed_iters, max_iters = c->cfg.cg_max_iters;
     const int32_t refresh = c->cfg.cg_refresh > 0 ? c->cfg.cg_refresh : (1 << 30);
@@ -1000,14 +1050,47 @@ prg_status solve_all(prg_ctx* c, prg_solve_stats* stats) {
             jobs.pnt_row[jobs.count] = d == 0 ? -1 : c->pnt_off[d];
             jobs.count++;
         }
-    // chain 0: the finest depth; chain 1: every other large depth, together;
-    // chain 2: a warm-started depth (other than the finest), after the
-    // network's inference on its own stream
+    // chain 0: the finest depth; chain 1: every other large depth, together
+    // (with the finest depth in chain 0 when they are few, below); chain 2: a
+    // warm-started depth (other than the finest), after the network's
+    // inference on its own stream
     constexpr int kChains = 3;
     Chain ch[kChains];
     const bool warm_large = warm_depth >= 0 && c->counts[warm_depth] > kSmallRows;
     for (int d = 0; d <= D; d++)
         if (c->counts[d] > kSmallRows) ch[d == D ? 0 : (warm_large && d == warm_depth ? 2 : 1)].depths.push_back(d);
+    // A chain's SpMV instance (cells per thread for its largest tile), dynamic
+    // LDS (cell values of that tile) and one resident round of workgroups.
+    struct Shape {
+        int inst;
+        size_t lds;
+        int64_t tiles, budget;
+    };
+    auto shape_of = [&](const std::vector<int>& depths) {
+        int32_t cnt = 1;
+        int64_t tiles = 0;
+        for (int d : depths) {
+            cnt = std::max(cnt, c->plan_maxcount[d]);
+            tiles += tiles_of(c->counts[d]);
+        }
+        const int inst = spmv_instance((8 * cnt + kSpmvThreads - 1) / kSpmvThreads);
+        const size_t lds = size_t(8) * 4 * size_t(cnt);
+        return Shape{inst, lds, tiles, int64_t(spmv_wg_per_cu(inst, lds)) * std::max(1, c->num_cu)};
+    };
+    // One chain when every tile of all these depths has a workgroup of its own
+    // in one resident round: an iteration is then bound by its launches, and
+    // one chain issues half of them.  Larger depths keep two chains, which
+    // fill each other's gaps and leave the finest depth the whole chip once
+    // the others are done.
+    if (!serial && !ch[0].depths.empty() && !ch[1].depths.empty()) {
+        std::vector<int> all = ch[1].depths;
+        all.push_back(D);
+        const Shape f = shape_of(all);
+        if (f.tiles <= f.budget && !(warm_depth == D && c->counts[D] > kSmallRows)) {
+            ch[0].depths = all;
+            ch[1].depths.clear();
+        }
+    }
     ch[0].s = s;
     ch[1].s = serial ? s : c->stream2;
     ch[2].s = serial ? s : c->stream4;
@@ -1023,9 +1106,7 @@ prg_status solve_all(prg_ctx* c, prg_solve_stats* stats) {
         }
         return c->ev_pool[ev_used++];
     };
-    std::vector<hipEvent_t> dbeg(D + 1, nullptr), dend(D + 1, nullptr);
     std::vector<double> ms(D + 1, 0.0);
-    std::vector<double> ov(size_t(4) * (D + 1), 0.0);
     prg_status result = PRG_OK;
     auto stencil_of = [&](int d) {
         Stencil S;
@@ -1040,11 +1121,10 @@ prg_status solve_all(prg_ctx* c, prg_solve_stats* stats) {
     int nsegs = 0;
     for (auto& h : ch) nsegs += int(h.depths.size());
     if (nsegs > kMaxSegs) throw Error{PRG_E_ARG, "too many large depths"};
-    static_assert(kMaxSegs * sizeof(CgState) <= kHostStates, "chain states exceed their pinned area");
-    static_assert(kHostStates + kMaxSegs * sizeof(Seg) <= kHostPlanMax, "segment table exceeds the pinned staging area");
-    static_assert(kHostPlanSum + (kMaxDepth + 1) * 8 <= 4092, "plan counts exceed the pinned area (its last 4 bytes hold the owned-corner count)");
-    CgState* hst = static_cast<CgState*>(c->cg_host);
-    Seg* hseg = reinterpret_cast<Seg*>(static_cast<uint8_t*>(c->cg_host) + kHostStates);
+    uint8_t* host = static_cast<uint8_t*>(c->cg_host);
+    CgState* hst = reinterpret_cast<CgState*>(host);
+    int32_t* hdone = reinterpret_cast<int32_t*>(host + kHostDone);
+    Seg* hseg = reinterpret_cast<Seg*>(host + kHostSegs);
     Seg* dseg = reinterpret_cast<Seg*>(c->cg_seg.reserve(std::max<size_t>(1, size_t(nsegs)) * sizeof(Seg)));
     {
         int si = 0;
@@ -1055,11 +1135,7 @@ prg_status solve_all(prg_ctx* c, prg_solve_stats* stats) {
             if (!cnt) continue;
             // vectors: one 64-float-aligned segment per depth
             std::vector<int64_t> voff(cnt + 1, 0);
-            int64_t tiles_all = 0;
-            for (int i = 0; i < cnt; i++) {
-                voff[i + 1] = voff[i] + ((c->counts[h.depths[i]] + 63) / 64) * 64;
-                tiles_all += tiles_of(c->counts[h.depths[i]]);
-            }
+            for (int i = 0; i < cnt; i++) voff[i + 1] = voff[i] + ((c->counts[h.depths[i]] + 63) / 64) * 64;
             float* V[5];
             for (int v = 0; v < 5; v++) V[v] = c->cg_vec[k][v].reserve(size_t(voff[cnt]));
             double* rr = c->cg_part[k][0].reserve(size_t(cnt) * 2 * kMaxWG);
@@ -1067,16 +1143,13 @@ prg_status solve_all(prg_ctx* c, prg_solve_stats* stats) {
             double* bb = c->cg_part[k][2].reserve(size_t(cnt) * std::max(kMaxWG, kMaxSpmvWG));
             h.st = reinterpret_cast<CgState*>(c->cg_state[k].reserve(size_t(cnt) * sizeof(CgState)));
             h.hst = hst + si;
+            h.hdone = hdone + si;
+            h.beg = new_event();
             h.ev = new_event();
-            // the chain's SpMV instance (cells per thread for its largest tile)
-            // and workgroups: one resident round, shared by tile count
-            int32_t kc = 1;
-            for (int i = 0; i < cnt; i++)
-                kc = std::max(kc, (8 * std::max(1, c->plan_maxcount[h.depths[i]]) + kSpmvThreads - 1) / kSpmvThreads);
-            h.inst = spmv_instance(kc);
-            size_t lds = 0;  // cell values of the largest tile among the chain's depths
-            for (int i = 0; i < cnt; i++) lds = std::max(lds, size_t(8) * 4 * std::max(1, c->plan_maxcount[h.depths[i]]));
-            const int64_t budget = int64_t(spmv_wg_per_cu(h.inst, lds)) * std::max(1, c->num_cu);
+            // workgroups: one resident round, shared by tile count
+            const Shape f = shape_of(h.depths);
+            const int64_t tiles_all = f.tiles, budget = f.budget;
+            h.inst = f.inst;
             int32_t wg = 0, vwg = 0;
             for (int i = 0; i < cnt; i++) {
                 const int d = h.depths[i];
@@ -1103,12 +1176,20 @@ prg_status solve_all(prg_ctx* c, prg_solve_stats* stats) {
                 g.pq = pq + size_t(i) * kMaxSpmvWG;
                 g.bb = bb + size_t(i) * std::max(kMaxWG, kMaxSpmvWG);
                 g.st = h.st + i;
+                g.pnt = c->pnt.get() + 27 * c->pnt_off[d];
+                g.b = c->div.get() + c->bases[d];
+                g.X = X + c->bases[d];
+                g.hst = h.hst + i;
+                g.hdone = h.hdone + i;
+                g.hout = ov + 4 * d;
+                g.zero_x = d == warm_depth ? 0 : 1;
+                h.hdone[i] = 0;
                 const Stencil S = stencil_of(d);
                 for (int j = 0; j < 27; j++) g.L[j] = S.L[j];
             }
             h.nwg = wg;
             h.nvwg = vwg;
-            h.lds = lds;
+            h.lds = f.lds;
             si += cnt;
         }
     }
@@ -1119,7 +1200,9 @@ prg_status solve_all(prg_ctx* c, prg_solve_stats* stats) {
         if (nsegs) PRG_HIP(hipMemcpyAsync(dseg, hseg, size_t(nsegs) * sizeof(Seg), hipMemcpyHostToDevice, s));
         hipEvent_t es0 = new_event(), es1 = new_event();
         PRG_HIP(hipEventRecord(es0, s));
-        for (hipStream_t x : {c->stream2, c->stream3, c->stream4}) PRG_HIP(hipStreamWaitEvent(x, es0, 0));
+        if (!ch[1].depths.empty()) PRG_HIP(hipStreamWaitEvent(c->stream2, es0, 0));
+        if (jobs.count || warm_depth >= 0) PRG_HIP(hipStreamWaitEvent(c->stream3, es0, 0));
+        if (!ch[2].depths.empty()) PRG_HIP(hipStreamWaitEvent(c->stream4, es0, 0));
         // The network runs ahead of the solve of its depth: on that depth's
         // chain stream when the depth is large (the finest depth's chain or
         // chain 2), else on the small depths' stream.  A chain on the same
@@ -1136,7 +1219,7 @@ prg_status solve_all(prg_ctx* c, prg_solve_stats* stats) {
             PRG_HIP(hipEventRecord(es0, small_s));
             k_cg_small<<<jobs.count, kSmallBlock, 0, small_s>>>(jobs, c->d_stencil.get(), c->pnt.get(),
                                                                 c->div.get(), X, warm_depth, tol, fixed, max_iters,
-                                                                refresh, outv);
+                                                                refresh, ov);
             PRG_CHECK_LAUNCH();
             PRG_HIP(hipEventRecord(es1, small_s));
         }
@@ -1144,29 +1227,25 @@ prg_status solve_all(prg_ctx* c, prg_solve_stats* stats) {
         auto begin_chain = [&](Chain& h) {
             if (ew && std::find(h.depths.begin(), h.depths.end(), warm_depth) != h.depths.end())
                 PRG_HIP(hipStreamWaitEvent(h.s, ew, 0));
-            for (size_t i = 0; i < h.depths.size(); i++) {
-                const int d = h.depths[i];
-                const Seg& g = hseg[h.seg0 + i];
-                const int64_t n = c->counts[d], base = c->bases[d];
-                dbeg[d] = new_event();
-                dend[d] = new_event();
-                PRG_HIP(hipEventRecord(dbeg[d], h.s));
+            PRG_HIP(hipEventRecord(h.beg, h.s));
+            double bytes = 0.0;
+            for (int d : h.depths) bytes += (d == warm_depth ? kPntRowBytes + 20.0 : 16.0) * double(c->counts[d]);
+            {
                 // b read, xs, r, p written; x0 read and A x0 formed unless x0 = 0
-                TimedScope ts(c->kt, "cg_init", (d == warm_depth ? kPntRowBytes + 20.0 : 16.0) * double(n));
-                k_cg_init<<<g.nvwg, kVecThreads, 0, h.s>>>(c->pnt.get() + 27 * c->pnt_off[d], n, stencil_of(d),
-                                                          c->div.get() + base, X + base, d == warm_depth ? 0 : 1,
-                                                          g.XS, g.R, g.P0, g.rr, g.bb, g.st);
+                TimedScope ts(c->kt, "cg_init", bytes);
+                k_cg_init<<<h.nvwg, kVecThreads, 0, h.s>>>(dseg + h.seg0, int32_t(h.depths.size()));
                 PRG_CHECK_LAUNCH();
-                if (d == warm_depth) {
-                    k_warm_reset_decide<<<1, kVecThreads, 0, h.s>>>(g.rr, g.bb, g.nvwg, g.st);
-                    PRG_CHECK_LAUNCH();
-                    k_warm_reset_apply<<<g.nvwg, kVecThreads, 0, h.s>>>(n, c->div.get() + base, g.XS, g.R, g.P0,
-                                                                        g.rr, g.bb, g.st);
-                    PRG_CHECK_LAUNCH();
-                }
+            }
+            for (size_t i = 0; i < h.depths.size(); i++) {
+                if (h.depths[i] != warm_depth) continue;
+                const Seg& g = hseg[h.seg0 + i];
+                k_warm_reset_decide<<<1, kVecThreads, 0, h.s>>>(g.rr, g.bb, g.nvwg, g.st);
+                PRG_CHECK_LAUNCH();
+                k_warm_reset_apply<<<g.nvwg, kVecThreads, 0, h.s>>>(g.n, g.b, g.XS, g.R, g.P0, g.rr, g.bb, g.st);
+                PRG_CHECK_LAUNCH();
             }
             h.issued = 0;
-            h.batch = kFirstBatch;
+            h.launched.clear();
         };
         // iteration `it` (1-based) of a chain: SpMV, update, and the residual
         // refresh when due
@@ -1195,82 +1274,69 @@ prg_status solve_all(prg_ctx* c, prg_solve_stats* stats) {
                 PRG_CHECK_LAUNCH();
             }
             if ((it % refresh) == 0) {
-                for (int i = 0; i < cnt; i++) {
-                    const int d = h.depths[i];
-                    const Seg& g = hseg[h.seg0 + i];
-                    TimedScope ts(c->kt, "cg_refresh", kResidualRowBytes * double(g.n));
-                    h.launched.emplace_back(ts.idx, it);
-                    k_cg_refresh<<<g.nvwg, kVecThreads, 0, h.s>>>(c->pnt.get() + 27 * c->pnt_off[d], g.n,
-                                                                 stencil_of(d), c->div.get() + c->bases[d], g.XS,
-                                                                 g.R, g.rr + (it & 1) * kMaxWG, g.st);
-                    PRG_CHECK_LAUNCH();
-                }
+                TimedScope ts(c->kt, "cg_refresh", kResidualRowBytes * double(rows));
+                h.launched.emplace_back(ts.idx, it);
+                k_cg_refresh<<<h.nvwg, kVecThreads, 0, h.s>>>(dseg + h.seg0, cnt, it);
+                PRG_CHECK_LAUNCH();
             }
         };
-        // the chain's states read back after its queued iterations
+        auto chain_done = [&](const Chain& h) {
+            for (size_t i = 0; i < h.depths.size(); i++)
+                if (!__atomic_load_n(h.hdone + i, __ATOMIC_RELAXED)) return false;
+            return true;
+        };
+        // Behind the queued iterations, without waiting for them: the true
+        // residuals, the solution and the states (queued again, and
+        // superseding these, if more iterations follow).
         auto end_batch = [&](Chain& h) {
-            h.issued += h.batch;
-            PRG_HIP(hipMemcpyAsync(h.hst, h.st, h.depths.size() * sizeof(CgState), hipMemcpyDeviceToHost, h.s));
+            double bytes = 0.0;
+            for (int d : h.depths) bytes += kResidualRowBytes * double(c->counts[d]);
+            {
+                TimedScope ts(c->kt, "cg_true_residual", bytes);
+                h.end_idx = ts.idx;
+                k_true_residual<<<h.nvwg, kVecThreads, 0, h.s>>>(dseg + h.seg0, int32_t(h.depths.size()));
+                PRG_CHECK_LAUNCH();
+            }
+            k_true_residual_finish<<<unsigned(h.depths.size()), kVecThreads, 0, h.s>>>(dseg + h.seg0);
+            PRG_CHECK_LAUNCH();
             PRG_HIP(hipEventRecord(h.ev, h.s));
             h.waiting = true;
         };
-        auto issue_batch = [&](Chain& h) {
+        // up to `count` iterations, fewer once the host sees the chain's flags
+        auto issue_batch = [&](Chain& h, int count) {
             h.launched.clear();
-            for (int k = 0; k < h.batch; k++) launch_iter(h, h.issued + k + 1);
+            for (int k = 0; k < count && !chain_done(h); k++) launch_iter(h, ++h.issued);
             end_batch(h);
         };
-        auto end_chain = [&](Chain& h) {
-            for (size_t i = 0; i < h.depths.size(); i++) {
-                const int d = h.depths[i];
-                const Seg& g = hseg[h.seg0 + i];
-                const int64_t n = c->counts[d], base = c->bases[d];
-                {
-                    TimedScope ts(c->kt, "cg_true_residual", kResidualRowBytes * double(n));
-                    k_true_residual<<<g.nvwg, kVecThreads, 0, h.s>>>(c->pnt.get() + 27 * c->pnt_off[d], n,
-                                                                    stencil_of(d), c->div.get() + base, g.XS, g.bb);
-                    PRG_CHECK_LAUNCH();
-                }
-                k_true_residual_finish<<<1, kVecThreads, 0, h.s>>>(g.bb, g.nvwg, g.rr, g.nvwg, kMaxWG, g.st,
-                                                                  outv + 4 * d);
-                PRG_CHECK_LAUNCH();
-                PRG_HIP(hipMemcpyAsync(X + base, g.XS, size_t(n) * 4, hipMemcpyDeviceToDevice, h.s));
-                PRG_HIP(hipEventRecord(dend[d], h.s));
-            }
-        };
 
-        // Each chain: init, batches of iterations with a state read-back after
-        // each, true residuals; the host polls the chains so none waits for
-        // another.  Serial mode runs chain 2, then 1, the finest depth last.
+        // Each chain: init, batches of iterations with their end behind them;
+        // the host polls the chains so none waits for another.  Serial mode
+        // runs chain 2, then 1, the finest depth last.
         std::vector<int> serial_order;
         for (int k = kChains - 1; k >= 0; k--)
             if (!ch[k].depths.empty()) serial_order.push_back(k);
         size_t serial_next = 0;
         auto start_chain = [&](int k) {
             begin_chain(ch[k]);
-            issue_batch(ch[k]);
+            issue_batch(ch[k], kFirstBatch);
         };
         if (serial) {
             if (!serial_order.empty()) start_chain(serial_order[serial_next++]);
         } else {
             // every chain's init, then the first batches one iteration at a
-            // time across the chains, so no chain waits for another's launches
+            // time across the chains, so no chain waits for another's
+            // launches.  The first batch usually covers the whole solve.
             for (int k = 0; k < kChains; k++)
-                if (!ch[k].depths.empty()) {
-                    begin_chain(ch[k]);
-                    ch[k].launched.clear();
-                }
-            for (int i = 0; i < kFirstBatch; i++)
-                for (int k = 0; k < kChains; k++)
-                    if (!ch[k].depths.empty()) launch_iter(ch[k], i + 1);
-            // The first batch usually covers the whole solve, so each chain's
-            // true residuals and solution copy go right behind it (they are
-            // queued again, and supersede these, if more iterations follow);
-            // the end of a chain then waits for no host poll.
-            for (int k = 0; k < kChains; k++)
-                if (!ch[k].depths.empty()) {
-                    end_batch(ch[k]);
-                    end_chain(ch[k]);
-                    ch[k].ended = true;
+                if (!ch[k].depths.empty()) begin_chain(ch[k]);
+            for (int i = 0; i <= kFirstBatch; i++)
+                for (int k = 0; k < kChains; k++) {
+                    Chain& h = ch[k];
+                    if (h.depths.empty() || h.waiting) continue;
+                    if (i == kFirstBatch || chain_done(h)) {
+                        end_batch(h);
+                    } else {
+                        launch_iter(h, ++h.issued);
+                    }
                 }
         }
         while (true) {
@@ -1292,13 +1358,10 @@ prg_status solve_all(prg_ctx* c, prg_solve_stats* stats) {
                 for (const auto& l : h.launched)
                     if (l.second > last && all_done) c->kt.relabel(l.first, "cg_idle");
                 if (all_done) {
-                    if (!h.ended) end_chain(h);
                     if (serial && serial_next < serial_order.size()) start_chain(serial_order[serial_next++]);
                 } else {
-                    h.batch = 6;
-                    issue_batch(h);
-                    h.ended = !serial;
-                    if (h.ended) end_chain(h);
+                    c->kt.relabel(h.end_idx, "cg_idle");  // superseded
+                    issue_batch(h, kNextBatch);
                 }
             }
             if (!active) break;
@@ -1311,21 +1374,14 @@ prg_status solve_all(prg_ctx* c, prg_solve_stats* stats) {
             c->kt.recs["cg_small"].launches += 1;
             c->kt.recs["cg_small"].total_ms += t;
         }
-        for (int d = 0; d <= D; d++)
-            if (dbeg[d]) {
-                PRG_HIP(hipEventSynchronize(dend[d]));
-                float t = 0.0f;
-                PRG_HIP(hipEventElapsedTime(&t, dbeg[d], dend[d]));
-                ms[d] = t;
-            }
-        // the context stream continues after every chain and the small solves
-        for (hipStream_t x : {c->stream2, c->stream3, c->stream4}) {
-            hipEvent_t ej = new_event();
-            PRG_HIP(hipEventRecord(ej, x));
-            PRG_HIP(hipStreamWaitEvent(s, ej, 0));
+        for (const Chain& h : ch) {
+            if (h.depths.empty()) continue;
+            float t = 0.0f;  // a chain's depths are solved together
+            PRG_HIP(hipEventElapsedTime(&t, h.beg, h.ev));
+            for (int d : h.depths) ms[d] = t;
         }
-        PRG_HIP(hipMemcpyAsync(ov.data(), outv, ov.size() * 8, hipMemcpyDeviceToHost, s));
-        PRG_HIP(hipStreamSynchronize(s));
+        // the context stream continues after every chain and the small solves
+        for (hipStream_t x : {c->stream2, c->stream3, c->stream4, s}) PRG_HIP(hipStreamSynchronize(x));
     } catch (...) {
         for (hipStream_t x : {c->stream2, c->stream3, c->stream4}) (void)hipStreamSynchronize(x);
         (void)hipStreamSynchronize(s);
