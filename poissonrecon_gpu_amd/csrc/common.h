@@ -16,9 +16,15 @@ namespace prg {
 
 constexpr int kMaxDepth = 10;  // 3D key bits must fit in uint32
 
-// A context's pinned read-back area; its last 4 bytes hold the owned-corner count.
+// A context's pinned read-back area: the solver's part, then counts that
+// kernels write there themselves (a copy behind the kernel would cost about
+// 10 us): non-empty nodes per depth, the mesh's vertices and triangles, the
+// owned corners.
 constexpr size_t kCgHostBytes = 8192;
+constexpr size_t kCgHostLevels = kCgHostBytes - 64;
+constexpr size_t kCgHostMesh = kCgHostBytes - 16;
 constexpr size_t kCgHostTopo = kCgHostBytes - 4;
+static_assert(kCgHostLevels + 4 * (kMaxDepth + 1) <= kCgHostMesh, "counts overlap");
 
 // ---- errors ------------------------------------------------------------------
 struct Error {

@@ -500,14 +500,13 @@ void start_topology(prg_ctx* c) {
     const int D = c->D;
     const int64_t MD = c->MD(), baseD = c->bases[D];
     KernelTimer& kt = c->kt;
-    PoolBuf<int32_t> cmask{&c->pool[78]}, oref{&c->pool[79]}, cbase{&c->pool[80]}, vtot{&c->pool[81]},
+    PoolBuf<int32_t> cmask{&c->pool[78]}, oref{&c->pool[79]}, cbase{&c->pool[80]},
         ccount{&c->pool[92]};
     PoolBuf<float> btab{&c->pool[91]};
     cmask.reserve(MD);
     ccount.reserve(MD);
     oref.reserve(8 * MD);
     cbase.reserve(MD);
-    vtot.reserve(1);
     // stage time: events on the stream the topology runs on
     resolve_stage(c, PRG_STAGE_MC_TOPOLOGY);
     PRG_HIP(hipEventRecord(c->stage_ev[PRG_STAGE_MC_TOPOLOGY][0], s));
@@ -519,8 +518,7 @@ void start_topology(prg_ctx* c) {
                                                                MD, cmask.get(), ccount.get(), oref.get());
         PRG_CHECK_LAUNCH();
     }
-    scan_exclusive(ccount.get(), cbase.get(), MD, vtot.get(), s, scr, kt);
-    PRG_HIP(hipMemcpyAsync(topo_count_host(c), vtot.get(), 4, hipMemcpyDeviceToHost, s));
+    scan_exclusive(ccount.get(), cbase.get(), MD, topo_count_host(c), s, scr, kt);
     const int64_t nbt = int64_t(D + 1) * (int64_t(1) << D) * 2;
     btab.reserve(4 * nbt);
     k_corner_basis<<<grid_for(nbt, kBlock), kBlock, 0, s>>>(c->d_base_fn.get(), D, btab.get());
@@ -541,11 +539,11 @@ void extract_leaf_mesh(prg_ctx* c) {
     // per leaf slot: owned-corner mask and count, their scan (corner ids);
     // owned sign-change edge mask and count, their scan (vertex ids)
     PoolBuf<int32_t> cmask{&c->pool[78]}, oref{&c->pool[79]}, cbase{&c->pool[80]}, emask{&c->pool[82]},
-        eref{&c->pool[83]}, ebase{&c->pool[84]}, etot{&c->pool[85]}, ntri{&c->pool[86]}, toff{&c->pool[87]},
-        ttot{&c->pool[88]}, ecount{&c->pool[93]};
+        eref{&c->pool[83]}, ebase{&c->pool[84]}, ntri{&c->pool[86]}, toff{&c->pool[87]}, ecount{&c->pool[93]};
     PoolBuf<float> vval{&c->pool[89]}, btab{&c->pool[91]};
     float* CV = c->corner_vals.reserve(8 * MD);
     int32_t NV = 0, NT = 0;
+    int32_t* counts = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(c->cg_host) + kCgHostMesh);
     if (c->topo_gen != c->tree_gen) start_topology(c);
     if (c->topo_pending) {
         PRG_HIP(hipEventSynchronize(c->topo_ev));
@@ -574,10 +572,8 @@ void extract_leaf_mesh(prg_ctx* c) {
         ecount.reserve(MD);
         eref.reserve(12 * MD);
         ebase.reserve(MD);
-        etot.reserve(1);
         ntri.reserve(MD);
         toff.reserve(MD);
-        ttot.reserve(1);
         PoolBuf<uint8_t> cubes{&c->pool[94]};
         cubes.reserve(MD);
         {
@@ -592,11 +588,10 @@ void extract_leaf_mesh(prg_ctx* c) {
                                                                    ecount.get(), eref.get());
             PRG_CHECK_LAUNCH();
         }
-        scan_exclusive2(ecount.get(), ebase.get(), etot.get(), ntri.get(), toff.get(), ttot.get(), MD, s, c->scratch,
-                        kt);
-        PRG_HIP(hipMemcpyAsync(&NV, etot.get(), 4, hipMemcpyDeviceToHost, s));
-        PRG_HIP(hipMemcpyAsync(&NT, ttot.get(), 4, hipMemcpyDeviceToHost, s));
+        scan_exclusive2(ecount.get(), ebase.get(), counts, ntri.get(), toff.get(), counts + 1, MD, s, c->scratch, kt);
         PRG_HIP(hipStreamSynchronize(s));
+        NV = counts[0];
+        NT = counts[1];
         float* MV = c->mesh_v.reserve(size_t(3) * NV);
         int32_t* MT = c->mesh_t.reserve(size_t(3) * NT);
         // caller buffers that hold the mesh: the vertex copy (second stream)

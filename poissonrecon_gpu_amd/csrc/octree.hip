@@ -87,7 +87,7 @@ __global__ void __launch_bounds__(kBlock) k_bbox_partial(const float* xyz, int64
 
 // Scale and centre from the block minima / maxima, in the reference's float
 // operations (main.cu:539-545): tr = (centre x, y, z, scale).
-__global__ void __launch_bounds__(1024) k_bbox_final(const float* part, int nb, float* tr) {
+__global__ void __launch_bounds__(1024) k_bbox_final(const float* part, int nb, float* tr, float* tr_host) {
     // minima and maxima are exact in any order: one partial per thread, then a tree
     __shared__ float red[6][1024];
     const int tid = threadIdx.x;
@@ -119,8 +119,8 @@ __global__ void __launch_bounds__(1024) k_bbox_final(const float* part, int nb, 
         center[a] = (mx[a] + mn[a]) / 2;
     }
     scale = scale * 1.25f;
-    for (int a = 0; a < 3; a++) tr[a] = center[a] - scale / 2;
-    tr[3] = scale;
+    for (int a = 0; a < 3; a++) tr_host[a] = tr[a] = center[a] - scale / 2;
+    tr_host[3] = tr[3] = scale;
 }
 
 // one 32-byte record per point (x, y, z, nx, ny, nz, 0, 0), so the sort's
@@ -438,7 +438,8 @@ struct LevelArrays {
 // The bottom-up step (k_level_up) for depths
 // ds .. 1: per depth, chunks of the compact nodes with a workgroup scan of
 // the parent-run heads carried across chunks.
-__global__ void __launch_bounds__(kSmallThreads) k_levels_up_small(LevelArrays A, int32_t* ne, int ds, int D) {
+__global__ void __launch_bounds__(kSmallThreads) k_levels_up_small(LevelArrays A, int32_t* ne, int ds, int D,
+                                                                   int32_t* host_ne) {
     __shared__ int32_t sc[kSmallThreads];
     __shared__ int32_t carry;
     const int tid = threadIdx.x;
@@ -481,6 +482,7 @@ __global__ void __launch_bounds__(kSmallThreads) k_levels_up_small(LevelArrays A
         if (tid == 0) ne[d - 1] = carry;
         __syncthreads();
     }
+    if (tid <= D) host_ne[tid] = ne[tid];  // pinned
 }
 
 struct SmallLevels {
@@ -586,7 +588,7 @@ void normalize_points(prg_ctx* c, const float* xyz, const float* nxyz, int64_t n
         PRG_CHECK_LAUNCH();
     }
     {
-        k_bbox_final<<<1, 1024, 0, s>>>(part.get(), blocks, c->transform_dev.reserve(4));
+        k_bbox_final<<<1, 1024, 0, s>>>(part.get(), blocks, c->transform_dev.reserve(4), c->transform_host);
         PRG_CHECK_LAUNCH();
     }
     c->N = n;
@@ -597,8 +599,7 @@ void normalize_points(prg_ctx* c, const float* xyz, const float* nxyz, int64_t n
         PRG_CHECK_LAUNCH();
     }
     c->points_sorted = false;
-    // the host copy of (centre, scale) arrives with the next synchronisation
-    PRG_HIP(hipMemcpyAsync(c->transform_host, c->transform_dev.get(), 16, hipMemcpyDeviceToHost, s));
+    // the host copy of (centre, scale), in pinned memory, is there after the next synchronisation
     c->transform_pending = true;
     if (!on_device) PRG_HIP(hipStreamSynchronize(s));  // the staging copies must finish before the caller reuses its arrays
 }
@@ -740,15 +741,14 @@ void build_octree(prg_ctx* c) {
         LA.ndi[d] = NDI[d]->get();
         LA.pos[d] = POS[d]->get();
     }
+    int32_t* hne = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(c->cg_host) + kCgHostLevels);
     {
         // (ds >= 1: depth 1 has at most 8 nodes)
         TimedScope ts(kt, "level_up_small", 28.0 * double(ub[ds]));
-        k_levels_up_small<<<1, kSmallThreads, 0, s>>>(LA, ne_dev.get(), ds, D);
+        k_levels_up_small<<<1, kSmallThreads, 0, s>>>(LA, ne_dev.get(), ds, D, hne);
         PRG_CHECK_LAUNCH();
     }
     {
-        std::vector<int32_t> hne(D + 1);
-        PRG_HIP(hipMemcpyAsync(hne.data(), ne_dev.get(), size_t(D + 1) * 4, hipMemcpyDeviceToHost, s));
         PRG_HIP(hipStreamSynchronize(s));
         for (int d = 0; d <= D; d++) NE[d] = hne[d];
         if (c->transform_pending) {

@@ -884,7 +884,7 @@ static_assert(kHostDone + kMaxSegs * 4 <= kHostOut, "flags exceed their pinned a
 static_assert(kHostOut + (kMaxDepth + 1) * 4 * 8 <= kHostSegs, "results exceed their pinned area");
 static_assert(kHostSegs + kMaxSegs * sizeof(Seg) <= kHostPlanMax, "segment table exceeds the pinned staging area");
 static_assert(kHostPlanMax + (kMaxDepth + 1) * 4 <= kHostPlanSum && kHostPlanSum % 8 == 0, "plan read-back layout");
-static_assert(kHostPlanSum + (kMaxDepth + 1) * 8 <= kCgHostTopo, "plan counts exceed the pinned area");
+static_assert(kHostPlanSum + (kMaxDepth + 1) * 8 <= kCgHostLevels, "plan counts exceed the pinned area");
 
 int32_t* plan_maxcount_host(prg_ctx* c) {
     return reinterpret_cast<int32_t*>(static_cast<uint8_t*>(c->cg_host) + kHostPlanMax);
@@ -940,7 +940,7 @@ int64_t tiles_of(int64_t n) { return (n / 8 + kTile - 1) / kTile; }
 
 // Tile plans of every depth above kSmallRows rows, once per octree: on the
 // second stream after the build (on the context stream when kernels are
-// timed), with the per-depth largest tile count copied to pinned memory.
+// timed), with the per-depth tile counts written to pinned memory.
 void start_plans(prg_ctx* c) {
     hipStream_t s = c->kt.enabled ? c->stream : c->stream2;
     const int D = c->D;
@@ -975,11 +975,9 @@ void start_plans(prg_ctx* c) {
     {
         PlanOffsets P{};
         for (int d = 0; d <= D + 1; d++) P.off[d] = c->plan_tile_off[d];
-        k_plan_max<<<unsigned(D + 1), 1024, 0, s>>>(cnt, P, mx, sm);
+        k_plan_max<<<unsigned(D + 1), 1024, 0, s>>>(cnt, P, plan_maxcount_host(c), plan_sumcount_host(c));
         PRG_CHECK_LAUNCH();
     }
-    PRG_HIP(hipMemcpyAsync(plan_maxcount_host(c), mx, size_t(D + 1) * 4, hipMemcpyDeviceToHost, s));
-    PRG_HIP(hipMemcpyAsync(plan_sumcount_host(c), sm, size_t(D + 1) * 8, hipMemcpyDeviceToHost, s));
     PRG_HIP(hipEventRecord(c->plan_ev, s));
     c->plan_pending = true;
     c->plan_gen = c->tree_gen;

@@ -44,6 +44,7 @@
 #include <vector>
 
 #include "ctx.h"
+#include "lookback.h"
 #include "mc_common.h"
 #include "tile.h"
 
@@ -193,14 +194,105 @@ __global__ void __launch_bounds__(kBlockS) k_face_marks_up(int64_t base, int64_t
     if (faces) face_visit(Y, faces, key, pnt, L, parent, d, D, inter, up);
 }
 
-__global__ void __launch_bounds__(kBlockS) k_flag_coarse_leaves(const int32_t* child_base, int64_t n, int32_t* flag) {
-    const int64_t i = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
-    if (i < n) flag[i] = (i >= 1 && child_base[i] < 0) ? 1 : 0;
+// The same for depths ds .. 0, of at most kSmallUp nodes each, by one
+// workgroup: a launch per depth costs about 4 us whatever it does.  The
+// faces of a depth are ORed in L2; the fence completes them before the
+// barrier, and the loads read them there.
+constexpr int kUpBlock = 1024;
+constexpr int64_t kSmallUp = 4096;
+__global__ void __launch_bounds__(kUpBlock) k_face_marks_up_small(int ds, const uint32_t* key, const int32_t* pnt,
+                                                                  Levels L, const int32_t* parent, int D,
+                                                                  uint8_t* inter, uint32_t* up) {
+    for (int d = ds; d >= 0; d--) {
+        for (int64_t Y = L.base[d] + threadIdx.x; Y < L.base[d + 1]; Y += kUpBlock) {
+            const uint32_t w = __hip_atomic_load(up + (Y >> 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const uint32_t faces = (w >> (8 * (Y & 3))) & 0xffu;
+            if (faces) face_visit(Y, faces, key, pnt, L, parent, d, D, inter, up);
+        }
+        __threadfence();
+        __syncthreads();
+    }
 }
 
-__global__ void __launch_bounds__(kBlockS) k_compact(const int32_t* flag, const int32_t* off, int64_t n, int32_t* out) {
-    const int64_t i = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
-    if (i < n && flag[i]) out[off[i]] = int32_t(i);
+// bytes of a buffer set to a repeated value, by a whole grid (16-byte stores, then the tail)
+__device__ __forceinline__ void fill_bytes(void* p, int64_t bytes, uint32_t v, int64_t gid, int64_t gsize) {
+    uint4* q = static_cast<uint4*>(p);
+    const int64_t n16 = bytes >> 4;
+    for (int64_t i = gid; i < n16; i += gsize) q[i] = uint4{v, v, v, v};
+    uint8_t* b = static_cast<uint8_t*>(p) + 16 * n16;
+    if (gid < (bytes & 15)) b[gid] = uint8_t(v);
+}
+
+// Everything the subdivision starts cleared: counters, face marks, the up
+// bytes, the needed corners; root_of to -1.
+__global__ void __launch_bounds__(kBlockS) k_sub_init(int32_t* cnt, uint8_t* inter, uint32_t* up, uint8_t* need,
+                                                      int32_t* root_of, int64_t M, int64_t baseD) {
+    const int64_t gid = int64_t(blockIdx.x) * kBlockS + threadIdx.x, gsize = int64_t(gridDim.x) * kBlockS;
+    fill_bytes(cnt, kCntSlots * 4, 0, gid, gsize);
+    fill_bytes(inter, 6 * M, 0, gid, gsize);
+    fill_bytes(up, 4 * ((M + 3) / 4), 0, gid, gsize);
+    fill_bytes(need, 8 * baseD, 0, gid, gsize);
+    fill_bytes(root_of, 4 * M, 0xffffffffu, gid, gsize);
+}
+
+constexpr int kSelItems = 16;
+constexpr int kSelTile = kBlockS * kSelItems;
+
+// In one launch (lookback.h), the list of the i < n with a mark, in order:
+// LEAF: the coarse leaves (no children; the root is none), from child_base;
+// else: the bytes of `marks` that are not 0, and each one's place in nid.
+template <bool LEAF>
+__global__ void __launch_bounds__(kBlockS) k_select(const int32_t* __restrict__ child_base,
+                                                    const uint8_t* __restrict__ marks, int64_t n, uint32_t tiles,
+                                                    uint64_t* state, int32_t* __restrict__ list,
+                                                    int32_t* __restrict__ nid, int32_t* count) {
+    __shared__ int32_t lds[kBlockS / 64];
+    __shared__ int32_t s_before;
+    const LookTile t = look_begin(state, tiles);
+    if (t.tile >= tiles) return;
+    const int64_t base = int64_t(t.tile) * kSelTile + int64_t(threadIdx.x) * kSelItems;
+    uint32_t m = 0;
+    if (LEAF) {
+        int32_t v[kSelItems];
+        if (base + kSelItems <= n) {
+#pragma unroll
+            for (int j = 0; j < kSelItems; j += 4)
+                *reinterpret_cast<int4*>(v + j) = *reinterpret_cast<const int4*>(child_base + base + j);
+        } else {
+#pragma unroll
+            for (int j = 0; j < kSelItems; j++) v[j] = base + j < n ? child_base[base + j] : 0;
+        }
+#pragma unroll
+        for (int j = 0; j < kSelItems; j++) m |= (v[j] < 0 && base + j >= 1) ? 1u << j : 0u;
+    } else {
+        uint8_t v[kSelItems];
+        if (base + kSelItems <= n) {
+            *reinterpret_cast<uint4*>(v) = *reinterpret_cast<const uint4*>(marks + base);
+        } else {
+#pragma unroll
+            for (int j = 0; j < kSelItems; j++) v[j] = base + j < n ? marks[base + j] : 0;
+        }
+#pragma unroll
+        for (int j = 0; j < kSelItems; j++) m |= v[j] ? 1u << j : 0u;
+    }
+    int32_t total;
+    const int32_t ex = block_exclusive_scan(__popc(m), lds, total);
+    if (threadIdx.x < 64) {
+        const int32_t b = look_back(state + kLookHeader, t, tiles, total);
+        if (threadIdx.x == 0) {
+            s_before = b;
+            if (t.tile == tiles - 1) *count = b + total;
+        }
+    }
+    __syncthreads();
+    look_end(state, t, tiles);
+    int32_t at = s_before + ex;
+    for (; m; m &= m - 1) {
+        const int64_t i = base + __builtin_ctz(m);
+        list[at] = int32_t(i);
+        if (!LEAF) nid[i] = at;
+        at++;
+    }
 }
 
 // Corner owners of the coarse leaves' corners among the same-depth nodes
@@ -208,7 +300,7 @@ __global__ void __launch_bounds__(kBlockS) k_compact(const int32_t* flag, const 
 // ncl (device) coarse leaves in cl.
 __global__ void __launch_bounds__(kBlockS) k_coarse_corner_owner(const int32_t* cl, const int32_t* ncl,
                                                                  const uint32_t* key, const int32_t* pnt, Levels L,
-                                                                 int D, int32_t* oref, int32_t* need) {
+                                                                 int D, int32_t* oref, uint8_t* need) {
     const int64_t g = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
     if (g >= 8 * int64_t(*ncl)) return;
     const int64_t X = cl[g >> 3];
@@ -340,18 +432,13 @@ __global__ void __launch_bounds__(kBlockS, 5) k_coarse_corner_value(const int32_
 }
 
 // hasTriangle || hasIntersection for each coarse leaf (ProcessLeafNodesAtOtherDepth
-// + ifSubdivide, main.cu:2957-2992); 0 past the ncl coarse leaves, so a scan
-// over all n slots counts the roots.
-__global__ void __launch_bounds__(kBlockS) k_coarse_select(const int32_t* cl, const int32_t* ncl, int64_t n,
-                                                           const int32_t* oref, const int32_t* nid, const float* cv,
-                                                           const uint32_t* key, const int32_t* pnt, Levels L, int D,
-                                                           const uint8_t* inter, int32_t* rflag) {
+// + ifSubdivide, main.cu:2957-2992).
+__global__ void __launch_bounds__(kBlockS) k_coarse_select(const int32_t* cl, const int32_t* ncl, const int32_t* oref,
+                                                           const int32_t* nid, const float* cv, const uint32_t* key,
+                                                           const int32_t* pnt, Levels L, int D, const uint8_t* inter,
+                                                           uint8_t* rflag) {
     const int64_t c = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
-    if (c >= n) return;
-    if (c >= *ncl) {
-        rflag[c] = 0;
-        return;
-    }
+    if (c >= *ncl) return;
     const int64_t X = cl[c];
     // vertices[0] is the (0,0,0) corner in either numbering
     const float v0 = cv[nid[oref[8 * c]]];
@@ -374,30 +461,6 @@ constexpr int kBrickPts = ((1 << kBrickLog) + 1) * ((1 << kBrickLog) + 1) * ((1 
 
 __device__ __forceinline__ int brick_log(int D, int r) { return D - r < kBrickLog ? D - r : kBrickLog; }
 
-// Per root (q < nroots): its real index, bricks and virtual leaves; zero past
-// the roots, so scans over all n slots give the brick and leaf offsets.
-__global__ void __launch_bounds__(kBlockS) k_root_info(const int32_t* cl, const int32_t* ridx, const int32_t* nroots,
-                                                       int64_t n, Levels L, int D, int32_t* roots, int32_t* rbricks,
-                                                       int32_t* rleaves) {
-    const int64_t q = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
-    if (q >= n) return;
-    if (q >= *nroots) {
-        rbricks[q] = 0;
-        rleaves[q] = 0;
-        return;
-    }
-    const int32_t rho = cl[ridx[q]];
-    const int r = depth_of(rho, L, D);
-    roots[q] = rho;
-    rbricks[q] = 1 << (3 * (D - r - brick_log(D, r)));
-    rleaves[q] = 1 << (3 * (D - r));
-}
-
-__global__ void __launch_bounds__(kBlockS) k_root_of(const int32_t* roots, const int32_t* nroots, int32_t* root_of) {
-    const int64_t i = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
-    if (i < *nroots) root_of[roots[i]] = int32_t(i);
-}
-
 // The place in a list (its length in *counter) of each lane with `want`: one
 // atomic per wave, lanes in order.
 __device__ __forceinline__ int32_t wave_append(bool want, int32_t* counter) {
@@ -410,31 +473,98 @@ __device__ __forceinline__ int32_t wave_append(bool want, int32_t* counter) {
     return at + int32_t(__popcll(m & ((uint64_t(1) << lane) - 1)));
 }
 
-// The roots of 2^3 and of 4^3 leaves in lists of their own, and each one's
-// place in its list (sidx).
-__global__ void __launch_bounds__(kBlockS) k_list_small_roots(const int32_t* roots, const int32_t* nroots, Levels L,
-                                                              int D, int32_t* list1, int32_t* list2, int32_t* sidx,
-                                                              int32_t* cnt) {
-    const int64_t q = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
-    const int kb = q < *nroots ? D - depth_of(roots[q], L, D) : 0;
-    const int32_t a1 = wave_append(kb == 1, cnt + kCntSmall1), a2 = wave_append(kb == 2, cnt + kCntSmall2);
-    if (kb == 1) {
-        list1[a1] = int32_t(q);
-        sidx[q] = a1;
+constexpr int kRootBlock = 320;  // one wave per look-back
+constexpr int kRootItems = 16;
+constexpr int kRootTile = kRootBlock * kRootItems;
+
+// The roots, in order, from the marked coarse leaves, in one launch
+// (lookback.h): each root's real index and first brick, its number at its
+// node (root_of), and the roots of 2^3 and of 4^3 leaves in lists of their
+// own with each one's place in its list (sidx).  The last tile leaves the
+// counts in cnt and in pinned memory.  (As flags, compaction, sizes, two
+// scans and an append these were five launches over the upper bound n.)
+__global__ void __launch_bounds__(kRootBlock) k_list_all_roots(const int32_t* __restrict__ cl,
+                                                               const uint8_t* __restrict__ rflag, uint32_t tiles,
+                                                               uint64_t* state, Levels L, int D,
+                                                               int32_t* __restrict__ roots, int32_t* __restrict__ boff,
+                                                               int32_t* __restrict__ root_of,
+                                                               int32_t* __restrict__ list1,
+                                                               int32_t* __restrict__ list2, int32_t* __restrict__ sidx,
+                                                               int32_t* cnt, int32_t* host_cnt) {
+    __shared__ int32_t lds[kRootBlock / 64];
+    __shared__ int32_t s_before[5];
+    const int64_t n = cnt[kCntCoarse];
+    const LookTile t = look_begin(state, tiles);
+    if (t.tile >= tiles) return;
+    const int64_t base = int64_t(t.tile) * kRootTile + int64_t(threadIdx.x) * kRootItems;
+    uint32_t m = 0;
+    if (base < n) {
+        uint8_t v[kRootItems];
+        // (whole 16-byte words lie inside the array, which is sized for the upper bound)
+        *reinterpret_cast<uint4*>(v) = *reinterpret_cast<const uint4*>(rflag + base);
+#pragma unroll
+        for (int j = 0; j < kRootItems; j++) m |= (base + j < n && v[j]) ? 1u << j : 0u;
     }
-    if (kb == 2) {
-        list2[a2] = int32_t(q);
-        sidx[q] = a2;
+    int32_t bricks = 0, leaves = 0, n1 = 0, n2 = 0;
+    for (uint32_t w = m; w; w &= w - 1) {
+        const int kb = D - depth_of(cl[base + __builtin_ctz(w)], L, D);
+        bricks += 1 << (3 * (kb - min(kb, kBrickLog)));
+        leaves += 1 << (3 * kb);
+        n1 += kb == 1;
+        n2 += kb == 2;
+    }
+    int32_t tot[5];
+    int32_t q = block_exclusive_scan(__popc(m), lds, tot[0]);
+    int32_t b = block_exclusive_scan(bricks, lds, tot[1]);
+    (void)block_exclusive_scan(leaves, lds, tot[2]);
+    int32_t a1 = block_exclusive_scan(n1, lds, tot[3]);
+    int32_t a2 = block_exclusive_scan(n2, lds, tot[4]);
+    const int wave = threadIdx.x >> 6;
+    const int32_t mine = wave == 0 ? tot[0] : wave == 1 ? tot[1] : wave == 2 ? tot[2] : wave == 3 ? tot[3] : tot[4];
+    const int32_t x = look_back(state + kLookHeader + int64_t(wave) * tiles, t, tiles, mine);
+    if ((threadIdx.x & 63) == 0) {
+        s_before[wave] = x;
+        if (t.tile == tiles - 1) {
+            const int slot = wave == 0 ? kCntRoots : wave == 1 ? kCntBricks : wave == 2 ? kCntLeaves
+                             : wave == 3 ? kCntSmall1 : kCntSmall2;
+            cnt[slot] = x + mine;
+            host_cnt[slot] = x + mine;
+        }
+    }
+    __syncthreads();
+    look_end(state, t, tiles);
+    q += s_before[0];
+    b += s_before[1];
+    a1 += s_before[3];
+    a2 += s_before[4];
+    for (; m; m &= m - 1) {
+        const int32_t rho = cl[base + __builtin_ctz(m)];
+        const int kb = D - depth_of(rho, L, D);
+        roots[q] = rho;
+        boff[q] = b;
+        root_of[rho] = q;
+        if (kb == 1) {
+            list1[a1] = q;
+            sidx[q] = a1++;
+        }
+        if (kb == 2) {
+            list2[a2] = q;
+            sidx[q] = a2++;
+        }
+        b += 1 << (3 * (kb - min(kb, kBrickLog)));
+        q++;
     }
 }
 
-// counts and signs of n bricks to 0
-__global__ void __launch_bounds__(kBlockS) k_clear_bricks(int32_t* bnv, int32_t* bnt, int8_t* sign, int64_t n) {
+// counts and signs of n bricks to 0, no brick listed for evaluation
+__global__ void __launch_bounds__(kBlockS) k_clear_bricks(int32_t* bnv, int32_t* bnt, int8_t* sign, int32_t* didx,
+                                                          int64_t n) {
     const int64_t i = int64_t(blockIdx.x) * kBlockS + threadIdx.x;
     if (i >= n) return;
     bnv[i] = 0;
     bnt[i] = 0;
     sign[i] = 0;
+    didx[i] = -1;
 }
 
 struct SubArgs {
@@ -450,7 +580,7 @@ struct SubArgs {
     int D;
     const float* iso;
     const int32_t* roots;
-    const int32_t* boff;     // first brick of each root (exclusive scan, nroots + 1 entries)
+    const int32_t* boff;     // first brick of each root
     const int32_t* root_of;  // per real node: its root number, or -1
     const int32_t* cnt;      // device counters
     const int32_t* bmap;     // root number of each brick
@@ -2223,22 +2353,24 @@ void extract_subdivision(prg_ctx* c) {
     if (rd < D - 1) throw Error{PRG_E_STATE, "coarse rows missing"};
 
     // pool slots 97..159
-    PoolBuf<uint8_t> inter{&c->pool[97]};
-    PoolBuf<int32_t> cnt{&c->pool[98]}, flag{&c->pool[99]}, off{&c->pool[100]}, cl{&c->pool[101]},
-        oref{&c->pool[102]}, need{&c->pool[103]}, nid{&c->pool[104]}, clist{&c->pool[105]}, rflag{&c->pool[107]},
-        roff{&c->pool[108]}, ridx{&c->pool[109]}, roots{&c->pool[110]}, rbricks{&c->pool[111]},
-        boff{&c->pool[112]}, rleaves{&c->pool[113]}, loff{&c->pool[114]}, root_of{&c->pool[115]};
+    PoolBuf<uint8_t> inter{&c->pool[97]}, need{&c->pool[103]}, rflag{&c->pool[107]};
+    PoolBuf<int32_t> cnt{&c->pool[98]}, cl{&c->pool[101]}, oref{&c->pool[102]}, nid{&c->pool[104]},
+        clist{&c->pool[105]}, roots{&c->pool[110]}, boff{&c->pool[112]}, root_of{&c->pool[115]};
+    PoolBuf<uint32_t> up{&c->pool[140]};
     PoolBuf<float> cv{&c->pool[106]};
     int32_t* C = cnt.reserve(kCntSlots);
-    PRG_HIP(hipMemsetAsync(C, 0, kCntSlots * 4, s));
+    int32_t* H = c->sub_host;  // pinned; the counts that kernels write there, and copies of C
+    std::fill(H, H + kCntSlots, 0);
+    inter.reserve(6 * M);
+    up.reserve((M + 3) / 4);
+    need.reserve(8 * baseD);
+    root_of.reserve(M);
+    k_sub_init<<<unsigned(std::min<int64_t>(4 * std::max(1, c->num_cu), grid_for(M, kBlockS))), kBlockS, 0, s>>>(
+        C, inter.get(), up.get(), need.get(), root_of.get(), M, baseD);
+    PRG_CHECK_LAUNCH();
 
     // faces touched by the leaf-level surface, and up the parent chains
-    inter.reserve(6 * M);
-    PRG_HIP(hipMemsetAsync(inter.get(), 0, size_t(6 * M), s));
     {
-        PoolBuf<uint32_t> up{&c->pool[140]};
-        up.reserve((M + 3) / 4);
-        PRG_HIP(hipMemsetAsync(up.get(), 0, size_t((M + 3) / 4) * 4, s));
         // bytes: the cube index of each leaf-level node and the face byte of
         // each coarser node, read once (the face visits' gathers come on top)
         TimedScope ts(kt, "face_marks", double(M));
@@ -2247,35 +2379,42 @@ void extract_subdivision(prg_ctx* c) {
         k_face_marks<<<grid_for(MD, kBlockS), kBlockS, 0, s>>>(cubes.get(), MD, baseD, c->key.get(), c->pnt.get(),
                                                                 Lv, c->parent.get(), D, inter.get(), up.get());
         PRG_CHECK_LAUNCH();
-        for (int d = D - 1; d >= 0; d--) {
+        int d = D - 1;
+        for (; c->counts[d] > kSmallUp; d--) {
             k_face_marks_up<<<grid_for(c->counts[d], kBlockS), kBlockS, 0, s>>>(
                 c->bases[d], c->counts[d], d, c->key.get(), c->pnt.get(), Lv, c->parent.get(), D, inter.get(),
                 up.get());
             PRG_CHECK_LAUNCH();
         }
+        k_face_marks_up_small<<<1, kUpBlock, 0, s>>>(d, c->key.get(), c->pnt.get(), Lv, c->parent.get(), D, inter.get(),
+                                                     up.get());
+        PRG_CHECK_LAUNCH();
     }
     // coarse leaves (counts stay on the device; launches are sized by upper bounds)
-    flag.reserve(baseD);
-    off.reserve(baseD);
     cl.reserve(baseD);
-    k_flag_coarse_leaves<<<grid_for(baseD, kBlockS), kBlockS, 0, s>>>(c->child_base.get(), baseD, flag.get());
-    PRG_CHECK_LAUNCH();
-    scan_exclusive(flag.get(), off.get(), baseD, C + kCntCoarse, s, c->scratch, kt);
-    k_compact<<<grid_for(baseD, kBlockS), kBlockS, 0, s>>>(flag.get(), off.get(), baseD, cl.get());
-    PRG_CHECK_LAUNCH();
+    auto select_tiles = [&](int64_t n, int tile) { return uint32_t((n + tile - 1) / tile); };
+    {
+        const uint32_t tiles = select_tiles(baseD, kSelTile);
+        uint64_t* state = look_state(c->scratch, tiles, s);
+        k_select<true><<<tiles, kBlockS, 0, s>>>(c->child_base.get(), nullptr, baseD, tiles, state, cl.get(), nullptr,
+                                                 C + kCntCoarse);
+        PRG_CHECK_LAUNCH();
+    }
     // their corner values
     oref.reserve(8 * baseD);
-    need.reserve(8 * baseD);
     nid.reserve(8 * baseD);
     clist.reserve(8 * baseD);
     cv.reserve(8 * baseD);
-    PRG_HIP(hipMemsetAsync(need.get(), 0, size_t(8 * baseD) * 4, s));
     k_coarse_corner_owner<<<grid_for(8 * baseD, kBlockS), kBlockS, 0, s>>>(cl.get(), C + kCntCoarse, c->key.get(),
                                                                             c->pnt.get(), Lv, D, oref.get(), need.get());
     PRG_CHECK_LAUNCH();
-    scan_exclusive(need.get(), nid.get(), 8 * baseD, C + kCntCorners, s, c->scratch, kt);
-    k_compact<<<grid_for(8 * baseD, kBlockS), kBlockS, 0, s>>>(need.get(), nid.get(), 8 * baseD, clist.get());
-    PRG_CHECK_LAUNCH();
+    {
+        const uint32_t tiles = select_tiles(8 * baseD, kSelTile);
+        uint64_t* state = look_state(c->scratch, tiles, s);
+        k_select<false><<<tiles, kBlockS, 0, s>>>(nullptr, need.get(), 8 * baseD, tiles, state, clist.get(), nid.get(),
+                                                  C + kCntCorners);
+        PRG_CHECK_LAUNCH();
+    }
     {
         TimedScope ts(kt, "coarse_corner_value", 24.0 * double(baseD));
         k_coarse_corner_value<<<grid_for(8 * baseD, kBlockS), kBlockS, 0, s>>>(
@@ -2284,45 +2423,31 @@ void extract_subdivision(prg_ctx* c) {
         PRG_CHECK_LAUNCH();
     }
     // roots, their bricks and virtual leaves
-    rflag.reserve(baseD);
-    roff.reserve(baseD);
-    ridx.reserve(baseD);
+    rflag.reserve(baseD + 16);
     roots.reserve(baseD);
-    rbricks.reserve(baseD);
     boff.reserve(baseD);
-    rleaves.reserve(baseD);
-    loff.reserve(baseD);
-    k_coarse_select<<<grid_for(baseD, kBlockS), kBlockS, 0, s>>>(cl.get(), C + kCntCoarse, baseD, oref.get(),
-                                                                  nid.get(), cv.get(), c->key.get(), c->pnt.get(), Lv,
-                                                                  D, inter.get(), rflag.get());
+    k_coarse_select<<<grid_for(baseD, kBlockS), kBlockS, 0, s>>>(cl.get(), C + kCntCoarse, oref.get(), nid.get(),
+                                                                  cv.get(), c->key.get(), c->pnt.get(), Lv, D,
+                                                                  inter.get(), rflag.get());
     PRG_CHECK_LAUNCH();
-    scan_exclusive(rflag.get(), roff.get(), baseD, C + kCntRoots, s, c->scratch, kt);
-    k_compact<<<grid_for(baseD, kBlockS), kBlockS, 0, s>>>(rflag.get(), roff.get(), baseD, ridx.get());
-    PRG_CHECK_LAUNCH();
-    k_root_info<<<grid_for(baseD, kBlockS), kBlockS, 0, s>>>(cl.get(), ridx.get(), C + kCntRoots, baseD, Lv, D,
-                                                              roots.get(), rbricks.get(), rleaves.get());
-    PRG_CHECK_LAUNCH();
-    scan_exclusive2(rbricks.get(), boff.get(), C + kCntBricks, rleaves.get(), loff.get(), C + kCntLeaves, baseD, s,
-                    c->scratch, kt);
     PoolBuf<int32_t> slist1{&c->pool[144]}, slist2{&c->pool[145]}, sidx{&c->pool[146]};
     slist1.reserve(baseD);
     slist2.reserve(baseD);
     sidx.reserve(baseD);
-    k_list_small_roots<<<grid_for(baseD, kBlockS), kBlockS, 0, s>>>(roots.get(), C + kCntRoots, Lv, D, slist1.get(),
-                                                                     slist2.get(), sidx.get(), C);
-    PRG_CHECK_LAUNCH();
-    int32_t* H = c->sub_host;
-    PRG_HIP(hipMemcpyAsync(H, C, kCntSlots * 4, hipMemcpyDeviceToHost, s));
+    {
+        const uint32_t tiles = select_tiles(baseD, kRootTile);
+        uint64_t* state = look_state(c->scratch, 5 * int64_t(tiles), s);
+        k_list_all_roots<<<tiles, kRootBlock, 0, s>>>(cl.get(), rflag.get(), tiles, state, Lv, D, roots.get(),
+                                                      boff.get(), root_of.get(), slist1.get(), slist2.get(),
+                                                      sidx.get(), C, H);
+        PRG_CHECK_LAUNCH();
+    }
     PRG_HIP(hipStreamSynchronize(s));
     const int64_t nr = H[kCntRoots], nb = H[kCntBricks];
     c->sub_roots = nr;
     c->sub_leaves = H[kCntLeaves];
     if (nr == 0) return;
     if (nb <= 0 || H[kCntLeaves] <= 0) throw Error{PRG_E_HIP, "subdivision: inconsistent brick counts"};
-    root_of.reserve(M);
-    PRG_HIP(hipMemsetAsync(root_of.get(), 0xff, size_t(M) * 4, s));
-    k_root_of<<<grid_for(nr, kBlockS), kBlockS, 0, s>>>(roots.get(), C + kCntRoots, root_of.get());
-    PRG_CHECK_LAUNCH();
 
     PoolBuf<float> btab{&c->pool[91]};
     SubArgs A{c->key.get(),
@@ -2358,7 +2483,9 @@ void extract_subdivision(prg_ctx* c) {
     xlist.reserve(nb);
     glist.reserve(nb);
     bsign.reserve(nb);
-    k_clear_bricks<<<grid_for(nb, kBlockS), kBlockS, 0, s>>>(bnv.get(), bnt.get(), bsign.get(), nb);
+    PoolBuf<int32_t> didx{&c->pool[135]};
+    didx.reserve(nb);
+    k_clear_bricks<<<grid_for(nb, kBlockS), kBlockS, 0, s>>>(bnv.get(), bnt.get(), bsign.get(), didx.get(), nb);
     PRG_CHECK_LAUNCH();
     // the small roots: values, cubes and counts
     const int32_t n1 = H[kCntSmall1], n2 = H[kCntSmall2];
@@ -2442,18 +2569,15 @@ void extract_subdivision(prg_ctx* c) {
     }
     const int64_t ndense = nb3 > 0 ? H[kCntDense] : 0;
     PoolBuf<float> gvals{&c->pool[134]};
-    PoolBuf<int32_t> didx{&c->pool[135]};
     PoolBuf<uint16_t> lofs_tab{&c->pool[124]}, emask_tab{&c->pool[125]};
     PoolBuf<uint8_t> cube_tab{&c->pool[126]};
     LeafTabs T3{};
     if (ndense > 0) {
         gvals.reserve(size_t(ndense) * kBrickPts);
-        didx.reserve(nb);
         T3.lofs = lofs_tab.reserve(size_t(ndense) * kBrickLeaves);
         T3.emask = emask_tab.reserve(size_t(ndense) * kBrickLeaves);
         T3.cube = cube_tab.reserve(size_t(ndense) * kBrickLeaves);
         TimedScope ts(kt, "subdivide_count", 0.0);
-        PRG_HIP(hipMemsetAsync(didx.get(), 0xff, size_t(nb) * 4, s));
         int per_cu = 0;
         PRG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_brick_values, kWave, 0));
         const int64_t resident = int64_t(std::max(1, per_cu)) * std::max(1, c->num_cu);
@@ -2467,9 +2591,8 @@ void extract_subdivision(prg_ctx* c) {
                                                                 didx.get());
         PRG_CHECK_LAUNCH();
     }
-    scan_exclusive2(bnv.get(), bvoff.get(), C + kCntVerts, bnt.get(), btoff.get(), C + kCntTris, nb, s, c->scratch,
+    scan_exclusive2(bnv.get(), bvoff.get(), H + kCntVerts, bnt.get(), btoff.get(), H + kCntTris, nb, s, c->scratch,
                     kt);
-    PRG_HIP(hipMemcpyAsync(H, C, kCntSlots * 4, hipMemcpyDeviceToHost, s));
     PRG_HIP(hipStreamSynchronize(s));
     const int64_t snv = H[kCntVerts], snt = H[kCntTris];
     c->sub_bricks = nb;
@@ -2502,22 +2625,21 @@ void extract_subdivision(prg_ctx* c) {
         TimedScope ts(kt, "subdivide_triangles", 12.0 * double(snt));
         if (n1) {
             k_small_triangles<1><<<lw1, kWave, 0, s>>>(A, slist1.get(), n1, sidx.get(), T1, bvoff.get(), btoff.get(),
-                                                       c->mesh_nv, ST, C + kCntErr);
+                                                       c->mesh_nv, ST, H + kCntErr);
             PRG_CHECK_LAUNCH();
         }
         if (n2) {
             k_small_triangles<2><<<lw2, kWave, 0, s>>>(A, slist2.get(), n2, sidx.get(), T2, bvoff.get(), btoff.get(),
-                                                       c->mesh_nv, ST, C + kCntErr);
+                                                       c->mesh_nv, ST, H + kCntErr);
             PRG_CHECK_LAUNCH();
         }
         if (ndense > 0) {
             k_brick_triangles<<<unsigned(ndense), kBrickLeaves, 0, s>>>(A, dlist.get(), didx.get(), T3, bnt.get(),
                                                                         bvoff.get(), btoff.get(), c->mesh_nv, ST,
-                                                                        C + kCntErr);
+                                                                        H + kCntErr);
             PRG_CHECK_LAUNCH();
         }
     }
-    PRG_HIP(hipMemcpyAsync(H + kCntErr, C + kCntErr, 4, hipMemcpyDeviceToHost, s));
     PRG_HIP(hipStreamSynchronize(s));
     if (H[kCntErr]) throw Error{PRG_E_HIP, "subdivision: a triangle edge has no owner vertex"};
     c->sub_nv = snv;
