@@ -233,6 +233,174 @@ __global__ void __launch_bounds__(kT) k_conv3(ConvIn src, const short* __restric
         }
 }
 
+// The same sums, in the same order, on grids of 8^3 and more, where a tile is
+// a run of voxels: ZL = 16 voxels of a z row, or two rows of 8.
+//
+// A workgroup of 4 waves, WX x WY in space by WN in output channels (16
+// each); a wave computes RX x RY tiles.  The halo lies in LDS one 16-channel
+// slice at a time (the next slice loads while this one is used), a slice as
+// four planes of 4 channels, so the 16 voxels of a fragment read are
+// consecutive 8-byte words (no bank conflict).  A fragment, shifted in z by a
+// tap, serves every tile it lies next to: 48 reads instead of 108 for the 27
+// taps of 2 x 2 tiles.  All 27 weight fragments of a slice sit in registers;
+// each is replaced by the next slice's after its last use.  The weights are
+// the MFMA's first operand, so a lane ends with 4 channels of one voxel and
+// stores 16 bytes.
+// Sizes known at compile time keep the index arithmetic to shifts and
+// constants; it had bounded these convolutions (3300 vector instructions a
+// wave against 108 MFMAs of 16 -> 16 channels).
+template <int LZ, int RX, int RY, int WX, int WY, int WN>
+struct ConvTile {
+    static constexpr int ZL = 1 << LZ, YS = 16 >> LZ;  // a tile: YS rows of ZL voxels
+    static constexpr int BX = WX * RX, BY = WY * RY * YS;
+    static constexpr int HX = BX + 2, HY = BY + 2, HZ = ZL + 2, H = HX * HY * HZ;
+    // words (of 4 channels) per plane, 160 bytes past a multiple of 256: the
+    // staging's writes of a half-wave, 8 voxels in 4 planes, meet no bank
+    // more often than their 256 bytes need
+    static constexpr int P = H + ((20 - H % 32) + 32) % 32;
+    static constexpr int L = (4 * H + kT - 1) / kT;  // staging loads per thread
+};
+
+template <int LZ, int RX, int RY, int WX, int WY, int WN, bool MULTI>
+__global__ void __launch_bounds__(kT, RX * RY > 1 ? (MULTI ? 2 : 4) : (MULTI ? 3 : 5)) k_conv3_rows(
+    ConvIn src, const short* __restrict__ w, const float* __restrict__ bias, int G, int relu, float* __restrict__ out,
+    int cout, int ntg) {
+    using C = ConvTile<LZ, RX, RY, WX, WY, WN>;
+    static_assert(WX * WY * WN * 64 == kT, "one wave per part");
+    constexpr int FY = C::YS * (RY - 1) + 3;
+    __shared__ s4 halo[(MULTI ? 2 : 1) * 4 * C::P];
+    const int cin = src.clo + src.cskip;
+    src = sample_of(src, G);
+    out += sample_offset(G, cout);
+    const int nbz = G >> LZ, nby = G / C::BY;
+    // workgroups are dealt to the 8 XCDs in turn: each XCD takes one
+    // contiguous range of bricks, whose halos meet in its L2
+    int b = blockIdx.x;
+    if ((gridDim.x & 7) == 0) b = (b & 7) * int(gridDim.x >> 3) + (b >> 3);
+    const int oz = (b & (nbz - 1)) << LZ;  // (both counts are powers of two)
+    b >>= log2i(nbz);
+    const int oy = (b & (nby - 1)) * C::BY, ox = (b >> log2i(nby)) * C::BX;
+    const int tid = threadIdx.x, l = tid & 63, i = l & 15, kq = l >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wx = wave % WX, wy = (wave / WX) % WY, wn = wave / (WX * WY);
+    const int S = cin >> 4, Q = S * (ntg / WN);
+    int nt = blockIdx.z * ntg + wn, sl = 0;
+
+    // staging: this thread's words, word k of halo voxel (tid + k kT) / 4
+    const int c4 = tid & 3;
+    int vox[C::L];
+    float4 st[C::L];
+    auto stage_load = [&](int slice) {
+        const bool lo = slice * 16 < src.clo;
+        if (slice == 0 || slice * 16 == src.clo) {
+            // voxel indices in this source (-1 outside the grid)
+#pragma unroll
+            for (int k = 0; k < C::L; k++) {
+                const int h = (tid + k * kT) >> 2;
+                const int hxy = h / C::HZ, hz = h - hxy * C::HZ, hx = hxy / C::HY, hy = hxy - hx * C::HY;
+                const int gx = ox + hx - 1, gy = oy + hy - 1, gz = oz + hz - 1;
+                const bool in = h < C::H && uint32_t(gx) < uint32_t(G) && uint32_t(gy) < uint32_t(G) &&
+                                uint32_t(gz) < uint32_t(G);
+                const int sh = lo ? 1 : 0, Gs = G >> sh;
+                vox[k] = in ? ((gx >> sh) * Gs + (gy >> sh)) * Gs + (gz >> sh) : -1;
+            }
+        }
+        const int c = lo ? src.clo : src.cskip;
+        const float* p = (lo ? src.lo + slice * 16 : src.skip + (slice * 16 - src.clo)) + 4 * c4;
+#pragma unroll
+        for (int k = 0; k < C::L; k++) {
+            st[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (vox[k] >= 0) st[k] = *reinterpret_cast<const float4*>(p + int64_t(vox[k]) * c);
+        }
+    };
+    auto stage_store = [&](int buf) {
+        s4* d = halo + (buf * 4 + c4) * C::P + (tid >> 2);
+#pragma unroll
+        for (int k = 0; k < C::L; k++)
+            if (4 * C::H % kT == 0 || k + 1 < C::L || tid + k * kT < 4 * C::H)
+                d[k * (kT / 4)] = s4{bf(st[k].x), bf(st[k].y), bf(st[k].z), bf(st[k].w)};
+    };
+    const int64_t tstep = int64_t(cout) * cin;
+    auto weights = [&](int ntile, int slice) { return w + (int64_t(ntile) * 16 + i) * cin + slice * 16 + 4 * kq; };
+    s4 wr[27];
+    {
+        const short* wl = weights(nt, 0);
+#pragma unroll
+        for (int t = 0; t < 27; t++) wr[t] = *reinterpret_cast<const s4*>(wl + t * tstep);
+    }
+    stage_load(0);
+    stage_store(0);
+    const int vy = i >> LZ, vz = i & (C::ZL - 1);  // the lane's voxel of a tile
+    const int frag0 = kq * C::P + ((wx * RX) * C::HY + wy * RY * C::YS + vy) * C::HZ + vz;
+    // three partial sums, one per dz, keep independent MFMAs in flight
+    f4 acc[3][RX][RY];
+    for (int q = 0;; q++) {
+        const bool more = MULTI && q + 1 < Q;
+        const int nsl = sl + 1 < S ? sl + 1 : 0, nnt = sl + 1 < S ? nt : nt + WN;
+        const bool restage = more && S > 1;
+        if (restage) stage_load(nsl);
+        if (q == 0 || S > 1) __syncthreads();
+        const short* wnext = weights(more ? nnt : nt, more ? nsl : sl);  // (the last re-reads its own: unused)
+        if (sl == 0)
+#pragma unroll
+            for (int z = 0; z < 3; z++)
+#pragma unroll
+                for (int x = 0; x < RX; x++)
+#pragma unroll
+                    for (int y = 0; y < RY; y++) acc[z][x][y] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        const s4* frag = halo + (MULTI && S > 1 ? (q & 1) * 4 * C::P : 0) + frag0;
+#pragma unroll
+        for (int fx = 0; fx < RX + 2; fx++)
+#pragma unroll
+            for (int fy = 0; fy < FY; fy++)
+#pragma unroll
+                for (int z = 0; z < 3; z++) {
+                    const s4 a = frag[(fx * C::HY + fy) * C::HZ + z];
+#pragma unroll
+                    for (int x = 0; x < RX; x++)
+#pragma unroll
+                        for (int y = 0; y < RY; y++) {
+                            const int dx = fx - x, dy = fy - C::YS * y;
+                            if (dx < 0 || dx > 2 || dy < 0 || dy > 2) continue;
+                            const int t = (dx * 3 + dy) * 3 + z;
+                            acc[z][x][y] =
+                                __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wr[t], a, acc[z][x][y], 0, 0, 0);
+                        }
+                    if (MULTI) {
+                        const int dx = fx - (RX - 1), dy = fy - C::YS * (RY - 1);
+                        if (dx >= 0 && dy >= 0) {
+                            const int t = (dx * 3 + dy) * 3 + z;
+                            wr[t] = *reinterpret_cast<const s4*>(wnext + t * tstep);
+                        }
+                    }
+                }
+        if (sl == S - 1) {
+            float4 bv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (bias) bv = *reinterpret_cast<const float4*>(bias + nt * 16 + 4 * kq);
+#pragma unroll
+            for (int x = 0; x < RX; x++)
+#pragma unroll
+                for (int y = 0; y < RY; y++) {
+                    const int gx = ox + wx * RX + x, gy = oy + (wy * RY + y) * C::YS + vy, gz = oz + vz;
+                    float v[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        v[e] = (acc[0][x][y][e] + acc[1][x][y][e]) + acc[2][x][y][e];
+                        const float be = e == 0 ? bv.x : e == 1 ? bv.y : e == 2 ? bv.z : bv.w;
+                        if (bias) v[e] = v[e] + be;
+                        if (relu) v[e] = v[e] > 0.0f ? v[e] : 0.0f;
+                    }
+                    *reinterpret_cast<float4*>(out + (int64_t(gx * G + gy) * G + gz) * cout + nt * 16 + 4 * kq) =
+                        make_float4(v[0], v[1], v[2], v[3]);
+                }
+        }
+        if (!more) break;
+        if (restage) stage_store((q + 1) & 1);
+        sl = nsl;
+        nt = nnt;
+    }
+}
+
 // dW partials: part[ch][t][co][ci] = sum over the chunk's voxels v of
 // bf16(g[v, co]) * bf16(in[v + off_t, ci]), 16 voxels per MFMA in voxel order.
 //
@@ -831,24 +999,24 @@ namespace {
 const int kConvDef[14][3] = {{16, 16, 0}, {16, 16, 0}, {16, 32, 1}, {32, 32, 1}, {32, 64, 2}, {64, 64, 2}, {64, 64, 3},
                              {64, 64, 3}, {128, 64, 2}, {64, 64, 2}, {96, 32, 1}, {32, 32, 1}, {48, 16, 0}, {16, 16, 0}};
 
-// Brick and wave split of a convolution with output grid G and NT = cout / 16
-// N-tiles: few voxels and many channels per workgroup on the small grids, so
-// every grid gives the chip enough workgroups.
+// Brick and wave split of k_conv3 (grids under 8^3) with output grid G and
+// NT = cout / 16 N-tiles.
 struct ConvPlan {
     int BX, BY, BZ, MA, NA, MG;
 };
 
 ConvPlan conv_plan(int G, int NT) {
     ConvPlan p{};
-    p.BZ = G < 16 ? G : 16;
+    p.BZ = G;
+    p.MA = 1;
     int bxy = 1;  // BX = BY = bxy before small-grid widening
     switch (NT) {
-        case 1: bxy = int64_t(G) * G * G >= int64_t(256) * 1024 ? 4 : 2; p.MA = bxy == 4 ? 4 : 1; p.NA = 1; break;
-        case 2: p.MA = 1; p.NA = 1; break;
-        case 3: bxy = 2; p.MA = 1; p.NA = 3; break;
-        case 4: p.MA = 1; p.NA = 1; break;
-        case 6: p.MA = 1; p.NA = 3; break;
-        case 8: p.MA = 1; p.NA = 2; break;
+        case 1: bxy = 2; p.NA = 1; break;
+        case 2: p.NA = 1; break;
+        case 3: bxy = 2; p.NA = 3; break;
+        case 4: p.NA = 1; break;
+        case 6: p.NA = 3; break;
+        case 8: p.NA = 2; break;
         default: throw Error{PRG_E_ARG, "unsupported channel count"};
     }
     p.BX = bxy < G ? bxy : G;
@@ -867,29 +1035,61 @@ ConvPlan conv_plan(int G, int NT) {
 
 bool pow2_channels(int c) { return c == 16 || c == 32 || c == 64; }
 
+// Tiles of 16 voxels and 16 channels from which a wave takes 2 x 2 of them
+// (below: one, for the waves that fill the chip).
+constexpr int64_t kConvManyTiles = 4096;
+
+template <int LZ, int RX, int RY, int WX, int WY, int WN>
+void launch_conv_rows(hipStream_t s, ConvIn src, const short* w, const float* bias, int G, int relu, float* out,
+                      int cout, int B) {
+    using C = ConvTile<LZ, RX, RY, WX, WY, WN>;
+    const int NT = cout / 16, S = (src.clo + src.cskip) / 16;
+    if (NT % WN || G % C::BX || G % C::BY || G % C::ZL) throw Error{PRG_E_ARG, "convolution tile does not divide"};
+    // one slice: its halo is staged once for all N-tiles
+    const int ntg = S == 1 ? NT : WN;
+    const dim3 grid(unsigned((G / C::BX) * (G / C::BY) * (G / C::ZL)), unsigned(B), unsigned(NT / ntg));
+    if (S * (ntg / WN) > 1)
+        k_conv3_rows<LZ, RX, RY, WX, WY, WN, true><<<grid, kT, 0, s>>>(src, w, bias, G, relu, out, cout, ntg);
+    else
+        k_conv3_rows<LZ, RX, RY, WX, WY, WN, false><<<grid, kT, 0, s>>>(src, w, bias, G, relu, out, cout, ntg);
+    PRG_CHECK_LAUNCH();
+}
+
+template <int LZ>
+void launch_conv_grid(hipStream_t s, ConvIn src, const short* w, const float* bias, int G, int relu, float* out,
+                      int cout, int B) {
+    const int NT = cout / 16;
+    const bool many = int64_t(B) * G * G * G / 16 * NT >= kConvManyTiles && G >= 8;
+    if (NT % 4 == 0) {
+        if (many) launch_conv_rows<LZ, 2, 2, 1, 1, 4>(s, src, w, bias, G, relu, out, cout, B);
+        else launch_conv_rows<LZ, 1, 1, 1, 1, 4>(s, src, w, bias, G, relu, out, cout, B);
+    } else if (NT % 2 == 0) {
+        if (many) launch_conv_rows<LZ, 2, 2, 2, 1, 2>(s, src, w, bias, G, relu, out, cout, B);
+        else launch_conv_rows<LZ, 1, 1, 1, 2, 2>(s, src, w, bias, G, relu, out, cout, B);
+    } else {
+        if (many) launch_conv_rows<LZ, 2, 2, 2, 2, 1>(s, src, w, bias, G, relu, out, cout, B);
+        else launch_conv_rows<LZ, 1, 1, 2, 2, 1>(s, src, w, bias, G, relu, out, cout, B);
+    }
+}
+
 void launch_conv(hipStream_t s, ConvIn src, const short* w, const float* bias, int G, int relu, float* out, int cout,
                  int B) {
     const int cin = src.clo + src.cskip;
     if (!pow2_channels(src.cskip) || (src.clo && !pow2_channels(src.clo)) || cout % 16 || cout <= 0 ||
         (src.clo && G < 2))
         throw Error{PRG_E_ARG, "unsupported convolution channels"};
+    if (G >= 16) return launch_conv_grid<4>(s, src, w, bias, G, relu, out, cout, B);
+    if (G == 8) return launch_conv_grid<3>(s, src, w, bias, G, relu, out, cout, B);
     const ConvPlan p = conv_plan(G, cout / 16);
     const size_t lds = size_t(p.BX + 2) * (p.BY + 2) * (p.BZ + 2) * cin * 2;
     if (lds > 64 * 1024) throw Error{PRG_E_ARG, "convolution halo exceeds 64 KiB of LDS"};
-    const unsigned nb = unsigned((G / p.BX) * (G / p.BY) * (G / p.BZ));
-    const int MA = p.MA, NA = p.NA;
-#define PRG_CONV(ma, na)                                                                                         \
-    if (MA == ma && NA == na) {                                                                                   \
-        k_conv3<ma, na><<<dim3(nb, unsigned(B)), kT, lds, s>>>(src, w, bias, G, p.BX, p.BY, p.BZ, p.MG, relu, out, cout);             \
-        PRG_CHECK_LAUNCH();                                                                                       \
-        return;                                                                                                   \
+    const dim3 grid(unsigned((G / p.BX) * (G / p.BY) * (G / p.BZ)), unsigned(B));
+    switch (p.NA) {
+        case 1: k_conv3<1, 1><<<grid, kT, lds, s>>>(src, w, bias, G, p.BX, p.BY, p.BZ, p.MG, relu, out, cout); break;
+        case 2: k_conv3<1, 2><<<grid, kT, lds, s>>>(src, w, bias, G, p.BX, p.BY, p.BZ, p.MG, relu, out, cout); break;
+        default: k_conv3<1, 3><<<grid, kT, lds, s>>>(src, w, bias, G, p.BX, p.BY, p.BZ, p.MG, relu, out, cout);
     }
-    PRG_CONV(4, 1)
-    PRG_CONV(1, 1)
-    PRG_CONV(1, 2)
-    PRG_CONV(1, 3)
-#undef PRG_CONV
-    throw Error{PRG_E_ARG, "no convolution kernel for the plan"};
+    PRG_CHECK_LAUNCH();
 }
 
 void pack_all(prg_unet* n) {
