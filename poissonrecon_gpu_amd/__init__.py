@@ -12,6 +12,7 @@ from __future__ import annotations
 import ctypes as C
 from dataclasses import dataclass
 from pathlib import Path
+import weakref
 
 import numpy as np
 
@@ -209,6 +210,29 @@ class Mesh:
         return (self.vertices * np.float32(self.scale)) + self.center.astype(np.float32)
 
 
+class _HostArray:
+    """An array the library allocated, to be viewed by numpy (np.asarray) and
+    freed with its last view."""
+
+    def __init__(self, pointer, rows: int, dtype, **field):
+        self.__array_interface__ = {"data": (C.cast(pointer, C.c_void_p).value, False), "shape": (int(rows), 3),
+                                    "typestr": np.dtype(dtype).str, "version": 3}
+        m = PrgMesh()
+        for name in field:  # prg_mesh_release frees the arrays that are set
+            setattr(m, name, field[name])
+        weakref.finalize(self, lib().prg_mesh_release, C.pointer(m)).atexit = False
+
+
+def _adopt_mesh(m: PrgMesh) -> tuple[np.ndarray, np.ndarray]:
+    """The vertices and triangles of a mesh the library allocated, without a
+    copy; the mesh gives them up."""
+    v = np.asarray(_HostArray(m.vertices, m.n_vertices, np.float32, vertices=m.vertices))
+    t = np.asarray(_HostArray(m.triangles, m.n_triangles, np.int32, triangles=m.triangles))
+    m.vertices = C.POINTER(C.c_float)()
+    m.triangles = C.POINTER(C.c_int32)()
+    return v, t
+
+
 class Reconstructor:
     """One reconstruction context (prg_ctx) on one HIP device."""
 
@@ -285,9 +309,8 @@ class Reconstructor:
         m = PrgMesh()
         self._call("prg_extract_mesh", int(subdivide), C.byref(m))
         try:
-            v = np.ctypeslib.as_array(m.vertices, shape=(max(m.n_vertices, 1) * 3,))[: 3 * m.n_vertices]
-            t = np.ctypeslib.as_array(m.triangles, shape=(max(m.n_triangles, 1) * 3,))[: 3 * m.n_triangles]
-            return Mesh(v.reshape(-1, 3).copy(), t.reshape(-1, 3).copy(), np.array(m.center[:], np.float32),
+            v, t = _adopt_mesh(m)
+            return Mesh(v, t, np.array(m.center[:], np.float32),
                         float(m.scale), m.n_leaf_vertices, m.n_leaf_triangles)
         finally:
             lib().prg_mesh_release(C.byref(m))
@@ -305,7 +328,7 @@ class Reconstructor:
         m.n_leaf_vertices, m.n_leaf_triangles = int(mesh.n_leaf_vertices), int(mesh.n_leaf_triangles)
         merged = C.c_int64()
         self._call("prg_weld_mesh_noalloc" if noalloc else "prg_weld_mesh", C.byref(m), C.byref(merged))
-        return (Mesh(v[: m.n_vertices].copy(), t, mesh.center, mesh.scale, m.n_leaf_vertices, m.n_leaf_triangles),
+        return (Mesh(v[: m.n_vertices], t, mesh.center, mesh.scale, m.n_leaf_vertices, m.n_leaf_triangles),
                 merged.value)
 
     def subdivision_info(self) -> tuple[int, int]:
@@ -505,9 +528,7 @@ def reconstruct_batch(clouds, depths, concurrency: int = 4, subdivide: bool = Tr
                  ms=float(it.ms), max_true_rel_residual=float(it.max_true_rel_residual),
                  total_iters=int(it.total_iters))
         if return_meshes and it.mesh.vertices:
-            nv, nt = it.mesh.n_vertices, it.mesh.n_triangles
-            r["mesh_vertices"] = np.ctypeslib.as_array(it.mesh.vertices, shape=(max(nv, 1) * 3,))[: 3 * nv].reshape(-1, 3).copy()
-            r["mesh_triangles"] = np.ctypeslib.as_array(it.mesh.triangles, shape=(max(nt, 1) * 3,))[: 3 * nt].reshape(-1, 3).copy()
+            r["mesh_vertices"], r["mesh_triangles"] = _adopt_mesh(it.mesh)
         out.append(r)
         lib().prg_mesh_release(C.byref(it.mesh))
     return st, out

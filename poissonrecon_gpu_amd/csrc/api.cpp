@@ -1,6 +1,8 @@
 // C ABI of the library (include/prg.h): argument checks, state machine,
 // error capture and host <-> device buffer access.  Every entry point
 // catches prg::Error and returns its status; nothing aborts the process.
+#include <sys/mman.h>
+
 #include <cstdlib>
 #include <cstring>
 #include <new>
@@ -19,6 +21,7 @@ prg_status fail(prg_ctx* c, prg_status st, const std::string& msg) {
 template <class F>
 prg_status guarded(prg_ctx* c, F&& f) {
     if (!c) return PRG_E_ARG;
+    const prg::ArenaScope scope(&c->arena);
     try {
         return f();
     } catch (const Error& e) {
@@ -58,6 +61,16 @@ int64_t buffer_bytes(const prg_ctx* c, int which) {
         case PRG_BUF_LEAF_CORNER_VALUES: return (c->mesh_nv > 0 || c->mesh_nt > 0 || c->corner_vals.get()) ? 32 * MD : -1;
         default: return -1;
     }
+}
+
+// Memory for std::free: large arrays on 2 MiB pages where the system grants
+// them, since the copy that fills a fresh array is the one to touch its pages.
+void* host_alloc(size_t bytes) {
+    constexpr size_t kHuge = size_t(2) << 20;
+    void* p = nullptr;
+    if (bytes < 2 * kHuge || posix_memalign(&p, kHuge, bytes) != 0) return std::malloc(bytes);
+    (void)madvise(p, bytes / kHuge * kHuge, MADV_HUGEPAGE);
+    return p;
 }
 
 void d2h(prg_ctx* c, void* dst, const void* src, size_t bytes) {
@@ -117,7 +130,7 @@ prg_status prg_create(prg_ctx** out, const prg_config* cfg) {
         PRG_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
         PRG_HIP(hipStreamCreateWithFlags(&c->stream2, hipStreamNonBlocking));
         PRG_HIP(hipStreamCreateWithFlags(&c->stream3, hipStreamNonBlocking));
-        PRG_HIP(hipStreamCreateWithFlags(&c->stream4, hipStreamNonBlocking));
+        c->arena.streams = {&c->stream, &c->stream2, &c->stream3, &c->stream4};
         PRG_HIP(hipEventCreateWithFlags(&c->plan_ev, hipEventDisableTiming));
         PRG_HIP(hipEventCreate(&c->topo_ev));
         PRG_HIP(hipEventCreate(&c->mesh_ev));
@@ -126,9 +139,10 @@ prg_status prg_create(prg_ctx** out, const prg_config* cfg) {
             PRG_HIP(hipEventCreate(&e[0]));
             PRG_HIP(hipEventCreate(&e[1]));
         }
-        PRG_HIP(hipHostMalloc(&c->transform_host, 16, hipHostMallocCoherent));
-        PRG_HIP(hipHostMalloc(&c->cg_host, prg::kCgHostBytes, hipHostMallocCoherent));
-        PRG_HIP(hipHostMalloc(reinterpret_cast<void**>(&c->sub_host), 256, hipHostMallocCoherent));
+        // one pinned allocation: the solver's area, the subdivision's counters, the transform
+        PRG_HIP(hipHostMalloc(&c->cg_host, prg::kCgHostBytes + 256 + 16, hipHostMallocCoherent));
+        c->sub_host = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(c->cg_host) + prg::kCgHostBytes);
+        c->transform_host = reinterpret_cast<float*>(c->sub_host + 64);
         PRG_HIP(hipDeviceGetAttribute(&c->num_cu, hipDeviceAttributeMultiprocessorCount, cf.device));
         prg::weld_noalloc_scratch(cf.device);  // the fixed weld array's address on this device, once
         if (const char* lim = std::getenv("PRG_TILE_LDS_LIMIT")) c->tile_limit = std::max(0, std::atoi(lim));
@@ -159,9 +173,7 @@ void prg_destroy(prg_ctx* c) {
     for (auto& e : c->stage_ev)
         for (hipEvent_t x : e)
             if (x) (void)hipEventDestroy(x);
-    if (c->transform_host) (void)hipHostFree(c->transform_host);
     if (c->cg_host) (void)hipHostFree(c->cg_host);
-    if (c->sub_host) (void)hipHostFree(c->sub_host);
     for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
     hipStream_t ss[4] = {c->stream, c->stream2, c->stream3, c->stream4};
     delete c;  // releases device buffers
@@ -176,7 +188,8 @@ prg_status prg_set_max_depth(prg_ctx* c, int32_t max_depth) {
         if (max_depth < 2 || max_depth > prg::kMaxDepth) return fail(c, PRG_E_ARG, "max_depth must be in [2, 10]");
         PRG_HIP(hipSetDevice(c->cfg.device));
         // work of the previous octree still queued on the other streams ends first
-        for (hipStream_t x : {c->stream, c->stream2, c->stream3, c->stream4}) PRG_HIP(hipStreamSynchronize(x));
+        for (hipStream_t x : {c->stream, c->stream2, c->stream3, c->stream4})
+            if (x) PRG_HIP(hipStreamSynchronize(x));
         c->plan_pending = c->topo_pending = false;
         c->cfg.max_depth = max_depth;
         c->D = max_depth;
@@ -368,8 +381,8 @@ prg_status prg_extract_mesh(prg_ctx* c, int32_t subdivide, prg_mesh* out) {
         if (!c->iso_ready) return fail(c, PRG_E_STATE, "prg_isovalue or prg_set_isovalue first");
         if (!out) return fail(c, PRG_E_ARG, "null mesh");
         build_mesh(c, subdivide, out);
-        out->vertices = static_cast<float*>(std::malloc(size_t(3 * out->n_vertices + 1) * 4));
-        out->triangles = static_cast<int32_t*>(std::malloc(size_t(3 * out->n_triangles + 1) * 4));
+        out->vertices = static_cast<float*>(host_alloc(size_t(3 * out->n_vertices + 1) * 4));
+        out->triangles = static_cast<int32_t*>(host_alloc(size_t(3 * out->n_triangles + 1) * 4));
         if (!out->vertices || !out->triangles) {
             prg_mesh_release(out);
             return fail(c, PRG_E_NOMEM, "mesh host allocation");

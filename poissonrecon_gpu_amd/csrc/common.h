@@ -43,17 +43,64 @@ struct Error {
 #define PRG_CHECK_LAUNCH() PRG_HIP(hipGetLastError())
 
 // ---- device buffers ------------------------------------------------------------
-// Owning device allocation that only grows (re-used across calls of a context).
+// Device memory of one context: buffers are parts of a few large allocations,
+// given back to the device with the context.  A context's about 170 buffers
+// as allocations of their own cost 20 us each to make, and 270 us each to free
+// beside other contexts at work (hipFree waits for the whole device).
+// A part given back may still be read by work queued on the context's
+// streams: it is only handed out again after those streams were waited for.
+// Used by one thread at a time, like its context (arena.cpp).
+class Arena {
+public:
+    Arena() = default;
+    Arena(const Arena&) = delete;
+    Arena& operator=(const Arena&) = delete;
+    ~Arena();
+    void* take(size_t bytes);
+    void give(void* p, size_t bytes);
+    std::vector<const hipStream_t*> streams;  // of the context (null ones are not made yet)
+
+private:
+    struct Part {
+        uint8_t* p;
+        size_t bytes;
+        bool queued;  // work using it may still be queued
+        int chunk;
+    };
+    struct Chunk {
+        uint8_t* p;
+        size_t bytes;
+    };
+    bool add_chunk(size_t bytes);
+    std::vector<Part> free_;  // by address; neighbours of one chunk are joined
+    std::vector<Chunk> chunks_;
+    size_t total_ = 0;
+};
+
+// The arena that buffers reserved by this thread come from (null: allocations
+// of their own), for a scope: a context's entry points set theirs.
+Arena*& current_arena();
+struct ArenaScope {
+    Arena* before;
+    explicit ArenaScope(Arena* a) : before(current_arena()) { current_arena() = a; }
+    ~ArenaScope() { current_arena() = before; }
+    ArenaScope(const ArenaScope&) = delete;
+    ArenaScope& operator=(const ArenaScope&) = delete;
+};
+
+// Owning device buffer that only grows (re-used across calls of a context).
 template <class T>
 struct DBuf {
     T* p = nullptr;
     size_t n = 0;  // capacity in elements
+    Arena* arena = nullptr;  // where p comes from (null: hipMalloc)
     DBuf() = default;
     DBuf(const DBuf&) = delete;
     DBuf& operator=(const DBuf&) = delete;
     ~DBuf() { release(); }
     void release() {
-        if (p) (void)hipFree(p);
+        if (p && arena) arena->give(p, n * sizeof(T));
+        else if (p) (void)hipFree(p);
         p = nullptr;
         n = 0;
     }
@@ -61,7 +108,9 @@ struct DBuf {
         if (count <= n && p) return p;
         release();
         size_t c = count ? count : 1;
-        PRG_HIP(hipMalloc(&p, c * sizeof(T)));
+        arena = current_arena();
+        if (arena) p = static_cast<T*>(arena->take(c * sizeof(T)));
+        else PRG_HIP(hipMalloc(&p, c * sizeof(T)));
         n = c;
         return p;
     }

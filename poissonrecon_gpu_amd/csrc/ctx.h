@@ -27,7 +27,8 @@ struct prg_ctx {
     hipStream_t stream = nullptr;
     hipStream_t stream2 = nullptr;  // independent work overlapping `stream` (CG chains, small-depth solves)
     hipStream_t stream3 = nullptr;
-    hipStream_t stream4 = nullptr;  // the warm-started depth (after the network's inference)
+    hipStream_t stream4 = nullptr;  // the warm-started depth (after the network's inference); made when first used
+    prg::Arena arena;  // before every buffer: released after them
     std::string err;
     prg::KernelTimer kt;
     prg::Scratch scratch;

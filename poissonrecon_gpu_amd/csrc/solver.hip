@@ -1091,6 +1091,7 @@ prg_status solve_all(prg_ctx* c, prg_solve_stats* stats) {
     }
     ch[0].s = s;
     ch[1].s = serial ? s : c->stream2;
+    if (!ch[2].depths.empty() && !c->stream4) PRG_HIP(hipStreamCreateWithFlags(&c->stream4, hipStreamNonBlocking));
     ch[2].s = serial ? s : c->stream4;
     hipStream_t small_s = serial ? s : c->stream3;
 
@@ -1379,9 +1380,11 @@ prg_status solve_all(prg_ctx* c, prg_solve_stats* stats) {
             for (int d : h.depths) ms[d] = t;
         }
         // the context stream continues after every chain and the small solves
-        for (hipStream_t x : {c->stream2, c->stream3, c->stream4, s}) PRG_HIP(hipStreamSynchronize(x));
+        for (hipStream_t x : {c->stream2, c->stream3, c->stream4, s})
+            if (x) PRG_HIP(hipStreamSynchronize(x));
     } catch (...) {
-        for (hipStream_t x : {c->stream2, c->stream3, c->stream4}) (void)hipStreamSynchronize(x);
+        for (hipStream_t x : {c->stream2, c->stream3, c->stream4})
+            if (x) (void)hipStreamSynchronize(x);
         (void)hipStreamSynchronize(s);
         throw;
     }

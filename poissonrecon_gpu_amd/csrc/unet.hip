@@ -1338,6 +1338,7 @@ prg_status unet_guard(prg_unet* n, F&& f) {
 }  // namespace
 
 void unet_warm_start(prg_ctx* c, int depth, hipStream_t s) {
+    const ArenaScope scope(nullptr);  // the network's buffers outlive the context
     prg_unet* n = c->warm_net;
     if (!n || (int64_t(1) << depth) != n->G) throw Error{PRG_E_STATE, "warm-start network does not match the depth"};
     if (n->device != c->cfg.device) throw Error{PRG_E_ARG, "warm-start network is on another device"};
