@@ -58,6 +58,14 @@ struct ConvIn {
     int cskip;
 };
 
+// Output of a convolution: channels [0, split) to `lo`, [split, cout) to `hi`,
+// each a tensor of its own (split = cout for a plain output).
+struct ConvOut {
+    float* lo;
+    int split;
+    float* hi;
+};
+
 // The workgroup's sample of a batch (blockIdx.y): tensors hold their samples
 // one after another.
 __device__ __forceinline__ int64_t sample_offset(int G, int c) { return int64_t(blockIdx.y) * G * G * G * c; }
@@ -68,7 +76,7 @@ __device__ __forceinline__ ConvIn sample_of(ConvIn s, int G) {
     return s;
 }
 
-__device__ __forceinline__ int log2i(int v) { return 31 - __builtin_clz(v); }
+__host__ __device__ __forceinline__ int log2i(int v) { return 31 - __builtin_clz(v); }
 
 // a / d for 0 <= a < 2^20 and 1 <= d < 2^10 (inv = 1.0f / d): the float
 // estimate is within one of the quotient and is corrected
@@ -121,6 +129,7 @@ __device__ __forceinline__ void load_halo(s4* halo4, int H, int HY, int HZ, cons
 }
 
 // out[v, co] = act(bias[co] + sum_t sum_ci bf16(in[v + off_t, ci]) * w[t][co][ci])
+// (w as packed_at lays it out)
 //
 // One workgroup per brick of BX x BY x BZ output voxels (x, y, z; z fastest).
 // The brick's input halo, (BX + 2)(BY + 2)(BZ + 2) voxels, is staged in LDS
@@ -133,13 +142,12 @@ __device__ __forceinline__ void load_halo(s4* halo4, int H, int HY, int HZ, cons
 // over slices, then taps; a slice's 27 weight fragments are loaded together.
 template <int MA, int NA>
 __global__ void __launch_bounds__(kT) k_conv3(ConvIn src, const short* __restrict__ w, const float* __restrict__ bias,
-                                             int G, int BX, int BY, int BZ, int MG, int relu, float* __restrict__ out,
+                                             int G, int BX, int BY, int BZ, int MG, int relu, ConvOut dst,
                                              int cout) {
     extern __shared__ s4 halo4[];
     const short* halo = reinterpret_cast<const short*>(halo4);
     const int cin = src.clo + src.cskip;
     src = sample_of(src, G);
-    out += sample_offset(G, cout);
     const int HY = BY + 2, HZ = BZ + 2, HYZ = HY * HZ, H = (BX + 2) * HYZ;
     const int nbz = G / BZ, nby = G / BY;
     int b = blockIdx.x;
@@ -153,12 +161,12 @@ __global__ void __launch_bounds__(kT) k_conv3(ConvIn src, const short* __restric
     const int NT = cout >> 4, S = cin >> 4, nvox = BX * BY * BZ;
     const bool active = (ng + 1) * NA <= NT;
     // the first slice's weight fragments are in flight while the halo loads
-    const short* wl = w + int64_t((active ? ng : 0) * NA * 16 + i) * cin + 4 * kq;
+    const short* wl = w + ((active ? ng : 0) * NA * 16 + i) * 16 + 4 * kq;
     s4 wr[27][NA];
 #pragma unroll
     for (int t = 0; t < 27; t++)
 #pragma unroll
-        for (int n = 0; n < NA; n++) wr[t][n] = *reinterpret_cast<const s4*>(wl + (int64_t(t) * cout + n * 16) * cin);
+        for (int n = 0; n < NA; n++) wr[t][n] = *reinterpret_cast<const s4*>(wl + (t * cout + n * 16) * 16);
     if (src.clo) load_halo<true>(halo4, H, HY, HZ, src.lo, src.clo, 0, ox, oy, oz, G);
     load_halo<false>(halo4, H, HY, HZ, src.skip, src.cskip, src.clo, ox, oy, oz, G);
     __syncthreads();
@@ -210,7 +218,7 @@ __global__ void __launch_bounds__(kT) k_conv3(ConvIn src, const short* __restric
                     for (int m = 0; m < MA; m++)
                         acc[j % 3][m][n] =
                             __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[j][m], wr[t][n], acc[j % 3][m][n], 0, 0, 0);
-                    wr[t][n] = *reinterpret_cast<const s4*>(wl + (int64_t(t) * cout + n * 16) * cin + nsl * 16);
+                    wr[t][n] = *reinterpret_cast<const s4*>(wl + ((nsl * 27 + t) * cout + n * 16) * 16);
                 }
             }
         }
@@ -222,13 +230,17 @@ __global__ void __launch_bounds__(kT) k_conv3(ConvIn src, const short* __restric
             const int q = (mg * MA + m) * 16 + 4 * kq + e;
             if (q >= nvox) continue;
             const int gx = ox + q / (BY * BZ), gy = oy + (q / BZ) % BY, gz = oz + q % BZ;
-            float* o = out + ((int64_t(gx) * G + gy) * G + gz) * cout + ng * NA * 16 + i;
+            const int64_t v = (int64_t(gx) * G + gy) * G + gz;
 #pragma unroll
             for (int n = 0; n < NA; n++) {
+                const int co = (ng * NA + n) * 16 + i;
+                const bool hi = co >= dst.split;
+                const int oc = hi ? cout - dst.split : dst.split;
+                float* o = (hi ? dst.hi : dst.lo) + sample_offset(G, oc) + v * oc + co - (hi ? dst.split : 0);
                 float val = (acc[0][m][n][e] + acc[1][m][n][e]) + acc[2][m][n][e];
-                if (bias) val = val + bias[(ng * NA + n) * 16 + i];
+                if (bias) val = val + bias[co];
                 if (relu) val = val > 0.0f ? val : 0.0f;
-                o[n * 16] = val;
+                *o = val;
             }
         }
 }
@@ -263,15 +275,14 @@ struct ConvTile {
 
 template <int LZ, int RX, int RY, int WX, int WY, int WN, bool MULTI>
 __global__ void __launch_bounds__(kT, RX * RY > 1 ? (MULTI ? 2 : 4) : (MULTI ? 3 : 5)) k_conv3_rows(
-    ConvIn src, const short* __restrict__ w, const float* __restrict__ bias, int G, int relu, float* __restrict__ out,
-    int cout, int ntg) {
+    ConvIn src, const short* __restrict__ w, const float* __restrict__ bias, int G, int relu, ConvOut dst, int cout,
+    int ntg) {
     using C = ConvTile<LZ, RX, RY, WX, WY, WN>;
     static_assert(WX * WY * WN * 64 == kT, "one wave per part");
     constexpr int FY = C::YS * (RY - 1) + 3;
     __shared__ s4 halo[(MULTI ? 2 : 1) * 4 * C::P];
     const int cin = src.clo + src.cskip;
     src = sample_of(src, G);
-    out += sample_offset(G, cout);
     const int nbz = G >> LZ, nby = G / C::BY;
     // workgroups are dealt to the 8 XCDs in turn: each XCD takes one
     // contiguous range of bricks, whose halos meet in its L2
@@ -320,8 +331,8 @@ __global__ void __launch_bounds__(kT, RX * RY > 1 ? (MULTI ? 2 : 4) : (MULTI ? 3
             if (4 * C::H % kT == 0 || k + 1 < C::L || tid + k * kT < 4 * C::H)
                 d[k * (kT / 4)] = s4{bf(st[k].x), bf(st[k].y), bf(st[k].z), bf(st[k].w)};
     };
-    const int64_t tstep = int64_t(cout) * cin;
-    auto weights = [&](int ntile, int slice) { return w + (int64_t(ntile) * 16 + i) * cin + slice * 16 + 4 * kq; };
+    const int tstep = cout * 16;
+    auto weights = [&](int ntile, int slice) { return w + (slice * 27 * cout + ntile * 16 + i) * 16 + 4 * kq; };
     s4 wr[27];
     {
         const short* wl = weights(nt, 0);
@@ -375,6 +386,9 @@ __global__ void __launch_bounds__(kT, RX * RY > 1 ? (MULTI ? 2 : 4) : (MULTI ? 3
                     }
                 }
         if (sl == S - 1) {
+            const bool hi = nt * 16 >= dst.split;
+            const int oc = hi ? cout - dst.split : dst.split;
+            float* out = (hi ? dst.hi - dst.split : dst.lo) + sample_offset(G, oc) + nt * 16 + 4 * kq;
             float4 bv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             if (bias) bv = *reinterpret_cast<const float4*>(bias + nt * 16 + 4 * kq);
 #pragma unroll
@@ -390,7 +404,7 @@ __global__ void __launch_bounds__(kT, RX * RY > 1 ? (MULTI ? 2 : 4) : (MULTI ? 3
                         if (bias) v[e] = v[e] + be;
                         if (relu) v[e] = v[e] > 0.0f ? v[e] : 0.0f;
                     }
-                    *reinterpret_cast<float4*>(out + (int64_t(gx * G + gy) * G + gz) * cout + nt * 16 + 4 * kq) =
+                    *reinterpret_cast<float4*>(out + (int64_t(gx * G + gy) * G + gz) * oc) =
                         make_float4(v[0], v[1], v[2], v[3]);
                 }
         }
@@ -600,15 +614,30 @@ __global__ void __launch_bounds__(kT) k_grad_finish(const float* __restrict__ pa
     }
 }
 
-// bf16 copies: wb[t][co][ci] = bf16(w[t][co][ci]); wf[t][ci][co] = bf16(w[26 - t][co][ci])
-__global__ void k_pack(const float* w, int cin, int cout, short* wb, short* wf) {
-    const int64_t k = int64_t(blockIdx.x) * kT + threadIdx.x;
-    const int64_t n = int64_t(27) * cout * cin;
-    if (k >= n) return;
-    const int ci = int(k % cin), co = int((k / cin) % cout), t = int(k / (int64_t(cin) * cout));
-    const short h = bf(w[k]);
-    wb[k] = h;
-    wf[(int64_t(26 - t) * cin + ci) * cout + co] = h;
+// Where the weight of tap t, output channel co and input channel ci lies in a
+// convolution's BF16 weights, [ci / 16][t][co][ci % 16]: a wave's fragment of
+// 16 output by 16 input channels is 512 consecutive bytes (with all input
+// channels of a row together it was 32 bytes each of 16 lines).
+__device__ __forceinline__ int64_t packed_at(int t, int co, int ci, int cout) {
+    return ((int64_t(ci >> 4) * 27 + t) * cout + co) * 16 + (ci & 15);
+}
+
+struct PackJobs {
+    int64_t woff[14];
+    int32_t cin[14], cout[14];
+    short *wb[14], *wf[14];
+};
+
+// The BF16 weights of every convolution (blockIdx.y) and of its data gradient:
+// wb holds w[t][co][ci], wf the flipped and transposed w[26 - t][ci][co].
+__global__ void __launch_bounds__(kT) k_pack(const float* __restrict__ params, PackJobs J) {
+    const int k = blockIdx.y, cin = J.cin[k], cout = J.cout[k];
+    const int64_t j = int64_t(blockIdx.x) * kT + threadIdx.x;
+    if (j >= int64_t(27) * cout * cin) return;
+    const int ci = int(j % cin), co = int((j / cin) % cout), t = int(j / (int64_t(cin) * cout));
+    const short h = bf(params[J.woff[k] + j]);
+    J.wb[k][packed_at(t, co, ci, cout)] = h;
+    J.wf[k][packed_at(26 - t, ci, co, cin)] = h;
 }
 
 // Sums a float4 per thread over the threads with the same t % q4 (q4 = 4, 8
@@ -631,15 +660,21 @@ __device__ __forceinline__ float4 quad_sum(float4 v, int q4, float4* red) {
     return red[t];
 }
 
-// g[v, c] *= (y[v, c] > 0), and the bias gradient's workgroup partials
-// bp[w][c] over the workgroup's `per` voxels (a multiple of 4 kT / C): one
-// pass over g and y for both.  (The bias gradient alone, one workgroup per
-// channel with strided loads, took 325 us for 16 channels on 64^3.)
-__global__ void __launch_bounds__(kT) k_relu_bias(float* __restrict__ g, const float* __restrict__ y, int64_t V, int C,
-                                                 int64_t per, float* __restrict__ bp) {
+// g[v, c] *= (y[v, c] > 0), after adding the gradient pg of the output's
+// average pooling (grid G / 2; null: none), and the bias gradient's workgroup
+// partials bp[w][c] over the workgroup's `per` voxels (a multiple of
+// 4 kT / C): one pass over g and y for all three.  (The bias gradient alone,
+// one workgroup per channel with strided loads, took 325 us for 16 channels
+// on 64^3; the pooling's as a pass of its own 130 us for 8 samples.)
+__global__ void __launch_bounds__(kT) k_relu_bias(float* __restrict__ g, const float* __restrict__ y,
+                                                 const float* __restrict__ pg, int lg, int C, int64_t per,
+                                                 float* __restrict__ bp) {
+    const int G = 1 << lg;
+    const int64_t V = int64_t(1) << (3 * lg);
     __shared__ float4 red[kT];
     g += int64_t(blockIdx.y) * V * C;
     y += int64_t(blockIdx.y) * V * C;
+    pg += pg ? sample_offset(G >> 1, C) : 0;
     bp += int64_t(blockIdx.y) * gridDim.x * C;
     const int q4 = C >> 2, q = threadIdx.x & (q4 - 1), step = kT / q4;
     const int64_t v0 = int64_t(blockIdx.x) * per, v1 = v0 + per < V ? v0 + per : V;
@@ -649,6 +684,15 @@ __global__ void __launch_bounds__(kT) k_relu_bias(float* __restrict__ g, const f
         float4* gp = reinterpret_cast<float4*>(g + v * C) + q;
         const float4 a = *(reinterpret_cast<const float4*>(y + v * C) + q);
         float4 b = *gp;
+        if (pg) {
+            const int z = int(v) & (G - 1), yy = int(v >> lg) & (G - 1), x = int(v >> (2 * lg));
+            const int64_t u = (((int64_t(x >> 1) << (lg - 1)) + (yy >> 1)) << (lg - 1)) + (z >> 1);
+            const float4 h = *(reinterpret_cast<const float4*>(pg + u * C) + q);
+            b.x = b.x + h.x * 0.125f;
+            b.y = b.y + h.y * 0.125f;
+            b.z = b.z + h.z * 0.125f;
+            b.w = b.w + h.w * 0.125f;
+        }
         if (!(a.x > 0.0f)) b.x = 0.0f;
         if (!(a.y > 0.0f)) b.y = 0.0f;
         if (!(a.z > 0.0f)) b.z = 0.0f;
@@ -663,73 +707,57 @@ __global__ void __launch_bounds__(kT) k_relu_bias(float* __restrict__ g, const f
     if (threadIdx.x < q4) *(reinterpret_cast<float4*>(bp + int64_t(blockIdx.x) * C) + threadIdx.x) = s;
 }
 
-// average pooling 2x2x2 (G -> G/2) and its gradient
-__global__ void k_pool(const float* in, int G, int C, float* out) {
-    const int H = G / 2;
+// a 2x2x2 cell's eight voxels summed in order, four channels per thread: out
+// (G / 2) = f * sum.  Channels C = 2^lc, G = 2^lg.
+__device__ __forceinline__ void sum_cells(const float* __restrict__ in, int lc, int lg, float f,
+                                          float* __restrict__ out) {
+    const int lh = lg - 1, G = 1 << lg, C = 1 << lc;
     const int64_t k = int64_t(blockIdx.x) * kT + threadIdx.x;
-    if (k >= int64_t(H) * H * H * C) return;
+    if (k >= int64_t(1) << (3 * lh + lc - 2)) return;
     in += sample_offset(G, C);
-    out += sample_offset(H, C);
-    const int c = int(k % C);
-    const int64_t v = k / C;
-    const int x = int(v / (int64_t(H) * H)), y = int((v / H) % H), z = int(v % H);
-    float s = 0.0f;
-    for (int q = 0; q < 8; q++) {
-        const int64_t u = (int64_t(2 * x + (q >> 2)) * G + 2 * y + ((q >> 1) & 1)) * G + 2 * z + (q & 1);
-        s += in[u * C + c];
+    out += sample_offset(G >> 1, C);
+    const int q = int(k) & ((C >> 2) - 1);
+    const int64_t v = k >> (lc - 2);
+    const int z = int(v) & ((1 << lh) - 1), y = int(v >> lh) & ((1 << lh) - 1), x = int(v >> (2 * lh));
+    float4 a[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const int64_t u = (((int64_t(2 * x + (j >> 2)) << lg) + 2 * y + ((j >> 1) & 1)) << lg) + 2 * z + (j & 1);
+        a[j] = reinterpret_cast<const float4*>(in)[(u << (lc - 2)) + q];
     }
-    out[k] = s * 0.125f;
-}
-
-__global__ void k_pool_back(const float* g, int G, int C, float* gin, int accumulate) {
-    const int H = G / 2;
-    const int64_t k = int64_t(blockIdx.x) * kT + threadIdx.x;
-    if (k >= int64_t(G) * G * G * C) return;
-    g += sample_offset(H, C);
-    gin += sample_offset(G, C);
-    const int c = int(k % C);
-    const int64_t u = k / C;
-    const int x = int(u / (int64_t(G) * G)), y = int((u / G) % G), z = int(u % G);
-    const float val = g[((int64_t(x / 2) * H + y / 2) * H + z / 2) * C + c] * 0.125f;
-    gin[k] = accumulate ? gin[k] + val : val;
-}
-
-// gradient of a decoder input, concat(nearest upsampling of lo, skip): g_lo
-// (sum of 8 children, fixed order) and the skip part
-__global__ void k_up_concat_back_lo(const float* g, int C, int S, int G, float* glo) {
-    const int W = C + S, H = G / 2;
-    const int64_t k = int64_t(blockIdx.x) * kT + threadIdx.x;
-    if (k >= int64_t(H) * H * H * C) return;
-    g += sample_offset(G, W);
-    glo += sample_offset(H, C);
-    const int c = int(k % C);
-    const int64_t v = k / C;
-    const int x = int(v / (int64_t(H) * H)), y = int((v / H) % H), z = int(v % H);
-    float s = 0.0f;
-    for (int q = 0; q < 8; q++) {
-        const int64_t u = (int64_t(2 * x + (q >> 2)) * G + 2 * y + ((q >> 1) & 1)) * G + 2 * z + (q & 1);
-        s += g[u * W + c];
+    float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        s.x += a[j].x;
+        s.y += a[j].y;
+        s.z += a[j].z;
+        s.w += a[j].w;
     }
-    glo[k] = s;
+    reinterpret_cast<float4*>(out)[k] = make_float4(s.x * f, s.y * f, s.z * f, s.w * f);
 }
 
-__global__ void k_up_concat_back_skip(const float* g, int C, int S, int G, float* gskip) {
-    const int W = C + S;
-    const int64_t k = int64_t(blockIdx.x) * kT + threadIdx.x;
-    if (k >= int64_t(G) * G * G * S) return;
-    g += sample_offset(G, W);
-    gskip += sample_offset(G, S);
-    const int64_t u = k / S;
-    gskip[k] = g[u * W + C + int(k % S)];
+// average pooling 2x2x2 (its gradient is added by k_relu_bias)
+__global__ void __launch_bounds__(kT) k_pool(const float* in, int lc, int lg, float* out) {
+    sum_cells(in, lc, lg, 0.125f, out);
 }
 
-// head: pred[v] = b + sum_c w[c] * in[v, c] (float, c = 0..15 in order)
-__global__ void k_head(const float* in, const float* w, int64_t V, float* pred) {
+// gradient of nearest upsampling
+__global__ void __launch_bounds__(kT) k_up_back(const float* g, int lc, int lg, float* glo) {
+    sum_cells(g, lc, lg, 1.0f, glo);
+}
+
+// head: pred[v] = f * (b + sum_c w[c] * in[v, c]) (float, c = 0..15 in order)
+__global__ void __launch_bounds__(kT) k_head(const float* __restrict__ in, const float* __restrict__ w, int64_t V,
+                                            float f, float* __restrict__ pred) {
     const int64_t v = int64_t(blockIdx.x) * kT + threadIdx.x;
     if (v >= V) return;
+    float a[16];
+#pragma unroll
+    for (int c = 0; c < 16; c += 4) *reinterpret_cast<float4*>(a + c) = *reinterpret_cast<const float4*>(in + v * 16 + c);
     float s = 0.0f;
-    for (int c = 0; c < 16; c++) s += w[c] * in[v * 16 + c];
-    pred[v] = s + w[16];
+#pragma unroll
+    for (int c = 0; c < 16; c++) s += w[c] * a[c];
+    pred[v] = (s + w[16]) * f;
 }
 
 // Two doubles per thread summed over the workgroup (a fixed tree).
@@ -1040,7 +1068,7 @@ bool pow2_channels(int c) { return c == 16 || c == 32 || c == 64; }
 constexpr int64_t kConvManyTiles = 4096;
 
 template <int LZ, int RX, int RY, int WX, int WY, int WN>
-void launch_conv_rows(hipStream_t s, ConvIn src, const short* w, const float* bias, int G, int relu, float* out,
+void launch_conv_rows(hipStream_t s, ConvIn src, const short* w, const float* bias, int G, int relu, ConvOut out,
                       int cout, int B) {
     using C = ConvTile<LZ, RX, RY, WX, WY, WN>;
     const int NT = cout / 16, S = (src.clo + src.cskip) / 16;
@@ -1056,7 +1084,7 @@ void launch_conv_rows(hipStream_t s, ConvIn src, const short* w, const float* bi
 }
 
 template <int LZ>
-void launch_conv_grid(hipStream_t s, ConvIn src, const short* w, const float* bias, int G, int relu, float* out,
+void launch_conv_grid(hipStream_t s, ConvIn src, const short* w, const float* bias, int G, int relu, ConvOut out,
                       int cout, int B) {
     const int NT = cout / 16;
     const bool many = int64_t(B) * G * G * G / 16 * NT >= kConvManyTiles && G >= 8;
@@ -1072,7 +1100,7 @@ void launch_conv_grid(hipStream_t s, ConvIn src, const short* w, const float* bi
     }
 }
 
-void launch_conv(hipStream_t s, ConvIn src, const short* w, const float* bias, int G, int relu, float* out, int cout,
+void launch_conv(hipStream_t s, ConvIn src, const short* w, const float* bias, int G, int relu, ConvOut out, int cout,
                  int B) {
     const int cin = src.clo + src.cskip;
     if (!pow2_channels(src.cskip) || (src.clo && !pow2_channels(src.clo)) || cout % 16 || cout <= 0 ||
@@ -1093,26 +1121,34 @@ void launch_conv(hipStream_t s, ConvIn src, const short* w, const float* bias, i
 }
 
 void pack_all(prg_unet* n) {
-    for (auto& L : n->conv) {
-        const int64_t cnt = int64_t(27) * L.cout * L.cin;
-        k_pack<<<blocks(cnt), kT, 0, n->stream>>>(n->params.get() + L.woff, L.cin, L.cout, L.wb.get(), L.wf.get());
-        PRG_CHECK_LAUNCH();
+    PackJobs J{};
+    int64_t most = 0;
+    for (int k = 0; k < 14; k++) {
+        auto& L = n->conv[k];
+        J.woff[k] = L.woff;
+        J.cin[k] = L.cin;
+        J.cout[k] = L.cout;
+        J.wb[k] = L.wb.get();
+        J.wf[k] = L.wf.get();
+        most = std::max(most, int64_t(27) * L.cout * L.cin);
     }
+    k_pack<<<dim3(blocks(most), 14), kT, 0, n->stream>>>(n->params.get(), J);
+    PRG_CHECK_LAUNCH();
 }
 
-// prediction of the B samples in x0
-void forward(prg_unet* n, int B) {
+// prediction of the B samples in x0, times f
+void forward(prg_unet* n, int B, float f = 1.0f) {
     hipStream_t s = n->stream;
     const int G = n->G;
     auto& C = n->conv;
     auto run = [&](int k) {
         auto& L = C[k];
         launch_conv(s, ConvIn{L.lo, L.clo, L.skip, L.cin - L.clo}, L.wb.get(), n->params.get() + L.boff, L.G, 1,
-                    L.out, L.cout, B);
+                    ConvOut{L.out, L.cout, nullptr}, L.cout, B);
     };
     auto pool = [&](const float* in, int g, int c, float* out) {
         const int64_t h = g / 2;
-        k_pool<<<dim3(blocks(h * h * h * c), unsigned(B)), kT, 0, s>>>(in, g, c, out);
+        k_pool<<<dim3(blocks(h * h * h * c / 4), unsigned(B)), kT, 0, s>>>(in, log2i(c), log2i(g), out);
         PRG_CHECK_LAUNCH();
     };
     run(0);
@@ -1133,7 +1169,7 @@ void forward(prg_unet* n, int B) {
     run(12);
     run(13);
     const int64_t V = int64_t(G) * G * G * B;
-    k_head<<<blocks(V), kT, 0, s>>>(C[13].out, n->params.get() + (n->nparams - 17), V, n->pred.get());
+    k_head<<<blocks(V), kT, 0, s>>>(C[13].out, n->params.get() + (n->nparams - 17), V, f, n->pred.get());
     PRG_CHECK_LAUNCH();
 }
 
@@ -1151,16 +1187,19 @@ BiasPlan bias_plan(int64_t V, int C) {
     return {unsigned((V + per - 1) / per), per};
 }
 
-// gradient of conv k for incoming gradient g (in place: ReLU mask, unless
-// `masked`: g has it and the bias gradient is accumulated); writes the input
-// gradient to gin unless gin is null; accumulates dW and db.
-void conv_back(prg_unet* n, int B, int k, float* g, float* gin, bool masked = false) {
+// Gradient of conv k for incoming gradient g (in place: the pooled gradient
+// `pg` of its output added, then the ReLU mask; unless `masked`: g has both
+// and the bias gradient is accumulated).  Writes the input gradient to gin
+// unless it is null (of a concatenated input: the upsampled channels to gin,
+// the skip's to gskip); accumulates dW and db.
+void conv_back(prg_unet* n, int B, int k, float* g, float* gin, float* gskip = nullptr, const float* pg = nullptr,
+               bool masked = false) {
     hipStream_t s = n->stream;
     auto& L = n->conv[k];
     const int64_t V = int64_t(L.G) * L.G * L.G;
     const BiasPlan bp = bias_plan(V, L.cout);
     if (!masked) {
-        k_relu_bias<<<dim3(bp.wg, unsigned(B)), kT, 0, s>>>(g, L.out, V, L.cout, bp.per, n->bpart.get());
+        k_relu_bias<<<dim3(bp.wg, unsigned(B)), kT, 0, s>>>(g, L.out, pg, log2i(L.G), L.cout, bp.per, n->bpart.get());
         PRG_CHECK_LAUNCH();
     }
     const int nchunk = int((V + kWChunk - 1) / kWChunk);
@@ -1181,7 +1220,9 @@ void conv_back(prg_unet* n, int B, int k, float* g, float* gin, bool masked = fa
         n->part.get(), nchunk, nw, n->grads.get() + L.woff, n->bpart.get(), int(bp.wg), L.cout,
         n->grads.get() + L.boff, B);
     PRG_CHECK_LAUNCH();
-    if (gin) launch_conv(s, ConvIn{nullptr, 0, g, L.cout}, L.wf.get(), nullptr, L.G, 0, gin, L.cin, B);
+    if (gin)
+        launch_conv(s, ConvIn{nullptr, 0, g, L.cout}, L.wf.get(), nullptr, L.G, 0,
+                    gskip ? ConvOut{gin, L.clo, gskip} : ConvOut{gin, L.cin, nullptr}, L.cin, B);
 }
 
 // the losses of the B samples `forward` ran on, and their gradients for every
@@ -1206,44 +1247,35 @@ void backward(prg_unet* n, int B) {
     k_head_finish<<<(kHeadCols + 3) / 4, kT, 0, s>>>(n->bpart.get(), nh, n->grads.get() + head,
                                                      n->grads.get() + C[13].boff, B);
     PRG_CHECK_LAUNCH();
+    auto up_back = [&](const float* g, int c, int g1, float* glo) {
+        const int64_t h = g1 / 2;
+        k_up_back<<<dim3(blocks(h * h * h * c / 4), unsigned(B)), kT, 0, s>>>(g, log2i(c), log2i(g1), glo);
+        PRG_CHECK_LAUNCH();
+    };
+    float *ge0 = n->ge0.get(), *ge1 = n->ge1.get(), *ge2 = n->ge2.get();
     // d0
-    conv_back(n, B, 13, ga, gb, true);
-    conv_back(n, B, 12, gb, ga);  // ga: gradient of c0 (48 channels)
-    k_up_concat_back_skip<<<dim3(blocks(V0 * 16), unsigned(B)), kT, 0, s>>>(ga, 32, 16, G, n->ge0.get());
-    PRG_CHECK_LAUNCH();
-    k_up_concat_back_lo<<<dim3(blocks(V1 * 32), unsigned(B)), kT, 0, s>>>(ga, 32, 16, G, gb);
-    PRG_CHECK_LAUNCH();
+    conv_back(n, B, 13, ga, gb, nullptr, nullptr, true);
+    conv_back(n, B, 12, gb, ga, ge0);  // ga: gradient of d1's output upsampled (G, 32)
+    up_back(ga, 32, G, gb);
     // d1 (gb: gradient of d1 output, G/2, 32 channels)
     conv_back(n, B, 11, gb, ga);
-    conv_back(n, B, 10, ga, gb);  // gb: c1 gradient (96)
-    k_up_concat_back_skip<<<dim3(blocks(V1 * 32), unsigned(B)), kT, 0, s>>>(gb, 64, 32, G / 2, n->ge1.get());
-    PRG_CHECK_LAUNCH();
-    k_up_concat_back_lo<<<dim3(blocks(V2 * 64), unsigned(B)), kT, 0, s>>>(gb, 64, 32, G / 2, ga);
-    PRG_CHECK_LAUNCH();
+    conv_back(n, B, 10, ga, gb, ge1);  // gb: gradient of d2's output upsampled (G/2, 64)
+    up_back(gb, 64, G / 2, ga);
     // d2 (ga: gradient of d2 output, G/4, 64)
     conv_back(n, B, 9, ga, gb);
-    conv_back(n, B, 8, gb, ga);  // ga: c2 gradient (128)
-    k_up_concat_back_skip<<<dim3(blocks(V2 * 64), unsigned(B)), kT, 0, s>>>(ga, 64, 64, G / 4, n->ge2.get());
-    PRG_CHECK_LAUNCH();
-    k_up_concat_back_lo<<<dim3(blocks(V2 / 8 * 64), unsigned(B)), kT, 0, s>>>(ga, 64, 64, G / 4, gb);
-    PRG_CHECK_LAUNCH();
+    conv_back(n, B, 8, gb, ga, ge2);  // ga: gradient of the bottleneck's output upsampled (G/4, 64)
+    up_back(ga, 64, G / 4, gb);
     // bottleneck (gb: G/8, 64)
     conv_back(n, B, 7, gb, ga);
     conv_back(n, B, 6, ga, gb);  // gb: gradient of p3 (G/8, 64)
-    k_pool_back<<<dim3(blocks(V2 * 64), unsigned(B)), kT, 0, s>>>(gb, G / 4, 64, n->ge2.get(), 1);
-    PRG_CHECK_LAUNCH();
     // e2
-    conv_back(n, B, 5, n->ge2.get(), ga);
+    conv_back(n, B, 5, ge2, ga, nullptr, gb);
     conv_back(n, B, 4, ga, gb);  // gb: gradient of p2 (G/4, 32)
-    k_pool_back<<<dim3(blocks(V1 * 32), unsigned(B)), kT, 0, s>>>(gb, G / 2, 32, n->ge1.get(), 1);
-    PRG_CHECK_LAUNCH();
     // e1
-    conv_back(n, B, 3, n->ge1.get(), ga);
+    conv_back(n, B, 3, ge1, ga, nullptr, gb);
     conv_back(n, B, 2, ga, gb);  // gb: gradient of p1 (G/2, 16)
-    k_pool_back<<<dim3(blocks(V0 * 16), unsigned(B)), kT, 0, s>>>(gb, G, 16, n->ge0.get(), 1);
-    PRG_CHECK_LAUNCH();
     // e0
-    conv_back(n, B, 1, n->ge0.get(), ga);
+    conv_back(n, B, 1, ge0, ga, nullptr, gb);
     conv_back(n, B, 0, ga, nullptr);
 }
 
@@ -1484,9 +1516,7 @@ prg_status prg_unet_predict(prg_unet* n, const float* bgrid, const float* mask, 
         const int64_t V = int64_t(n->G) * n->G * n->G;
         prg::reserve_batch(n, 1);
         prg::load_samples(n, bgrid, mask, nullptr, &scale, 1);
-        prg::forward(n, 1);
-        prg::k_scale<<<prg::blocks(V), prg::kT, 0, n->stream>>>(n->pred.get(), V, scale, nullptr);
-        PRG_CHECK_LAUNCH();
+        prg::forward(n, 1, scale);
         PRG_HIP(hipMemcpyAsync(out, n->pred.get(), size_t(V) * 4, hipMemcpyDeviceToHost, n->stream));
         PRG_HIP(hipStreamSynchronize(n->stream));
         return PRG_OK;
