@@ -195,9 +195,14 @@ __global__ void __launch_bounds__(kBlock) k_vector_field(const int32_t* pntD, co
 // kVfPoints points reads them from global memory instead, and a tile with
 // more than kTileBlocks listed blocks takes the per-row path (the choices are
 // per workgroup).
-constexpr int kVfPoints = 768;
+constexpr int kVfPoints = 768;        // 52 KB of LDS, three workgroups per CU
+// For clouds of kVfDense points and more per sibling block, whose tiles mostly
+// exceed kVfPoints: 77 KB, two workgroups per CU.
+constexpr int kVfPointsDense = 1280;
+constexpr double kVfDense = 4.0;
 
-__global__ void __launch_bounds__(kTileThreads, 6) k_vector_field_tiles(TilePlan P, int64_t nblk,
+template <int POINTS>
+__global__ void __launch_bounds__(kTileThreads, POINTS > kVfPoints ? 4 : 6) k_vector_field_tiles(TilePlan P, int64_t nblk,
                                                                      const int32_t* __restrict__ pntD,
                                                                      const int32_t* __restrict__ pidx,
                                                                      const int32_t* __restrict__ pnum,
@@ -213,7 +218,7 @@ __global__ void __launch_bounds__(kTileThreads, 6) k_vector_field_tiles(TilePlan
     // a cell's first point is bfirst[block] + coff[cell] - coff[8 block].
     __shared__ int32_t bfirst[kTileBlocks];        // first point of each listed block
     __shared__ int32_t coff[8 * kTileBlocks + 1];  // LDS offsets of the cells' points
-    __shared__ float pw[12 * kVfPoints];           // 9 weights and the normal, one array per component
+    __shared__ float pw[12 * POINTS];           // 9 weights and the normal, one array per component
     __shared__ int16_t rid[kTileEntries];
     __shared__ int32_t wtot[kTileThreads / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -268,10 +273,10 @@ __global__ void __launch_bounds__(kTileThreads, 6) k_vector_field_tiles(TilePlan
             }
             const int64_t q = int64_t(bfirst[lo >> 3]) + (i - coff[lo & ~7]);
 #pragma unroll
-            for (int k = 0; k < 9; k++) pw[k * kVfPoints + i] = W[9 * q + k];
-            pw[9 * kVfPoints + i] = nx[q];
-            pw[10 * kVfPoints + i] = ny[q];
-            pw[11 * kVfPoints + i] = nz[q];
+            for (int k = 0; k < 9; k++) pw[k * POINTS + i] = W[9 * q + k];
+            pw[9 * POINTS + i] = nx[q];
+            pw[10 * POINTS + i] = ny[q];
+            pw[11 * POINTS + i] = nz[q];
         }
     }
     __syncthreads();
@@ -290,13 +295,13 @@ __global__ void __launch_bounds__(kTileThreads, 6) k_vector_field_tiles(TilePlan
         const int kx = 2 - j / 9, ky = 2 - (j / 3) % 3, kz = 2 - j % 3;  // 1 - delta
         if (staged) {
             for (int32_t q = o; q < e; q++) {
-                const float fx = pw[kx * kVfPoints + q], fy = pw[(3 + ky) * kVfPoints + q],
-                            fz = pw[(6 + kz) * kVfPoints + q];
+                const float fx = pw[kx * POINTS + q], fy = pw[(3 + ky) * POINTS + q],
+                            fz = pw[(6 + kz) * POINTS + q];
                 float w = fx * fy;
                 w = w * fz;
-                vx = vx + w * pw[9 * kVfPoints + q];
-                vy = vy + w * pw[10 * kVfPoints + q];
-                vz = vz + w * pw[11 * kVfPoints + q];
+                vx = vx + w * pw[9 * POINTS + q];
+                vy = vy + w * pw[10 * POINTS + q];
+                vz = vz + w * pw[11 * POINTS + q];
             }
         } else {
             const int64_t p0 = int64_t(bfirst[cell >> 3]) + (o - coff[cell & ~7]);
@@ -780,7 +785,9 @@ void compute_divergence(prg_ctx* c) {
     // LDS capacities of the tile kernels; a smaller limit (a test setting)
     // sends more tiles down the per-row and global-memory paths
     const int32_t lim_blocks = c->tile_limit > 0 ? std::min(c->tile_limit, kTileBlocks) : kTileBlocks;
-    const int32_t lim_points = c->tile_limit > 0 ? std::min(c->tile_limit, kVfPoints) : kVfPoints;
+    const bool dense = double(c->N) >= kVfDense * double(MD / 8);
+    const int32_t vf_points = dense ? kVfPointsDense : kVfPoints;
+    const int32_t lim_points = c->tile_limit > 0 ? std::min(c->tile_limit, vf_points) : vf_points;
     float* VX = c->vfx.reserve(MD);
     float* VY = c->vfy.reserve(MD);
     float* VZ = c->vfz.reserve(MD);
@@ -799,7 +806,8 @@ void compute_divergence(prg_ctx* c) {
         TilePlan P{};
         if (tile_plan_on(c, D, &P, s)) {
             const int64_t nblk = MD / 8, ntiles = (nblk + kTile - 1) / kTile;
-            k_vector_field_tiles<<<unsigned(ntiles), kTileThreads, 0, s>>>(
+            const auto kernel = dense ? k_vector_field_tiles<kVfPointsDense> : k_vector_field_tiles<kVfPoints>;
+            kernel<<<unsigned(ntiles), kTileThreads, 0, s>>>(
                 P, nblk, c->pnt.get() + 27 * c->pnt_off[D], c->pidx.get(), c->pnum.get(), W.get(), c->nx.get(),
                 c->ny.get(), c->nz.get(), baseD, VX, VY, VZ, lim_blocks, lim_points);
         } else {

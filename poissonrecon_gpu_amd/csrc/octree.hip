@@ -371,25 +371,34 @@ constexpr int kLvlBlock = 256;
 constexpr int kLvlItems = 8;
 constexpr int kLvlTile = kLvlBlock * kLvlItems;
 
-__device__ __forceinline__ int32_t head_flag(const uint32_t* nk, int64_t i, int64_t n, int hs) {
-    return (i < n && (i == 0 || (nk[i] >> hs) != (nk[i - 1] >> hs))) ? 1 : 0;
-}
-
 __global__ void __launch_bounds__(kLvlBlock) k_level_up(const uint32_t* nk, const int32_t* np, const int32_t* ndi,
-                                                        int32_t* ne, int hs, int D, int d, uint32_t tiles,
-                                                        uint64_t* state, int32_t* pos, uint32_t* pk, int32_t* pp,
-                                                        int32_t* pdi) {
+                                                        int32_t* ne, int hs, int D, int d, uint64_t* state,
+                                                        int32_t* pos, uint32_t* pk, int32_t* pp, int32_t* pdi) {
     __shared__ int32_t lds[kLvlBlock / 64];
     __shared__ int32_t s_before;
+    // only the tiles that hold nodes (the launch is sized for an upper bound:
+    // the empty ones' turns in the look-back had taken most of the time)
+    const int64_t n = ne[d];
+    const uint32_t tiles = uint32_t((n + kLvlTile - 1) / kLvlTile);
+    if (blockIdx.x >= tiles) return;
     const LookTile t = look_begin(state, tiles);
     if (t.tile >= tiles) return;
-    const int64_t n = ne[d], base = int64_t(t.tile) * kLvlTile + int64_t(threadIdx.x) * kLvlItems;
+    const int64_t base = int64_t(t.tile) * kLvlTile + int64_t(threadIdx.x) * kLvlItems;
     const int sh = 3 * (D - d);
+    uint32_t key[kLvlItems];
+    const uint32_t prev = base > 0 && base - 1 < n ? nk[base - 1] : 0u;
+    if (base + kLvlItems <= n) {
+#pragma unroll
+        for (int k = 0; k < kLvlItems; k += 4) *reinterpret_cast<uint4*>(key + k) = *reinterpret_cast<const uint4*>(nk + base + k);
+    } else {
+#pragma unroll
+        for (int k = 0; k < kLvlItems; k++) key[k] = base + k < n ? nk[base + k] : 0u;
+    }
     int32_t f[kLvlItems];
     int32_t acc = 0;
 #pragma unroll
     for (int k = 0; k < kLvlItems; k++) {
-        f[k] = head_flag(nk, base + k, n, hs);
+        f[k] = base + k < n && (base + k == 0 || (key[k] >> hs) != ((k ? key[k - 1] : prev) >> hs)) ? 1 : 0;
         acc += f[k];
     }
     int32_t tot;
@@ -409,10 +418,9 @@ __global__ void __launch_bounds__(kLvlBlock) k_level_up(const uint32_t* nk, cons
         const int64_t i = base + k;
         if (i < n) {
             const int32_t b = ex + f[k] - 1;  // parent block: heads up to i, inclusive, minus one
-            const uint32_t key = nk[i];
-            pos[i] = 8 * b + int32_t((key >> sh) & 7u);
+            pos[i] = 8 * b + int32_t((key[k] >> sh) & 7u);
             if (f[k]) {
-                pk[b] = key & ~(7u << sh);
+                pk[b] = key[k] & ~(7u << sh);
                 pp[b] = np[i];
                 pdi[b] = (d == D) ? 8 * b : ndi[i];
             }
@@ -723,8 +731,8 @@ void build_octree(prg_ctx* c) {
         const int hs = 3 * (D - d + 1);
         TimedScope ts(kt, "level_up", 28.0 * double(ub[d]));
         k_level_up<<<unsigned(tiles), kLvlBlock, 0, s>>>(NK[d]->get(), NP[d]->get(), NDI[d]->get(), ne_dev.get(), hs, D,
-                                                         d, uint32_t(tiles), state, POS[d]->get(), NK[d - 1]->get(),
-                                                         NP[d - 1]->get(), NDI[d - 1]->get());
+                                                         d, state, POS[d]->get(), NK[d - 1]->get(), NP[d - 1]->get(),
+                                                         NDI[d - 1]->get());
         PRG_CHECK_LAUNCH();
     }
     LevelArrays LA{};

@@ -96,7 +96,8 @@ static_assert(kCntSlots * 4 <= 256 && kCntCells + kMaxDepth < kCntTaken && kCntT
 
 __device__ __forceinline__ int depth_of(int64_t i, const Levels& L, int D) {
     int d = 0;
-    while (d < D && i >= L.base[d + 1]) d++;
+#pragma unroll
+    for (int k = 1; k <= kMaxDepth; k++) d += k <= D && i >= L.base[k] ? 1 : 0;
     return d;
 }
 
@@ -144,28 +145,36 @@ __device__ __forceinline__ void face_visit(int64_t Y, uint32_t faces, const uint
                                            const int32_t* __restrict__ pnt, const Levels& L,
                                            const int32_t* __restrict__ parent, int d, int D, uint8_t* inter,
                                            uint32_t* up) {
+    // the face record (face_rec): owned by the smaller key of Y and its
+    // neighbour across the face, both at depth d.  The six neighbours' loads
+    // go out together, then their keys'.
     const uint32_t ky = key[Y];
+    const int64_t loc = Y - L.base[d];
+    const int s = int(loc & 7);
+    const int32_t* row = pnt + 27 * (L.pnt_off[d] + (loc >> 3));
+    int32_t nb[6];
+    uint32_t kn[6];
+#pragma unroll
+    for (int j = 0; j < 6; j++) {
+        const int o3 = j >> 1, dl = (j & 1) ? 1 : -1;
+        int entry, child;
+        tile_neighbour(s, nidx(o3 == 0 ? dl : 0, o3 == 1 ? dl : 0, o3 == 2 ? dl : 0), entry, child);
+        // (the tree's root has no neighbour and no row)
+        const int32_t cb = d > 0 && ((faces >> j) & 1u) ? row[entry] : -1;
+        nb[j] = cb < 0 ? -1 : int32_t(L.base[d] + cb + child);
+    }
+#pragma unroll
+    for (int j = 0; j < 6; j++) kn[j] = nb[j] < 0 ? 0xffffffffu : key[nb[j]];
     uint32_t cont = 0;
+#pragma unroll
     for (int j = 0; j < 6; j++) {
         if (!((faces >> j) & 1u)) continue;
-        // the face record (face_rec): owned by the smaller key of Y and its
-        // neighbour across the face, both at depth d
-        const int o3 = j >> 1, dl = (j & 1) ? 1 : -1;
-        const int32_t nb = neighbour_of(pnt, L, d, Y, nidx(o3 == 0 ? dl : 0, o3 == 1 ? dl : 0, o3 == 2 ? dl : 0));
-        int64_t owner = Y;
-        int kind = j;
-        uint32_t ko = ky;
-        if (nb != -1) {
-            const uint32_t kn = key[nb];
-            if (kn < ky) {
-                owner = nb;
-                kind = j ^ 1;
-                ko = kn;
-            }
-        }
+        const bool far = nb[j] >= 0 && kn[j] < ky;
+        const int64_t owner = far ? nb[j] : Y;
+        const int kind = far ? j ^ 1 : j;
         inter[6 * owner + kind] = 1;
         // only the root (depth 0) has no parent
-        if (d > 0 && c_parent_face[(ko >> (3 * (D - d))) & 7u][kind] != -1) cont |= 1u << j;
+        if (d > 0 && c_parent_face[((far ? kn[j] : ky) >> (3 * (D - d))) & 7u][kind] != -1) cont |= 1u << j;
     }
     if (cont) {
         const int64_t P = parent[Y];
@@ -196,8 +205,7 @@ __global__ void __launch_bounds__(kBlockS) k_face_marks_up(int64_t base, int64_t
 
 // The same for depths ds .. 0, of at most kSmallUp nodes each, by one
 // workgroup: a launch per depth costs about 4 us whatever it does.  The
-// faces of a depth are ORed in L2; the fence completes them before the
-// barrier, and the loads read them there.
+// faces of a depth are ORed in L2, and the loads read them there.
 constexpr int kUpBlock = 1024;
 constexpr int64_t kSmallUp = 4096;
 __global__ void __launch_bounds__(kUpBlock) k_face_marks_up_small(int ds, const uint32_t* key, const int32_t* pnt,
@@ -209,7 +217,10 @@ __global__ void __launch_bounds__(kUpBlock) k_face_marks_up_small(int ds, const 
             const uint32_t faces = (w >> (8 * (Y & 3))) & 0xffu;
             if (faces) face_visit(Y, faces, key, pnt, L, parent, d, D, inter, up);
         }
-        __threadfence();
+        // (the waits complete the ORs in L2, where one workgroup's are ordered
+        // without a device-scope fence, which writes the L2 back)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
     }
 }
@@ -484,8 +495,8 @@ constexpr int kRootTile = kRootBlock * kRootItems;
 // counts in cnt and in pinned memory.  (As flags, compaction, sizes, two
 // scans and an append these were five launches over the upper bound n.)
 __global__ void __launch_bounds__(kRootBlock) k_list_all_roots(const int32_t* __restrict__ cl,
-                                                               const uint8_t* __restrict__ rflag, uint32_t tiles,
-                                                               uint64_t* state, Levels L, int D,
+                                                               const uint8_t* __restrict__ rflag, uint64_t* state,
+                                                               Levels L, int D,
                                                                int32_t* __restrict__ roots, int32_t* __restrict__ boff,
                                                                int32_t* __restrict__ root_of,
                                                                int32_t* __restrict__ list1,
@@ -494,6 +505,9 @@ __global__ void __launch_bounds__(kRootBlock) k_list_all_roots(const int32_t* __
     __shared__ int32_t lds[kRootBlock / 64];
     __shared__ int32_t s_before[5];
     const int64_t n = cnt[kCntCoarse];
+    // (the launch is sized for the upper bound)
+    const uint32_t tiles = n > 0 ? uint32_t((n + kRootTile - 1) / kRootTile) : 1;
+    if (blockIdx.x >= tiles) return;
     const LookTile t = look_begin(state, tiles);
     if (t.tile >= tiles) return;
     const int64_t base = int64_t(t.tile) * kRootTile + int64_t(threadIdx.x) * kRootItems;
@@ -2437,7 +2451,7 @@ void extract_subdivision(prg_ctx* c) {
     {
         const uint32_t tiles = select_tiles(baseD, kRootTile);
         uint64_t* state = look_state(c->scratch, 5 * int64_t(tiles), s);
-        k_list_all_roots<<<tiles, kRootBlock, 0, s>>>(cl.get(), rflag.get(), tiles, state, Lv, D, roots.get(),
+        k_list_all_roots<<<tiles, kRootBlock, 0, s>>>(cl.get(), rflag.get(), state, Lv, D, roots.get(),
                                                       boff.get(), root_of.get(), slist1.get(), slist2.get(),
                                                       sidx.get(), C, H);
         PRG_CHECK_LAUNCH();
