@@ -633,7 +633,8 @@ constexpr int kP = (1 << kBrickLog) + 1;  // grid points per brick side (at most
 // at most (D - 3 - r) blocks of 4^3 cells and blocks of 5^3, 7^3 and 11^3
 // cells at the three finest depths.
 constexpr int kXBlk = 2304;
-constexpr int kXBlkScreen = 512;  // and in the screens' LDS
+constexpr int kXBlkScreen = 768;        // and in the screens' LDS: of cells of 16^3 leaves and more,
+constexpr int kXBlkScreenBrick = 2176;  // and of bricks
 
 // LDS of one brick's wave: the root's neighbourhood, the brick's basis
 // tables and blocks (BrickCore).
@@ -655,18 +656,25 @@ struct BrickCore {
     // D, D - 2, .. and D - 1, D - 3, ..: up to 5^3 and 7^3 cells
     int32_t CB0[125], CB1[343];
     int32_t NB[27], NBK[27], NBR[27];  // the root's neighbours, their child bases, their root numbers (group)
-    float tmax[kMaxDepth + 1];         // brick_abs_bound: per depth, the largest |basis value|
-    float xsum[kMaxDepth + 1];         // and the sum of |coefficients|
 };
 
-// A screened cell's: the chain's polynomial and blocks of up to kXBlkScreen
-// floats and 5^3 cells above depth D (a cell that needs more is not settled).
+// A screened cell's: the chain's polynomial and blocks of up to FLOATS
+// coefficients and 7^3 cells above depth D (a cell that needs more is not
+// settled).
+template <int FLOATS>
 struct CellLds {
     float P[27];
-    float XB[kXBlkScreen];
+    float XB[FLOATS];
     int32_t xb_off[kMaxDepth + 1];
-    int32_t CB0[125], CB1[125];
+    int32_t CB0[343], CB1[343];
     int32_t NBK[27], NBR[27];
+};
+
+// A brick's for the per-corner certificate: a cell's, with the basis table
+// entries (BrickCore's T) of the three finest depths, (e, a, i) for depth
+// D - kBrickLog + 1 + e.
+struct CertLds : CellLds<kXBlk> {
+    BasisT T[kBrickLog * 3 * kP];
 };
 
 __device__ __forceinline__ void decode_cell(uint32_t k, int32_t c[3]) {
@@ -730,15 +738,21 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
-// The record of root q (one wave per root).
-__global__ void __launch_bounds__(kWave) k_root_records(SubArgs A, int32_t* rec) {
-    const int D = A.D, lane = threadIdx.x;
-    const int32_t q = blockIdx.x;
-    const int32_t rho = A.roots[q];
+// The records of roots 2 w and 2 w + 1, half a wave each: following a root's
+// ancestors row by row is a chain of dependent loads, so the waves' number is
+// what counts (one root per wave: 324 us for 294,344 roots).
+__global__ void __launch_bounds__(kWave) k_root_records(SubArgs A, int32_t nr, int32_t* rec) {
+    const int D = A.D, lane = threadIdx.x & 31;
+    const int32_t q = 2 * blockIdx.x + (threadIdx.x >> 5);
+    __shared__ float Xs[2][(kMaxDepth + 1) * 27];
+    float* X = Xs[threadIdx.x >> 5];
+    const bool in = q < nr;
+    const int32_t rho = A.roots[in ? q : 0];
     const int r = depth_of(rho, A.L, D);
     int32_t* R = rec + int64_t(q) * kRecWords;
-    __shared__ float X[(kMaxDepth + 1) * 27];
-    if (lane < 27) {
+    const bool use = in && lane < 27;
+    const int l27 = lane < 27 ? lane : 0;
+    if (use) {
         const int32_t nb = neighbour_of(A.pnt, A.L, r, rho, lane);
         R[kRecNB + lane] = nb;
         R[kRecNBK + lane] = nb < 0 ? -1 : A.child_base[nb];
@@ -751,24 +765,26 @@ __global__ void __launch_bounds__(kWave) k_root_records(SubArgs A, int32_t* rec)
     int32_t a = A.parent[rho];
     for (int d = r - 1; d >= 1; d--) {
         const float* Row = A.rows + kRowFloats * (int64_t(a) - A.L.base[1]);
-        if (lane < 27) {
-            R[kRecX + 27 * d + lane] = __float_as_int(Row[lane]);
-            X[27 * d + lane] = Row[lane];
+        const float xv = Row[l27];
+        a = __float_as_int(Row[27]);
+        if (use) {
+            R[kRecX + 27 * d + lane] = __float_as_int(xv);
+            X[27 * d + lane] = xv;
         }
-        a = __builtin_amdgcn_readfirstlane(__float_as_int(Row[27]));
     }
-    if (lane == 0) {
+    if (in && lane == 0) {
         R[kRecX] = __float_as_int(A.x[0]);
         R[kRecRho] = rho;
         R[kRecR] = r;
         R[kRecKey] = int32_t(A.key[rho]);
     }
-    if (D - r < kBrickLog) return;  // (uniform) no cells to screen
+    const bool cells = in && D - r >= kBrickLog;  // cells to screen
+    if (__builtin_amdgcn_ballot_w64(cells) == 0) return;
     if (lane < 27) X[lane] = lane == 13 ? A.x[0] : 0.0f;  // depth 0: the tree's root has no neighbours
     __syncthreads();
+    if (!cells) return;  // (no barrier follows; a half's shuffles stay inside it)
     int32_t rc[3];
     decode_cell(A.key[rho], rc);
-    const int l27 = lane < 27 ? lane : 0;
     float val = 0.0f, err = 0.0f;
     for (int d = 0; d <= r; d++) {
         float w[3][3];
@@ -776,9 +792,12 @@ __global__ void __launch_bounds__(kWave) k_root_records(SubArgs A, int32_t* rec)
         for (int a3 = 0; a3 < 3; a3++)
             spline_weights(rc[a3] >> (D - r), r - d, a3 == 0 ? l27 / 9 : a3 == 1 ? (l27 / 3) % 3 : l27 % 3, w[a3]);
         val += sum27(X + 27 * d, 9, 3, w);
-        err += A.dev[d] * wave_max(fabsf(X[27 * d + l27]));
+        float m = fabsf(X[27 * d + l27]);
+#pragma unroll
+        for (int o = 16; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 32));
+        err += A.dev[d] * m;
     }
-    if (lane < 27) R[kRecPoly + lane] = __float_as_int(val);
+    if (use) R[kRecPoly + lane] = __float_as_int(val);
     if (lane == 0) R[kRecErr] = __float_as_int(err);
 }
 
@@ -825,29 +844,28 @@ __device__ __forceinline__ void set_kids(Brick& B, const L& S) {
 
 // Loads the root record of brick b (8^3 leaves) into LDS (its neighbours and
 // its chain's values) and sets the brick's geometry.
-// q_loaded: the root whose record S already holds (the previous brick's, in a
-// kernel that walks a list), or -1.
 template <class L>
-__device__ __forceinline__ void brick_setup(const SubArgs& A, int32_t b, Brick& B, L& S, int32_t q_loaded = -1) {
+__device__ __forceinline__ void brick_setup(const SubArgs& A, int32_t b, Brick& B, L& S) {
     const int lane = threadIdx.x;
     B.q = __builtin_amdgcn_readfirstlane(A.bmap[b]);
     const int32_t* R = A.rec + int64_t(B.q) * kRecWords;
     cell_geometry(A, b, kBrickLog, R, B);
-    if (B.q != q_loaded) {
-        for (int w = lane; w < kRecX; w += kWave) {
-            const int32_t v = R[w];
-            if (w < kRecNBK) S.NB[w] = v;
-            else if (w < kRecNBR) S.NBK[w - kRecNBK] = v;
-            else S.NBR[w - kRecNBR] = v;
-        }
-        for (int w = lane; w < 27 * (B.r + 1); w += kWave) S.X[w] = __int_as_float(R[kRecX + w]);
+    for (int w = lane; w < kRecX; w += kWave) {
+        const int32_t v = R[w];
+        if (w < kRecNBK) S.NB[w] = v;
+        else if (w < kRecNBR) S.NBK[w - kRecNBK] = v;
+        else S.NBR[w - kRecNBR] = v;
     }
+    for (int w = lane; w < 27 * (B.r + 1); w += kWave) S.X[w] = __int_as_float(R[kRecX + w]);
     __syncthreads();
     set_kids(B, S);
 }
 
-// The same for a screened cell of 2^k leaves a side.
-__device__ __forceinline__ void cell_setup(const SubArgs& A, int32_t b, int k, Brick& B, CellLds& S, int32_t q_loaded) {
+// Loads a screened cell's part of its root's record into LDS and sets the
+// cell's geometry.  q_loaded: the root whose record S already holds (the
+// previous cell's, in a kernel that walks a list), or -1.
+template <class L>
+__device__ __forceinline__ void cell_setup(const SubArgs& A, int32_t b, int k, Brick& B, L& S, int32_t q_loaded) {
     const int lane = threadIdx.x;
     B.q = __builtin_amdgcn_readfirstlane(A.bmap[b]);
     const int32_t* R = A.rec + int64_t(B.q) * kRecWords;
@@ -1256,123 +1274,19 @@ __device__ __forceinline__ void leaf_cube(const Brick& B, const L& S, const floa
     *emask = m;
 }
 
-// The separable contraction of one depth's coefficients over z and y for
-// the lane's weights: Y[m] = sum_n wy[n] sum_l wz[l] X[m][n][l].
-// contract27: the root's chain at a depth 1..r, whose 27 neighbours all lie
-// around the owners' common ancestor (3 slots per axis, weights (t.x, t.y,
-// t.z)).  contract64: a 4^3 block (cells A - 2 .. A + 1 around the brick's
-// ancestor A) with 4-slot weights.
-__device__ __forceinline__ void contract27(const float* X27, BasisT ty, BasisT tz, float Y[3]) {
-    const float wy[3] = {ty.x, ty.y, ty.z}, wz[3] = {tz.x, tz.y, tz.z};
-    float xv[27];
-#pragma unroll
-    for (int q = 0; q < 27; q++) xv[q] = X27[q];
-#pragma unroll
-    for (int m = 0; m < 3; m++) {
-        float y = 0.0f;
-#pragma unroll
-        for (int n = 0; n < 3; n++) {
-            float z = 0.0f;
-#pragma unroll
-            for (int l = 0; l < 3; l++) z = __builtin_fmaf(xv[9 * m + 3 * n + l], wz[l], z);
-            y = __builtin_fmaf(wy[n], z, y);
-        }
-        Y[m] = y;
-    }
-}
-
-__device__ __forceinline__ void contract64(const float* X64, const float wy[4], const float wz[4], float Y[4]) {
-#pragma unroll
-    for (int m = 0; m < 4; m++) {
-        float xv[16];
-#pragma unroll
-        for (int q = 0; q < 16; q++) xv[q] = X64[16 * m + q];
-        float y = 0.0f;
-#pragma unroll
-        for (int n = 0; n < 4; n++) {
-            float z = 0.0f;
-#pragma unroll
-            for (int l = 0; l < 4; l++) z = __builtin_fmaf(xv[4 * n + l], wz[l], z);
-            y = __builtin_fmaf(wy[n], z, y);
-        }
-        Y[m] = y;
-    }
-}
-
-// An upper bound of A(g) = sum over depths and the owner's 27 neighbours of
-// |x_k b_x b_y b_z| for every corner g of the brick owned inside its root:
-// per depth, the sum of |x| over the depth's block (which holds every
-// owner's 27 neighbours) times the cube of the largest |basis value| among
-// the brick's table entries at that depth.  The float sums of non-negative
-// terms are within 0.1% of their exact values.
-template <class L>
-__device__ __forceinline__ float brick_abs_bound(const Brick& B, L& S, int D) {
-    const int lane = threadIdx.x, P = (1 << B.kb) + 1, dlast = D - B.kb;
-    if (lane <= kMaxDepth) S.tmax[lane] = S.xsum[lane] = 0.0f;
-    __syncthreads();
-    // |basis values| (non-negative floats order as their bit patterns)
-    constexpr int TP = kP;
-    for (int e = lane; e < (D + 1) * 3 * TP; e += kWave) {
-        const int d = e / (3 * TP), i = e % TP;
-        if (i >= P || (d > B.r && S.xb_off[d] < 0)) continue;
-        const BasisT t = S.T[e];
-        const float m = fmaxf(fabsf(t.x), fmaxf(fabsf(t.y), fabsf(t.z)));
-        atomicMax(reinterpret_cast<int*>(&S.tmax[d]), __float_as_int(m));
-    }
-    // |coefficients|: the chain, then the blocks
-    for (int e = lane; e < 27 * B.r; e += kWave) atomicAdd(&S.xsum[1 + e / 27], fabsf(S.X[27 + e]));
-    if (lane == 0) atomicAdd(&S.xsum[0], fabsf(S.X[0]));
-    for (int d = B.r + 1; d <= D; d++) {
-        if (S.xb_off[d] < 0) continue;
-        const int W = d <= dlast ? 4 : block_width(D, B.kb, d), n = W * W * W;
-        float sx = 0.0f;
-        for (int e = lane; e < n; e += kWave) sx += fabsf(S.XB[S.xb_off[d] + e]);
-        if (sx != 0.0f) atomicAdd(&S.xsum[d], sx);
-    }
-    __syncthreads();
-    float bound = 0.0f;
-#pragma unroll
-    for (int d = 0; d <= kMaxDepth; d++) {
-        const float tm = S.tmax[d];
-        if (d <= D) bound += S.xsum[d] * (tm * tm * tm);
-    }
-    return 1.001f * bound;
-}
-
-// The basis weights over the 4 block slots along axis ax for grid coordinate
-// org[ax] + i at depth d <= D - kb: the owner's three values, placed at its
-// ancestor's offset (-1 or 0) from the brick's ancestor.
-template <class L>
-__device__ __forceinline__ void axis_weights4(const Brick& B, const L& S, int D, int d, int ax, int i,
-                                              float w[4]) {
-    const int32_t g = B.org[ax] + i, o = own_cell(g, B.R0[ax]);
-    const int delta = (o >> (D - d)) - (B.org[ax] >> (D - d));
-    const BasisT t = S.T[3 * kP * d + kP * ax + i];
-    if (delta == 0) {
-        w[0] = 0.0f;
-        w[1] = t.x;
-        w[2] = t.y;
-        w[3] = t.z;
-    } else {
-        w[0] = t.x;
-        w[1] = t.y;
-        w[2] = t.z;
-        w[3] = 0.0f;
-    }
-}
-
-// A sign for every corner of the cell that its root owns.  The depths up to
-// the cell's own are one polynomial over the cell: the chain's (restricted
-// from the root's) plus, per depth r + 1 .. D - k, the spline of the block's
-// three cells per axis around the cell's ancestor.  A corner's owner may be a
-// leaf of the cell below along an axis; its 27 neighbours then reach one cell
+// The function over a cell from the depths up to its own (c = D - kb), lane i
+// < 27 returning control value i of its polynomial: the chain's (restricted
+// from the root's) plus, per depth r + 1 .. c, the spline of the block's three
+// cells per axis around the cell's ancestor.  A corner's owner may be a leaf
+// of the cell below along an axis; its 27 neighbours then reach one cell
 // further down and one less up, and the spline of the cell left out is 0
-// there.  Its range lies between the smallest and the largest control value.
-// The depths below the cell's add at most their largest |x| times big[d]
-// each; the float evaluation differs from the spline by at most dev[d] times
-// the largest |x| per depth (depth_bounds, the rounding of all sums
-// included).  The cell is settled when all of that is clear of iso.
-__device__ __forceinline__ int cell_sign(const SubArgs& A, const Brick& B, const CellLds& S) {
+// there.  The corners' float values differ from it by at most *slack: dev[d]
+// times the largest |x| per depth (depth_bounds, the rounding of all sums
+// included).  *finite: false in a lane that saw a coefficient that is not (a
+// maximum passes over NaN; it also makes every control value NaN).
+template <class L>
+__device__ __forceinline__ float cell_polynomial(const SubArgs& A, const Brick& B, const L& S, float* slack,
+                                                 bool* finite) {
     const int D = A.D, lane = threadIdx.x, c = D - B.kb;
     const int l27 = lane < 27 ? lane : 0;
     const int i3[3] = {l27 / 9, (l27 / 3) % 3, l27 % 3};
@@ -1382,9 +1296,32 @@ __device__ __forceinline__ int cell_sign(const SubArgs& A, const Brick& B, const
     for (int a = 0; a < 3; a++)
         bernstein_weights(float(B.org[a] - B.R0[a]) * inv, float(1 << B.kb) * inv, i3[a], w[a]);
     float val = sum27(S.P, 9, 3, w);
+    *slack = __int_as_float(__builtin_amdgcn_readfirstlane(A.rec[int64_t(B.q) * kRecWords + kRecErr]));
+    for (int d = B.r + 1; d <= c; d++) {
+        const int o = S.xb_off[d];  // (uniform)
+        if (o < 0) continue;
+        const float x = fabsf(S.XB[o + lane]);  // 4^3 cells
+        *finite = *finite && x < INFINITY;
+#pragma unroll
+        for (int a = 0; a < 3; a++) spline_weights(B.org[a] >> B.kb, c - d, i3[a], w[a]);
+        val += sum27(S.XB + o + 21, 16, 4, w);  // slots 1..3 along each axis
+        *slack += A.dev[d] * wave_max(x);
+    }
+    *finite = *finite && fabsf(val) < INFINITY;
+    return val;
+}
+
+// A sign for every corner of the cell that its root owns: the polynomial's
+// range lies between the smallest and the largest control value; the depths
+// below the cell's add at most their largest |x| times big[d] each.  The cell
+// is settled when all of that is clear of iso.
+template <class L>
+__device__ __forceinline__ int cell_sign(const SubArgs& A, const Brick& B, const L& S) {
+    const int D = A.D, lane = threadIdx.x, c = D - B.kb;
     bool finite = true;
-    float slack = __int_as_float(__builtin_amdgcn_readfirstlane(A.rec[int64_t(B.q) * kRecWords + kRecErr]));
-    for (int d = B.r + 1; d <= D; d++) {
+    float slack;
+    const float val = cell_polynomial(A, B, S, &slack, &finite);
+    for (int d = c + 1; d <= D; d++) {
         const int o = S.xb_off[d];  // (uniform)
         if (o < 0) continue;
         const int W = block_width(D, B.kb, d), n = W * W * W;
@@ -1394,19 +1331,8 @@ __device__ __forceinline__ int cell_sign(const SubArgs& A, const Brick& B, const
             m = fmaxf(m, x);
             finite = finite && x < INFINITY;
         }
-        m = wave_max(m);
-        if (d <= c) {
-#pragma unroll
-            for (int a = 0; a < 3; a++) spline_weights(B.org[a] >> B.kb, c - d, i3[a], w[a]);
-            val += sum27(S.XB + o + 21, 16, 4, w);  // slots 1..3 along each axis
-            slack += A.dev[d] * m;
-        } else {
-            slack += (A.big[d] + A.dev[d]) * m;
-        }
+        slack += (A.big[d] + A.dev[d]) * wave_max(m);
     }
-    // (a maximum passes over NaN; a coefficient that is not finite makes every
-    // control value NaN, or is one of the deeper depths')
-    finite = finite && fabsf(val) < INFINITY;
     if (__builtin_amdgcn_ballot_w64(!finite) != 0) return 0;
     const float hi = wave_max(val), lo = -wave_max(-val);
     const float iso = *A.iso;
@@ -1440,31 +1366,6 @@ __device__ __forceinline__ uint32_t brick_group_deps(const Brick& B, const L& S,
     return deps;
 }
 
-// Proves, when it can, that every corner value of the brick has one strict
-// sign, so the brick has no crossing edge and no triangle.  For each depth
-// the sum S(g) = sum_k x_k b_x b_y b_z over the corner owner's 27 neighbours
-// is evaluated from the same float coefficients and basis table entries the
-// evaluation reads, as a separable contraction: each lane owns the column of
-// grid points (*, j, k), contracts the depth's coefficients over z and y
-// with its own weights, then over x for the nine points of its column.  At
-// the chain depths 1..r every owner has the root's ancestor, whose 27
-// neighbours are the chain; at depths r+1..D-kb (the whole brick in one cell)
-// the owners' ancestors are that cell or the one below it, which a 4x4x4
-// block covers; at the finer depths, where the brick spans several cells, the
-// owner's 27 terms are read from the brick's block point by point.  The float
-// value the evaluation computes, a sum of n <= 27 (D+1) + 1 products of
-// three roundings each, differs from S(g) by at most (n+3) 2^-24 A(g) with
-// A(g) = sum_k |x_k b_x b_y b_z| (recursive summation bound); the
-// contraction's own rounding adds less than 60 2^-24 A(g).  A(g) is bounded
-// for the whole brick by brick_abs_bound.  The brick is certified when
-// |S(g) - iso| exceeds 560 2^-24 times that bound (plus the rounding of the
-// subtraction) with one sign at every corner its root owns.  A corner on the
-// root's boundary may be owned by a leaf of another root of the group: its
-// value is the one that root's brick holding the owner computes for its own
-// corner (the same owner, table entries and order), so the sign is compared
-// with that brick's afterwards (k_group_check).  Returns +1 or -1 (every
-// corner the brick's root owns has this sign) or 0 (not proven).
-
 // Whether the brick touches a face, edge or corner its root shares with
 // another root of the group (whose leaves may own corners of the brick).
 template <class L>
@@ -1487,77 +1388,109 @@ __device__ __forceinline__ bool brick_in_group(const Brick& B, const L& S) {
     return group;
 }
 
-template <class L>
-__device__ __forceinline__ int brick_certify(const SubArgs& A, const Brick& B, L& S, bool group) {
-    const int D = A.D, kb = B.kb, P = (1 << kb) + 1;
-    const int lane = threadIdx.x;
+// Proves, when it can, that every corner value of the 8^3 brick has one strict
+// sign, so the brick has no crossing edge and no triangle.  Each lane owns the
+// column of grid points (*, j, k).  The depths up to D - 3, whose cell holds
+// the whole brick, are one polynomial (cell_polynomial), contracted over z and
+// y to three values per column and then evaluated at its nine points.  At the
+// three finer depths d, where the brick spans several cells, the sum
+// S(g) = sum_k x_k b_x b_y b_z over the corner owner's 27 neighbours is formed
+// from the same float coefficients and basis table entries the evaluation
+// reads, contracted over z and y per x slot of the block and added to the
+// points whose owners see the slot.  The float value the evaluation computes,
+// a sum of n <= 27 (D + 1) + 1 products of three roundings each, differs from
+// S(g) by at most (n + 3) 2^-24 A(g) with A(g) = sum_k |x_k b_x b_y b_z|
+// (recursive summation bound); the contraction's own rounding adds less than
+// 60 2^-24 A(g), and A(g) is at most the block's sum of |x| times the cube of
+// the largest |basis value| among the entries: 560 2^-24 of that covers both
+// (float sums of non-negative terms are within 0.1%).  The polynomial's share
+// of the distance is cell_polynomial's slack, its evaluation here less than 40
+// roundings of its largest control value.  The brick is certified when the
+// distance to iso exceeds all of it with one sign at every corner its root
+// owns.  A corner on the root's boundary may be owned by a leaf of another
+// root of the group: its value is the one that root's brick holding the owner
+// computes for its own corner (the same owner, table entries and order), so
+// the sign is compared with that brick's afterwards (k_group_check).  Returns
+// +1 or -1 (every corner the brick's root owns has this sign) or 0 (not
+// proven).  Depth by depth over the columns, all from the tables, this took
+// 33 ns a brick; the list was half as long again.
+__device__ __forceinline__ int brick_certify(const SubArgs& A, const Brick& B, const CertLds& S, bool group) {
+    const int D = A.D, lane = threadIdx.x, c = D - kBrickLog;
     const float iso = *A.iso;
-    const int dlast = D - kb;  // deepest depth whose cell holds the whole brick
-    const float marginA = 560.0f * 5.9604645e-8f * brick_abs_bound(B, S, D) + 1e-15f;
+    bool finite = true;
+    float slack;
+    const float val = cell_polynomial(A, B, S, &slack, &finite);
+    float fine = 0.0f;
+    for (int d = c + 1; d <= D; d++) {
+        const int o = S.xb_off[d];  // (uniform)
+        if (o < 0) continue;
+        const int W = block_width(D, kBrickLog, d), n = W * W * W;
+        float sx = 0.0f;
+        for (int e = lane; e < n; e += kWave) sx += fabsf(S.XB[o + e]);
+#pragma unroll
+        for (int h = 32; h > 0; h >>= 1) sx += __shfl_xor(sx, h, kWave);
+        const BasisT t = S.T[3 * kP * (d - c - 1) + (lane < 3 * kP ? lane : 0)];
+        const float tm = wave_max(fmaxf(fabsf(t.x), fmaxf(fabsf(t.y), fabsf(t.z))));
+        fine += sx * (tm * tm * tm);
+    }
+    finite = finite && fine < INFINITY;
+    if (__builtin_amdgcn_ballot_w64(!finite) != 0) return 0;
+    const float margin0 = 1.001f * slack + 1.001f * (560.0f * 5.9604645e-8f) * fine +
+                          2.4e-6f * wave_max(fabsf(val)) + 1e-15f;
+    float Q[27];  // the control values, uniform
+#pragma unroll
+    for (int q = 0; q < 27; q++) Q[q] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(val), q));
     bool ok = true, pos = false, neg = false;
     for (int pp = lane; pp < kP * kP; pp += kWave) {
         const int j = pp % kP, k = pp / kP;
-        if (j >= P || k >= P) continue;
+        const float tj = float(j) * 0.125f, tk = float(k) * 0.125f;
+        const float wj[3] = {(1.0f - tj) * (1.0f - tj), 2.0f * tj * (1.0f - tj), tj * tj};
+        const float wk[3] = {(1.0f - tk) * (1.0f - tk), 2.0f * tk * (1.0f - tk), tk * tk};
+        float Y[3];
+#pragma unroll
+        for (int m = 0; m < 3; m++) {
+            float y = 0.0f;
+#pragma unroll
+            for (int n = 0; n < 3; n++) {
+                float z = 0.0f;
+#pragma unroll
+                for (int l = 0; l < 3; l++) z = __builtin_fmaf(Q[9 * m + 3 * n + l], wk[l], z);
+                y = __builtin_fmaf(wj[n], z, y);
+            }
+            Y[m] = y;
+        }
         float v[kP];
 #pragma unroll
-        for (int i = 0; i < kP; i++) v[i] = 0.0f;
-        // (points i >= P of a smaller brick are accumulated from unset table
-        // entries and never checked)
-        {  // depth 0: the tree's root, one coefficient
-            const float y = (S.X[0] * S.T[2 * kP + k].y) * S.T[kP + j].y;
-#pragma unroll
-            for (int i = 0; i < kP; i++) v[i] = __builtin_fmaf(S.T[i].y, y, v[i]);
-        }
-        for (int d = 1; d <= B.r; d++) {  // the chain: all owners share their ancestor
-            float Y[3];
-            contract27(S.X + 27 * d, S.T[3 * kP * d + kP + j], S.T[3 * kP * d + 2 * kP + k], Y);
-#pragma unroll
-            for (int i = 0; i < kP; i++) {
-                const BasisT t = S.T[3 * kP * d + i];
-                v[i] = __builtin_fmaf(t.x, Y[0], v[i]);
-                v[i] = __builtin_fmaf(t.y, Y[1], v[i]);
-                v[i] = __builtin_fmaf(t.z, Y[2], v[i]);
-            }
-        }
-        for (int d = B.r + 1; d <= dlast; d++) {  // 4^3 blocks of real nodes
-            if (S.xb_off[d] < 0) continue;
-            float w1[4], w2[4], Y[4];
-            axis_weights4(B, S, D, d, 1, j, w1);
-            axis_weights4(B, S, D, d, 2, k, w2);
-            contract64(S.XB + S.xb_off[d], w1, w2, Y);
-#pragma unroll
-            for (int i = 0; i < kP; i++) {
-                float w0[4];
-                axis_weights4(B, S, D, d, 0, i, w0);
-#pragma unroll
-                for (int m = 0; m < 4; m++) v[i] = __builtin_fmaf(w0[m], Y[m], v[i]);
-            }
+        for (int i = 0; i < kP; i++) {
+            const float t = float(i) * 0.125f;  // (constants: i is unrolled)
+            v[i] = __builtin_fmaf(t * t, Y[2], __builtin_fmaf(2.0f * t * (1.0f - t), Y[1], (1.0f - t) * (1.0f - t) * Y[0]));
         }
         // the finer depths, where the brick spans several cells: per x slot m
         // of the block, Y_m = sum over the lane's 3 y and 3 z slots, then
         // each point adds its owner's three x slots' Y (the slots a point's
         // owner sees follow from grid coordinates alone: uniform per i)
-        for (int d = dlast + 1; d <= D; d++) {
+        for (int d = c + 1; d <= D; d++) {
             const int slot = S.xb_off[d];
             if (slot < 0) continue;
-            const int sh = D - d, W = block_width(D, kb, d);
+            const int sh = D - d, W = block_width(D, kBrickLog, d);
+            const BasisT* T = S.T + 3 * kP * (d - c - 1);
             const int b1 = (own_cell(B.org[1] + j, B.R0[1]) >> sh) - 1 - ((B.org[1] >> sh) - 2);
             const int b2 = (own_cell(B.org[2] + k, B.R0[2]) >> sh) - 1 - ((B.org[2] >> sh) - 2);
-            const BasisT ty = S.T[3 * kP * d + kP + j], tz = S.T[3 * kP * d + 2 * kP + k];
+            const BasisT ty = T[kP + j], tz = T[2 * kP + k];
             const float by[3] = {ty.x, ty.y, ty.z}, bz[3] = {tz.x, tz.y, tz.z};
             int b0[kP];
             float bx[kP][3];
 #pragma unroll
             for (int i = 0; i < kP; i++) {
                 b0[i] = (own_cell(B.org[0] + i, B.R0[0]) >> sh) - 1 - ((B.org[0] >> sh) - 2);
-                const BasisT tx = S.T[3 * kP * d + i];
+                const BasisT tx = T[i];
                 bx[i][0] = tx.x;
                 bx[i][1] = tx.y;
                 bx[i][2] = tx.z;
             }
 #pragma unroll
             for (int m = 0; m < 11; m++) {  // W <= 11
-                if (m >= W || m < b0[0] || m > b0[P - 1] + 2) continue;  // (uniform) a slot no point sees
+                if (m >= W || m < b0[0] || m > b0[kP - 1] + 2) continue;  // (uniform) a slot no point sees
                 const float* Xm = S.XB + slot + m * W * W;
                 float y = 0.0f;
 #pragma unroll
@@ -1570,7 +1503,7 @@ __device__ __forceinline__ int brick_certify(const SubArgs& A, const Brick& B, L
 #pragma unroll
                 for (int i = 0; i < kP; i++) {
                     const int q = m - b0[i];  // uniform
-                    if (i < P && q >= 0 && q <= 2) v[i] = __builtin_fmaf(q == 0 ? bx[i][0] : q == 1 ? bx[i][1] : bx[i][2], y, v[i]);
+                    if (q >= 0 && q <= 2) v[i] = __builtin_fmaf(q == 0 ? bx[i][0] : q == 1 ? bx[i][1] : bx[i][2], y, v[i]);
                 }
             }
         }
@@ -1578,7 +1511,6 @@ __device__ __forceinline__ int brick_certify(const SubArgs& A, const Brick& B, L
                               B.org[2] + k < B.R0[2] + B.Sr;
 #pragma unroll
         for (int i = 0; i < kP; i++) {
-            if (i >= P) continue;
             const int32_t gx = B.org[0] + i;
             if (group && !(jk_inner && gx > B.R0[0] && gx < B.R0[0] + B.Sr)) {
                 // on the root's boundary: is the owner a leaf of another root?
@@ -1586,11 +1518,11 @@ __device__ __forceinline__ int brick_certify(const SubArgs& A, const Brick& B, L
                 int32_t o[3];
                 if (corner_owner(B, S, D, g, o) != 13) continue;
             }
-            const float val = v[i] - iso;
-            const float margin = marginA + 1.2e-7f * (fabsf(v[i]) + fabsf(iso));
-            ok = ok && fabsf(val) > margin;
-            pos = pos || val > 0;
-            neg = neg || val < 0;
+            const float dist = v[i] - iso;
+            const float margin = margin0 + 1.2e-7f * (fabsf(v[i]) + fabsf(iso));
+            ok = ok && fabsf(dist) > margin;
+            pos = pos || dist > 0;
+            neg = neg || dist < 0;
         }
     }
     const bool lane_good = ok && !(pos && neg);
@@ -1627,10 +1559,11 @@ __global__ void __launch_bounds__(kBlockS) k_list_roots(const int32_t* roots, co
 // surface and settles in large cells: the 1,036,945 bricks of 2 M points at
 // depth 10 took 1.85 ms as 122,256 cells of 16^3 and then 238,786 bricks, each
 // bounded by intervals depth by depth.
-__global__ void __launch_bounds__(kWave, 5) k_cell_screen(SubArgs A, int k, const int32_t* list, int32_t* parts,
+template <int FLOATS>
+__global__ void __launch_bounds__(kWave, FLOATS > kXBlkScreen ? 3 : 5) k_cell_screen(SubArgs A, int k, const int32_t* list, int32_t* parts,
                                                        int32_t* xlist, int8_t* sign, int32_t* glist, int32_t* cnt,
                                                        int certify) {
-    __shared__ CellLds S;
+    __shared__ CellLds<FLOATS> S;
     const int lane = threadIdx.x;
     const int32_t n = cnt[kCntCells + k];
     // up to 16 entries, at least about four grabs per workgroup
@@ -1699,11 +1632,9 @@ __global__ void __launch_bounds__(kWave, 5) k_cell_screen(SubArgs A, int k, cons
 // screen left; the bricks it does not settle are listed for the evaluation.
 // A resident grid takes chunks of consecutive entries from a counter; entries
 // of one root often follow each other, and its record then stays in LDS.
-// Compiled for three waves per SIMD (168 VGPRs, a few spilled): the waves wait
-// on memory about half their time, and two per SIMD hid less.
 __global__ void __launch_bounds__(kWave, 3) k_brick_exact(SubArgs A, const int32_t* xlist, int8_t* sign, int32_t* list,
                                                        int32_t* glist, int32_t* cnt, int certify) {
-    __shared__ BrickCore S;
+    __shared__ CertLds S;
     const int lane = threadIdx.x;
     const int32_t n = cnt[kCntExact];
     // chunks of up to 8 entries, at least about four per workgroup
@@ -1721,12 +1652,20 @@ __global__ void __launch_bounds__(kWave, 3) k_brick_exact(SubArgs A, const int32
         const int32_t b = xlist[it++];
         Brick B;
         __syncthreads();  // the previous brick's LDS reads are done
-        brick_setup(A, b, B, S, q_loaded);
+        cell_setup(A, b, kBrickLog, B, S, q_loaded);
         q_loaded = B.q;
-        brick_tables(A, B, S);
-        brick_blocks(A, B, S);
+        if (lane < kBrickLog * kP) {
+            const int d = A.D - kBrickLog + 1 + lane / kP, i = lane % kP;
+#pragma unroll
+            for (int ax = 0; ax < 3; ax++) {
+                const int32_t g = B.org[ax] + i, o = own_cell(g, B.R0[ax]);
+                const float4 t = A.btab[((int64_t(d) << A.D) + o) * 2 + (g - o)];
+                S.T[3 * kP * (lane / kP) + kP * ax + i] = BasisT{t.x, t.y, t.z};
+            }
+        }
+        const bool fits = brick_blocks(A, B, S);
         const bool group = brick_in_group(B, S);
-        const int s = certify ? brick_certify(A, B, S, group) : 0;
+        const int s = certify && fits ? brick_certify(A, B, S, group) : 0;
         if (lane == 0) {
             sign[b] = int8_t(s);
             if (s == 0) list[atomicAdd(cnt + kCntDense, 1)] = b;
@@ -2479,7 +2418,7 @@ void extract_subdivision(prg_ctx* c) {
     bmap.reserve(size_t(nb));
     A.rec = rec.get();
     A.bmap = bmap.get();
-    k_root_records<<<unsigned(nr), kWave, 0, s>>>(A, rec.get());
+    k_root_records<<<unsigned((nr + 1) / 2), kWave, 0, s>>>(A, int32_t(nr), rec.get());
     PRG_CHECK_LAUNCH();
     k_brick_map<<<grid_for(nb, kBlockS), kBlockS, 0, s>>>(boff.get(), C, nb, bmap.get());
     PRG_CHECK_LAUNCH();
@@ -2565,7 +2504,8 @@ void extract_subdivision(prg_ctx* c) {
         int kmax = D - 1;
         while (kmax > kBrickLog && (int64_t(1) << (3 * (kmax - kBrickLog))) > nb3) kmax--;
         for (int k = kmax; k >= kBrickLog; k--) {
-            k_cell_screen<<<resident(reinterpret_cast<const void*>(k_cell_screen), (nb3 >> (3 * (k - kBrickLog))) + 1),
+            const auto screen = k == kBrickLog ? k_cell_screen<kXBlkScreenBrick> : k_cell_screen<kXBlkScreen>;
+            screen<<<resident(reinterpret_cast<const void*>(screen), (nb3 >> (3 * (k - kBrickLog))) + 1),
                             kWave, 0, s>>>(A, k, lists.at[k], k > kBrickLog ? lists.at[k - 1] : nullptr, xlist.get(),
                                            bsign.get(), glist.get(), C, int(c->sub_certify));
             PRG_CHECK_LAUNCH();
