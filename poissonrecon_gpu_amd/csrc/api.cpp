@@ -476,7 +476,8 @@ static prg_status weld_checked(prg_ctx* c, prg_mesh* mesh, int64_t* n_merged, bo
         if (n >= (int64_t(1) << 31)) return fail(c, PRG_E_ARG, "more than 2^31 - 1 vertices");
         if (noalloc && (n > PRG_WELD_NOALLOC_MAX_VERTICES || m > PRG_WELD_NOALLOC_MAX_TRIANGLES))
             return fail(c, PRG_E_ARG, "mesh larger than the fixed weld array (PRG_WELD_NOALLOC_MAX_*)");
-        for (int64_t i = 0; i < 3 * m; i++)
+        // (with more vertices the weld itself finds an index out of range)
+        for (int64_t i = 0; n <= 1 && i < 3 * m; i++)
             if (mesh->triangles[i] < 0 || mesh->triangles[i] >= n)
                 return fail(c, PRG_E_ARG, "triangle index out of range");
         PRG_HIP(hipSetDevice(c->cfg.device));

@@ -25,6 +25,7 @@ constexpr size_t kCgHostLevels = kCgHostBytes - 64;
 constexpr size_t kCgHostMesh = kCgHostBytes - 16;
 constexpr size_t kCgHostTopo = kCgHostBytes - 4;
 static_assert(kCgHostLevels + 4 * (kMaxDepth + 1) <= kCgHostMesh, "counts overlap");
+constexpr int kWeldHost = 56;  // the weld's three counts in sub_host (behind the subdivision's counters)
 
 // ---- errors ------------------------------------------------------------------
 struct Error {
