@@ -844,19 +844,18 @@ __device__ __forceinline__ void set_kids(Brick& B, const L& S) {
 
 // Loads the root record of brick b (8^3 leaves) into LDS (its neighbours and
 // its chain's values) and sets the brick's geometry.
-template <class L>
+template <int kThreads, class L>
 __device__ __forceinline__ void brick_setup(const SubArgs& A, int32_t b, Brick& B, L& S) {
-    const int lane = threadIdx.x;
     B.q = __builtin_amdgcn_readfirstlane(A.bmap[b]);
     const int32_t* R = A.rec + int64_t(B.q) * kRecWords;
     cell_geometry(A, b, kBrickLog, R, B);
-    for (int w = lane; w < kRecX; w += kWave) {
+    for (int w = threadIdx.x; w < kRecX; w += kThreads) {
         const int32_t v = R[w];
         if (w < kRecNBK) S.NB[w] = v;
         else if (w < kRecNBR) S.NBK[w - kRecNBK] = v;
         else S.NBR[w - kRecNBR] = v;
     }
-    for (int w = lane; w < 27 * (B.r + 1); w += kWave) S.X[w] = __int_as_float(R[kRecX + w]);
+    for (int w = threadIdx.x; w < 27 * (B.r + 1); w += kThreads) S.X[w] = __int_as_float(R[kRecX + w]);
     __syncthreads();
     set_kids(B, S);
 }
@@ -910,11 +909,11 @@ __device__ __forceinline__ int32_t own_cell(int32_t g, int32_t R0) { return g ==
 // The smallest-key leaf around a grid point, when it is a leaf of the
 // brick's own root, is own_cell along every axis, so every corner the
 // brick's root owns reads its three basis values per depth from S.T.
-template <class L>
+template <int kThreads, class L>
 __device__ __forceinline__ void brick_tables(const SubArgs& A, const Brick& B, L& S) {
     const int D = A.D, P = (1 << B.kb) + 1;
     constexpr int TP = kP;
-    for (int e = threadIdx.x; e < (D + 1) * TP; e += kWave) {
+    for (int e = threadIdx.x; e < (D + 1) * TP; e += kThreads) {
         const int d = e / TP, i = e % TP;
         if (i >= P) continue;
 #pragma unroll
@@ -924,6 +923,13 @@ __device__ __forceinline__ void brick_tables(const SubArgs& A, const Brick& B, L
             S.T[3 * TP * d + TP * ax + i] = BasisT{t.x, t.y, t.z};
         }
     }
+}
+
+// Whether v holds in any thread of the workgroup.
+template <int kThreads>
+__device__ __forceinline__ bool any_thread(bool v) {
+    if (kThreads == kWave) return __builtin_amdgcn_ballot_w64(v) != 0;
+    return __syncthreads_or(v) != 0;
 }
 
 // Fills the brick's blocks (depths r+1..D), level by level: each cell's
@@ -936,7 +942,8 @@ __device__ __forceinline__ void brick_tables(const SubArgs& A, const Brick& B, L
 // LDS (109,000 of 160,000 bricks missed the interval screen for those alone).
 // A depth whose block holds no nonzero coefficient gets none.  Returns false
 // when the caller's LDS cannot hold the blocks.
-template <class L>
+// (kThreads: of the workgroup, all of which take part.)
+template <int kThreads = kWave, class L>
 __device__ __forceinline__ bool brick_blocks(const SubArgs& A, const Brick& B, L& S) {
     constexpr int kCap = int(sizeof(S.XB) / sizeof(float));
     constexpr int kCapC[2] = {int(sizeof(S.CB0) / sizeof(int32_t)), int(sizeof(S.CB1) / sizeof(int32_t))};
@@ -959,7 +966,7 @@ __device__ __forceinline__ bool brick_blocks(const SubArgs& A, const Brick& B, L
         const int Wp = dd > B.r + 1 ? block_width(D, B.kb, dd - 1) : 0;
         const int32_t plo[3] = {(B.org[0] >> (sh + 1)) - 2, (B.org[1] >> (sh + 1)) - 2, (B.org[2] >> (sh + 1)) - 2};
         bool kids = false, nz = false;
-        for (int e = lane; e < n; e += kWave) {
+        for (int e = lane; e < n; e += kThreads) {
             // l / W and l / W^2 for l < W^3 <= 1331 by a 16-bit reciprocal (exact: l / W
             // has a fractional part of at most (W-1)/W, the reciprocal's excess adds < 0.03)
             const int q1 = int((uint32_t(e) * rw) >> 16), q2 = int((uint32_t(q1) * rw) >> 16);
@@ -985,8 +992,8 @@ __device__ __forceinline__ bool brick_blocks(const SubArgs& A, const Brick& B, L
             nz = nz || xv != 0.0f;
             kids = kids || ck >= 0;
         }
-        const bool any = __builtin_amdgcn_ballot_w64(nz) != 0;
-        on = __builtin_amdgcn_ballot_w64(kids) != 0;
+        const bool any = any_thread<kThreads>(nz);
+        on = any_thread<kThreads>(kids);
         if (any && lane == 0) S.xb_off[dd] = total;
         total += n;
         __syncthreads();  // this depth's child bases are read by the next
@@ -1201,8 +1208,6 @@ __device__ __forceinline__ float grid_value(const SubArgs& A, const Brick& B, co
     tt = tt * b0z;
     return f + tt - *A.iso;
 }
-
-constexpr int kValRounds = (kBrickPts + kWave - 1) / kWave;
 
 // Owner of edge e of leaf v among the virtual leaves sharing it
 // (initSubdivideEdgeArray, main.cu:1867-2019): its cell and the edge kind seen
@@ -1675,22 +1680,25 @@ __global__ void __launch_bounds__(kWave, 3) k_brick_exact(SubArgs A, const int32
 }
 
 // The corner values of the bricks the certificates left (grid_value): gv at
-// kBrickPts per listed brick.  `slices` waves share a brick's rounds of 64
-// points (each sets up the brick's tables and blocks itself): a list shorter
-// than the chip's waves leaves each of them a part of a brick's serial chain
-// of loads and sums instead of all of it (921 bricks, 35,947 points at depth
-// 8: 401 us one wave per brick).
-__global__ void __launch_bounds__(kWave) k_brick_values(SubArgs A, const int32_t* list, int slices, float* gv) {
+// kBrickPts per listed brick.  A value is a serial chain of LDS reads and
+// sums, so what counts is the waves in flight; a brick's tables and blocks are
+// 16 KB of LDS, which held them to 2.5 per SIMD as one wave per brick (532 us
+// for 3,338 bricks; 250 us with four).  `slices` workgroups share the rounds
+// of a brick (each sets up its own tables and blocks): a list shorter than the
+// chip leaves each of them one round instead of all three.
+constexpr int kValThreads = 256;
+constexpr int kValRounds = (kBrickPts + kValThreads - 1) / kValThreads;
+__global__ void __launch_bounds__(kValThreads, 5) k_brick_values(SubArgs A, const int32_t* list, int slices, float* gv) {
     __shared__ BrickCore S;
     const int32_t it = int32_t(blockIdx.x) / slices;
-    const int slice = int(blockIdx.x) % slices, per = (kValRounds + slices - 1) / slices;
+    const int per = kValRounds / slices, first = (int(blockIdx.x) % slices) * per;
     Brick B;
-    brick_setup(A, list[it], B, S);
-    brick_tables(A, B, S);
-    brick_blocks(A, B, S);
+    brick_setup<kValThreads>(A, list[it], B, S);
+    brick_tables<kValThreads>(A, B, S);
+    brick_blocks<kValThreads>(A, B, S);
     float* out = gv + int64_t(it) * kBrickPts;
-    for (int t = slice * per; t < std::min(kValRounds, slice * per + per); t++) {
-        const int p = threadIdx.x + kWave * t;
+    for (int t = first; t < first + per; t++) {
+        const int p = threadIdx.x + kValThreads * t;
         if (p >= kBrickPts) break;
         const int32_t g[3] = {B.org[0] + p % kP, B.org[1] + (p / kP) % kP, B.org[2] + p / (kP * kP)};
         out[p] = grid_value(A, B, S, g);
@@ -2532,14 +2540,9 @@ void extract_subdivision(prg_ctx* c) {
         T3.emask = emask_tab.reserve(size_t(ndense) * kBrickLeaves);
         T3.cube = cube_tab.reserve(size_t(ndense) * kBrickLeaves);
         TimedScope ts(kt, "subdivide_count", 0.0);
-        int per_cu = 0;
-        PRG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_brick_values, kWave, 0));
-        const int64_t resident = int64_t(std::max(1, per_cu)) * std::max(1, c->num_cu);
-        // about two resident grids of waves, in whole rounds
-        int slices = int(std::min<int64_t>(kValRounds, std::max<int64_t>(1, 2 * resident / ndense)));
-        while (kValRounds % slices) slices--;
-        if (ndense * slices >= (int64_t(1) << 31)) throw Error{PRG_E_NOMEM, "too many bricks to evaluate"};
-        k_brick_values<<<unsigned(ndense * slices), kWave, 0, s>>>(A, dlist.get(), slices, gvals.get());
+        // one workgroup per round while that fills no more than the chip
+        const int slices = ndense * kValRounds <= 4 * std::max(1, c->num_cu) ? kValRounds : 1;
+        k_brick_values<<<unsigned(ndense * slices), kValThreads, 0, s>>>(A, dlist.get(), slices, gvals.get());
         PRG_CHECK_LAUNCH();
         k_brick_cubes<<<unsigned(ndense), kBrickLeaves, 0, s>>>(A, dlist.get(), gvals.get(), T3, bnv.get(), bnt.get(),
                                                                 didx.get());
