@@ -348,6 +348,7 @@ static void build_mesh(prg_ctx* c, int32_t subdivide, prg_mesh* out) {
     PRG_HIP(hipSetDevice(c->cfg.device));
     prg::extract_leaf_mesh(c);
     c->sub_nv = c->sub_nt = 0;
+    c->sub_v_copied = false;
     if (subdivide) prg::extract_subdivision(c);
     std::memset(out, 0, sizeof(*out));
     resolve_transform(c);
@@ -367,7 +368,7 @@ static void copy_mesh(prg_ctx* c, float* vertices, int32_t* triangles) {
         if (c->mesh_nv) d2h(c, vertices, c->mesh_v.get(), size_t(3 * c->mesh_nv) * 4);
         if (c->mesh_nt) d2h(c, triangles, c->mesh_t.get(), size_t(3 * c->mesh_nt) * 4);
     }
-    if (c->sub_nv) d2h(c, vertices + 3 * c->mesh_nv, c->sub_v.get(), size_t(3 * c->sub_nv) * 4);
+    if (c->sub_nv && !c->sub_v_copied) d2h(c, vertices + 3 * c->mesh_nv, c->sub_v.get(), size_t(3 * c->sub_nv) * 4);
     if (c->sub_nt) d2h(c, triangles + 3 * c->mesh_nt, c->sub_t.get(), size_t(3 * c->sub_nt) * 4);
     if (c->out_copied && c->out_async) PRG_HIP(hipStreamWaitEvent(c->stream, c->mesh_ev, 0));
     PRG_HIP(hipStreamSynchronize(c->stream));

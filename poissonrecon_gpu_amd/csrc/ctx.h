@@ -96,6 +96,7 @@ struct prg_ctx {
     // stream behind mesh_ev while the subdivision runs (mesh_ev2 orders them
     // after the triangle emission)
     bool out_async = false;
+    bool sub_v_copied = false;  // the subdivision's vertices are on their way too (mesh_ev)
     hipEvent_t mesh_ev = nullptr;
     hipEvent_t mesh_ev2 = nullptr;
     bool topo_pending = false;

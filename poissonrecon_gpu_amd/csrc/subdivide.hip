@@ -2306,6 +2306,7 @@ void extract_subdivision(prg_ctx* c) {
     KernelTimer& kt = c->kt;
     const Levels Lv = levels_of(c);
     c->sub_nv = c->sub_nt = 0;
+    c->sub_v_copied = false;
     c->sub_roots = c->sub_leaves = 0;
     c->sub_bricks = c->sub_exact = c->sub_evaluated = 0;
     if (baseD <= 1) return;
@@ -2578,6 +2579,11 @@ void extract_subdivision(prg_ctx* c) {
             PRG_CHECK_LAUNCH();
         }
     }
+    // into the caller's buffers, when they hold the whole mesh, the vertices go
+    // on the second stream while the triangles are emitted
+    const bool direct = c->out_copied && c->out_async && 3 * (c->mesh_nv + snv) <= c->out_vcap &&
+                        3 * (c->mesh_nt + snt) <= c->out_tcap && snv > 0;
+    if (direct) PRG_HIP(hipEventRecord(c->mesh_ev2, s));
     {
         TimedScope ts(kt, "subdivide_triangles", 12.0 * double(snt));
         if (n1) {
@@ -2596,6 +2602,12 @@ void extract_subdivision(prg_ctx* c) {
                                                                         H + kCntErr);
             PRG_CHECK_LAUNCH();
         }
+    }
+    if (direct) {
+        PRG_HIP(hipStreamWaitEvent(c->stream2, c->mesh_ev2, 0));
+        PRG_HIP(hipMemcpyAsync(c->out_v + 3 * c->mesh_nv, SV, size_t(3 * snv) * 4, hipMemcpyDeviceToHost, c->stream2));
+        PRG_HIP(hipEventRecord(c->mesh_ev, c->stream2));
+        c->sub_v_copied = true;
     }
     PRG_HIP(hipStreamSynchronize(s));
     if (H[kCntErr]) throw Error{PRG_E_HIP, "subdivision: a triangle edge has no owner vertex"};
