@@ -429,7 +429,8 @@ __global__ void __launch_bounds__(kT, RX * RY > 1 ? (MULTI ? 2 : 4) : (MULTI ? 3
 // replaced by zeros.  The channel strides are 4 words past a multiple of 32
 // (no bank conflict beyond the two cycles a half-wave's 256 bytes need).
 // What bounds it is the staging (each element is read for 3 dx and per tile
-// of the other operand), not the matrix cores.  One wave per (chunk, tap,
+// of the other operand), not the matrix cores; a stage's loads are in flight
+// during the products of the one before.  One wave per (chunk, tap,
 // tiles) with scalar loads straight from memory and 64-bit divisions per
 // element took 440 us for 16 -> 16 channels on 64^3 and 990 us for 48 -> 16.
 constexpr int kWStage = 512;  // voxels per stage
@@ -470,56 +471,70 @@ __global__ void __launch_bounds__(192) k_wgrad_rows(ConvIn src, const float* __r
 #pragma unroll
     for (int z = 0; z < 3; z++) acc[z] = f4{0.0f, 0.0f, 0.0f, 0.0f};
     const int v0 = ch * kWChunk, v1 = v0 + kWChunk < V ? v0 + kWChunk : V;
+    // a stage's loads: pairs of voxels along z, four channels each
+    constexpr int NI = (ROWS * G * 2 + 191) / 192, NG = (kWStage * 2 + 191) / 192;
+    float4 ia[NI], ib[NI], ga[NG], gb[NG];
+    const int zstep = lo ? 0 : sc;  // to the second voxel (upsampled: the same)
+    auto load_stage = [&](int vs) {
+        const int row0 = vs >> LG;  // first row (x G + y) of the stage
+#pragma unroll
+        for (int k = 0; k < NI; k++) {
+            const int t = tid + k * 192, cq = t & 3, zp = (t >> 2) & (G / 2 - 1), r = t >> (LG + 1);
+            const int row = row0 - 1 + r, x = (row >> LG) + dx, y = row & (G - 1);
+            ia[k] = ib[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (r < ROWS && row >= 0 && row < G * G && x >= 0 && x < G) {
+                const int vox = lo ? (((x >> 1) << (LG - 1)) + (y >> 1)) * (G / 2) + zp : ((x << LG) + y) * G + 2 * zp;
+                const float* q = sp + int64_t(vox) * sc + 4 * cq;
+                ia[k] = *reinterpret_cast<const float4*>(q);
+                ib[k] = *reinterpret_cast<const float4*>(q + zstep);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < NG; k++) {
+            const int t = tid + k * 192, cq = t & 3, vp = t >> 2;
+            const float* q = gp + int64_t(vs + 2 * (vp < kWStage / 2 ? vp : 0)) * cout + 4 * cq;
+            ga[k] = *reinterpret_cast<const float4*>(q);
+            gb[k] = *reinterpret_cast<const float4*>(q + cout);
+        }
+    };
+    load_stage(v0);
     for (int vs = v0; vs < v1; vs += kWStage) {
         __syncthreads();  // the previous stage's reads
-        const int row0 = vs >> LG;  // first row (x G + y) of the stage
-#pragma unroll 4
-        for (int t = tid; t < ROWS * G * 2; t += 192) {
-            const int cq = t & 3, zp = (t >> 2) & (G / 2 - 1), r = t >> (LG + 1);
-            const int row = row0 - 1 + r, x = (row >> LG) + dx, y = row & (G - 1);
-            float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f), c = a;
-            if (row >= 0 && row < G * G && x >= 0 && x < G) {
-                if (lo) {
-                    a = *reinterpret_cast<const float4*>(
-                        sp + int64_t((((x >> 1) << (LG - 1)) + (y >> 1)) * (G / 2) + zp) * sc + 4 * cq);
-                    c = a;
-                } else {
-                    const float* q = sp + int64_t(((x << LG) + y) * G + 2 * zp) * sc + 4 * cq;
-                    a = *reinterpret_cast<const float4*>(q);
-                    c = *reinterpret_cast<const float4*>(q + sc);
-                }
-            }
+        const int row0 = vs >> LG;
+#pragma unroll
+        for (int k = 0; k < NI; k++) {
+            const int t = tid + k * 192, cq = t & 3, zp = (t >> 2) & (G / 2 - 1), r = t >> (LG + 1);
+            if (r >= ROWS) continue;
             uint32_t* d = si + 4 * cq * CW + r * (RS / 2) + 2 + zp;
-            d[0] = bf2(a.x, c.x);
-            d[CW] = bf2(a.y, c.y);
-            d[2 * CW] = bf2(a.z, c.z);
-            d[3 * CW] = bf2(a.w, c.w);
+            d[0] = bf2(ia[k].x, ib[k].x);
+            d[CW] = bf2(ia[k].y, ib[k].y);
+            d[2 * CW] = bf2(ia[k].z, ib[k].z);
+            d[3 * CW] = bf2(ia[k].w, ib[k].w);
         }
-#pragma unroll 4
-        for (int t = tid; t < kWStage * 2; t += 192) {
-            const int cq = t & 3, vp = t >> 2;
-            const float* q = gp + int64_t(vs + 2 * vp) * cout + 4 * cq;
-            const float4 a = *reinterpret_cast<const float4*>(q);
-            const float4 c = *reinterpret_cast<const float4*>(q + cout);
+#pragma unroll
+        for (int k = 0; k < NG; k++) {
+            const int t = tid + k * 192, cq = t & 3, vp = t >> 2;
+            if (vp >= kWStage / 2) continue;
             uint32_t* d = sg + 4 * cq * GW + vp;
-            d[0] = bf2(a.x, c.x);
-            d[GW] = bf2(a.y, c.y);
-            d[2 * GW] = bf2(a.z, c.z);
-            d[3 * GW] = bf2(a.w, c.w);
+            d[0] = bf2(ga[k].x, gb[k].x);
+            d[GW] = bf2(ga[k].y, gb[k].y);
+            d[2 * GW] = bf2(ga[k].z, gb[k].z);
+            d[3 * GW] = bf2(ga[k].w, gb[k].w);
         }
         __syncthreads();
+        if (vs + kWStage < v1) load_stage(vs + kWStage);  // in flight during the products
 #pragma unroll 4
         for (int st = 0; st < kWStage / 16; st++) {
             const int v = st * 16 + 4 * kq;  // the lane's first voxel in the stage
             const int r = v >> LG, z = v & (G - 1), y = (row0 + r) & (G - 1);
-            const uint2 ga = *reinterpret_cast<const uint2*>(sg + i * GW + (v >> 1));
+            const uint2 gv = *reinterpret_cast<const uint2*>(sg + i * GW + (v >> 1));
             const uint32_t* q = si + i * CW + (r + 1 + dy) * (RS / 2) + 2 + (z >> 1);
             uint2 m = *reinterpret_cast<const uint2*>(q);
             uint32_t w0 = q[-1], w3 = q[2];
             if (y + dy < 0 || y + dy >= G) m.x = m.y = w0 = w3 = 0;
             const uint32_t s0 = __builtin_amdgcn_alignbit(m.x, w0, 16), s1 = __builtin_amdgcn_alignbit(m.y, m.x, 16),
                            s2 = __builtin_amdgcn_alignbit(w3, m.y, 16);
-            const s4 av = __builtin_bit_cast(s4, ga);
+            const s4 av = __builtin_bit_cast(s4, gv);
             acc[0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, __builtin_bit_cast(s4, make_uint2(s0, s1)), acc[0],
                                                                0, 0, 0);
             acc[1] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, __builtin_bit_cast(s4, m), acc[1], 0, 0, 0);
@@ -576,23 +591,41 @@ __global__ void __launch_bounds__(kT) k_wgrad_small(ConvIn src, const float* __r
     for (int e = 0; e < 4; e++) dst[int64_t(cot * 16 + 4 * kq + e) * cin + ci] = acc[e];
 }
 
-// Sum over workgroup partials bp[w][col], w = 0 .. nw - 1, by one wave: lane
-// strides, then a tree (a fixed order).  Every lane returns the sum.
-__device__ __forceinline__ float wave_col_sum(const float* __restrict__ bp, int nw, int cols, int col) {
-    float s = 0.0f;
-#pragma unroll 8
-    for (int w = threadIdx.x & 63; w < nw; w += 64) s += bp[int64_t(w) * cols + col];
+// ---- sums over a sample's voxels in one fixed order ----
+// A bias or head gradient is a sum over all voxels in float, and a training
+// step amplifies its rounding (Adam divides small gradients by their own
+// size), so its order is part of the results: kChains running sums, chain t
+// over the voxels t, t + kChains, .. in order, then a binary tree over the
+// chains.  A group of workgroup-wide loads feeds the running sums through
+// LDS: the voxels of kSteps steps are read (and their other work done) by all
+// threads, kStepLanes lanes a step, and kStepLanes lanes then add them up step
+// by step.  (One workgroup per channel, each thread following its own chain
+// in memory, took 325 us for 16 channels on 64^3.)
+constexpr int kChains = 256;
+constexpr int kSumT = 512;        // threads
+constexpr int kStepLanes = 32;    // lanes of a step: kStepLanes / (C / 4) chains of C channels
+constexpr int kSteps = 32;        // steps in LDS at a time
+constexpr int kStepLoads = kSteps * kStepLanes / kSumT;  // of each thread
+
+// the tree over the chains' sums of one column, by one wave (every lane)
+__device__ __forceinline__ float chain_tree(const float* __restrict__ bp, int cols, int col) {
+    const int l = threadIdx.x & 63;
+    float v0 = bp[int64_t(l) * cols + col], v1 = bp[int64_t(l + 64) * cols + col];
+    const float v2 = bp[int64_t(l + 128) * cols + col], v3 = bp[int64_t(l + 192) * cols + col];
+    v0 += v2;
+    v1 += v3;
+    v0 += v1;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    return s;
+    for (int o = 32; o > 0; o >>= 1) v0 += __shfl_down(v0, o, 64);
+    return __shfl(v0, 0, 64);
 }
 
 // For each of B samples in turn, grad[k] += sum over its chunks (in order) of
-// part[b][ch][k], k < n, and in the workgroups past those db[c] += sum over
-// its nw workgroup partials bp[b][w][c], one wave per channel
+// part[b][ch][k], k < n, and in the workgroups past those db[c] += the tree
+// over its chains' sums bp[b][t][c], one wave per channel
 __global__ void __launch_bounds__(kT) k_grad_finish(const float* __restrict__ part, int nchunk, int64_t n,
-                                                   float* __restrict__ grad, const float* __restrict__ bp, int nw,
-                                                   int C, float* __restrict__ db, int B) {
+                                                   float* __restrict__ grad, const float* __restrict__ bp, int C,
+                                                   float* __restrict__ db, int B) {
     const int64_t nb = (n + kT - 1) / kT;
     if (int64_t(blockIdx.x) < nb) {
         const int64_t k = int64_t(blockIdx.x) * kT + threadIdx.x;
@@ -609,7 +642,7 @@ __global__ void __launch_bounds__(kT) k_grad_finish(const float* __restrict__ pa
         const int c = int(int64_t(blockIdx.x) - nb) * (kT / 64) + (threadIdx.x >> 6);
         if (c >= C) return;
         float total = db[c];
-        for (int b = 0; b < B; b++) total += wave_col_sum(bp + int64_t(b) * nw * C, nw, C, c);
+        for (int b = 0; b < B; b++) total += chain_tree(bp + int64_t(b) * kChains * C, C, c);
         if ((threadIdx.x & 63) == 0) db[c] = total;
     }
 }
@@ -640,71 +673,72 @@ __global__ void __launch_bounds__(kT) k_pack(const float* __restrict__ params, P
     J.wf[k][packed_at(26 - t, ci, co, cin)] = h;
 }
 
-// Sums a float4 per thread over the threads with the same t % q4 (q4 = 4, 8
-// or 16 channel quads); the first q4 threads return the sums.
-__device__ __forceinline__ float4 quad_sum(float4 v, int q4, float4* red) {
-    const int t = threadIdx.x;
-    __syncthreads();
-    red[t] = v;
-    __syncthreads();
-    for (int o = kT / 2; o >= q4; o >>= 1) {
-        if (t < o) {
-            const float4 b = red[t + o];
-            red[t].x += b.x;
-            red[t].y += b.y;
-            red[t].z += b.z;
-            red[t].w += b.w;
-        }
-        __syncthreads();
-    }
-    return red[t];
-}
-
 // g[v, c] *= (y[v, c] > 0), after adding the gradient pg of the output's
-// average pooling (grid G / 2; null: none), and the bias gradient's workgroup
-// partials bp[w][c] over the workgroup's `per` voxels (a multiple of
-// 4 kT / C): one pass over g and y for all three.  (The bias gradient alone,
-// one workgroup per channel with strided loads, took 325 us for 16 channels
-// on 64^3; the pooling's as a pass of its own 130 us for 8 samples.)
-__global__ void __launch_bounds__(kT) k_relu_bias(float* __restrict__ g, const float* __restrict__ y,
-                                                 const float* __restrict__ pg, int lg, int C, int64_t per,
-                                                 float* __restrict__ bp) {
+// average pooling (grid G / 2; null: none), and the bias gradient's running
+// sums bp[t][c]: one pass over g and y for all three (the pooling's as a pass
+// of its own took 130 us for 8 samples).
+__global__ void __launch_bounds__(kSumT) k_relu_bias(float* __restrict__ g, const float* __restrict__ y,
+                                                    const float* __restrict__ pg, int lg, int C,
+                                                    float* __restrict__ bp) {
+    __shared__ float4 buf[2][kSteps][kStepLanes];
     const int G = 1 << lg;
     const int64_t V = int64_t(1) << (3 * lg);
-    __shared__ float4 red[kT];
     g += int64_t(blockIdx.y) * V * C;
     y += int64_t(blockIdx.y) * V * C;
     pg += pg ? sample_offset(G >> 1, C) : 0;
-    bp += int64_t(blockIdx.y) * gridDim.x * C;
-    const int q4 = C >> 2, q = threadIdx.x & (q4 - 1), step = kT / q4;
-    const int64_t v0 = int64_t(blockIdx.x) * per, v1 = v0 + per < V ? v0 + per : V;
-    float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-#pragma unroll 4
-    for (int64_t v = v0 + threadIdx.x / q4; v < v1; v += step) {
-        float4* gp = reinterpret_cast<float4*>(g + v * C) + q;
-        const float4 a = *(reinterpret_cast<const float4*>(y + v * C) + q);
-        float4 b = *gp;
-        if (pg) {
-            const int z = int(v) & (G - 1), yy = int(v >> lg) & (G - 1), x = int(v >> (2 * lg));
-            const int64_t u = (((int64_t(x >> 1) << (lg - 1)) + (yy >> 1)) << (lg - 1)) + (z >> 1);
-            const float4 h = *(reinterpret_cast<const float4*>(pg + u * C) + q);
-            b.x = b.x + h.x * 0.125f;
-            b.y = b.y + h.y * 0.125f;
-            b.z = b.z + h.z * 0.125f;
-            b.w = b.w + h.w * 0.125f;
+    bp += int64_t(blockIdx.y) * kChains * C;
+    const int lq = log2i(C) - 2, l = threadIdx.x & (kStepLanes - 1), sl = threadIdx.x / kStepLanes;
+    const int q = l & ((1 << lq) - 1), t = (int(blockIdx.x) * kStepLanes + l) >> lq;  // this lane's chain
+    const int nsteps = int((V + kChains - 1) / kChains);
+    float4 a[kStepLoads], b[kStepLoads];
+    auto load = [&](int kb) {
+#pragma unroll
+        for (int u = 0; u < kStepLoads; u++) {
+            const int64_t v = t + int64_t(kChains) * (kb + sl + u * (kSumT / kStepLanes));
+            a[u] = b[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (v >= V) continue;
+            a[u] = *(reinterpret_cast<const float4*>(y + v * C) + q);
+            b[u] = *(reinterpret_cast<const float4*>(g + v * C) + q);
+            if (pg) {
+                const int z = int(v) & (G - 1), yy = int(v >> lg) & (G - 1), x = int(v >> (2 * lg));
+                const int64_t w = (((int64_t(x >> 1) << (lg - 1)) + (yy >> 1)) << (lg - 1)) + (z >> 1);
+                const float4 h = *(reinterpret_cast<const float4*>(pg + w * C) + q);
+                b[u].x = b[u].x + h.x * 0.125f;
+                b[u].y = b[u].y + h.y * 0.125f;
+                b[u].z = b[u].z + h.z * 0.125f;
+                b[u].w = b[u].w + h.w * 0.125f;
+            }
         }
-        if (!(a.x > 0.0f)) b.x = 0.0f;
-        if (!(a.y > 0.0f)) b.y = 0.0f;
-        if (!(a.z > 0.0f)) b.z = 0.0f;
-        if (!(a.w > 0.0f)) b.w = 0.0f;
-        *gp = b;
-        s.x += b.x;
-        s.y += b.y;
-        s.z += b.z;
-        s.w += b.w;
+    };
+    load(0);
+    float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int kb = 0, cur = 0; kb < nsteps; kb += kSteps, cur ^= 1) {
+#pragma unroll
+        for (int u = 0; u < kStepLoads; u++) {
+            const int k = sl + u * (kSumT / kStepLanes);
+            const int64_t v = t + int64_t(kChains) * (kb + k);
+            if (!(a[u].x > 0.0f)) b[u].x = 0.0f;
+            if (!(a[u].y > 0.0f)) b[u].y = 0.0f;
+            if (!(a[u].z > 0.0f)) b[u].z = 0.0f;
+            if (!(a[u].w > 0.0f)) b[u].w = 0.0f;
+            if (v < V) *(reinterpret_cast<float4*>(g + v * C) + q) = b[u];
+            buf[cur][k][l] = b[u];
+        }
+        __syncthreads();
+        if (kb + kSteps < nsteps) load(kb + kSteps);  // in flight during the sums
+        if (threadIdx.x < kStepLanes) {
+            // (steps past the last voxel hold +0, which changes no sum that is not -0)
+#pragma unroll 8
+            for (int k = 0; k < kSteps; k++) {
+                const float4 x = buf[cur][k][l];
+                s.x += x.x;
+                s.y += x.y;
+                s.z += x.z;
+                s.w += x.w;
+            }
+        }
     }
-    s = quad_sum(s, q4, red);
-    if (threadIdx.x < q4) *(reinterpret_cast<float4*>(bp + int64_t(blockIdx.x) * C) + threadIdx.x) = s;
+    if (threadIdx.x < kStepLanes) *(reinterpret_cast<float4*>(bp + int64_t(t) * C) + q) = s;
 }
 
 // a 2x2x2 cell's eight voxels summed in order, four channels per thread: out
@@ -761,12 +795,13 @@ __global__ void __launch_bounds__(kT) k_head(const float* __restrict__ in, const
 }
 
 // Two doubles per thread summed over the workgroup (a fixed tree).
+template <int kThreads = kT>
 __device__ __forceinline__ void pair_sum(double& a, double& b, double* ra, double* rb) {
     const int t = threadIdx.x;
     ra[t] = a;
     rb[t] = b;
     __syncthreads();
-    for (int o = kT / 2; o > 0; o >>= 1) {
+    for (int o = kThreads / 2; o > 0; o >>= 1) {
         if (t < o) {
             ra[t] += ra[t + o];
             rb[t] += rb[t + o];
@@ -778,7 +813,6 @@ __device__ __forceinline__ void pair_sum(double& a, double& b, double* ra, doubl
 }
 
 constexpr int kLossVox = 2048;  // voxels per workgroup of k_loss_part
-constexpr int kHeadVox = 1024;  // and of k_loss_back
 constexpr int kHeadCols = 33;   // its partials: head weights (16), head bias, d0b's bias (16)
 
 // masked MSE: per-workgroup partials of sum_v m and sum_v m (p - t)^2 (double)
@@ -807,84 +841,116 @@ __global__ void __launch_bounds__(kT) k_loss_part(const float* __restrict__ pred
 // The loss, sum_v m (p - t)^2 / sum_v m, from the nl partials (each workgroup
 // sums them in the same order), its gradient gp = 2 m (p - t) / sum m at each
 // voxel, and through the head to the last convolution's pre-activation:
-// gin[v, c] = gp w[c] where in[v, c] > 0, else 0.  hp: per-workgroup partials
+// gin[v, c] = gp w[c] where in[v, c] > 0, else 0.  hp[t][..]: the running sums
 // of the head's weight and bias gradients and of that convolution's bias
 // gradient.  (The loss in one workgroup took 530 us on 64^3 and the head's
 // weight gradient in 17 took 350 us.)
-__global__ void __launch_bounds__(kT) k_loss_back(const float* __restrict__ pred, const float* __restrict__ tgt,
-                                                 const float* __restrict__ mask, const float* __restrict__ in,
-                                                 const float* __restrict__ w, int64_t V, const double* __restrict__ lp,
-                                                 int nl, double* __restrict__ loss, float* __restrict__ gin,
-                                                 float* __restrict__ hp) {
-    __shared__ double r1[kT], r2[kT];
-    __shared__ float4 red[kT];
+__global__ void __launch_bounds__(kSumT) k_loss_back(const float* __restrict__ pred, const float* __restrict__ tgt,
+                                                    const float* __restrict__ mask, const float* __restrict__ in,
+                                                    const float* __restrict__ w, int64_t V,
+                                                    const double* __restrict__ lp, int nl, double* __restrict__ loss,
+                                                    float* __restrict__ gin, float* __restrict__ hp) {
+    __shared__ double r1[kSumT], r2[kSumT];
+    __shared__ float4 bw[2][kSteps][kStepLanes], bb[2][kSteps][kStepLanes];
+    __shared__ float bg[2][kSteps][kStepLanes / 4];
     pred += int64_t(blockIdx.y) * V;
     tgt += int64_t(blockIdx.y) * V;
     mask += int64_t(blockIdx.y) * V;
     in += int64_t(blockIdx.y) * V * 16;
     gin += int64_t(blockIdx.y) * V * 16;
     lp += 2 * int64_t(blockIdx.y) * nl;
-    hp += int64_t(blockIdx.y) * gridDim.x * kHeadCols;
-    double sm = 0.0, sl = 0.0;
-    for (int k = threadIdx.x; k < nl; k += kT) {
+    hp += int64_t(blockIdx.y) * kChains * kHeadCols;
+    double sm = 0.0, sl2 = 0.0;
+    for (int k = threadIdx.x; k < nl; k += kSumT) {
         sm += lp[2 * k];
-        sl += lp[2 * k + 1];
+        sl2 += lp[2 * k + 1];
     }
-    pair_sum(sm, sl, r1, r2);
+    pair_sum<kSumT>(sm, sl2, r1, r2);
     const double msum = sm;
-    if (blockIdx.x == 0 && threadIdx.x == 0) loss[blockIdx.y] = msum > 0.0 ? sl / msum : 0.0;
-    const int q = threadIdx.x & 3;
+    if (blockIdx.x == 0 && threadIdx.x == 0) loss[blockIdx.y] = msum > 0.0 ? sl2 / msum : 0.0;
+    const int l = threadIdx.x & (kStepLanes - 1), sl = threadIdx.x / kStepLanes;
+    const int q = l & 3, t = (int(blockIdx.x) * kStepLanes + l) >> 2;
     const float4 wq = make_float4(w[4 * q], w[4 * q + 1], w[4 * q + 2], w[4 * q + 3]);
-    const int64_t v0 = int64_t(blockIdx.x) * kHeadVox, v1 = v0 + kHeadVox < V ? v0 + kHeadVox : V;
+    const int nsteps = int((V + kChains - 1) / kChains);
+    float4 a[kStepLoads];
+    float m[kStepLoads], p[kStepLoads], tg[kStepLoads];
+    auto load = [&](int kb) {
+#pragma unroll
+        for (int u = 0; u < kStepLoads; u++) {
+            const int64_t v = t + int64_t(kChains) * (kb + sl + u * (kSumT / kStepLanes));
+            a[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            m[u] = p[u] = tg[u] = 0.0f;
+            if (v >= V) continue;
+            a[u] = *(reinterpret_cast<const float4*>(in + v * 16) + q);
+            m[u] = mask[v];
+            p[u] = pred[v];
+            tg[u] = tgt[v];
+        }
+    };
+    load(0);
     float4 sw = make_float4(0.0f, 0.0f, 0.0f, 0.0f), sb = sw;
     float sg = 0.0f;
-#pragma unroll 4
-    for (int64_t v = v0 + (threadIdx.x >> 2); v < v1; v += kT / 4) {
-        const float4 a = *(reinterpret_cast<const float4*>(in + v * 16) + q);
-        const float gp = msum > 0.0 ? float(2.0 * mask[v] * (double(pred[v]) - double(tgt[v])) / msum) : 0.0f;
-        const float4 b = make_float4(a.x > 0.0f ? gp * wq.x : 0.0f, a.y > 0.0f ? gp * wq.y : 0.0f,
-                                     a.z > 0.0f ? gp * wq.z : 0.0f, a.w > 0.0f ? gp * wq.w : 0.0f);
-        *(reinterpret_cast<float4*>(gin + v * 16) + q) = b;
-        sw.x += gp * a.x;
-        sw.y += gp * a.y;
-        sw.z += gp * a.z;
-        sw.w += gp * a.w;
-        sb.x += b.x;
-        sb.y += b.y;
-        sb.z += b.z;
-        sb.w += b.w;
-        sg += gp;
+    for (int kb = 0, cur = 0; kb < nsteps; kb += kSteps, cur ^= 1) {
+#pragma unroll
+        for (int u = 0; u < kStepLoads; u++) {
+            const int k = sl + u * (kSumT / kStepLanes);
+            const int64_t v = t + int64_t(kChains) * (kb + k);
+            const float gp = msum > 0.0 ? float(2.0 * m[u] * (double(p[u]) - double(tg[u])) / msum) : 0.0f;
+            const float4 b = make_float4(a[u].x > 0.0f ? gp * wq.x : 0.0f, a[u].y > 0.0f ? gp * wq.y : 0.0f,
+                                         a[u].z > 0.0f ? gp * wq.z : 0.0f, a[u].w > 0.0f ? gp * wq.w : 0.0f);
+            if (v < V) *(reinterpret_cast<float4*>(gin + v * 16) + q) = b;
+            bw[cur][k][l] = make_float4(gp * a[u].x, gp * a[u].y, gp * a[u].z, gp * a[u].w);
+            bb[cur][k][l] = b;
+            if (q == 0) bg[cur][k][l >> 2] = gp;
+        }
+        __syncthreads();
+        if (kb + kSteps < nsteps) load(kb + kSteps);
+        // the head's weights and bias in one wave, the convolution's bias in another
+        if (threadIdx.x < kStepLanes) {
+#pragma unroll 8
+            for (int k = 0; k < kSteps; k++) {
+                const float4 x = bw[cur][k][l];
+                sw.x += x.x;
+                sw.y += x.y;
+                sw.z += x.z;
+                sw.w += x.w;
+                sg += bg[cur][k][l >> 2];
+            }
+        } else if (threadIdx.x >= 64 && threadIdx.x < 64 + kStepLanes) {
+#pragma unroll 8
+            for (int k = 0; k < kSteps; k++) {
+                const float4 x = bb[cur][k][l];
+                sb.x += x.x;
+                sb.y += x.y;
+                sb.z += x.z;
+                sb.w += x.w;
+            }
+        }
     }
-    float* dst = hp + int64_t(blockIdx.x) * kHeadCols;
-    const int t = threadIdx.x;
-    sw = quad_sum(sw, 4, red);
-    if (t < 4) {
-        dst[4 * t] = sw.x;
-        dst[4 * t + 1] = sw.y;
-        dst[4 * t + 2] = sw.z;
-        dst[4 * t + 3] = sw.w;
+    float* dst = hp + int64_t(t) * kHeadCols;
+    if (threadIdx.x < kStepLanes) {
+        dst[4 * q] = sw.x;
+        dst[4 * q + 1] = sw.y;
+        dst[4 * q + 2] = sw.z;
+        dst[4 * q + 3] = sw.w;
+        if (q == 0) dst[16] = sg;
+    } else if (threadIdx.x >= 64 && threadIdx.x < 64 + kStepLanes) {
+        dst[17 + 4 * q] = sb.x;
+        dst[17 + 4 * q + 1] = sb.y;
+        dst[17 + 4 * q + 2] = sb.z;
+        dst[17 + 4 * q + 3] = sb.w;
     }
-    sb = quad_sum(sb, 4, red);
-    if (t < 4) {
-        dst[17 + 4 * t] = sb.x;
-        dst[17 + 4 * t + 1] = sb.y;
-        dst[17 + 4 * t + 2] = sb.z;
-        dst[17 + 4 * t + 3] = sb.w;
-    }
-    // (every thread of a quad saw the same voxels)
-    const float4 sh = quad_sum(make_float4(sg, 0.0f, 0.0f, 0.0f), 4, red);
-    if (t == 0) dst[16] = sh.x;
 }
 
 // the head's gradients (dw: 16 weights, bias) and the last convolution's bias
-// gradient from k_loss_back's nw partials, sample by sample; one wave per column
-__global__ void __launch_bounds__(kT) k_head_finish(const float* __restrict__ hp, int nw, float* __restrict__ dw,
+// gradient from k_loss_back's running sums, sample by sample; one wave per column
+__global__ void __launch_bounds__(kT) k_head_finish(const float* __restrict__ hp, float* __restrict__ dw,
                                                    float* __restrict__ db, int B) {
     const int c = int(blockIdx.x) * (kT / 64) + (threadIdx.x >> 6);
     if (c >= kHeadCols) return;
     float* dst = c < 17 ? dw + c : db + (c - 17);
     float total = *dst;
-    for (int b = 0; b < B; b++) total += wave_col_sum(hp + int64_t(b) * nw * kHeadCols, nw, kHeadCols, c);
+    for (int b = 0; b < B; b++) total += chain_tree(hp + int64_t(b) * kChains * kHeadCols, kHeadCols, c);
     if ((threadIdx.x & 63) == 0) *dst = total;
 }
 
@@ -1173,20 +1239,6 @@ void forward(prg_unet* n, int B, float f = 1.0f) {
     PRG_CHECK_LAUNCH();
 }
 
-// Workgroups of k_relu_bias for V voxels of C channels, and the voxels of each.
-struct BiasPlan {
-    unsigned wg;
-    int64_t per;
-};
-
-BiasPlan bias_plan(int64_t V, int C) {
-    const int64_t step = 4 * kT / C;  // voxels per workgroup round
-    const int64_t rounds = (V + step - 1) / step;
-    const int64_t wg = std::min<int64_t>(512, std::max<int64_t>(1, rounds / 2));
-    const int64_t per = (rounds + wg - 1) / wg * step;
-    return {unsigned((V + per - 1) / per), per};
-}
-
 // Gradient of conv k for incoming gradient g (in place: the pooled gradient
 // `pg` of its output added, then the ReLU mask; unless `masked`: g has both
 // and the bias gradient is accumulated).  Writes the input gradient to gin
@@ -1197,9 +1249,9 @@ void conv_back(prg_unet* n, int B, int k, float* g, float* gin, float* gskip = n
     hipStream_t s = n->stream;
     auto& L = n->conv[k];
     const int64_t V = int64_t(L.G) * L.G * L.G;
-    const BiasPlan bp = bias_plan(V, L.cout);
     if (!masked) {
-        k_relu_bias<<<dim3(bp.wg, unsigned(B)), kT, 0, s>>>(g, L.out, pg, log2i(L.G), L.cout, bp.per, n->bpart.get());
+        k_relu_bias<<<dim3(unsigned(kChains * L.cout / 4 / kStepLanes), unsigned(B)), kSumT, 0, s>>>(
+            g, L.out, pg, log2i(L.G), L.cout, n->bpart.get());
         PRG_CHECK_LAUNCH();
     }
     const int nchunk = int((V + kWChunk - 1) / kWChunk);
@@ -1217,7 +1269,7 @@ void conv_back(prg_unet* n, int B, int k, float* g, float* gin, float* gskip = n
     }
     PRG_CHECK_LAUNCH();
     k_grad_finish<<<blocks(nw) + (masked ? 0 : L.cout / (kT / 64)), kT, 0, s>>>(
-        n->part.get(), nchunk, nw, n->grads.get() + L.woff, n->bpart.get(), int(bp.wg), L.cout,
+        n->part.get(), nchunk, nw, n->grads.get() + L.woff, n->bpart.get(), L.cout,
         n->grads.get() + L.boff, B);
     PRG_CHECK_LAUNCH();
     if (gin)
@@ -1235,16 +1287,16 @@ void backward(prg_unet* n, int B) {
     float* ga = n->ga.get();
     float* gb = n->gb.get();
     // loss, head and the last ReLU
-    const int nl = int((V0 + kLossVox - 1) / kLossVox), nh = int((V0 + kHeadVox - 1) / kHeadVox);
+    const int nl = int((V0 + kLossVox - 1) / kLossVox);
     const int64_t head = n->nparams - 17;
     k_loss_part<<<dim3(unsigned(nl), unsigned(B)), kT, 0, s>>>(n->pred.get(), n->target.get(), n->mask.get(), V0,
                                                                n->lpart.get());
     PRG_CHECK_LAUNCH();
-    k_loss_back<<<dim3(unsigned(nh), unsigned(B)), kT, 0, s>>>(n->pred.get(), n->target.get(), n->mask.get(), C[13].out,
-                                            n->params.get() + head, V0, n->lpart.get(), nl, n->loss.get(), ga,
-                                            n->bpart.get());
+    k_loss_back<<<dim3(unsigned(kChains * 4 / kStepLanes), unsigned(B)), kSumT, 0, s>>>(
+        n->pred.get(), n->target.get(), n->mask.get(), C[13].out, n->params.get() + head, V0, n->lpart.get(), nl,
+        n->loss.get(), ga, n->bpart.get());
     PRG_CHECK_LAUNCH();
-    k_head_finish<<<(kHeadCols + 3) / 4, kT, 0, s>>>(n->bpart.get(), nh, n->grads.get() + head,
+    k_head_finish<<<(kHeadCols + 3) / 4, kT, 0, s>>>(n->bpart.get(), n->grads.get() + head,
                                                      n->grads.get() + C[13].boff, B);
     PRG_CHECK_LAUNCH();
     auto up_back = [&](const float* g, int c, int g1, float* glo) {
@@ -1328,7 +1380,7 @@ void reserve_batch(prg_unet* n, int B) {
     n->ge1.reserve(V0 / 8 * 32);
     n->ge2.reserve(V0 / 64 * 64);
     n->part.reserve(pc);
-    n->bpart.reserve(std::max<size_t>(size_t(512) * 64 * B, (V0 + size_t(kHeadVox) * B) / kHeadVox * kHeadCols));
+    n->bpart.reserve(size_t(kChains) * 64 * B);
     n->lpart.reserve(2 * ((V0 + size_t(kLossVox) * B) / kLossVox));
     n->loss.reserve(B);
     n->inv.reserve(B);
