@@ -977,11 +977,11 @@ __global__ void __launch_bounds__(kT) k_input(const float* __restrict__ b, const
     o[1] = o[2] = o[3] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 }
 
-// a[v] *= f, or by f[sample] when fs is given (V values per sample)
-__global__ void k_scale(float* a, int64_t V, float f, const float* fs) {
+// a[v] *= f[sample] (V values per sample)
+__global__ void __launch_bounds__(kT) k_scale(float* a, int64_t V, const float* f) {
     const int64_t v = int64_t(blockIdx.x) * kT + threadIdx.x;
     if (v >= V) return;
-    a[int64_t(blockIdx.y) * V + v] *= fs ? fs[blockIdx.y] : f;
+    a[int64_t(blockIdx.y) * V + v] *= f[blockIdx.y];
 }
 
 // ---- dense grids of one depth of a context ----
@@ -1071,6 +1071,8 @@ struct prg_unet {
     int device = 0;
     int G = 64;
     hipStream_t stream = nullptr;
+    hipStream_t copy_stream = nullptr;  // the targets' upload, made when first used
+    hipEvent_t copied = nullptr;
     std::string err;
     int64_t nparams = 0;
     prg::DBuf<float> params, grads, adam_m, adam_v;
@@ -1335,21 +1337,32 @@ void upload(prg_unet* n, float* dst, const float* src, int64_t count) {
     PRG_HIP(hipMemcpyAsync(dst, src, size_t(count) * 4, hipMemcpyHostToDevice, n->stream));
 }
 
-// B samples' inputs (divergence and mask grids) and, for training, targets,
-// normalised by their scales
-void load_samples(prg_unet* n, const float* bgrid, const float* mask, const float* target, const float* scale, int B) {
+// B samples' inputs (divergence and mask grids), normalised by their scales
+void load_samples(prg_unet* n, const float* bgrid, const float* mask, const float* scale, int B) {
     const int64_t V = int64_t(n->G) * n->G * n->G;
     for (int b = 0; b < B; b++) n->inv_host[b] = 1.0f / scale[b];
     upload(n, n->inv.get(), n->inv_host, B);
     upload(n, n->bgrid.get(), bgrid, V * B);
     upload(n, n->mask.get(), mask, V * B);
-    const dim3 grid(blocks(V), unsigned(B));
-    if (target) {
-        upload(n, n->target.get(), target, V * B);
-        k_scale<<<grid, kT, 0, n->stream>>>(n->target.get(), V, 1.0f, n->inv.get());
-        PRG_CHECK_LAUNCH();
+    k_input<<<dim3(blocks(V), unsigned(B)), kT, 0, n->stream>>>(n->bgrid.get(), n->mask.get(), n->inv.get(), V,
+                                                               n->x0.get());
+    PRG_CHECK_LAUNCH();
+}
+
+// Their targets, normalised likewise: up on a stream of their own, beside the
+// forward pass queued before (0.3 ms of a training step of 8 at 64^3).
+// Nothing queued uses the buffer: every step and gradient call ends with a
+// synchronisation.
+void load_targets(prg_unet* n, const float* target, int B) {
+    const int64_t V = int64_t(n->G) * n->G * n->G;
+    if (!n->copy_stream) {
+        PRG_HIP(hipStreamCreateWithFlags(&n->copy_stream, hipStreamNonBlocking));
+        PRG_HIP(hipEventCreateWithFlags(&n->copied, hipEventDisableTiming));
     }
-    k_input<<<grid, kT, 0, n->stream>>>(n->bgrid.get(), n->mask.get(), n->inv.get(), V, n->x0.get());
+    PRG_HIP(hipMemcpyAsync(n->target.get(), target, size_t(V * B) * 4, hipMemcpyHostToDevice, n->copy_stream));
+    PRG_HIP(hipEventRecord(n->copied, n->copy_stream));
+    PRG_HIP(hipStreamWaitEvent(n->stream, n->copied, 0));
+    k_scale<<<dim3(blocks(V), unsigned(B)), kT, 0, n->stream>>>(n->target.get(), V, n->inv.get());
     PRG_CHECK_LAUNCH();
 }
 
@@ -1530,6 +1543,11 @@ prg_status prg_unet_create(prg_unet** out, int32_t device, int32_t grid, uint64_
 void prg_unet_destroy(prg_unet* n) {
     if (!n) return;
     (void)hipSetDevice(n->device);
+    if (n->copy_stream) {
+        (void)hipStreamSynchronize(n->copy_stream);
+        (void)hipStreamDestroy(n->copy_stream);
+    }
+    if (n->copied) (void)hipEventDestroy(n->copied);
     if (n->stream) {
         (void)hipStreamSynchronize(n->stream);
         (void)hipStreamDestroy(n->stream);
@@ -1567,7 +1585,7 @@ prg_status prg_unet_predict(prg_unet* n, const float* bgrid, const float* mask, 
         if (!bgrid || !mask || !out || !(scale > 0.0f)) return PRG_E_ARG;
         const int64_t V = int64_t(n->G) * n->G * n->G;
         prg::reserve_batch(n, 1);
-        prg::load_samples(n, bgrid, mask, nullptr, &scale, 1);
+        prg::load_samples(n, bgrid, mask, &scale, 1);
         prg::forward(n, 1, scale);
         PRG_HIP(hipMemcpyAsync(out, n->pred.get(), size_t(V) * 4, hipMemcpyDeviceToHost, n->stream));
         PRG_HIP(hipStreamSynchronize(n->stream));
@@ -1581,8 +1599,9 @@ prg_status prg_unet_gradients(prg_unet* n, const float* bgrid, const float* mask
         if (!bgrid || !mask || !target || !grads || !loss || !(scale > 0.0f)) return PRG_E_ARG;
         PRG_HIP(hipMemsetAsync(n->grads.get(), 0, size_t(n->nparams) * 4, n->stream));
         prg::reserve_batch(n, 1);
-        prg::load_samples(n, bgrid, mask, target, &scale, 1);
+        prg::load_samples(n, bgrid, mask, &scale, 1);
         prg::forward(n, 1);
+        prg::load_targets(n, target, 1);
         prg::backward(n, 1);
         PRG_HIP(hipMemcpyAsync(grads, n->grads.get(), size_t(n->nparams) * 4, hipMemcpyDeviceToHost, n->stream));
         PRG_HIP(hipMemcpyAsync(loss, n->loss.get(), 8, hipMemcpyDeviceToHost, n->stream));
@@ -1614,8 +1633,9 @@ prg_status prg_unet_train_step(prg_unet* n, const float* bgrids, const float* ma
         double total = 0.0;
         for (int b0 = 0; b0 < batch; b0 += sub) {
             const int B = std::min(sub, batch - b0);
-            prg::load_samples(n, bgrids + b0 * V, masks + b0 * V, targets + b0 * V, scales + b0, B);
+            prg::load_samples(n, bgrids + b0 * V, masks + b0 * V, scales + b0, B);
             prg::forward(n, B);
+            prg::load_targets(n, targets + b0 * V, B);
             prg::backward(n, B);
             double l[prg::kMaxBatch];
             PRG_HIP(hipMemcpyAsync(l, n->loss.get(), size_t(B) * 8, hipMemcpyDeviceToHost, n->stream));
