@@ -946,14 +946,14 @@ __device__ __forceinline__ bool any_thread(bool v) {
 template <int kThreads = kWave, class L>
 __device__ __forceinline__ bool brick_blocks(const SubArgs& A, const Brick& B, L& S) {
     constexpr int kCap = int(sizeof(S.XB) / sizeof(float));
+    constexpr int kBatch = kThreads == kWave ? 3 : 1;
     constexpr int kCapC[2] = {int(sizeof(S.CB0) / sizeof(int32_t)), int(sizeof(S.CB1) / sizeof(int32_t))};
     const int D = A.D, lane = threadIdx.x;
     bool on = B.deep;  // (uniform) the next depth may have real cells
     int total = 0;
     if (lane <= kMaxDepth) S.xb_off[lane] = -1;
-#pragma unroll
-    for (int dd = 1; dd <= kMaxDepth; dd++) {
-        if (!on || dd <= B.r || dd > D) continue;
+#pragma unroll 1
+    for (int dd = B.r + 1; dd <= D && on; dd++) {  // (unrolled, its code came from memory at every launch)
         const int W = block_width(D, B.kb, dd), sh = D - dd, n = W * W * W;
         // child bases of depth dd - 1 in one buffer, of dd in the other
         const bool odd = (sh & 1) != 0;
@@ -966,31 +966,43 @@ __device__ __forceinline__ bool brick_blocks(const SubArgs& A, const Brick& B, L
         const int Wp = dd > B.r + 1 ? block_width(D, B.kb, dd - 1) : 0;
         const int32_t plo[3] = {(B.org[0] >> (sh + 1)) - 2, (B.org[1] >> (sh + 1)) - 2, (B.org[2] >> (sh + 1)) - 2};
         bool kids = false, nz = false;
-        for (int e = lane; e < n; e += kThreads) {
-            // l / W and l / W^2 for l < W^3 <= 1331 by a 16-bit reciprocal (exact: l / W
-            // has a fractional part of at most (W-1)/W, the reciprocal's excess adds < 0.03)
-            const int q1 = int((uint32_t(e) * rw) >> 16), q2 = int((uint32_t(q1) * rw) >> 16);
-            const int32_t c[3] = {lo[0] + q2, lo[1] + (q1 - q2 * W), lo[2] + (e - q1 * W)};
-            int32_t cb = -1;
-            if (uint32_t(c[0]) < uint32_t(width) && uint32_t(c[1]) < uint32_t(width) && uint32_t(c[2]) < uint32_t(width)) {
-                if (dd == B.r + 1) {
-                    const int ox = (c[0] >> 1) - B.R[0], oy = (c[1] >> 1) - B.R[1], oz = (c[2] >> 1) - B.R[2];
-                    cb = (ox | oy | oz) ? S.NBK[nidx(ox, oy, oz)] : -1;
-                } else {
-                    cb = CBp[(((c[0] >> 1) - plo[0]) * Wp + ((c[1] >> 1) - plo[1])) * Wp + ((c[2] >> 1) - plo[2])];
+        // kBatch cells per thread at a time: their loads go out together
+        for (int e0 = lane; e0 < n; e0 += kBatch * kThreads) {
+            int32_t node[kBatch], ck[kBatch];
+            float xv[kBatch];
+#pragma unroll
+            for (int u = 0; u < kBatch; u++) {
+                // e / W and e / W^2 for e < W^3 <= 1331 by a 16-bit reciprocal (exact: e / W
+                // has a fractional part of at most (W-1)/W, the reciprocal's excess adds < 0.03)
+                const int e = e0 + u * kThreads;
+                const int q1 = int((uint32_t(e) * rw) >> 16), q2 = int((uint32_t(q1) * rw) >> 16);
+                const int32_t c[3] = {lo[0] + q2, lo[1] + (q1 - q2 * W), lo[2] + (e - q1 * W)};
+                int32_t cb = -1;
+                if (e < n && uint32_t(c[0]) < uint32_t(width) && uint32_t(c[1]) < uint32_t(width) &&
+                    uint32_t(c[2]) < uint32_t(width)) {
+                    if (dd == B.r + 1) {
+                        const int ox = (c[0] >> 1) - B.R[0], oy = (c[1] >> 1) - B.R[1], oz = (c[2] >> 1) - B.R[2];
+                        cb = (ox | oy | oz) ? S.NBK[nidx(ox, oy, oz)] : -1;
+                    } else {
+                        cb = CBp[(((c[0] >> 1) - plo[0]) * Wp + ((c[1] >> 1) - plo[1])) * Wp + ((c[2] >> 1) - plo[2])];
+                    }
                 }
+                node[u] = cb < 0 ? -1 : cb + (((c[0] & 1) << 2) | ((c[1] & 1) << 1) | (c[2] & 1));
             }
-            float xv = 0.0f;
-            int32_t ck = -1;
-            if (cb >= 0) {
-                const int32_t node = cb + (((c[0] & 1) << 2) | ((c[1] & 1) << 1) | (c[2] & 1));
-                xv = A.x[node];
-                if (dd < D) ck = A.child_base[node];
+#pragma unroll
+            for (int u = 0; u < kBatch; u++) {
+                xv[u] = node[u] < 0 ? 0.0f : A.x[node[u]];
+                ck[u] = node[u] < 0 || dd >= D ? -1 : A.child_base[node[u]];
             }
-            S.XB[total + e] = xv;
-            if (dd < D) CBn[e] = ck;
-            nz = nz || xv != 0.0f;
-            kids = kids || ck >= 0;
+#pragma unroll
+            for (int u = 0; u < kBatch; u++) {
+                const int e = e0 + u * kThreads;
+                if (e >= n) continue;
+                S.XB[total + e] = xv[u];
+                if (dd < D) CBn[e] = ck[u];
+                nz = nz || xv[u] != 0.0f;
+                kids = kids || ck[u] >= 0;
+            }
         }
         const bool any = any_thread<kThreads>(nz);
         on = any_thread<kThreads>(kids);
