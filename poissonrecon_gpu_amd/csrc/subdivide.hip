@@ -87,11 +87,11 @@ __constant__ CubeFaces c_cube_faces = make_cube_faces();
 __constant__ int8_t c_children_vertex_kind[8] = {0, 1, 3, 2, 4, 5, 7, 6};
 
 // slots of the device counter array; the cells of 2^k leaves a side listed at
-// kCntCells + k, and taken from the list at kCntTaken + k
+// kCntCells + k
 enum { kCntCoarse = 0, kCntCorners = 1, kCntRoots = 2, kCntBricks = 3, kCntVerts = 4, kCntTris = 5, kCntLeaves = 6,
-       kCntErr = 7, kCntDense = 8, kCntExact = 9, kCntExactTaken = 10, kCntSmall1 = 11, kCntSmall2 = 12,
-       kCntGroup = 13, kCntCells = 16, kCntTaken = 32, kCntSlots = 48 };
-static_assert(kCntSlots * 4 <= 256 && kCntCells + kMaxDepth < kCntTaken && kCntTaken + kMaxDepth < kCntSlots,
+       kCntErr = 7, kCntDense = 8, kCntExact = 9, kCntSmall1 = 11, kCntSmall2 = 12,
+       kCntGroup = 13, kCntCells = 16, kCntSlots = 32 };
+static_assert(kCntSlots * 4 <= 256 && kCntCells + kMaxDepth < kCntSlots && kCntSlots <= kWeldHost,
               "the pinned counter copy holds 64 ints");
 
 __device__ __forceinline__ int depth_of(int64_t i, const Levels& L, int D) {
@@ -1567,35 +1567,68 @@ __global__ void __launch_bounds__(kBlockS) k_list_roots(const int32_t* roots, co
     }
 }
 
+// Entries a wave has found for a list, in LDS until there are kWaveList: one
+// atomic on the list's counter for all of them.  (An atomic per entry, and one
+// per few entries taken from the input list, was most of the screens' and the
+// certificate's time: thousands of waves on one counter wait for each other,
+// 43 us a cell in k_cell_screen.)
+constexpr int kWaveList = 128;
+struct WaveList {
+    int32_t e[kWaveList];
+};
+
+// Appends the n buffered entries times `each` (entry j * each + i: e[j] + (i << shift)).
+__device__ __forceinline__ void wave_flush(const WaveList& L, int32_t n, int32_t each, int shift, int32_t* counter,
+                                           int32_t* list) {
+    __syncthreads();  // (one wave: the buffered entries are in LDS)
+    int32_t at = 0;
+    if (threadIdx.x == 0 && n > 0) at = atomicAdd(counter, n * each);
+    at = __shfl(at, 0, kWave);
+    for (int32_t j = threadIdx.x; j < n * each; j += kWave) {
+        const int32_t q = each == 1 ? j : j >> 3, i = each == 1 ? 0 : j & 7;  // (each is 1 or 8)
+        list[at + j] = L.e[q] + (i << shift);
+    }
+    __syncthreads();
+}
+
+// Buffers v of the lanes with `want` (uniform n), flushing before it is full.
+__device__ __forceinline__ int32_t wave_push(WaveList& L, int32_t n, bool want, int32_t v, int32_t* counter,
+                                             int32_t* list) {
+    const uint64_t m = __builtin_amdgcn_ballot_w64(want);
+    if (m == 0) return n;
+    if (n + kWave > kWaveList) {
+        wave_flush(L, n, 1, 0, counter, list);
+        n = 0;
+    }
+    if (want) L.e[n + int32_t(__popcll(m & ((uint64_t(1) << threadIdx.x) - 1)))] = v;
+    return n + int32_t(__popcll(m));
+}
+
 // Pass 0: screens the listed cells of 2^k leaves a side, one wave each (a
-// resident grid takes chunks of the list from a counter).  A settled cell
-// gives its bricks its sign (their counts stay 0), and lists those that touch
-// another root of the group for k_group_check; of the others, a cell of more
-// than one brick lists its eight parts for the next size and a brick goes to
-// the per-corner certificate.  Most of the refined volume is far from the
-// surface and settles in large cells: the 1,036,945 bricks of 2 M points at
-// depth 10 took 1.85 ms as 122,256 cells of 16^3 and then 238,786 bricks, each
-// bounded by intervals depth by depth.
+// resident grid strides over the list).  A settled cell gives its bricks its
+// sign (their counts stay 0), and lists those that touch another root of the
+// group for k_group_check; of the others, a cell of more than one brick lists
+// its eight parts for the next size and a brick goes to the per-corner
+// certificate.  Most of the refined volume is far from the surface and settles
+// in large cells.  All passes of the screens, 2 M points at depth 10
+// (1,036,945 bricks): 1333 us with shared counters for the list's next entries
+// and for each entry found, 925 us without.
 template <int FLOATS>
 __global__ void __launch_bounds__(kWave, FLOATS > kXBlkScreen ? 3 : 5) k_cell_screen(SubArgs A, int k, const int32_t* list, int32_t* parts,
                                                        int32_t* xlist, int8_t* sign, int32_t* glist, int32_t* cnt,
                                                        int certify) {
     __shared__ CellLds<FLOATS> S;
+    __shared__ WaveList left, group;
     const int lane = threadIdx.x;
     const int32_t n = cnt[kCntCells + k];
-    // up to 16 entries, at least about four grabs per workgroup
-    const int32_t chunk = std::max(1, std::min(16, n / (4 * int32_t(gridDim.x))));
-    int32_t q_loaded = -1, it = 0, it_end = 0;
-    for (;;) {
-        if (it == it_end) {
-            int32_t c0 = 0;
-            if (lane == 0) c0 = atomicAdd(cnt + kCntTaken + k, chunk);
-            c0 = __shfl(c0, 0, kWave);
-            if (c0 >= n) break;
-            it = c0;
-            it_end = std::min(n, c0 + chunk);
-        }
-        const int32_t b = list[it++];
+    const bool brick = k == kBrickLog;
+    int32_t* const next = brick ? xlist : parts;
+    int32_t* const next_cnt = cnt + (brick ? int(kCntExact) : kCntCells + k - 1);
+    const int32_t each = brick ? 1 : 8;
+    const int shift = brick ? 0 : 3 * (k - 1 - kBrickLog);
+    int32_t q_loaded = -1, nleft = 0, ngroup = 0;
+    for (int32_t it = blockIdx.x; it < n; it += int32_t(gridDim.x)) {
+        const int32_t b = list[it];
         Brick B;
         __syncthreads();  // the previous cell's LDS reads are done
         cell_setup(A, b, k, B, S, q_loaded);
@@ -1603,15 +1636,12 @@ __global__ void __launch_bounds__(kWave, FLOATS > kXBlkScreen ? 3 : 5) k_cell_sc
         int s = 0;
         if (certify && brick_blocks(A, B, S)) s = cell_sign(A, B, S);
         if (s == 0) {
-            const int32_t np = k > kBrickLog ? 8 : 1;
-            int32_t at = 0;
-            if (lane == 0) at = atomicAdd(cnt + (k > kBrickLog ? kCntCells + k - 1 : int(kCntExact)), np);
-            at = __shfl(at, 0, kWave);
-            if (k > kBrickLog) {
-                if (lane < 8) parts[at + lane] = b + (lane << (3 * (k - 1 - kBrickLog)));
-            } else if (lane == 0) {
-                xlist[at] = b;
+            if (nleft == kWaveList) {
+                wave_flush(left, nleft, each, shift, next_cnt, next);
+                nleft = 0;
             }
+            if (lane == 0) left.e[nleft] = b;
+            nleft++;
             continue;
         }
         // the cell's bricks; those on a face, edge or corner shared with the group
@@ -1638,35 +1668,26 @@ __global__ void __launch_bounds__(kWave, FLOATS > kXBlkScreen ? 3 : 5) k_cell_sc
                     if (g + (1 << kBrickLog) == B.R0[a] + B.Sr) m[a] |= z << (2 * step);
                 }
                 const bool want = in && (m[0] & m[1] & m[2] & gm) != 0;
-                const int32_t at = wave_append(want, cnt + kCntGroup);
-                if (want) glist[at] = b + i;
+                ngroup = wave_push(group, ngroup, want, b + i, cnt + kCntGroup, glist);
             }
         }
     }
+    wave_flush(left, nleft, each, shift, next_cnt, next);
+    wave_flush(group, ngroup, 1, 0, cnt + kCntGroup, glist);
 }
 
 // Pass 0b: the per-corner certificate (brick_certify) for the bricks the
-// screen left; the bricks it does not settle are listed for the evaluation.
-// A resident grid takes chunks of consecutive entries from a counter; entries
-// of one root often follow each other, and its record then stays in LDS.
+// screen left (a resident grid strides over them); the bricks it does not
+// settle are listed for the evaluation.
 __global__ void __launch_bounds__(kWave, 3) k_brick_exact(SubArgs A, const int32_t* xlist, int8_t* sign, int32_t* list,
                                                        int32_t* glist, int32_t* cnt, int certify) {
     __shared__ CertLds S;
+    __shared__ WaveList left, group;
     const int lane = threadIdx.x;
     const int32_t n = cnt[kCntExact];
-    // chunks of up to 8 entries, at least about four per workgroup
-    const int32_t chunk = std::max(1, std::min(8, n / (4 * int32_t(gridDim.x))));
-    int32_t q_loaded = -1, it = 0, it_end = 0;
-    for (;;) {
-        if (it == it_end) {
-            int32_t c0 = 0;
-            if (lane == 0) c0 = atomicAdd(cnt + kCntExactTaken, chunk);
-            c0 = __shfl(c0, 0, kWave);
-            if (c0 >= n) break;
-            it = c0;
-            it_end = std::min(n, c0 + chunk);
-        }
-        const int32_t b = xlist[it++];
+    int32_t q_loaded = -1, nleft = 0, ngroup = 0;
+    for (int32_t it = blockIdx.x; it < n; it += int32_t(gridDim.x)) {
+        const int32_t b = xlist[it];
         Brick B;
         __syncthreads();  // the previous brick's LDS reads are done
         cell_setup(A, b, kBrickLog, B, S, q_loaded);
@@ -1681,14 +1702,14 @@ __global__ void __launch_bounds__(kWave, 3) k_brick_exact(SubArgs A, const int32
             }
         }
         const bool fits = brick_blocks(A, B, S);
-        const bool group = brick_in_group(B, S);
-        const int s = certify && fits ? brick_certify(A, B, S, group) : 0;
-        if (lane == 0) {
-            sign[b] = int8_t(s);
-            if (s == 0) list[atomicAdd(cnt + kCntDense, 1)] = b;
-            else if (group) glist[atomicAdd(cnt + kCntGroup, 1)] = b;
-        }
+        const bool in_group = brick_in_group(B, S);
+        const int s = certify && fits ? brick_certify(A, B, S, in_group) : 0;
+        if (lane == 0) sign[b] = int8_t(s);
+        nleft = wave_push(left, nleft, lane == 0 && s == 0, b, cnt + kCntDense, list);
+        ngroup = wave_push(group, ngroup, lane == 0 && s != 0 && in_group, b, cnt + kCntGroup, glist);
     }
+    wave_flush(left, nleft, 1, 0, cnt + kCntDense, list);
+    wave_flush(group, ngroup, 1, 0, cnt + kCntGroup, glist);
 }
 
 // The corner values of the bricks the certificates left (grid_value): gv at
@@ -1809,8 +1830,10 @@ __device__ __forceinline__ void brick_geometry(const SubArgs& A, int32_t b, Bric
 // owners themselves are looked up only when one does not.
 __global__ void __launch_bounds__(kWave) k_group_check(SubArgs A, const int32_t* glist, const int8_t* sign,
                                                        int32_t* list, int32_t* cnt) {
+    __shared__ WaveList left;
     const int lane = threadIdx.x, D = A.D;
     const int32_t n = cnt[kCntGroup];
+    int32_t nleft = 0;
     for (int32_t it = blockIdx.x; it < n; it += int32_t(gridDim.x)) {
         const int32_t b = glist[it];
         Brick B;
@@ -1841,9 +1864,10 @@ __global__ void __launch_bounds__(kWave) k_group_check(SubArgs A, const int32_t*
         const uint64_t around = __builtin_amdgcn_ballot_w64(other);
         const uint32_t deps = brick_group_deps(B, S, D);
         // (an owner in a brick outside the group's roots cannot be)
-        if ((deps & uint32_t(bad)) || (deps & ~uint32_t(around)))
-            if (lane == 0) list[atomicAdd(cnt + kCntDense, 1)] = b;
+        const bool listed = (deps & uint32_t(bad)) || (deps & ~uint32_t(around));
+        nleft = wave_push(left, nleft, lane == 0 && listed, b, cnt + kCntDense, list);
     }
+    wave_flush(left, nleft, 1, 0, cnt + kCntDense, list);
 }
 
 // Exclusive sum of v over the workgroup's 512 threads, and the total.
