@@ -253,9 +253,10 @@ prg_status prg_subdivision_info(prg_ctx* ctx, int64_t* n_roots, int64_t* n_virtu
 
 /* After a prg_extract_mesh* call with subdivide != 0: how the subdivision's
  * bricks (blocks of up to 8^3 virtual leaves) were settled: all of them, those
- * the one-interval certificate did not settle, and those whose corner values
- * were evaluated (the exact certificate did not settle them either).  No
- * counterpart in the reference, which evaluates every virtual leaf. */
+ * the bounds over whole cells did not settle, and those whose corner values
+ * were evaluated (the per-corner certificate did not settle them either).
+ * Roots of 2^3 and 4^3 leaves go to the evaluation at once and count in all
+ * three.  No counterpart in the reference, which evaluates every virtual leaf. */
 prg_status prg_subdivision_bricks(prg_ctx* ctx, int64_t* n_bricks, int64_t* n_exact, int64_t* n_evaluated);
 
 /* Whole pipeline: build, divergence, solve, isovalue, mesh. */

@@ -338,7 +338,7 @@ class Reconstructor:
         return a.value, b.value
 
     def subdivision_bricks(self) -> tuple[int, int, int]:
-        """(bricks, left by the interval certificate, evaluated) of the last subdivided mesh."""
+        """(bricks, left by the bounds over whole cells, evaluated) of the last subdivided mesh."""
         a, b, e = C.c_int64(), C.c_int64(), C.c_int64()
         self._call("prg_subdivision_bricks", C.byref(a), C.byref(b), C.byref(e))
         return a.value, b.value, e.value
