@@ -42,14 +42,12 @@ constexpr int kBlock = 256;
 constexpr int kMaxBlocks = 2048;
 constexpr int kSmallBlock = 1024;
 constexpr int64_t kSmallRows = 2048;
-// Algorithmic bytes per row of the kernels that gather through the
-// parent-neighbour table: the 27 entries of a row's 8-row sibling block (13.5 B
-// per row), plus the vectors each reads and writes once per row.  The SpMV
-// reads the tile plans instead (spmv_plan_bytes).  (The reference's
-// representation, 27 int32 neighbour indices + p_i read + (Ap)_i written,
-// would be 116 B per SpMV row.)
+// Algorithmic bytes per row of k_cg_init's residual (a warm start), which
+// gathers through the parent-neighbour table: the 27 entries of a row's 8-row
+// sibling block, 13.5 B per row.  The SpMV and the other residuals read the
+// tile plans (spmv_plan_bytes).  (The reference's representation, 27 int32
+// neighbour indices + p_i read + (Ap)_i written, would be 116 B per SpMV row.)
 constexpr double kPntRowBytes = 13.5;
-constexpr double kResidualRowBytes = kPntRowBytes + 12.0;  // x, b read; r written
 
 struct Stencil {
     float L[27];
@@ -158,7 +156,7 @@ __device__ __forceinline__ double sum_partials(const double* __restrict__ part, 
     return block_allsum<BS>(s, lds);
 }
 
-constexpr int kVecThreads = 512;  // init / update / refresh / true residual
+constexpr int kVecThreads = 512;  // init / update / the sums at the end
 constexpr int kMaxWG = 1024;       // workgroups of a depth in the vector kernels (its partial count)
 constexpr int kMaxSpmvWG = 2048;   // workgroups of a depth in the SpMV (its partial count)
 constexpr int kSpmvThreads = kTileThreads;  // one row per lane, kTile sibling blocks per tile
@@ -345,10 +343,13 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* p, uint64
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, int(nr), kBufWord3);
 }
 
-template <int K>
-__global__ void __launch_bounds__(kSpmvThreads, K <= kSpmvSmallK ? 8 : (K <= 8 ? 4 : 2)) k_cg_spmv(const Seg* __restrict__ segs,
-                                                                                 int32_t nseg, int32_t it,
-                                                          float tol, int32_t fixed, int32_t max_iters) {
+// What the tile loop works out: a CG iteration's first kernel, or r = b - A x
+// of the iterate, for a refresh of the recursive residual or at the end.
+enum SpmvMode { kModeIter, kModeRefresh, kModeEnd };
+
+template <int K, int MODE>
+__device__ __forceinline__ void spmv_tiles(const Seg* __restrict__ segs, int32_t nseg, int32_t it, float tol,
+                                           int32_t fixed, int32_t max_iters) {
     static_assert(K * kSpmvThreads <= 8 * kTileEntries, "cells per thread beyond a tile's plan");
     constexpr int kRidWords = kTileEntries / 2;  // row ids as 32-bit words
     extern __shared__ float cellv[];
@@ -364,9 +365,9 @@ __global__ void __launch_bounds__(kSpmvThreads, K <= kSpmvSmallK ? 8 : (K <= 8 ?
     __shared__ float grid[(kTile / 4) * 272];
     __shared__ double lds[kSpmvThreads / 64];
     const int16_t* rid = reinterpret_cast<const int16_t*>(rid32);
-    const Seg& sg = segs[seg_of(segs, nseg, blockIdx.x, false)];
+    const Seg& sg = segs[seg_of(segs, nseg, blockIdx.x, MODE != kModeIter)];
     CgState* st = sg.st;
-    if (st->done) return;
+    if (MODE != kModeEnd && st->done) return;
     const int64_t n = sg.n;
     // p_k and q of the tile's own rows (it == 1: p_1 is already in place, the
     // empty range drops those stores)
@@ -376,7 +377,9 @@ __global__ void __launch_bounds__(kSpmvThreads, K <= kSpmvSmallK ? 8 : (K <= 8 ?
     const double* bb_part = sg.bb;
     const int32_t np = sg.nvwg;
     double* pq_part = sg.pq;
-    const int bid = int(blockIdx.x) - sg.wg0, nblocks = sg.nwg;
+    // (a residual's partials take the place of the vector kernels': their workgroups)
+    const int bid = int(blockIdx.x) - (MODE == kModeIter ? sg.wg0 : sg.vwg0);
+    const int nblocks = MODE == kModeIter ? sg.nwg : sg.nvwg;
     const int k1 = it - 1;
     const bool first = (it == 1);
     const int tid = threadIdx.x;
@@ -436,7 +439,10 @@ __global__ void __launch_bounds__(kSpmvThreads, K <= kSpmvSmallK ? 8 : (K <= 8 ?
     // when the values reach LDS, so nothing waits for these loads before the
     // next tile.  it == 1: p_1 = r (k_cg_init copies r into p), so the second
     // load reads r again and the value is taken as it is.
-    const auto rs_r = buf_rsrc(sg.R, uint64_t(n) * sizeof(float));
+    // (a residual reads x alone)
+    const auto rs_r = buf_rsrc(MODE == kModeIter ? sg.R : sg.XS, uint64_t(n) * sizeof(float));
+    const auto rs_b = buf_rsrc(sg.b, uint64_t(n) * sizeof(float));
+    const auto rs_out = buf_rsrc(MODE == kModeRefresh ? sg.R : sg.X, uint64_t(n) * sizeof(float));
     const auto rs_p = buf_rsrc(first ? sg.R : ((it & 1) ? sg.P1 : sg.P0), uint64_t(n) * sizeof(float));
     auto load_cells = [&](const Plan& P, float vr[K], float vp[K]) {
 #pragma unroll
@@ -444,25 +450,28 @@ __global__ void __launch_bounds__(kSpmvThreads, K <= kSpmvSmallK ? 8 : (K <= 8 ?
             const int u = tid + k * kSpmvThreads;
             const uint32_t off = u < 8 * P.cnt ? 4u * (uint32_t(P.ub[k]) + uint32_t(u & 7)) : kBufOob;
             vr[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs_r, off, 0, 0));
-            vp[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs_p, off, 0, 0));
+            if (MODE == kModeIter) vp[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs_p, off, 0, 0));
         }
     };
     Plan pa{}, pb{};
     float va[K], vpa[K];
     load_plan(tbeg, pa);
-    // (the first plan is in flight while the partial sums load and reduce)
-    const double rr = sum_partials<kSpmvThreads>(rr_part, np, lds);
-    const double bb = (it == 1) ? sum_partials<kSpmvThreads>(bb_part, np, lds) : st->bb;
-    const double tol2 = double(tol) * double(tol) * bb;
-    const bool stop = (bb <= 0.0) || (k1 >= max_iters) || (rr == 0.0) || (fixed > 0 ? (k1 >= fixed) : (rr <= tol2));
-    const float bf = (it == 1) ? 0.0f : float(rr / st->rr_hist[(k1 - 1) & 1]);
-    if (bid == 0 && threadIdx.x == 0) {
-        if (it == 1) st->bb = bb;
-        st->rr_hist[k1 & 1] = rr;
-        st->rr = rr;
-        if (stop) set_done(sg, k1);
+    float bf = 0.0f;
+    if (MODE == kModeIter) {
+        // (the first plan is in flight while the partial sums load and reduce)
+        const double rr = sum_partials<kSpmvThreads>(rr_part, np, lds);
+        const double bb = (it == 1) ? sum_partials<kSpmvThreads>(bb_part, np, lds) : st->bb;
+        const double tol2 = double(tol) * double(tol) * bb;
+        const bool stop = (bb <= 0.0) || (k1 >= max_iters) || (rr == 0.0) || (fixed > 0 ? (k1 >= fixed) : (rr <= tol2));
+        bf = (it == 1) ? 0.0f : float(rr / st->rr_hist[(k1 - 1) & 1]);
+        if (bid == 0 && threadIdx.x == 0) {
+            if (it == 1) st->bb = bb;
+            st->rr_hist[k1 & 1] = rr;
+            st->rr = rr;
+            if (stop) set_done(sg, k1);
+        }
+        if (stop) return;
     }
-    if (stop) return;
     load_cells(pa, va, vpa);
     load_plan(tbeg + tstep, pb);
     double pq = 0.0;
@@ -474,10 +483,18 @@ __global__ void __launch_bounds__(kSpmvThreads, K <= kSpmvSmallK ? 8 : (K <= 8 ?
         for (int k = 0; k < K; k++) {
             const int u = tid + k * kSpmvThreads;
             if (u < 8 * pa.cnt) {
-                const float tp = bf * vpa[k];
-                cellv[u] = first ? va[k] : va[k] + tp;
+                if (MODE == kModeIter) {
+                    const float tp = bf * vpa[k];
+                    cellv[u] = first ? va[k] : va[k] + tp;
+                } else {
+                    cellv[u] = va[k];
+                }
             }
         }
+        const int64_t blk = tile * kTile + g;
+        const uint32_t off = blk < nblk ? 4u * uint32_t(8 * blk + s) : kBufOob;
+        float bv = 0.0f;
+        if (MODE != kModeIter) bv = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs_b, off, 0, 0));
         load_cells(pb, va, vpa);  // free again: the next tile's values
         pa = pb;
         load_plan(tile + 2 * tstep, pb);
@@ -497,7 +514,6 @@ __global__ void __launch_bounds__(kSpmvThreads, K <= kSpmvSmallK ? 8 : (K <= 8 ?
         // stores fall outside the descriptors and are dropped, so the stores
         // are issued without a branch and the loads of the next tiles are
         // waited for by count
-        const int64_t blk = tile * kTile + g;
         {
             // absent neighbours hold +0: adding L*0 leaves a float sum
             // unchanged, so the result equals the sum over present terms
@@ -508,18 +524,49 @@ __global__ void __launch_bounds__(kSpmvThreads, K <= kSpmvSmallK ? 8 : (K <= 8 ?
                 const float prod = sg.L[j] * gc[16 * (j / 9) + 4 * ((j / 3) % 3) + (j % 3)];
                 out = out + prod;
             }
-            const uint32_t off = blk < nblk ? 4u * uint32_t(8 * blk + s) : kBufOob;
             const float pt = gc[16 + 4 + 1];
+            if (MODE != kModeIter) {
+                const float rv = bv - out;
+                const double rd = MODE == kModeRefresh ? double(rv) : double(bv) - double(out);
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(MODE == kModeRefresh ? rv : pt), rs_out, off, 0, 0);
+                const double rrt = pq + rd * rd;
+                pq = blk < nblk ? rrt : pq;
+            } else {
             __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(pt), rs_pnew, off, 0, 0);
             __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(out), rs_q, off, 0, 0);
             const double pqt = pq + double(pt) * double(out);
             pq = blk < nblk ? pqt : pq;
+            }
         }
         __syncthreads();
     }
     const double sum = block_allsum<kSpmvThreads>(pq, lds);
-    if (tid == 0) pq_part[bid] = sum;
+    if (tid == 0) {
+        double* part = MODE == kModeIter ? pq_part : MODE == kModeRefresh ? sg.rr + (it & 1) * kMaxWG : sg.bb;
+        part[bid] = sum;
+    }
 }
+
+template <int K>
+__global__ void __launch_bounds__(kSpmvThreads, K <= kSpmvSmallK ? 8 : (K <= 8 ? 4 : 2)) k_cg_spmv(
+    const Seg* __restrict__ segs, int32_t nseg, int32_t it, float tol, int32_t fixed, int32_t max_iters) {
+    spmv_tiles<K, kModeIter>(segs, nseg, it, tol, fixed, max_iters);
+}
+
+// r = b - A x (every `refresh` iterations) and its r.r partial (slot it & 1),
+// for the unfinished depths of a chain; or, at the end of a chain, one launch
+// for its depths: ||b - A x||^2 of the final iterates, one FP64 partial per
+// workgroup (FP32 SpMV, FP64 sum of squares), and the solution copied out of
+// the aligned work vector.  Through the tile plans, as the SpMV: bound by the
+// same loop, less one vector read per cell.  2 M points at depth 10 (5,565,224
+// finest rows), both chains' launches together: 59 and 58 us; row by row, with
+// 27 gathers each bound by the texture-address unit, 151 and 149 us.
+template <int K, int MODE>
+__global__ void __launch_bounds__(kSpmvThreads, K <= kSpmvSmallK ? 8 : (K <= 8 ? 4 : 2)) k_cg_residual(
+    const Seg* __restrict__ segs, int32_t nseg, int32_t it) {
+    spmv_tiles<K, MODE>(segs, nseg, it, 0.0f, 0, 0);
+}
+
 
 // CG iteration `it`, second kernel: alpha = rr_{it-1} / p.q (every workgroup
 // sums the p.q partials; p.q <= 0 after the residual vanished stops the
@@ -583,52 +630,6 @@ __global__ void __launch_bounds__(kVecThreads) k_cg_update(const Seg* __restrict
         if (threadIdx.x == 0) rr_part[bid] = sum;
     }
     if (bid == 0 && threadIdx.x == 0) st->iters = it;
-}
-
-// r = b - A x (every `refresh` iterations) and its r.r partial (slot it & 1),
-// for the unfinished depths of a chain
-__global__ void __launch_bounds__(kVecThreads) k_cg_refresh(const Seg* __restrict__ segs, int32_t nseg, int32_t it) {
-    __shared__ double lds[kVecThreads / 64];
-    const Seg& sg = segs[seg_of(segs, nseg, blockIdx.x, true)];
-    if (sg.st->done) return;
-    const int64_t n = sg.n;
-    const int bid = int(blockIdx.x) - sg.vwg0;
-    const int32_t* pnt = sg.pnt;
-    const float *b = sg.b, *x = sg.XS;
-    float* r = sg.R;
-    const Stencil S = seg_stencil(sg);
-    double rr = 0.0;
-    for (int64_t t = int64_t(bid) * kVecThreads + threadIdx.x; t < n; t += int64_t(sg.nvwg) * kVecThreads) {
-        const float ax = spmv_pnt(pnt, t, x, S);
-        const float rv = b[t] - ax;
-        r[t] = rv;
-        rr += double(rv) * double(rv);
-    }
-    const double sum = block_allsum<kVecThreads>(rr, lds);
-    if (threadIdx.x == 0) sg.rr[(it & 1) * kMaxWG + bid] = sum;
-}
-
-// The end of a chain, one launch for its depths: ||b - A x||^2 of the final
-// iterates, one FP64 partial per workgroup (FP32 SpMV, FP64 sum of squares),
-// and the solution copied out of the aligned work vector.
-__global__ void __launch_bounds__(kVecThreads) k_true_residual(const Seg* __restrict__ segs, int32_t nseg) {
-    __shared__ double lds[kVecThreads / 64];
-    const Seg& sg = segs[seg_of(segs, nseg, blockIdx.x, true)];
-    const int64_t n = sg.n;
-    const int bid = int(blockIdx.x) - sg.vwg0;
-    const int32_t* pnt = sg.pnt;
-    const float *b = sg.b, *x = sg.XS;
-    float* X = sg.X;
-    const Stencil S = seg_stencil(sg);
-    double rr = 0.0;
-    for (int64_t t = int64_t(bid) * kVecThreads + threadIdx.x; t < n; t += int64_t(sg.nvwg) * kVecThreads) {
-        const float ax = spmv_pnt(pnt, t, x, S);
-        X[t] = x[t];
-        const double rv = double(b[t]) - double(ax);
-        rr += rv * rv;
-    }
-    const double sum = block_allsum<kVecThreads>(rr, lds);
-    if (threadIdx.x == 0) sg.bb[bid] = sum;
 }
 
 // One workgroup per depth of a chain: ||b - A x|| / ||b|| from the
@@ -931,6 +932,20 @@ void launch_spmv(int inst, int32_t nwg, size_t lds, hipStream_t s, const Seg* se
         default: PRG_SPMV(27); break;
     }
 #undef PRG_SPMV
+    PRG_CHECK_LAUNCH();
+}
+
+template <int MODE>
+void launch_residual(int inst, int32_t nwg, size_t lds, hipStream_t s, const Seg* segs, int32_t nseg, int32_t it) {
+#define PRG_RES(KC) k_cg_residual<KC, MODE><<<nwg, kSpmvThreads, lds, s>>>(segs, nseg, it)
+    switch (inst) {
+        case 0: PRG_RES(2); break;
+        case 1: PRG_RES(4); break;
+        case 2: PRG_RES(8); break;
+        case 4: PRG_RES(5); break;
+        default: PRG_RES(27); break;
+    }
+#undef PRG_RES
     PRG_CHECK_LAUNCH();
 }
 
@@ -1273,10 +1288,9 @@ prg_status solve_all(prg_ctx* c, prg_solve_stats* stats) {
                 PRG_CHECK_LAUNCH();
             }
             if ((it % refresh) == 0) {
-                TimedScope ts(c->kt, "cg_refresh", kResidualRowBytes * double(rows));
+                TimedScope ts(c->kt, "cg_refresh", spmv_bytes - 4.0 * double(rows));  // x, b read; r written
                 h.launched.emplace_back(ts.idx, it);
-                k_cg_refresh<<<h.nvwg, kVecThreads, 0, h.s>>>(dseg + h.seg0, cnt, it);
-                PRG_CHECK_LAUNCH();
+                launch_residual<kModeRefresh>(h.inst, h.nvwg, h.lds, h.s, dseg + h.seg0, cnt, it);
             }
         };
         auto chain_done = [&](const Chain& h) {
@@ -1289,12 +1303,11 @@ prg_status solve_all(prg_ctx* c, prg_solve_stats* stats) {
         // superseding these, if more iterations follow).
         auto end_batch = [&](Chain& h) {
             double bytes = 0.0;
-            for (int d : h.depths) bytes += kResidualRowBytes * double(c->counts[d]);
+            for (int d : h.depths) bytes += spmv_plan_bytes(c, d) - 4.0 * double(c->counts[d]);  // x, b read; x written
             {
                 TimedScope ts(c->kt, "cg_true_residual", bytes);
                 h.end_idx = ts.idx;
-                k_true_residual<<<h.nvwg, kVecThreads, 0, h.s>>>(dseg + h.seg0, int32_t(h.depths.size()));
-                PRG_CHECK_LAUNCH();
+                launch_residual<kModeEnd>(h.inst, h.nvwg, h.lds, h.s, dseg + h.seg0, int32_t(h.depths.size()), 0);
             }
             k_true_residual_finish<<<unsigned(h.depths.size()), kVecThreads, 0, h.s>>>(dseg + h.seg0);
             PRG_CHECK_LAUNCH();

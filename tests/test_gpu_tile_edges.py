@@ -71,3 +71,24 @@ def test_weld_at_tile_edges(prg, n, values):
                 assert removed == oremoved and m.n_leaf_vertices == onleaf
                 assert np.array_equal(m.vertices.view(np.uint32), ov.view(np.uint32))
                 assert np.array_equal(m.triangles, ot)
+
+
+@pytest.mark.parametrize("n,depth,refresh", [(900, 6, 1), (3000, 7, 1), (3000, 7, 3), (60000, 7, 2), (20000, 8, 4)])
+def test_residual_refresh_on_tiles(prg, n, depth, refresh):
+    """Solves that recompute r = b - A x every few iterations, ten iterations on
+    both sides (the tolerance of the solve without a refresh)."""
+    print(f"\n[refresh: {n} points at depth {depth}, every {refresh}]", flush=True)
+    p, q = prg.synth_torus(n, n)
+    g, o = _both(prg, p, q, depth)
+    g.close()
+    o.compute_divergence()
+    with prg.Reconstructor(max_depth=depth, cg_fixed_iters=10, cg_refresh=refresh) as g2:
+        g2.set_points(p, q)
+        g2.build_octree()
+        g2.write_buffer(prg.BUF_DIVERGENCE, o.read_buffer(prg.BUF_DIVERGENCE))
+        g2.solve()
+        xg = g2.read_buffer(prg.BUF_SOLUTION).astype(np.float64)
+    o.solve(mode=0, refresh=refresh, fixed_iters=10)
+    xo = o.read_buffer(prg.BUF_SOLUTION).astype(np.float64)
+    assert np.linalg.norm(xg - xo) <= 1e-5 * np.linalg.norm(xo)
+    o.close()
