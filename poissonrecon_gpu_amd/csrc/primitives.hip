@@ -18,9 +18,15 @@
 namespace prg {
 namespace {
 
-constexpr int kScanBlock = 256;
 constexpr int kScanItems = 16;  // consecutive elements per thread
-constexpr int kScanTile = kScanBlock * kScanItems;
+
+// Threads of a scan's workgroups: a tile costs about 50 ns of its own in the
+// chain of tiles (the ticket, the look-back), so beyond 2^20 elements a tile is
+// four times as large (5.6 M elements: 81 us with 1,359 tiles of 4,096, 51 us
+// with a quarter of them; two arrays 55 and 42); below, the smaller ones give
+// the chip more workgroups.
+constexpr int kScanSmall = 256, kScanLarge = 1024;
+int scan_block(int64_t n) { return n > (int64_t(1) << 20) ? kScanLarge : kScanSmall; }
 
 // v[k] = in[base + k], 0 from n on; `wide`: 16-byte loads where all are in range
 __device__ __forceinline__ int32_t load_items(const int32_t* __restrict__ in, int64_t base, int64_t n, bool wide,
@@ -59,15 +65,15 @@ __device__ __forceinline__ void store_items(int32_t* __restrict__ out, int64_t b
 // Exclusive scan of one array, or of two of the same length (TWO), in one
 // launch (lookback.h).  Bound by its launch (about 4 us) up to about 10^5
 // elements, then by the memory it reads and writes once.
-template <bool TWO>
-__global__ void __launch_bounds__(kScanBlock) k_scan(const int32_t* in_a, int32_t* out_a, int32_t* total_a,
+template <bool TWO, int BLOCK>
+__global__ void __launch_bounds__(BLOCK) k_scan(const int32_t* in_a, int32_t* out_a, int32_t* total_a,
                                                      const int32_t* in_b, int32_t* out_b, int32_t* total_b, int64_t n,
                                                      uint32_t tiles, bool wide, uint64_t* state) {
-    __shared__ int32_t w[kScanBlock / 64];
+    __shared__ int32_t w[BLOCK / 64];
     __shared__ int32_t before[2];
     const LookTile t = look_begin(state, tiles);
     if (t.tile >= tiles) return;  // (uniform; only if the state was damaged from outside)
-    const int64_t base = int64_t(t.tile) * kScanTile + int64_t(threadIdx.x) * kScanItems;
+    const int64_t base = int64_t(t.tile) * (BLOCK * kScanItems) + int64_t(threadIdx.x) * kScanItems;
     int32_t va[kScanItems], vb[kScanItems];
     const int32_t sa = load_items(in_a, base, n, wide, va);
     const int32_t sb = TWO ? load_items(in_b, base, n, wide, vb) : 0;
@@ -223,12 +229,14 @@ void scan_exclusive(const int32_t* d_in, int32_t* d_out, int64_t n, int32_t* d_t
         if (d_total) PRG_HIP(hipMemsetAsync(d_total, 0, sizeof(int32_t), s));
         return;
     }
-    const int64_t tiles = (n + kScanTile - 1) / kScanTile;
+    const int block = scan_block(n), tile = block * kScanItems;
+    const int64_t tiles = (n + tile - 1) / tile;
     uint64_t* state = look_state(scratch, tiles, s);
     const bool wide = ((reinterpret_cast<uintptr_t>(d_in) | reinterpret_cast<uintptr_t>(d_out)) & 15) == 0;
     TimedScope ts(kt, "scan_exclusive", 8.0 * double(n));
-    k_scan<false><<<unsigned(tiles), kScanBlock, 0, s>>>(d_in, d_out, d_total, nullptr, nullptr, nullptr, n,
-                                                         uint32_t(tiles), wide, state);
+    const auto kernel = block == kScanLarge ? k_scan<false, kScanLarge> : k_scan<false, kScanSmall>;
+    kernel<<<unsigned(tiles), block, 0, s>>>(d_in, d_out, d_total, nullptr, nullptr, nullptr, n, uint32_t(tiles), wide,
+                                             state);
     PRG_CHECK_LAUNCH();
 }
 
@@ -239,13 +247,15 @@ void scan_exclusive2(const int32_t* a_in, int32_t* a_out, int32_t* a_total, cons
         scan_exclusive(b_in, b_out, n, b_total, s, scratch, kt);
         return;
     }
-    const int64_t tiles = (n + kScanTile - 1) / kScanTile;
+    const int block = scan_block(n), tile = block * kScanItems;
+    const int64_t tiles = (n + tile - 1) / tile;
     uint64_t* state = look_state(scratch, 2 * tiles, s);
     const bool wide = ((reinterpret_cast<uintptr_t>(a_in) | reinterpret_cast<uintptr_t>(a_out) |
                         reinterpret_cast<uintptr_t>(b_in) | reinterpret_cast<uintptr_t>(b_out)) & 15) == 0;
     TimedScope ts(kt, "scan_exclusive", 16.0 * double(n));
-    k_scan<true><<<unsigned(tiles), kScanBlock, 0, s>>>(a_in, a_out, a_total, b_in, b_out, b_total, n, uint32_t(tiles),
-                                                        wide, state);
+    const auto kernel = block == kScanLarge ? k_scan<true, kScanLarge> : k_scan<true, kScanSmall>;
+    kernel<<<unsigned(tiles), block, 0, s>>>(a_in, a_out, a_total, b_in, b_out, b_total, n, uint32_t(tiles), wide,
+                                             state);
     PRG_CHECK_LAUNCH();
 }
 

@@ -247,21 +247,25 @@ __global__ void __launch_bounds__(kBlockS) k_sub_init(int32_t* cnt, uint8_t* int
 }
 
 constexpr int kSelItems = 16;
-constexpr int kSelTile = kBlockS * kSelItems;
+// Beyond 2^20 elements a tile is four times as large: each costs about 50 ns of
+// its own in the chain of tiles (12.4 M marks: 164 us with 3,021 tiles of 4,096,
+// 52 us with a quarter of them; 1.5 M nodes 15 and 12).
+constexpr int kSelSmall = kBlockS, kSelLarge = 4 * kBlockS;
+int select_block(int64_t n) { return n > (int64_t(1) << 20) ? kSelLarge : kSelSmall; }
 
 // In one launch (lookback.h), the list of the i < n with a mark, in order:
 // LEAF: the coarse leaves (no children; the root is none), from child_base;
 // else: the bytes of `marks` that are not 0, and each one's place in nid.
-template <bool LEAF>
-__global__ void __launch_bounds__(kBlockS) k_select(const int32_t* __restrict__ child_base,
+template <bool LEAF, int BLOCK>
+__global__ void __launch_bounds__(BLOCK) k_select(const int32_t* __restrict__ child_base,
                                                     const uint8_t* __restrict__ marks, int64_t n, uint32_t tiles,
                                                     uint64_t* state, int32_t* __restrict__ list,
                                                     int32_t* __restrict__ nid, int32_t* count) {
-    __shared__ int32_t lds[kBlockS / 64];
+    __shared__ int32_t lds[BLOCK / 64];
     __shared__ int32_t s_before;
     const LookTile t = look_begin(state, tiles);
     if (t.tile >= tiles) return;
-    const int64_t base = int64_t(t.tile) * kSelTile + int64_t(threadIdx.x) * kSelItems;
+    const int64_t base = int64_t(t.tile) * (BLOCK * kSelItems) + int64_t(threadIdx.x) * kSelItems;
     uint32_t m = 0;
     if (LEAF) {
         int32_t v[kSelItems];
@@ -2398,10 +2402,11 @@ void extract_subdivision(prg_ctx* c) {
     cl.reserve(baseD);
     auto select_tiles = [&](int64_t n, int tile) { return uint32_t((n + tile - 1) / tile); };
     {
-        const uint32_t tiles = select_tiles(baseD, kSelTile);
+        const int block = select_block(baseD);
+        const uint32_t tiles = select_tiles(baseD, block * kSelItems);
         uint64_t* state = look_state(c->scratch, tiles, s);
-        k_select<true><<<tiles, kBlockS, 0, s>>>(c->child_base.get(), nullptr, baseD, tiles, state, cl.get(), nullptr,
-                                                 C + kCntCoarse);
+        (block == kSelLarge ? k_select<true, kSelLarge> : k_select<true, kSelSmall>)<<<tiles, block, 0, s>>>(
+            c->child_base.get(), nullptr, baseD, tiles, state, cl.get(), nullptr, C + kCntCoarse);
         PRG_CHECK_LAUNCH();
     }
     // their corner values
@@ -2413,10 +2418,11 @@ void extract_subdivision(prg_ctx* c) {
                                                                             c->pnt.get(), Lv, D, oref.get(), need.get());
     PRG_CHECK_LAUNCH();
     {
-        const uint32_t tiles = select_tiles(8 * baseD, kSelTile);
+        const int block = select_block(8 * baseD);
+        const uint32_t tiles = select_tiles(8 * baseD, block * kSelItems);
         uint64_t* state = look_state(c->scratch, tiles, s);
-        k_select<false><<<tiles, kBlockS, 0, s>>>(nullptr, need.get(), 8 * baseD, tiles, state, clist.get(), nid.get(),
-                                                  C + kCntCorners);
+        (block == kSelLarge ? k_select<false, kSelLarge> : k_select<false, kSelSmall>)<<<tiles, block, 0, s>>>(
+            nullptr, need.get(), 8 * baseD, tiles, state, clist.get(), nid.get(), C + kCntCorners);
         PRG_CHECK_LAUNCH();
     }
     {

@@ -57,6 +57,16 @@ def test_small_roots_bit_exact(D, count, prg):
     _check_full_mesh("random", p, n, D, prg)
 
 
+@pytest.mark.parametrize("height", [0.77, 0.81])
+def test_selection_tile_sizes(height, prg):
+    """Clouds whose corner marks (eight per node above the leaf level) lie
+    below and above the 2^20 where the selection's tiles change size."""
+    rng = np.random.default_rng(7)
+    p = (rng.random((60000, 3)) * [1.0, 1.0, height]).astype(np.float32)
+    n = rng.standard_normal((60000, 3)).astype(np.float32)
+    _check_full_mesh("volume", p, n, 7, prg)
+
+
 def _check_full_mesh(name, p, n, D, prg):
     print(f"\n[case {name}: N={len(p)} D={D}]", flush=True)
     o = orc.Oracle(D)
