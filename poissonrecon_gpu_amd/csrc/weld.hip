@@ -39,9 +39,13 @@ __device__ __forceinline__ uint32_t hash_position(uint32_t x, uint32_t y, uint32
     return h ^ (h >> 16);
 }
 
-// the table empty, the counts of the call cleared
-__global__ void __launch_bounds__(kBlock) k_weld_init(int32_t* table, int64_t words, int32_t* host_counts) {
+// the table empty, the counts of the call cleared, and `look_words` words of
+// the scan's state (none of a context's, whose calls cannot overlap)
+__global__ void __launch_bounds__(kBlock) k_weld_init(int32_t* table, int64_t words, int32_t* host_counts,
+                                                      uint64_t* look, int look_words) {
     if (blockIdx.x == 0 && threadIdx.x < 3) host_counts[threadIdx.x] = 0;
+    if (blockIdx.x == 0)
+        for (int i = threadIdx.x; i < look_words; i += kBlock) look[i] = 0;
     int4* t4 = reinterpret_cast<int4*>(table);  // (a multiple of 4 words)
     for (int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x; i < words / 4; i += int64_t(gridDim.x) * kBlock)
         t4[i] = make_int4(-1, -1, -1, -1);
@@ -148,18 +152,19 @@ uint64_t table_slots(int64_t n) {
     return h;
 }
 
-// The weld proper on device arrays `b`, with the scan's state in `scr`.  The
-// triangles go up on the second stream, beside the vertices' kernels.
-void weld_core(prg_ctx* c, const WeldBufs& b, Scratch& scr, float* vertices, int64_t n, int32_t* triangles,
-               int64_t m, int64_t n_leaf, int64_t* n_out, int64_t* n_leaf_out) {
+// The weld proper on device arrays `b`, with the scan's state in `scr`, of
+// which the first `look_words` words are cleared first.  The triangles go up
+// on the second stream, beside the vertices' kernels.
+void weld_core(prg_ctx* c, const WeldBufs& b, Scratch& scr, int look_words, float* vertices, int64_t n,
+               int32_t* triangles, int64_t m, int64_t n_leaf, int64_t* n_out, int64_t* n_leaf_out) {
     hipStream_t s = c->stream;
     const uint64_t slots = table_slots(n);
     volatile int32_t* counts = c->sub_host + kWeldHost;  // kept vertices; kept among the first n_leaf; bad triangles
     const uint32_t tiles = uint32_t((n + kKeepTile - 1) / kKeepTile);
     uint64_t* state = look_state(scr, tiles, s);
     PRG_HIP(hipMemcpyAsync(b.V, vertices, size_t(3 * n) * 4, hipMemcpyHostToDevice, s));
-    k_weld_init<<<unsigned(std::min<uint64_t>(2048, slots / 1024 + 1)), kBlock, 0, s>>>(b.table, int64_t(slots),
-                                                                                      c->sub_host + kWeldHost);
+    k_weld_init<<<unsigned(std::min<uint64_t>(2048, slots / 1024 + 1)), kBlock, 0, s>>>(
+        b.table, int64_t(slots), c->sub_host + kWeldHost, state, look_words);
     PRG_CHECK_LAUNCH();
     k_weld_insert<<<grid_for(n, kBlock), kBlock, 0, s>>>(b.V, n, uint32_t(slots - 1), b.table, b.place);
     PRG_CHECK_LAUNCH();
@@ -178,6 +183,7 @@ void weld_core(prg_ctx* c, const WeldBufs& b, Scratch& scr, float* vertices, int
     PRG_HIP(hipStreamSynchronize(s));
     if (counts[2]) throw Error{PRG_E_ARG, "triangle index out of range"};  // the mesh is as it was
     const int64_t kept = counts[0];
+    if (kept < 1 || kept > n) throw Error{PRG_E_HIP, "weld: inconsistent vertex count"};  // the mesh is as it was
     PRG_HIP(hipMemcpyAsync(vertices, b.out, size_t(3 * kept) * 4, hipMemcpyDeviceToHost, s));
     if (m > 0) PRG_HIP(hipMemcpyAsync(triangles, b.T, size_t(3 * m) * 4, hipMemcpyDeviceToHost, s));
     PRG_HIP(hipStreamSynchronize(s));  // the device arrays are reused or freed after return
@@ -233,7 +239,7 @@ void weld_mesh(prg_ctx* c, float* vertices, int64_t n, int32_t* triangles, int64
     const size_t slots = size_t(table_slots(n));
     WeldBufs b{V.reserve(size_t(3 * n)), out.reserve(size_t(3 * n)), table.reserve(slots),
                number.reserve(slots),    place.reserve(size_t(n)),   m > 0 ? T.reserve(size_t(3 * m)) : nullptr};
-    weld_core(c, b, c->scratch, vertices, n, triangles, m, n_leaf, n_out, n_leaf_out);
+    weld_core(c, b, c->scratch, 0, vertices, n, triangles, m, n_leaf, n_out, n_leaf_out);
 }
 
 void weld_mesh_noalloc(prg_ctx* c, float* vertices, int64_t n, int32_t* triangles, int64_t m, int64_t n_leaf,
@@ -260,8 +266,9 @@ void weld_mesh_noalloc(prg_ctx* c, float* vertices, int64_t n, int32_t* triangle
     b.place = reinterpret_cast<uint32_t*>(take(4 * N));
     b.T = reinterpret_cast<int32_t*>(take(12 * kNoAllocTriangles));
     // the scan's state, lent to a Scratch whose buffer never grows past this
-    // capacity (so it is never reallocated or freed).  (It is zero when the
-    // library loads, and every scan leaves it ready for the next.)
+    // capacity (so it is never reallocated or freed).  Calls that overlap on
+    // a device race for the array, and what they leave in the state would spoil
+    // every later call, so each call clears it (2 KB, in its first kernel).
     Scratch scr;
     struct Lend {
         Scratch& s;
@@ -273,7 +280,7 @@ void weld_mesh_noalloc(prg_ctx* c, float* vertices, int64_t n, int32_t* triangle
     scr.look.p = reinterpret_cast<uint64_t*>(take(8 * kLookWords));
     scr.look.n = size_t(kLookWords);
     if (off > kNoAllocBytes) throw Error{PRG_E_HIP, "weld array layout exceeds its size"};
-    weld_core(c, b, scr, vertices, n, triangles, m, n_leaf, n_out, n_leaf_out);
+    weld_core(c, b, scr, int(kLookWords), vertices, n, triangles, m, n_leaf, n_out, n_leaf_out);
 }
 
 }  // namespace prg
