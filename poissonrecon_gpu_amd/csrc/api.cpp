@@ -139,14 +139,19 @@ prg_status prg_create(prg_ctx** out, const prg_config* cfg) {
             PRG_HIP(hipEventCreate(&e[0]));
             PRG_HIP(hipEventCreate(&e[1]));
         }
-        // one pinned allocation: the solver's area, the subdivision's counters, the transform
-        PRG_HIP(hipHostMalloc(&c->cg_host, prg::kCgHostBytes + 256 + 16, hipHostMallocCoherent));
+        // one pinned allocation: the solver's area, the subdivision's counters, the transform, the scans' error flags
+        PRG_HIP(hipHostMalloc(&c->cg_host, prg::kCgHostBytes + 256 + 16 + 8, hipHostMallocCoherent));
         c->sub_host = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(c->cg_host) + prg::kCgHostBytes);
         c->transform_host = reinterpret_cast<float*>(c->sub_host + 64);
+        int32_t* look_error = c->sub_host + 68;
+        look_error[0] = look_error[1] = 0;
+        c->scratch.look_error = look_error;
+        c->scratch2.look_error = look_error + 1;
         PRG_HIP(hipDeviceGetAttribute(&c->num_cu, hipDeviceAttributeMultiprocessorCount, cf.device));
         prg::weld_noalloc_scratch(cf.device);  // the fixed weld array's address on this device, once
         if (const char* lim = std::getenv("PRG_TILE_LDS_LIMIT")) c->tile_limit = std::max(0, std::atoi(lim));
         if (const char* ev = std::getenv("PRG_SUBDIVIDE_EVALUATE_ALL")) c->sub_certify = std::atoi(ev) == 0;
+        if (const char* sp = std::getenv("PRG_WELD_SPINS")) c->weld_spins = uint32_t(std::max(0, std::atoi(sp)));
         if (const char* ws = std::getenv("PRG_WARM_START_SCALE")) c->warm_scale = float(std::atof(ws));
         c->kt.enabled = cf.timing != 0;
         c->kt.stream = c->stream;

@@ -244,8 +244,18 @@ struct Scratch;  // grows on demand
 // two arrays of the same length (exclusive scans and totals), in one pass each
 void scan_exclusive2(const int32_t* a_in, int32_t* a_out, int32_t* a_total, const int32_t* b_in, int32_t* b_out,
                      int32_t* b_total, int64_t n, hipStream_t s, Scratch& scratch, KernelTimer& kt);
-// the state of the single-pass scans of one stream, with room for `words` tiles
-uint64_t* look_state(Scratch& scratch, int64_t words, hipStream_t s);
+// The state of the single-pass scans of one stream, as their kernels take it.
+struct LookState {
+    uint64_t* words;
+    int32_t* error;  // pinned: set by a tile that could not do its part
+    uint32_t spins;  // polls before a wait for another tile gives up
+};
+constexpr uint32_t kLookSpins = 1u << 22;  // seconds: every tile waited for runs already
+// ... with room for `words` tiles
+LookState look_state(Scratch& scratch, int64_t words, hipStream_t s);
+// Where the host has waited for scans of this state on stream s: throws if
+// one failed (the state is ready for the next).
+void look_check(Scratch& scratch, hipStream_t s);
 void scan_exclusive(const int32_t* d_in, int32_t* d_out, int64_t n, int32_t* d_total, hipStream_t s,
                     Scratch& scratch, KernelTimer& kt);
 // Stable LSD radix sort of (key, value) pairs on the low `bits` bits of the key.
@@ -255,6 +265,7 @@ void radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32
 
 struct Scratch {
     DBuf<uint64_t> look;  // the single-pass scans' state (look_state)
+    int32_t* look_error = nullptr;
     DBuf<int32_t> b, c;
     DBuf<uint8_t> bytes;
 };

@@ -137,13 +137,17 @@ struct prg_ctx {
     std::vector<hipEvent_t> ev_pool;  // the solver's events, reused across solves
     int num_cu = 0;                   // compute units of the device
     void* cg_host = nullptr;          // pinned, kCgHostBytes: CG state read-backs, plan counts, the segment table's staging
-    int32_t* sub_host = nullptr;      // pinned, 64 ints: the subdivision's counters
+    int32_t* sub_host = nullptr;      // pinned, 64 ints: the subdivision's counters (the transform and the scans' error flags behind them)
     // test setting (environment PRG_TILE_LDS_LIMIT at creation): caps the
     // listed blocks and points the leaf-level tile kernels stage in LDS, so
     // their per-row and global-memory paths run on ordinary inputs
     int32_t tile_limit = 0;
     // test knob (PRG_SUBDIVIDE_EVALUATE_ALL=1): evaluate every subdivision brick, no certificates
     bool sub_certify = true;
+    // test knob (PRG_WELD_SPINS): polls before a tile of the weld's scan gives up
+    // on the tiles before it (0: at once; the weld then reports PRG_E_HIP).
+    // The weld alone: nothing it runs indexes by what such a scan leaves.
+    uint32_t weld_spins = prg::kLookSpins;
     // test knob (PRG_WARM_START_SCALE): multiplies the learned warm start's prediction
     float warm_scale = 1.0f;
     // last solve: the warm-started depth (-1: none) and whether its start was

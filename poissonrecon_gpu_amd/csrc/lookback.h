@@ -30,17 +30,26 @@ struct LookTile {
     uint32_t tile, tag;
 };
 
-// The calling workgroup's tile number and the launch's tag (every thread).
-__device__ __forceinline__ LookTile look_begin(uint64_t* state, uint32_t tiles) {
+// A tile that cannot do its part: the launch's results are wrong, and the
+// host, which looks at the flag where it waits for them (look_check), says so.
+__device__ __forceinline__ void look_failed(const LookState& state) {
+    __hip_atomic_store(state.error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The calling workgroup's tile number and the launch's tag (every thread).  A
+// number past the launch's tiles (only if the state was damaged from outside)
+// is reported; the workgroup returns.
+__device__ __forceinline__ LookTile look_begin(const LookState& state, uint32_t tiles) {
     __shared__ LookTile t;
     if (threadIdx.x == 0) {
         if (tiles == 1) {
             t = LookTile{0, 0};
         } else {
-            uint32_t* h = reinterpret_cast<uint32_t*>(state);
+            uint32_t* h = reinterpret_cast<uint32_t*>(state.words);
             const uint32_t e = __hip_atomic_load(h + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             t.tile = __hip_atomic_fetch_add(h, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             t.tag = e + 1 < 0x3fffffffu ? e + 1 : 1;  // (never 0, the cleared words' tag)
+            if (t.tile >= tiles) look_failed(state);
         }
     }
     __syncthreads();
@@ -48,9 +57,11 @@ __device__ __forceinline__ LookTile look_begin(uint64_t* state, uint32_t tiles) 
 }
 
 // Called by one whole wave: publishes the tile's sum and returns the sum of
-// the tiles before it (every lane).
-__device__ __forceinline__ int32_t look_back(uint64_t* words, LookTile t, uint32_t tiles, int32_t sum) {
+// the tiles before it (every lane).  `row`: which of the launch's sums, each
+// with `tiles` words of its own.
+__device__ __forceinline__ int32_t look_back(const LookState& state, int row, LookTile t, uint32_t tiles, int32_t sum) {
     if (tiles == 1) return 0;
+    uint64_t* words = state.words + kLookHeader + int64_t(row) * tiles;
     const int lane = threadIdx.x & 63;
     const uint64_t tag = uint64_t(t.tag) << 34;
     if (lane == 0)
@@ -60,8 +71,9 @@ __device__ __forceinline__ int32_t look_back(uint64_t* words, LookTile t, uint32
     int32_t before = 0;
     int64_t top = int64_t(t.tile) - 1;  // the nearest tile not yet added
     // (bounded: every tile looked at has started, so its word comes; the bound
-    // ends the wave if the state was damaged from outside)
-    for (uint32_t spin = 0; spin < (1u << 22); spin++) {
+    // ends the wave, and reports it, if the state was damaged from outside)
+    bool found = false;
+    for (uint32_t spin = 0; spin < state.spins; spin++) {
         const int64_t i = top - lane;
         const uint64_t w =
             i >= 0 ? __hip_atomic_load(words + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
@@ -77,9 +89,13 @@ __device__ __forceinline__ int32_t look_back(uint64_t* words, LookTile t, uint32
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
         before += v;
-        if (pm) break;
+        if (pm) {
+            found = true;
+            break;
+        }
         top -= 64;
     }
+    if (!found && lane == 0) look_failed(state);
     if (lane == 0)
         __hip_atomic_store(words + t.tile, tag | (uint64_t(kLookPrefix) << 32) | uint32_t(before + sum),
                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -88,9 +104,9 @@ __device__ __forceinline__ int32_t look_back(uint64_t* words, LookTile t, uint32
 
 // After every look_back of the workgroup (a barrier in between): the last
 // tile to finish readies the state for the next launch.
-__device__ __forceinline__ void look_end(uint64_t* state, LookTile t, uint32_t tiles) {
+__device__ __forceinline__ void look_end(const LookState& state, LookTile t, uint32_t tiles) {
     if (tiles == 1 || threadIdx.x != 0) return;
-    uint32_t* h = reinterpret_cast<uint32_t*>(state);
+    uint32_t* h = reinterpret_cast<uint32_t*>(state.words);
     if (__hip_atomic_fetch_add(h + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == tiles - 1) {
         __hip_atomic_store(h, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(h + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -547,8 +547,12 @@ void extract_leaf_mesh(prg_ctx* c) {
     if (c->topo_gen != c->tree_gen) start_topology(c);
     if (c->topo_pending) {
         PRG_HIP(hipEventSynchronize(c->topo_ev));
-        c->topo_corners = *topo_count_host(c);
         c->topo_pending = false;
+        c->topo_gen = ~uint64_t(0);  // to be made again if its scan failed
+        if (kt.enabled) look_check(c->scratch, s);
+        else look_check(c->scratch2, c->stream2);
+        c->topo_gen = c->tree_gen;
+        c->topo_corners = *topo_count_host(c);
     }
     const int32_t V = c->topo_corners;
     bool direct = false;
@@ -590,6 +594,7 @@ void extract_leaf_mesh(prg_ctx* c) {
         }
         scan_exclusive2(ecount.get(), ebase.get(), counts, ntri.get(), toff.get(), counts + 1, MD, s, c->scratch, kt);
         PRG_HIP(hipStreamSynchronize(s));
+        look_check(c->scratch, s);
         NV = counts[0];
         NT = counts[1];
         float* MV = c->mesh_v.reserve(size_t(3) * NV);

@@ -203,7 +203,7 @@ __global__ void __launch_bounds__(kBlock) k_gather_points(const uint32_t* perm, 
 constexpr int kRunItems = 16;
 constexpr int kRunTile = kBlock * kRunItems;
 __global__ void __launch_bounds__(kBlock) k_unique(const uint32_t* __restrict__ key, int64_t n, uint32_t tiles,
-                                                   uint64_t* state, int32_t* __restrict__ rank,
+                                                   LookState state, int32_t* __restrict__ rank,
                                                    uint32_t* __restrict__ uk, int32_t* __restrict__ upidx,
                                                    int32_t* count) {
     __shared__ int32_t lds[kBlock / 64];
@@ -227,7 +227,7 @@ __global__ void __launch_bounds__(kBlock) k_unique(const uint32_t* __restrict__ 
     int32_t total;
     const int32_t ex = block_exclusive_scan(__popc(heads), lds, total);
     if (threadIdx.x < 64) {
-        const int32_t b = look_back(state + kLookHeader, t, tiles, total);
+        const int32_t b = look_back(state, 0, t, tiles, total);
         if (threadIdx.x == 0) {
             s_before = b;
             if (t.tile == tiles - 1) *count = b + total;
@@ -372,7 +372,7 @@ constexpr int kLvlItems = 8;
 constexpr int kLvlTile = kLvlBlock * kLvlItems;
 
 __global__ void __launch_bounds__(kLvlBlock) k_level_up(const uint32_t* nk, const int32_t* np, const int32_t* ndi,
-                                                        int32_t* ne, int hs, int D, int d, uint64_t* state,
+                                                        int32_t* ne, int hs, int D, int d, LookState state,
                                                         int32_t* pos, uint32_t* pk, int32_t* pp, int32_t* pdi) {
     __shared__ int32_t lds[kLvlBlock / 64];
     __shared__ int32_t s_before;
@@ -404,7 +404,7 @@ __global__ void __launch_bounds__(kLvlBlock) k_level_up(const uint32_t* nk, cons
     int32_t tot;
     int32_t ex = block_exclusive_scan(acc, lds, tot);
     if (threadIdx.x < 64) {
-        const int32_t b = look_back(state + kLookHeader, t, tiles, tot);
+        const int32_t b = look_back(state, 0, t, tiles, tot);
         if (threadIdx.x == 0) {
             s_before = b;
             if (t.tile == tiles - 1) ne[d - 1] = b + tot;
@@ -709,7 +709,7 @@ void build_octree(prg_ctx* c) {
     {
         TimedScope ts(kt, "unique", 16.0 * double(n));
         const int64_t tiles = (n + kRunTile - 1) / kRunTile;
-        uint64_t* state = look_state(c->scratch, tiles, s);
+        const LookState state = look_state(c->scratch, tiles, s);
         k_unique<<<unsigned(tiles), kBlock, 0, s>>>(key.get(), n, uint32_t(tiles), state, rank.get(), NK[D]->get(),
                                                     NP[D]->get(), ne_dev.get() + D);
         PRG_CHECK_LAUNCH();
@@ -727,7 +727,7 @@ void build_octree(prg_ctx* c) {
         NDI[d - 1]->reserve(ub[d - 1]);
         POS[d]->reserve(ub[d]);
         const int64_t tiles = (ub[d] + kLvlTile - 1) / kLvlTile;
-        uint64_t* state = look_state(c->scratch, tiles, s);
+        const LookState state = look_state(c->scratch, tiles, s);
         const int hs = 3 * (D - d + 1);
         TimedScope ts(kt, "level_up", 28.0 * double(ub[d]));
         k_level_up<<<unsigned(tiles), kLvlBlock, 0, s>>>(NK[d]->get(), NP[d]->get(), NDI[d]->get(), ne_dev.get(), hs, D,
@@ -758,6 +758,7 @@ void build_octree(prg_ctx* c) {
     }
     {
         PRG_HIP(hipStreamSynchronize(s));
+        look_check(c->scratch, s);
         for (int d = 0; d <= D; d++) NE[d] = hne[d];
         if (c->transform_pending) {
             for (int a = 0; a < 3; a++) c->center[a] = c->transform_host[a];

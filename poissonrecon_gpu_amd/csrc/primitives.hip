@@ -68,11 +68,11 @@ __device__ __forceinline__ void store_items(int32_t* __restrict__ out, int64_t b
 template <bool TWO, int BLOCK>
 __global__ void __launch_bounds__(BLOCK) k_scan(const int32_t* in_a, int32_t* out_a, int32_t* total_a,
                                                      const int32_t* in_b, int32_t* out_b, int32_t* total_b, int64_t n,
-                                                     uint32_t tiles, bool wide, uint64_t* state) {
+                                                     uint32_t tiles, bool wide, LookState state) {
     __shared__ int32_t w[BLOCK / 64];
     __shared__ int32_t before[2];
     const LookTile t = look_begin(state, tiles);
-    if (t.tile >= tiles) return;  // (uniform; only if the state was damaged from outside)
+    if (t.tile >= tiles) return;  // (uniform)
     const int64_t base = int64_t(t.tile) * (BLOCK * kScanItems) + int64_t(threadIdx.x) * kScanItems;
     int32_t va[kScanItems], vb[kScanItems];
     const int32_t sa = load_items(in_a, base, n, wide, va);
@@ -83,7 +83,7 @@ __global__ void __launch_bounds__(BLOCK) k_scan(const int32_t* in_a, int32_t* ou
     const int wave = threadIdx.x >> 6;
     if (wave == 0 || (TWO && wave == 1)) {
         const int32_t mine = wave == 0 ? ta : tb;
-        const int32_t x = look_back(state + kLookHeader + int64_t(wave) * tiles, t, tiles, mine);
+        const int32_t x = look_back(state, wave, t, tiles, mine);
         if ((threadIdx.x & 63) == 0) {
             before[wave] = x;
             int32_t* total = wave == 0 ? total_a : total_b;
@@ -214,13 +214,21 @@ __global__ void __launch_bounds__(kSortBlock) k_radix_downsweep(const uint32_t* 
 }  // namespace
 
 // The scan state of a stream for `words` tile words, cleared when it grows.
-uint64_t* look_state(Scratch& scratch, int64_t words, hipStream_t s) {
+LookState look_state(Scratch& scratch, int64_t words, hipStream_t s) {
     const size_t want = size_t(words) + kLookHeader;
     if (scratch.look.n < want || !scratch.look.p) {
         scratch.look.reserve(want + want / 4);
         PRG_HIP(hipMemsetAsync(scratch.look.p, 0, scratch.look.n * sizeof(uint64_t), s));
     }
-    return scratch.look.p;
+    return LookState{scratch.look.p, scratch.look_error, kLookSpins};
+}
+
+void look_check(Scratch& scratch, hipStream_t s) {
+    if (!__atomic_load_n(scratch.look_error, __ATOMIC_RELAXED)) return;
+    PRG_HIP(hipMemsetAsync(scratch.look.p, 0, scratch.look.n * sizeof(uint64_t), s));
+    PRG_HIP(hipStreamSynchronize(s));
+    __atomic_store_n(scratch.look_error, 0, __ATOMIC_RELAXED);
+    throw Error{PRG_E_HIP, "a scan over many tiles did not finish"};
 }
 
 void scan_exclusive(const int32_t* d_in, int32_t* d_out, int64_t n, int32_t* d_total, hipStream_t s,
@@ -231,7 +239,7 @@ void scan_exclusive(const int32_t* d_in, int32_t* d_out, int64_t n, int32_t* d_t
     }
     const int block = scan_block(n), tile = block * kScanItems;
     const int64_t tiles = (n + tile - 1) / tile;
-    uint64_t* state = look_state(scratch, tiles, s);
+    const LookState state = look_state(scratch, tiles, s);
     const bool wide = ((reinterpret_cast<uintptr_t>(d_in) | reinterpret_cast<uintptr_t>(d_out)) & 15) == 0;
     TimedScope ts(kt, "scan_exclusive", 8.0 * double(n));
     const auto kernel = block == kScanLarge ? k_scan<false, kScanLarge> : k_scan<false, kScanSmall>;
@@ -249,7 +257,7 @@ void scan_exclusive2(const int32_t* a_in, int32_t* a_out, int32_t* a_total, cons
     }
     const int block = scan_block(n), tile = block * kScanItems;
     const int64_t tiles = (n + tile - 1) / tile;
-    uint64_t* state = look_state(scratch, 2 * tiles, s);
+    const LookState state = look_state(scratch, 2 * tiles, s);
     const bool wide = ((reinterpret_cast<uintptr_t>(a_in) | reinterpret_cast<uintptr_t>(a_out) |
                         reinterpret_cast<uintptr_t>(b_in) | reinterpret_cast<uintptr_t>(b_out)) & 15) == 0;
     TimedScope ts(kt, "scan_exclusive", 16.0 * double(n));

@@ -259,7 +259,7 @@ int select_block(int64_t n) { return n > (int64_t(1) << 20) ? kSelLarge : kSelSm
 template <bool LEAF, int BLOCK>
 __global__ void __launch_bounds__(BLOCK) k_select(const int32_t* __restrict__ child_base,
                                                     const uint8_t* __restrict__ marks, int64_t n, uint32_t tiles,
-                                                    uint64_t* state, int32_t* __restrict__ list,
+                                                    LookState state, int32_t* __restrict__ list,
                                                     int32_t* __restrict__ nid, int32_t* count) {
     __shared__ int32_t lds[BLOCK / 64];
     __shared__ int32_t s_before;
@@ -293,7 +293,7 @@ __global__ void __launch_bounds__(BLOCK) k_select(const int32_t* __restrict__ ch
     int32_t total;
     const int32_t ex = block_exclusive_scan(__popc(m), lds, total);
     if (threadIdx.x < 64) {
-        const int32_t b = look_back(state + kLookHeader, t, tiles, total);
+        const int32_t b = look_back(state, 0, t, tiles, total);
         if (threadIdx.x == 0) {
             s_before = b;
             if (t.tile == tiles - 1) *count = b + total;
@@ -499,7 +499,7 @@ constexpr int kRootTile = kRootBlock * kRootItems;
 // counts in cnt and in pinned memory.  (As flags, compaction, sizes, two
 // scans and an append these were five launches over the upper bound n.)
 __global__ void __launch_bounds__(kRootBlock) k_list_all_roots(const int32_t* __restrict__ cl,
-                                                               const uint8_t* __restrict__ rflag, uint64_t* state,
+                                                               const uint8_t* __restrict__ rflag, LookState state,
                                                                Levels L, int D,
                                                                int32_t* __restrict__ roots, int32_t* __restrict__ boff,
                                                                int32_t* __restrict__ root_of,
@@ -539,7 +539,7 @@ __global__ void __launch_bounds__(kRootBlock) k_list_all_roots(const int32_t* __
     int32_t a2 = block_exclusive_scan(n2, lds, tot[4]);
     const int wave = threadIdx.x >> 6;
     const int32_t mine = wave == 0 ? tot[0] : wave == 1 ? tot[1] : wave == 2 ? tot[2] : wave == 3 ? tot[3] : tot[4];
-    const int32_t x = look_back(state + kLookHeader + int64_t(wave) * tiles, t, tiles, mine);
+    const int32_t x = look_back(state, wave, t, tiles, mine);
     if ((threadIdx.x & 63) == 0) {
         s_before[wave] = x;
         if (t.tile == tiles - 1) {
@@ -2404,7 +2404,7 @@ void extract_subdivision(prg_ctx* c) {
     {
         const int block = select_block(baseD);
         const uint32_t tiles = select_tiles(baseD, block * kSelItems);
-        uint64_t* state = look_state(c->scratch, tiles, s);
+        const LookState state = look_state(c->scratch, tiles, s);
         (block == kSelLarge ? k_select<true, kSelLarge> : k_select<true, kSelSmall>)<<<tiles, block, 0, s>>>(
             c->child_base.get(), nullptr, baseD, tiles, state, cl.get(), nullptr, C + kCntCoarse);
         PRG_CHECK_LAUNCH();
@@ -2420,7 +2420,7 @@ void extract_subdivision(prg_ctx* c) {
     {
         const int block = select_block(8 * baseD);
         const uint32_t tiles = select_tiles(8 * baseD, block * kSelItems);
-        uint64_t* state = look_state(c->scratch, tiles, s);
+        const LookState state = look_state(c->scratch, tiles, s);
         (block == kSelLarge ? k_select<false, kSelLarge> : k_select<false, kSelSmall>)<<<tiles, block, 0, s>>>(
             nullptr, need.get(), 8 * baseD, tiles, state, clist.get(), nid.get(), C + kCntCorners);
         PRG_CHECK_LAUNCH();
@@ -2446,13 +2446,14 @@ void extract_subdivision(prg_ctx* c) {
     sidx.reserve(baseD);
     {
         const uint32_t tiles = select_tiles(baseD, kRootTile);
-        uint64_t* state = look_state(c->scratch, 5 * int64_t(tiles), s);
+        const LookState state = look_state(c->scratch, 5 * int64_t(tiles), s);
         k_list_all_roots<<<tiles, kRootBlock, 0, s>>>(cl.get(), rflag.get(), state, Lv, D, roots.get(),
                                                       boff.get(), root_of.get(), slist1.get(), slist2.get(),
                                                       sidx.get(), C, H);
         PRG_CHECK_LAUNCH();
     }
     PRG_HIP(hipStreamSynchronize(s));
+    look_check(c->scratch, s);
     const int64_t nr = H[kCntRoots], nb = H[kCntBricks];
     c->sub_roots = nr;
     c->sub_leaves = H[kCntLeaves];
@@ -2600,6 +2601,7 @@ void extract_subdivision(prg_ctx* c) {
     scan_exclusive2(bnv.get(), bvoff.get(), H + kCntVerts, bnt.get(), btoff.get(), H + kCntTris, nb, s, c->scratch,
                     kt);
     PRG_HIP(hipStreamSynchronize(s));
+    look_check(c->scratch, s);
     const int64_t snv = H[kCntVerts], snt = H[kCntTris];
     c->sub_bricks = nb;
     c->sub_exact = int64_t(H[kCntExact]) + n1 + n2;

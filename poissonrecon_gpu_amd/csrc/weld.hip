@@ -83,7 +83,7 @@ constexpr int kKeepTile = kBlock * kKeepItems;
 // compacted; number[slot] = the output number of the slot's vertex.  The
 // output's vertices, and those of the first n_leaf, go to pinned memory.
 __global__ void __launch_bounds__(kBlock) k_weld_compact(const float* __restrict__ v, int64_t n, int64_t n_leaf,
-                                                         uint32_t tiles, uint64_t* state,
+                                                         uint32_t tiles, LookState state,
                                                          const int32_t* __restrict__ table,
                                                          const uint32_t* __restrict__ place,
                                                          int32_t* __restrict__ number, float* __restrict__ out,
@@ -103,7 +103,7 @@ __global__ void __launch_bounds__(kBlock) k_weld_compact(const float* __restrict
     int32_t total;
     const int32_t ex = block_exclusive_scan(__popc(keep), lds, total);
     if (threadIdx.x < 64) {
-        const int32_t b = look_back(state + kLookHeader, t, tiles, total);
+        const int32_t b = look_back(state, 0, t, tiles, total);
         if (threadIdx.x == 0) {
             s_before = b;
             if (t.tile == tiles - 1) host_counts[0] = b + total;
@@ -161,10 +161,11 @@ void weld_core(prg_ctx* c, const WeldBufs& b, Scratch& scr, int look_words, floa
     const uint64_t slots = table_slots(n);
     volatile int32_t* counts = c->sub_host + kWeldHost;  // kept vertices; kept among the first n_leaf; bad triangles
     const uint32_t tiles = uint32_t((n + kKeepTile - 1) / kKeepTile);
-    uint64_t* state = look_state(scr, tiles, s);
+    LookState state = look_state(scr, tiles, s);
+    state.spins = c->weld_spins;
     PRG_HIP(hipMemcpyAsync(b.V, vertices, size_t(3 * n) * 4, hipMemcpyHostToDevice, s));
     k_weld_init<<<unsigned(std::min<uint64_t>(2048, slots / 1024 + 1)), kBlock, 0, s>>>(
-        b.table, int64_t(slots), c->sub_host + kWeldHost, state, look_words);
+        b.table, int64_t(slots), c->sub_host + kWeldHost, state.words, look_words);
     PRG_CHECK_LAUNCH();
     k_weld_insert<<<grid_for(n, kBlock), kBlock, 0, s>>>(b.V, n, uint32_t(slots - 1), b.table, b.place);
     PRG_CHECK_LAUNCH();
@@ -181,6 +182,7 @@ void weld_core(prg_ctx* c, const WeldBufs& b, Scratch& scr, int look_words, floa
         PRG_CHECK_LAUNCH();
     }
     PRG_HIP(hipStreamSynchronize(s));
+    look_check(scr, s);
     if (counts[2]) throw Error{PRG_E_ARG, "triangle index out of range"};  // the mesh is as it was
     const int64_t kept = counts[0];
     if (kept < 1 || kept > n) throw Error{PRG_E_HIP, "weld: inconsistent vertex count"};  // the mesh is as it was
@@ -279,6 +281,7 @@ void weld_mesh_noalloc(prg_ctx* c, float* vertices, int64_t n, int32_t* triangle
     } lend{scr};
     scr.look.p = reinterpret_cast<uint64_t*>(take(8 * kLookWords));
     scr.look.n = size_t(kLookWords);
+    scr.look_error = c->scratch.look_error;
     if (off > kNoAllocBytes) throw Error{PRG_E_HIP, "weld array layout exceeds its size"};
     weld_core(c, b, scr, int(kLookWords), vertices, n, triangles, m, n_leaf, n_out, n_leaf_out);
 }

@@ -39,3 +39,34 @@ def test_noalloc_weld_whatever_the_array_holds(prg, nv):
                 assert removed == oremoved and wm.n_leaf_vertices == onleaf
                 assert np.array_equal(wm.vertices.view(np.uint32), ov.view(np.uint32))
                 assert np.array_equal(wm.triangles, ot)
+
+
+@pytest.mark.parametrize("noalloc", [False, True])
+@pytest.mark.parametrize("nv", [2048, 2049, 100000])
+def test_scan_that_gives_up_is_reported(prg, monkeypatch, noalloc, nv):
+    """A tile that stops waiting for the tiles before it (test setting: at
+    once) leaves no mesh behind that looks right: the call fails, the caller's
+    mesh is as it was, and other contexts are not touched."""
+    mesh = _mesh(prg, nv, 3000, nv)
+    v0, t0 = mesh.vertices.copy(), mesh.triangles.copy()
+    want = weld_ref.weld(mesh.vertices, mesh.triangles, mesh.n_leaf_vertices)
+    monkeypatch.setenv("PRG_WELD_SPINS", "0")
+    g = prg.Reconstructor(max_depth=5)
+    monkeypatch.delenv("PRG_WELD_SPINS")
+    h = prg.Reconstructor(max_depth=5)
+    for _ in range(2):
+        print(f"\n[weld of {nv} vertices that gives up at once, noalloc={noalloc}]", flush=True)
+        if nv <= 2048:  # one tile waits for none
+            wm, _ = g.weld_mesh(mesh, noalloc=noalloc)
+            assert np.array_equal(wm.vertices.view(np.uint32), want[0].view(np.uint32))
+        else:
+            with pytest.raises(prg.PrgError) as e:
+                g.weld_mesh(mesh, noalloc=noalloc)
+            assert e.value.status == prg.E_HIP
+        assert np.array_equal(mesh.vertices, v0) and np.array_equal(mesh.triangles, t0)
+        wm, removed = h.weld_mesh(mesh, noalloc=noalloc)
+        assert removed == want[3]
+        assert np.array_equal(wm.vertices.view(np.uint32), want[0].view(np.uint32))
+        assert np.array_equal(wm.triangles, want[1])
+    h.close()
+    g.close()
