@@ -23,6 +23,7 @@
 // order, so training is deterministic.
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <vector>
 
 #include "../../include/prg_unet.h"
@@ -1087,6 +1088,9 @@ struct prg_unet {
     float inv_host[prg::kMaxBatch];
     prg::DBuf<double> loss, lpart;
     int batch_cap = 0;  // samples the buffers hold
+    // test knob (PRG_UNET_FAIL_CALL at creation): the first call that uploads
+    // targets fails behind the upload
+    bool fail_call = false;
 };
 
 namespace prg {
@@ -1352,7 +1356,7 @@ void load_samples(prg_unet* n, const float* bgrid, const float* mask, const floa
 // Their targets, normalised likewise: up on a stream of their own, beside the
 // forward pass queued before (0.3 ms of a training step of 8 at 64^3).
 // Nothing queued uses the buffer: every step and gradient call ends with a
-// synchronisation.
+// synchronisation, failed ones in unet_guard.
 void load_targets(prg_unet* n, const float* target, int B) {
     const int64_t V = int64_t(n->G) * n->G * n->G;
     if (!n->copy_stream) {
@@ -1364,6 +1368,10 @@ void load_targets(prg_unet* n, const float* target, int B) {
     PRG_HIP(hipStreamWaitEvent(n->stream, n->copied, 0));
     k_scale<<<dim3(blocks(V), unsigned(B)), kT, 0, n->stream>>>(n->target.get(), V, n->inv.get());
     PRG_CHECK_LAUNCH();
+    if (n->fail_call) {
+        n->fail_call = false;
+        throw Error{PRG_E_HIP, "failed as PRG_UNET_FAIL_CALL asks"};
+    }
 }
 
 // Buffers for B samples at a time (they only grow) and the convolutions'
@@ -1420,13 +1428,21 @@ void reserve_batch(prg_unet* n, int B) {
 template <class F>
 prg_status unet_guard(prg_unet* n, F&& f) {
     if (!n) return PRG_E_ARG;
+    // what a failed call has queued ends before it returns: it reads the
+    // caller's arrays, and the next call's uploads are ordered behind nothing
+    auto quiet = [&] {
+        for (hipStream_t x : {n->stream, n->copy_stream})
+            if (x) (void)hipStreamSynchronize(x);
+    };
     try {
         PRG_HIP(hipSetDevice(n->device));
         return f();
     } catch (const Error& e) {
+        quiet();
         n->err = e.msg;
         return e.status;
     } catch (const std::bad_alloc&) {
+        quiet();
         n->err = "host allocation failed";
         return PRG_E_NOMEM;
     }
@@ -1482,6 +1498,7 @@ prg_status prg_unet_create(prg_unet** out, int32_t device, int32_t grid, uint64_
     prg_unet* n = new prg_unet();
     n->device = device;
     n->G = grid;
+    if (const char* fc = std::getenv("PRG_UNET_FAIL_CALL")) n->fail_call = std::atoi(fc) != 0;
     const prg_status st = prg::unet_guard(n, [&]() {
         PRG_HIP(hipStreamCreateWithFlags(&n->stream, hipStreamNonBlocking));
         int64_t off = 0;
