@@ -7,9 +7,19 @@ namespace prg {
 
 namespace {
 constexpr size_t kPartAlign = 512;
-// A new allocation holds at least kFirstChunk bytes and half of what there is
-// already, up to kMostSpare, or what is asked for: about ten allocations make
-// gigabytes, and at most a third of the memory is spare.
+// Buffers of kOwn bytes and more are allocations of their own, back with the
+// device as soon as they are outgrown: of clouds that fill the memory those
+// parts would not fit what comes after them.  The line is that high because a
+// hipFree slows the copies of pageable memory for several passes (6 M points,
+// 72 MB a copy: 21 ms instead of 5 for up to five passes after it), more than
+// the whole pass on a cloud whose buffers are smaller.
+constexpr size_t kOwn = size_t(1) << 30;
+// A new shared allocation holds at least kFirstChunk bytes, half of what the
+// shared ones hold already up to kMostSpare, or what is asked for if that is
+// more.  Their outgrown parts (each under kOwn) and the last one's rest are
+// what a context holds beyond its buffers: over clouds of 1, 2, 4 .. 32 M points
+// 13.5 GiB where the last alone takes 11.1 (12.6 and 11.1 when every buffer had
+// an allocation of its own).
 constexpr size_t kFirstChunk = size_t(32) << 20;
 constexpr size_t kMostSpare = size_t(1) << 30;
 constexpr size_t kTail = size_t(64) << 10;  // past every allocation's last part
@@ -25,15 +35,22 @@ Arena::~Arena() {
         if (c.p) (void)hipFree(c.p);
 }
 
-bool Arena::add_chunk(size_t bytes) {
+// an allocation, or null without room for it
+static uint8_t* device_alloc(size_t bytes) {
     void* p = nullptr;
-    const hipError_t e = hipMalloc(&p, bytes + kTail);
+    const hipError_t e = hipMalloc(&p, bytes);
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
-        return false;
+        return nullptr;
     }
     PRG_HIP(e);
-    const Part part{static_cast<uint8_t*>(p), bytes, false, int(chunks_.size())};
+    return static_cast<uint8_t*>(p);
+}
+
+bool Arena::add_chunk(size_t bytes) {
+    uint8_t* p = device_alloc(bytes + kTail);
+    if (!p) return false;
+    const Part part{p, bytes, false, int(chunks_.size())};
     chunks_.push_back(Chunk{part.p, bytes});
     total_ += bytes;
     free_.insert(std::lower_bound(free_.begin(), free_.end(), part.p, [](const Part& a, const uint8_t* b) { return a.p < b; }),
@@ -41,8 +58,32 @@ bool Arena::add_chunk(size_t bytes) {
     return true;
 }
 
+// shared allocations without a part in use go back to the device
+bool Arena::trim() {
+    bool freed = false;
+    for (size_t i = 0; i < free_.size();) {
+        Chunk& c = chunks_[size_t(free_[i].chunk)];
+        if (free_[i].p == c.p && free_[i].bytes == c.bytes) {
+            (void)hipFree(c.p);  // waits for the device
+            total_ -= c.bytes;
+            c = Chunk{nullptr, 0};
+            free_.erase(free_.begin() + ptrdiff_t(i));
+            freed = true;
+        } else {
+            i++;
+        }
+    }
+    return freed;
+}
+
 void* Arena::take(size_t bytes) {
     const size_t want = (bytes + kPartAlign - 1) / kPartAlign * kPartAlign;
+    if (want >= kOwn) {
+        uint8_t* p = device_alloc(want);
+        if (!p && trim()) p = device_alloc(want);
+        if (!p) throw Error{PRG_E_NOMEM, "out of device memory (" + std::to_string(bytes) + " bytes)"};
+        return p;
+    }
     for (int attempt = 0;; attempt++) {
         // the smallest part that holds it, one without queued work if there is one
         size_t best = free_.size();
@@ -73,26 +114,16 @@ void* Arena::take(size_t bytes) {
             attempt = 1;
             continue;
         }
-        // no room: allocations without a part in use go back to the device first
-        bool freed = false;
-        for (size_t i = 0; i < free_.size();) {
-            Chunk& c = chunks_[size_t(free_[i].chunk)];
-            if (free_[i].p == c.p && free_[i].bytes == c.bytes) {
-                (void)hipFree(c.p);  // waits for the device
-                total_ -= c.bytes;
-                c = Chunk{nullptr, 0};
-                free_.erase(free_.begin() + ptrdiff_t(i));
-                freed = true;
-            } else {
-                i++;
-            }
-        }
-        if (!freed || !add_chunk(want)) throw Error{PRG_E_NOMEM, "out of device memory (" + std::to_string(bytes) + " bytes)"};
+        if (!trim() || !add_chunk(want)) throw Error{PRG_E_NOMEM, "out of device memory (" + std::to_string(bytes) + " bytes)"};
     }
 }
 
 void Arena::give(void* p, size_t bytes) {
     Part part{static_cast<uint8_t*>(p), (bytes + kPartAlign - 1) / kPartAlign * kPartAlign, true, -1};
+    if (part.bytes >= kOwn) {
+        (void)hipFree(p);  // waits for the device
+        return;
+    }
     for (size_t i = 0; i < chunks_.size(); i++)
         if (chunks_[i].p && part.p >= chunks_[i].p && part.p < chunks_[i].p + chunks_[i].bytes) part.chunk = int(i);
     auto it = std::lower_bound(free_.begin(), free_.end(), part.p, [](const Part& a, const uint8_t* b) { return a.p < b; });

@@ -73,6 +73,7 @@ private:
         size_t bytes;
     };
     bool add_chunk(size_t bytes);
+    bool trim();
     std::vector<Part> free_;  // by address; neighbours of one chunk are joined
     std::vector<Chunk> chunks_;
     size_t total_ = 0;
