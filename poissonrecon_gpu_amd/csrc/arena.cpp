@@ -22,7 +22,6 @@ constexpr size_t kOwn = size_t(1) << 30;
 // an allocation of its own).
 constexpr size_t kFirstChunk = size_t(32) << 20;
 constexpr size_t kMostSpare = size_t(1) << 30;
-constexpr size_t kTail = size_t(64) << 10;  // past every allocation's last part
 }  // namespace
 
 Arena*& current_arena() {
@@ -48,7 +47,7 @@ static uint8_t* device_alloc(size_t bytes) {
 }
 
 bool Arena::add_chunk(size_t bytes) {
-    uint8_t* p = device_alloc(bytes + kTail);
+    uint8_t* p = device_alloc(bytes);
     if (!p) return false;
     const Part part{p, bytes, false, int(chunks_.size())};
     chunks_.push_back(Chunk{part.p, bytes});
