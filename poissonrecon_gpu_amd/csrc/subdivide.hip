@@ -474,8 +474,6 @@ constexpr int kBrickLog = 3;  // bricks of up to 8^3 virtual leaves
 constexpr int kBrickLeaves = 1 << (3 * kBrickLog);
 constexpr int kBrickPts = ((1 << kBrickLog) + 1) * ((1 << kBrickLog) + 1) * ((1 << kBrickLog) + 1);
 
-__device__ __forceinline__ int brick_log(int D, int r) { return D - r < kBrickLog ? D - r : kBrickLog; }
-
 // The place in a list (its length in *counter) of each lane with `want`: one
 // atomic per wave, lanes in order.
 __device__ __forceinline__ int32_t wave_append(bool want, int32_t* counter) {

@@ -132,19 +132,19 @@ __device__ __forceinline__ void load_halo(s4* halo4, int H, int HY, int HZ, cons
 // out[v, co] = act(bias[co] + sum_t sum_ci bf16(in[v + off_t, ci]) * w[t][co][ci])
 // (w as packed_at lays it out)
 //
-// One workgroup per brick of BX x BY x BZ output voxels (x, y, z; z fastest).
-// The brick's input halo, (BX + 2)(BY + 2)(BZ + 2) voxels, is staged in LDS
-// as BF16, 16-channel slice after slice: lds[s][h][16]; each wave loads whole
-// halo rows (contiguous in memory).  The brick's voxels in (x, y, z) order
-// form M-tiles of 16; wave w computes M-tiles [MA (w % MG), MA (w % MG) + MA)
-// for N-tiles [NA (w / MG), NA (w / MG) + NA) (16 output channels each).
+// On grids of 4^3 and 2^3, with 2, 4 or 8 N-tiles (16 output channels each):
+// one workgroup per brick of BX x BY x BZ output voxels (x, y, z; z fastest),
+// at most 16.  The brick's input halo, (BX + 2)(BY + 2)(BZ + 2) voxels, is
+// staged in LDS as BF16, 16-channel slice after slice: lds[s][h][16]; each
+// wave loads whole halo rows (contiguous in memory).  The brick's voxels in
+// (x, y, z) order are one M-tile; wave w computes it for N-tiles [NA w,
+// NA w + NA).
 // MFMA lane layout (16x16x16): lane l holds A[l % 16][4 (l / 16) + e],
 // B[4 (l / 16) + e][l % 16] and D[4 (l / 16) + e][l % 16], e = 0..3.  K runs
 // over slices, then taps; a slice's 27 weight fragments are loaded together.
-template <int MA, int NA>
+template <int NA>
 __global__ void __launch_bounds__(kT) k_conv3(ConvIn src, const short* __restrict__ w, const float* __restrict__ bias,
-                                             int G, int BX, int BY, int BZ, int MG, int relu, ConvOut dst,
-                                             int cout) {
+                                             int G, int BX, int BY, int BZ, int relu, ConvOut dst, int cout) {
     extern __shared__ s4 halo4[];
     const short* halo = reinterpret_cast<const short*>(halo4);
     const int cin = src.clo + src.cskip;
@@ -158,11 +158,10 @@ __global__ void __launch_bounds__(kT) k_conv3(ConvIn src, const short* __restric
     const int ox = (b / nby) * BX;
     const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
     const int i = l & 15, kq = l >> 4;
-    const int mg = wave % MG, ng = wave / MG;
     const int NT = cout >> 4, S = cin >> 4, nvox = BX * BY * BZ;
-    const bool active = (ng + 1) * NA <= NT;
+    const bool active = (wave + 1) * NA <= NT;
     // the first slice's weight fragments are in flight while the halo loads
-    const short* wl = w + ((active ? ng : 0) * NA * 16 + i) * 16 + 4 * kq;
+    const short* wl = w + ((active ? wave : 0) * NA * 16 + i) * 16 + 4 * kq;
     s4 wr[27][NA];
 #pragma unroll
     for (int t = 0; t < 27; t++)
@@ -172,25 +171,16 @@ __global__ void __launch_bounds__(kT) k_conv3(ConvIn src, const short* __restric
     load_halo<false>(halo4, H, HY, HZ, src.skip, src.cskip, src.clo, ox, oy, oz, G);
     __syncthreads();
     if (!active) return;  // idle wave; no barrier follows
-    // lanes past the brick's voxels (grids under 16^3) read the brick's first
-    // voxel, whose 27 neighbours are all in the halo, and use zeros
-    int hb[MA];
-    bool ok[MA];
-#pragma unroll
-    for (int m = 0; m < MA; m++) {
-        const int q = (mg * MA + m) * 16 + i;
-        ok[m] = q < nvox;
-        const int qx = q / (BY * BZ), qy = (q / BZ) % BY, qz = q % BZ;
-        hb[m] = ok[m] ? (qx + 1) * HYZ + (qy + 1) * HZ + qz + 1 : HYZ + HZ + 1;
-    }
+    // lanes past the brick's voxels (2^3 grids) read the brick's first voxel,
+    // whose 27 neighbours are all in the halo, and use zeros
+    const bool ok = i < nvox;
+    const int hb = ok ? (i / (BY * BZ) + 1) * HYZ + ((i / BZ) % BY + 1) * HZ + i % BZ + 1 : HYZ + HZ + 1;
     // three partial sums over alternating taps keep independent MFMAs in flight
-    f4 acc[3][MA][NA];
+    f4 acc[3][NA];
 #pragma unroll
     for (int x = 0; x < 3; x++)
 #pragma unroll
-        for (int m = 0; m < MA; m++)
-#pragma unroll
-            for (int n = 0; n < NA; n++) acc[x][m][n] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int n = 0; n < NA; n++) acc[x][n] = f4{0.0f, 0.0f, 0.0f, 0.0f};
     const s4 zero4 = s4{0, 0, 0, 0};
     for (int sl = 0; sl < S; sl++) {
         const short* hs = halo + sl * H * 16 + 4 * kq;
@@ -199,51 +189,43 @@ __global__ void __launch_bounds__(kT) k_conv3(ConvIn src, const short* __restric
 #pragma unroll
         for (int g = 0; g < 3; g++) {
             // the nine taps with dx = g - 1: their A fragments first, then the MFMAs
-            s4 a[9][MA];
+            s4 a[9];
 #pragma unroll
             for (int j = 0; j < 9; j++) {
                 const int toff = (g - 1) * HYZ + (j / 3 - 1) * HZ + (j % 3 - 1);
-#pragma unroll
-                for (int m = 0; m < MA; m++) a[j][m] = *reinterpret_cast<const s4*>(hs + (hb[m] + toff) * 16);
+                a[j] = *reinterpret_cast<const s4*>(hs + (hb + toff) * 16);
             }
 #pragma unroll
-            for (int j = 0; j < 9; j++)
-#pragma unroll
-                for (int m = 0; m < MA; m++) a[j][m] = ok[m] ? a[j][m] : zero4;
+            for (int j = 0; j < 9; j++) a[j] = ok ? a[j] : zero4;
 #pragma unroll
             for (int j = 0; j < 9; j++) {
                 const int t = 9 * g + j;
 #pragma unroll
                 for (int n = 0; n < NA; n++) {
-#pragma unroll
-                    for (int m = 0; m < MA; m++)
-                        acc[j % 3][m][n] =
-                            __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[j][m], wr[t][n], acc[j % 3][m][n], 0, 0, 0);
+                    acc[j % 3][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[j], wr[t][n], acc[j % 3][n], 0, 0, 0);
                     wr[t][n] = *reinterpret_cast<const s4*>(wl + ((nsl * 27 + t) * cout + n * 16) * 16);
                 }
             }
         }
     }
 #pragma unroll
-    for (int m = 0; m < MA; m++)
+    for (int e = 0; e < 4; e++) {
+        const int q = 4 * kq + e;
+        if (q >= nvox) continue;
+        const int gx = ox + q / (BY * BZ), gy = oy + (q / BZ) % BY, gz = oz + q % BZ;
+        const int64_t v = (int64_t(gx) * G + gy) * G + gz;
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int q = (mg * MA + m) * 16 + 4 * kq + e;
-            if (q >= nvox) continue;
-            const int gx = ox + q / (BY * BZ), gy = oy + (q / BZ) % BY, gz = oz + q % BZ;
-            const int64_t v = (int64_t(gx) * G + gy) * G + gz;
-#pragma unroll
-            for (int n = 0; n < NA; n++) {
-                const int co = (ng * NA + n) * 16 + i;
-                const bool hi = co >= dst.split;
-                const int oc = hi ? cout - dst.split : dst.split;
-                float* o = (hi ? dst.hi : dst.lo) + sample_offset(G, oc) + v * oc + co - (hi ? dst.split : 0);
-                float val = (acc[0][m][n][e] + acc[1][m][n][e]) + acc[2][m][n][e];
-                if (bias) val = val + bias[co];
-                if (relu) val = val > 0.0f ? val : 0.0f;
-                *o = val;
-            }
+        for (int n = 0; n < NA; n++) {
+            const int co = (wave * NA + n) * 16 + i;
+            const bool hi = co >= dst.split;
+            const int oc = hi ? cout - dst.split : dst.split;
+            float* o = (hi ? dst.hi : dst.lo) + sample_offset(G, oc) + v * oc + co - (hi ? dst.split : 0);
+            float val = (acc[0][n][e] + acc[1][n][e]) + acc[2][n][e];
+            if (bias) val = val + bias[co];
+            if (relu) val = val > 0.0f ? val : 0.0f;
+            *o = val;
         }
+    }
 }
 
 // The same sums, in the same order, on grids of 8^3 and more, where a tile is
@@ -1099,40 +1081,6 @@ namespace {
 const int kConvDef[14][3] = {{16, 16, 0}, {16, 16, 0}, {16, 32, 1}, {32, 32, 1}, {32, 64, 2}, {64, 64, 2}, {64, 64, 3},
                              {64, 64, 3}, {128, 64, 2}, {64, 64, 2}, {96, 32, 1}, {32, 32, 1}, {48, 16, 0}, {16, 16, 0}};
 
-// Brick and wave split of k_conv3 (grids under 8^3) with output grid G and
-// NT = cout / 16 N-tiles.
-struct ConvPlan {
-    int BX, BY, BZ, MA, NA, MG;
-};
-
-ConvPlan conv_plan(int G, int NT) {
-    ConvPlan p{};
-    p.BZ = G;
-    p.MA = 1;
-    int bxy = 1;  // BX = BY = bxy before small-grid widening
-    switch (NT) {
-        case 1: bxy = 2; p.NA = 1; break;
-        case 2: p.NA = 1; break;
-        case 3: bxy = 2; p.NA = 3; break;
-        case 4: p.NA = 1; break;
-        case 6: p.NA = 3; break;
-        case 8: p.NA = 2; break;
-        default: throw Error{PRG_E_ARG, "unsupported channel count"};
-    }
-    p.BX = bxy < G ? bxy : G;
-    p.BY = bxy < G ? bxy : G;
-    if (NT == 2 || NT == 6) p.BY = 2 < G ? 2 : G;
-    // at least one full M-tile of 16 voxels where the grid has them
-    while (p.BX * p.BY * p.BZ < 16 && p.BY < G) p.BY *= 2;
-    while (p.BX * p.BY * p.BZ < 16 && p.BX < G) p.BX *= 2;
-    const int MT = (p.BX * p.BY * p.BZ + 15) / 16;
-    if (MT % p.MA || NT % p.NA) throw Error{PRG_E_ARG, "convolution plan does not tile"};
-    p.MG = MT / p.MA;
-    if (p.MG * (NT / p.NA) > kT / 64) throw Error{PRG_E_ARG, "convolution plan needs more waves"};
-    if (G % p.BX || G % p.BY || G % p.BZ) throw Error{PRG_E_ARG, "convolution brick does not divide the grid"};
-    return p;
-}
-
 bool pow2_channels(int c) { return c == 16 || c == 32 || c == 64; }
 
 // Tiles of 16 voxels and 16 channels from which a wave takes 2 x 2 of them
@@ -1159,7 +1107,7 @@ template <int LZ>
 void launch_conv_grid(hipStream_t s, ConvIn src, const short* w, const float* bias, int G, int relu, ConvOut out,
                       int cout, int B) {
     const int NT = cout / 16;
-    const bool many = int64_t(B) * G * G * G / 16 * NT >= kConvManyTiles && G >= 8;
+    const bool many = int64_t(B) * G * G * G / 16 * NT >= kConvManyTiles;
     if (NT % 4 == 0) {
         if (many) launch_conv_rows<LZ, 2, 2, 1, 1, 4>(s, src, w, bias, G, relu, out, cout, B);
         else launch_conv_rows<LZ, 1, 1, 1, 1, 4>(s, src, w, bias, G, relu, out, cout, B);
@@ -1180,15 +1128,15 @@ void launch_conv(hipStream_t s, ConvIn src, const short* w, const float* bias, i
         throw Error{PRG_E_ARG, "unsupported convolution channels"};
     if (G >= 16) return launch_conv_grid<4>(s, src, w, bias, G, relu, out, cout, B);
     if (G == 8) return launch_conv_grid<3>(s, src, w, bias, G, relu, out, cout, B);
-    const ConvPlan p = conv_plan(G, cout / 16);
-    const size_t lds = size_t(p.BX + 2) * (p.BY + 2) * (p.BZ + 2) * cin * 2;
-    if (lds > 64 * 1024) throw Error{PRG_E_ARG, "convolution halo exceeds 64 KiB of LDS"};
-    const dim3 grid(unsigned((G / p.BX) * (G / p.BY) * (G / p.BZ)), unsigned(B));
-    switch (p.NA) {
-        case 1: k_conv3<1, 1><<<grid, kT, lds, s>>>(src, w, bias, G, p.BX, p.BY, p.BZ, p.MG, relu, out, cout); break;
-        case 2: k_conv3<1, 2><<<grid, kT, lds, s>>>(src, w, bias, G, p.BX, p.BY, p.BZ, p.MG, relu, out, cout); break;
-        default: k_conv3<1, 3><<<grid, kT, lds, s>>>(src, w, bias, G, p.BX, p.BY, p.BZ, p.MG, relu, out, cout);
-    }
+    // 4^3 in bricks of 1 x 4 x 4 voxels, 2^3 whole; a wave per N-tile, or two
+    // with eight of them (the grids under 8^3 are the levels of 32 and 64
+    // channels and of their concatenation)
+    const int NT = cout / 16, BX = G == 4 ? 1 : G;
+    if ((G != 4 && G != 2) || (NT != 2 && NT != 4 && NT != 8)) throw Error{PRG_E_ARG, "unsupported convolution"};
+    const size_t lds = size_t(BX + 2) * (G + 2) * (G + 2) * cin * 2;  // at most 27 KB
+    const dim3 grid(unsigned(G / BX), unsigned(B));
+    const auto kernel = NT == 8 ? k_conv3<2> : k_conv3<1>;
+    kernel<<<grid, kT, lds, s>>>(src, w, bias, G, BX, G, G, relu, out, cout);
     PRG_CHECK_LAUNCH();
 }
 
