@@ -328,7 +328,9 @@ class Reconstructor:
         m.n_leaf_vertices, m.n_leaf_triangles = int(mesh.n_leaf_vertices), int(mesh.n_leaf_triangles)
         merged = C.c_int64()
         self._call("prg_weld_mesh_noalloc" if noalloc else "prg_weld_mesh", C.byref(m), C.byref(merged))
-        return (Mesh(v[: m.n_vertices], t, mesh.center, mesh.scale, m.n_leaf_vertices, m.n_leaf_triangles),
+        # the tail of the merged vertices goes back in place (a view would keep it)
+        v.resize((m.n_vertices, 3), refcheck=False)
+        return (Mesh(v, t, mesh.center, mesh.scale, m.n_leaf_vertices, m.n_leaf_triangles),
                 merged.value)
 
     def subdivision_info(self) -> tuple[int, int]:
