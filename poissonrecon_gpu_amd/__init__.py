@@ -225,12 +225,12 @@ class _HostArray:
 
 def _adopt_mesh(m: PrgMesh) -> tuple[np.ndarray, np.ndarray]:
     """The vertices and triangles of a mesh the library allocated, without a
-    copy; the mesh gives them up."""
-    v = np.asarray(_HostArray(m.vertices, m.n_vertices, np.float32, vertices=m.vertices))
-    t = np.asarray(_HostArray(m.triangles, m.n_triangles, np.int32, triangles=m.triangles))
+    copy; the mesh gives each up as soon as it has another owner."""
+    v = _HostArray(m.vertices, m.n_vertices, np.float32, vertices=m.vertices)
     m.vertices = C.POINTER(C.c_float)()
+    t = _HostArray(m.triangles, m.n_triangles, np.int32, triangles=m.triangles)
     m.triangles = C.POINTER(C.c_int32)()
-    return v, t
+    return np.asarray(v), np.asarray(t)
 
 
 class Reconstructor:
