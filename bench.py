@@ -470,7 +470,8 @@ def main():
         "solve_vs_fp64_oracle": solve_fp64,
         "mesh": {"vertices": int(mesh[0]), "triangles": int(mesh[1]), "subdivision_roots": roots.value,
                  "virtual_leaves": vleaves.value,
-                 "subdivision_bricks": {"bricks": bricks[0], "left_by_interval_certificate": bricks[1],
+                 # (the roots of 2^3 and 4^3 leaves, evaluated at once, are in all three)
+                 "subdivision_bricks": {"bricks": bricks[0], "left_by_cell_bounds": bricks[1],
                                         "evaluated": bricks[2]}},
         "variants": variants,
         "kernels": kern,

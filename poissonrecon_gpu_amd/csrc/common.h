@@ -44,8 +44,9 @@ struct Error {
 #define PRG_CHECK_LAUNCH() PRG_HIP(hipGetLastError())
 
 // ---- device buffers ------------------------------------------------------------
-// Device memory of one context: buffers are parts of a few large allocations,
-// given back to the device with the context.  A context's about 170 buffers
+// Device memory of one context: buffers (under 1 GiB; larger ones are
+// allocations of their own) are parts of a few large allocations, given back to
+// the device with the context.  A context's about 170 buffers
 // as allocations of their own cost 20 us each to make, and 270 us each to free
 // beside other contexts at work (hipFree waits for the whole device).
 // A part given back may still be read by work queued on the context's

@@ -197,7 +197,12 @@ __global__ void __launch_bounds__(kBlock) k_vector_field(const int32_t* pntD, co
 // per workgroup).
 constexpr int kVfPoints = 768;        // 52 KB of LDS, three workgroups per CU
 // For clouds of kVfDense points and more per sibling block, whose tiles mostly
-// exceed kVfPoints: 77 KB, two workgroups per CU.
+// exceed kVfPoints: 77 KB, two workgroups per CU.  This instance against the
+// smaller one, superquadrics at depths 7 to 10 and a sphere at depth 8: with 2.8
+// points per block 37 and 28 us (100,000 points), with 2.9 428 and 332 us (2 M);
+// with 3.8 to 4.1 the same; with 4.2 27 and 37 us, with 4.9 611 and 1,087 us (4 M),
+// with 7 194 and 280 us (1 M); from 8 on most tiles exceed both (2,224 and 2,178
+// us with 8.6).
 constexpr int kVfPointsDense = 1280;
 constexpr double kVfDense = 4.0;
 

@@ -941,7 +941,8 @@ __device__ __forceinline__ bool any_thread(bool v) {
 // together.  The levels end where no cell of a block has children: most
 // bricks of a large root see real nodes of the first depths below it only,
 // and blocks of 5^3, 7^3 and 11^3 empty cells neither take time nor fill the
-// LDS (109,000 of 160,000 bricks missed the interval screen for those alone).
+// LDS (109,000 of the 160,000 bricks that a screen with all the blocks left were
+// left for those alone).
 // A depth whose block holds no nonzero coefficient gets none.  Returns false
 // when the caller's LDS cannot hold the blocks.
 // (kThreads: of the workgroup, all of which take part.)
@@ -1724,7 +1725,7 @@ __global__ void __launch_bounds__(kWave, 3) k_brick_exact(SubArgs A, const int32
 // kBrickPts per listed brick.  A value is a serial chain of LDS reads and
 // sums, so what counts is the waves in flight; a brick's tables and blocks are
 // 16 KB of LDS, which held them to 2.5 per SIMD as one wave per brick (532 us
-// for 3,338 bricks; 250 us with four).  `slices` workgroups share the rounds
+// for 3,338 bricks of 150,000 points at depth 10; 277 us with four, for 3,418).  `slices` workgroups share the rounds
 // of a brick (each sets up its own tables and blocks): a list shorter than the
 // chip leaves each of them one round instead of all three.
 constexpr int kValThreads = 256;

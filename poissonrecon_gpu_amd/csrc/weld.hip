@@ -28,6 +28,9 @@ namespace {
 
 constexpr int kBlock = 256;
 
+// The multipliers that fold the three words are the first three 32-bit primes
+// of xxHash (Yann Collet); the last four lines are the 32-bit mixer
+// "lowbias32" (Chris Wellons, hash-prospector).
 __device__ __forceinline__ uint32_t hash_position(uint32_t x, uint32_t y, uint32_t z) {
     uint32_t h = x * 0x9E3779B1u;
     h = ((h << 15) | (h >> 17)) ^ (y * 0x85EBCA77u);
